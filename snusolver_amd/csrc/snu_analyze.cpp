@@ -163,7 +163,7 @@ int build_leaf(const Plan &P, LeafPlan &L) {
     while (ptr < L.lu_rowptr[i + 1] && L.lu_colidx[ptr] < ls) ptr++;
     L.lu_bias[i] = ptr;
   }
-  // boundary rows / cols and the workspace column of every LU entry
+  // boundary rows / cols
   int nsep = core_n - ls;
   std::vector<int> binv(nsep, -1);
   for (int r = 0; r < ls; r++)
@@ -176,44 +176,6 @@ int build_leaf(const Plan &P, LeafPlan &L) {
   for (int r = ls; r < core_n; r++)
     if (L.lu_rowptr[r + 1] > L.lu_rowptr[r]) L.brow.push_back(r);
   L.nbr = (int)L.brow.size();
-  L.wcol.resize(L.lu_nnz);
-  for (int p = 0; p < L.lu_nnz; p++) {
-    int c = L.lu_colidx[p];
-    L.wcol[p] = c < ls ? c : ls + binv[c - ls];
-  }
-  // level sets of the leaf rows: factor/forward (L deps), backward (U deps)
-  std::vector<int> lev(ls, 0);
-  int nlev = 0;
-  for (int j = 0; j < ls; j++) {
-    int m = 0;
-    for (int p = L.lu_rowptr[j]; p < L.lu_diag[j]; p++) m = std::max(m, lev[L.lu_colidx[p]] + 1);
-    lev[j] = m;
-    nlev = std::max(nlev, m + 1);
-  }
-  L.lev_ptr.assign(nlev + 1, 0);
-  for (int j = 0; j < ls; j++) L.lev_ptr[lev[j] + 1]++;
-  for (int l = 0; l < nlev; l++) L.lev_ptr[l + 1] += L.lev_ptr[l];
-  L.lev_rows.resize(ls);
-  {
-    std::vector<int> f(L.lev_ptr.begin(), L.lev_ptr.end() - 1);
-    for (int j = 0; j < ls; j++) L.lev_rows[f[lev[j]]++] = j;
-  }
-  std::vector<int> ulev(ls, 0);
-  int nulev = 0;
-  for (int j = ls - 1; j >= 0; j--) {
-    int m = 0;
-    for (int p = L.lu_diag[j] + 1; p < L.lu_bias[j]; p++) m = std::max(m, ulev[L.lu_colidx[p]] + 1);
-    ulev[j] = m;
-    nulev = std::max(nulev, m + 1);
-  }
-  L.ulev_ptr.assign(nulev + 1, 0);
-  for (int j = 0; j < ls; j++) L.ulev_ptr[ulev[j] + 1]++;
-  for (int l = 0; l < nulev; l++) L.ulev_ptr[l + 1] += L.ulev_ptr[l];
-  L.ulev_rows.resize(ls);
-  {
-    std::vector<int> f(L.ulev_ptr.begin(), L.ulev_ptr.end() - 1);
-    for (int j = ls - 1; j >= 0; j--) L.ulev_rows[f[ulev[j]]++] = j;
-  }
   int frc = build_fronts(L);
   if (frc) return frc;
   // structural flops: every pivot of a row costs 1 division and 2 flops per

@@ -59,15 +59,16 @@ int ensure_rhs(snumat *h, int nrhs) {
   if (nrhs <= h->nrhs_cap) return SNU_OK;
   int rc;
   const size_t n = (size_t)h->P.n;
+  const size_t cols = (size_t)vec_groups(nrhs) * vec_width(nrhs);  // columns of the packed vectors
   auto vec = [&](auto &VV) -> int {
     drop_alloc(h, VV.bp);
-    drop_alloc(h, VV.cbuf);
+    drop_alloc(h, VV.wbuf);
     drop_alloc(h, VV.ys);
-    VV.bp = VV.cbuf = VV.ys = nullptr;
+    VV.bp = VV.wbuf = VV.ys = nullptr;
     VV.plan_nrhs = -1;
     int r;
-    if ((r = halloc(h, &VV.bp, n * nrhs)) || (r = halloc(h, &VV.ys, n * nrhs)) ||
-        (r = halloc(h, &VV.cbuf, (size_t)std::max(1, h->wd.cb_total) * nrhs)))
+    if ((r = halloc(h, &VV.bp, n * cols)) || (r = halloc(h, &VV.ys, n * cols)) ||
+        (r = halloc(h, &VV.wbuf, (size_t)h->wrows * cols)))
       return r;
     return SNU_OK;
   };
@@ -409,7 +410,7 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
   hipStream_t st = h->stream;
   h->t[15] = 0;
   const int n = h->P.n;
-  VecDev vd{0, n, nrhs};
+  VecDev vd{0, 0, n, nrhs, h->wrows, 0};
   PermDev pd[2];
   std::memset(pd, 0, sizeof(pd));
   pd[0] = PermDev{h->d_order, d_b, d_x, ldb, ldx, n, 0};
@@ -420,10 +421,11 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
   ss.perm = h->d_perm;
   ss.vec = h->d_vec;
   ss.nmat = 1;
-  ss.max_elems = (long long)n * nrhs;
-  ss.max_rhs = nrhs;
+  ss.max_groups = vec_groups(nrhs);
+  ss.max_elems = (long long)n * ss.max_groups;
+  ss.one = nrhs == 1;
+  ss.many = nrhs > 1;
   ss.wd = &h->wd;
-  ss.cb_ld = h->wd.cb_total;
   HIPCHK(hipEventRecord(h->ev[6], st));
   int rc = SNU_OK;
   if (h->prec == SNU_FP32) {
@@ -449,7 +451,7 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
     rs.max_steps = h->opts.ir_max_steps > 0 ? h->opts.ir_max_steps : h->opts.ir_max_steps < 0 ? 0 : 10;
     rs.tol = h->opts.ir_tol > 0 ? h->opts.ir_tol : 1e-15;
     std::vector<double> berr;
-    rc = run_refined(rs, (float *)B.bp, (float *)B.cbuf, *(const GemvPlan<float> *)B.plan, st, &h->ir_steps,
+    rc = run_refined(rs, (float *)B.bp, (float *)B.wbuf, *(const GemvPlan<float> *)B.plan, st, &h->ir_steps,
                      &berr);
     h->ir_berr = berr.empty() ? 0 : berr[0];
     if (rc == SNU_ERR_NOT_CONVERGED && fallback) {
@@ -462,7 +464,7 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
     }
     if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
   } else {
-    run_sweep<double>(ss, (double *)B.bp, (double *)B.cbuf, *(const GemvPlan<double> *)B.plan, st);
+    run_sweep<double>(ss, (double *)B.bp, (double *)B.wbuf, *(const GemvPlan<double> *)B.plan, st);
     h->ir_steps = 0;
     h->ir_berr = 0;
   }
@@ -485,12 +487,12 @@ int solve_dev(snumat *h, const double *d_b, long long ldb, double *d_x, long lon
   if (h->prec == SNU_FP32) {
     if ((rc = ensure_plan<float>(h, nrhs))) return rc;
     B.bp = h->v32.bp;
-    B.cbuf = h->v32.cbuf;
+    B.wbuf = h->v32.wbuf;
     B.plan = &h->v32.sp;
   } else {
     if ((rc = ensure_plan<double>(h, nrhs))) return rc;
     B.bp = h->v64.bp;
-    B.cbuf = h->v64.cbuf;
+    B.wbuf = h->v64.wbuf;
     B.plan = &h->v64.sp;
   }
   B.r = h->d_r;
@@ -526,75 +528,94 @@ extern "C" int snumat_solve_device(snumat_t *h, const double *d_b, double *d_x,
 
 namespace {
 // The solve of snumat_solve_device over buffers carved from the device's
-// scratch: permuted right-hand sides, dense-solve vectors, boundary
-// contributions, (SNU_FP32) residual, correction and column norms, then the
+// scratch: permuted right-hand sides, dense-solve vectors, the leaf fronts'
+// update rows, (SNU_FP32) residual, correction and column norms, then the
 // dense-solve descriptors and split-K partial sums.  Every buffer is written
 // before it is read within the call (the column norms are zeroed by their
 // own kernel), so no clearing is needed; the descriptors are copied in on
-// every call, as another handle's call may have overwritten them.
+// every call, as another handle's call may have overwritten them.  A call
+// whose padded column groups do not fit runs its columns one at a time, with
+// the handle's own one-column update rows when those do not fit either.
 template <typename T>
 int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
   unsigned char *base = nullptr;
   int rc = scratch_base(h->device, &base);
   if (rc) return rc;
   const size_t n = (size_t)h->P.n;
-  size_t off = 0;
-  auto carve = [&](size_t bytes) {
-    const size_t o = off;
-    off += (bytes + 255) & ~size_t(255);
-    return o;
-  };
-  const size_t o_bp = carve(sizeof(T) * n * nrhs);
-  const size_t o_ys = carve(sizeof(T) * n * nrhs);
-  const size_t o_cb = carve(sizeof(T) * (size_t)std::max(1, h->wd.cb_total) * nrhs);
-  size_t o_r = 0, o_dx = 0, o_cn = 0;
-  if (h->prec == SNU_FP32) {
-    o_r = carve(sizeof(double) * n * nrhs);
-    o_dx = carve(sizeof(double) * n * nrhs);
-    o_cn = carve(sizeof(double) * 3 * (size_t)nrhs);
-  }
-  Values<T> &VV = vals<T>(h);
-  GemvPlan<T> &g = VV.sp_scratch;
-  if (VV.scratch_nrhs != nrhs) {
-    VV.scratch_nrhs = -1;
-    g = GemvPlan<T>();  // device pointers point into the scratch: nothing to free
-    build_solve_plan<T>(h, (T *)(base + o_bp), (T *)(base + o_ys), nrhs, g);
-  }
-  const size_t need_part = layout_gemv_plan(g);
-  const size_t o_vp = carve(sizeof(GemvProbT<T>) * std::max<size_t>(1, g.vp.size()));
-  const size_t o_vs = carve(sizeof(GemvSegT<T>) * std::max<size_t>(1, g.vs.size()));
-  const size_t o_part = carve(sizeof(T) * std::max<size_t>(1, need_part));
-  if (off > kScratchBytes)
-    return set_error(SNU_ERR_BAD_INPUT, "allocation-free solve needs " + std::to_string(off) +
+  // the documented limit, independent of the layout used below: per column
+  // two vectors, the boundary contributions and (SNU_FP32) two FP64 vectors
+  size_t need = 2 * sizeof(T) * n + (h->prec == SNU_FP32 ? 16 * n : 0);
+  for (const LeafPlan &L : h->P.leaves) need += sizeof(T) * (size_t)L.nbr;
+  need *= nrhs;
+  if (need > kScratchBytes)
+    return set_error(SNU_ERR_BAD_INPUT, "allocation-free solve needs " + std::to_string(need) +
                                          " bytes of scratch for n = " + std::to_string(n) +
                                          ", nrhs = " + std::to_string(nrhs) + "; the limit is " +
                                          std::to_string(kScratchBytes) +
                                          " (use snumat_solve_device, or fewer columns per call)");
-  VV.scratch_nrhs = nrhs;
-  g.d_vp = (GemvProbT<T> *)(base + o_vp);
-  g.d_vs = (GemvSegT<T> *)(base + o_vs);
-  g.d_part = (T *)(base + o_part);
-  g.cap_vp = g.vp.size();
-  g.cap_vs = g.vs.size();
-  g.cap_part = need_part;
-  if (!g.vp.empty())
-    HIPCHK(hipMemcpyAsync(g.d_vp, g.vp.data(), g.vp.size() * sizeof(g.vp[0]), hipMemcpyHostToDevice,
-                          h->stream));
-  if (!g.vs.empty())
-    HIPCHK(hipMemcpyAsync(g.d_vs, g.vs.data(), g.vs.size() * sizeof(g.vs[0]), hipMemcpyHostToDevice,
-                          h->stream));
+  Values<T> &VV = vals<T>(h);
+  GemvPlan<T> &g = VV.sp_scratch;
   SolveBuffers B;
-  B.bp = base + o_bp;
-  B.cbuf = base + o_cb;
-  B.plan = &g;
-  if (h->prec == SNU_FP32) {
-    B.r = (double *)(base + o_r);
-    B.dx = (double *)(base + o_dx);
-    B.colnorms = (unsigned long long *)(base + o_cn);
+  // lay the buffers of a k-column solve out; own_w: update rows in the scratch
+  auto layout = [&](int k, bool own_w) -> bool {
+    size_t off = 0;
+    auto carve = [&](size_t bytes) {
+      const size_t o = off;
+      off += (bytes + 255) & ~size_t(255);
+      return base + o;
+    };
+    const size_t cols = (size_t)vec_groups(k) * vec_width(k);
+    T *bp = (T *)carve(sizeof(T) * n * cols), *ys = (T *)carve(sizeof(T) * n * cols);
+    B.bp = bp;
+    B.wbuf = own_w ? (void *)carve(sizeof(T) * (size_t)h->wrows * cols) : (void *)VV.w1;
+    if (h->prec == SNU_FP32) {
+      B.r = (double *)carve(sizeof(double) * n * k);
+      B.dx = (double *)carve(sizeof(double) * n * k);
+      B.colnorms = (unsigned long long *)carve(sizeof(double) * 3 * (size_t)k);
+    }
+    if (off > kScratchBytes) return false;
+    if (VV.scratch_nrhs != k || VV.scratch_own_w != own_w) {
+      VV.scratch_nrhs = -1;
+      g = GemvPlan<T>();  // device pointers point into the scratch: nothing to free
+      build_solve_plan<T>(h, bp, ys, k, g);
+      g.cap_part = layout_gemv_plan(g);
+      VV.scratch_nrhs = k;
+      VV.scratch_own_w = own_w;
+    }
+    g.cap_vp = g.vp.size();
+    g.cap_vs = g.vs.size();
+    g.d_vp = (GemvProbT<T> *)carve(sizeof(GemvProbT<T>) * std::max<size_t>(1, g.vp.size()));
+    g.d_vs = (GemvSegT<T> *)carve(sizeof(GemvSegT<T>) * std::max<size_t>(1, g.vs.size()));
+    g.d_part = (T *)carve(sizeof(T) * std::max<size_t>(1, g.cap_part));
+    B.plan = &g;
+    return off <= kScratchBytes;
+  };
+  int step = nrhs;
+  if (!layout(nrhs, true)) {
+    step = 1;
+    if (!layout(1, true) && !layout(1, false)) {
+      VV.scratch_nrhs = -1;
+      return set_error(SNU_ERR_BAD_INPUT, "allocation-free solve: one column does not fit the scratch of " +
+                                              std::to_string(kScratchBytes) + " bytes (n = " + std::to_string(n) + ")");
+    }
   }
   // no FP64 twin here: building one allocates (a stalled refinement
   // returns SNU_ERR_NOT_CONVERGED with x = the last iterate)
-  return solve_core(h, d_b, ld, d_x, ld, nrhs, B, false);
+  int worst = SNU_OK;
+  for (int c = 0; c < nrhs; c += step) {
+    if (c == 0) {
+      if (!g.vp.empty())
+        HIPCHK(hipMemcpyAsync(g.d_vp, g.vp.data(), g.vp.size() * sizeof(g.vp[0]), hipMemcpyHostToDevice,
+                              h->stream));
+      if (!g.vs.empty())
+        HIPCHK(hipMemcpyAsync(g.d_vs, g.vs.data(), g.vs.size() * sizeof(g.vs[0]), hipMemcpyHostToDevice,
+                              h->stream));
+    }
+    rc = solve_core(h, d_b + (size_t)c * ld, ld, d_x + (size_t)c * ld, ld, step, B, false);
+    if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
+    if (rc) worst = rc;
+  }
+  return worst;
 }
 }  // namespace
 
@@ -900,8 +921,12 @@ void executed_work(const snumat *h, double *w) {
   double gb = 0;
   for (const std::vector<Launch> *ls : {&sp.fwd, &sp.bwd})
     for (const Launch &L : *ls) gb += L.flops;  // matrix bytes read by the launch
-  double lb = 0;
-  for (const LeafPlan &L : h->P.leaves) lb += (double)(sizeof(T) + 4) * L.lu_nnz;
+  double lb = 0;  // the fronts' factors: L11 / U11, L21, U12
+  for (const LeafPlan &L : h->P.leaves)
+    for (size_t f = 0; f < L.ff.size(); f++) {
+      const double fo = L.ff[f], nb = fo - L.fnk[f];
+      lb += sizeof(T) * (fo * fo - nb * nb);
+    }
   w[0] = fl;
   w[1] = nl;
   w[2] = nd;

@@ -39,9 +39,9 @@ struct snubatch {
   FrontPlan<float> fr32;
   // solves (sized for the last right-hand-side pattern)
   std::vector<int> pattern;  // nrhs per matrix of the current solve plan
-  long long vec_cap = 0;
-  int cb_cap = 0, slot_cap = 0;
-  void *bp = nullptr, *ys = nullptr, *cbuf = nullptr;
+  long long vec_cap = 0, res_cap = 0, w_cap = 0;
+  int slot_cap = 0;
+  void *bp = nullptr, *ys = nullptr, *wbuf = nullptr;
   double *r = nullptr, *dx = nullptr;
   unsigned long long *norms = nullptr;
   int *d_active = nullptr;
@@ -51,6 +51,7 @@ struct snubatch {
   GemvPlan<double> s64;
   GemvPlan<float> s32;
   std::vector<VecDev> h_vec;
+  std::vector<long long> res_base;  // FP64 residual segment of each matrix
   std::vector<double> anorm;
   int ir_steps = 0;
   std::vector<double> berr;
@@ -119,34 +120,43 @@ template <typename T>
 int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   if (b->pattern == nrhs) return SNU_OK;
   const int nm = (int)b->mats.size();
-  long long tot = 0;
-  int cbt = 0, slots = 0;
+  // packed vectors (padded column groups), update rows, FP64 residuals
+  long long tot = 0, wtot = 0, rtot = 0;
+  int slots = 0;
   for (int m = 0; m < nm; m++) {
-    tot += (long long)b->mats[m]->P.n * nrhs[m];
-    cbt = std::max(cbt, nrhs[m]);
+    const long long cols = (long long)vec_groups(nrhs[m]) * vec_width(nrhs[m]);
+    tot += (long long)b->mats[m]->P.n * cols;
+    wtot += (long long)b->mats[m]->wrows * cols;
+    rtot += (long long)b->mats[m]->P.n * nrhs[m];
     slots += nrhs[m];
   }
   int rc;
+  b->pattern.clear();
   if (tot > b->vec_cap) {
     bfree(b, b->bp);
     bfree(b, b->ys);
-    bfree(b, b->r);
-    bfree(b, b->dx);
     b->bp = b->ys = nullptr;
-    b->r = b->dx = nullptr;
+    b->vec_cap = 0;
     if ((rc = balloc(b, &b->bp, sizeof(T) * tot)) || (rc = balloc(b, &b->ys, sizeof(T) * tot)))
-      return rc;
-    if (b->prec == SNU_FP32 &&
-        ((rc = balloc(b, (void **)&b->r, sizeof(double) * tot)) ||
-         (rc = balloc(b, (void **)&b->dx, sizeof(double) * tot))))
       return rc;
     b->vec_cap = tot;
   }
-  if (cbt > b->cb_cap) {
-    bfree(b, b->cbuf);
-    b->cbuf = nullptr;
-    if ((rc = balloc(b, &b->cbuf, sizeof(T) * (size_t)std::max(1, b->wd.cb_total) * cbt))) return rc;
-    b->cb_cap = cbt;
+  if (b->prec == SNU_FP32 && rtot > b->res_cap) {
+    bfree(b, b->r);
+    bfree(b, b->dx);
+    b->r = b->dx = nullptr;
+    b->res_cap = 0;
+    if ((rc = balloc(b, (void **)&b->r, sizeof(double) * rtot)) ||
+        (rc = balloc(b, (void **)&b->dx, sizeof(double) * rtot)))
+      return rc;
+    b->res_cap = rtot;
+  }
+  if (wtot > b->w_cap) {
+    bfree(b, b->wbuf);
+    b->wbuf = nullptr;
+    b->w_cap = 0;
+    if ((rc = balloc(b, &b->wbuf, sizeof(T) * (size_t)wtot))) return rc;
+    b->w_cap = wtot;
   }
   if (slots > b->slot_cap) {
     bfree(b, b->norms);
@@ -154,11 +164,17 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
     if ((rc = balloc(b, (void **)&b->norms, sizeof(unsigned long long) * 3 * (size_t)slots))) return rc;
     b->slot_cap = slots;
   }
-  b->h_vec.assign(nm, VecDev{0, 0, 0});
-  long long base = 0;
+  b->h_vec.assign(nm, VecDev());
+  b->res_base.assign(nm, 0);
+  long long base = 0, wbase = 0, rbase = 0;
   for (int m = 0; m < nm; m++) {
-    b->h_vec[m] = VecDev{base, b->mats[m]->P.n, nrhs[m]};
-    base += (long long)b->mats[m]->P.n * nrhs[m];
+    const snumat *h = b->mats[m];
+    const long long cols = (long long)vec_groups(nrhs[m]) * vec_width(nrhs[m]);
+    b->h_vec[m] = VecDev{base, wbase, h->P.n, nrhs[m], h->wrows, 0};
+    b->res_base[m] = rbase;
+    base += (long long)h->P.n * cols;
+    wbase += (long long)h->wrows * cols;
+    rbase += (long long)h->P.n * nrhs[m];
   }
   HIPCHK(hipMemcpyAsync(b->d_vec, b->h_vec.data(), sizeof(VecDev) * nm, hipMemcpyHostToDevice, b->stream));
   GemvPlan<T> &out = std::is_same<T, double>::value ? (GemvPlan<T> &)b->s64 : (GemvPlan<T> &)b->s32;
@@ -222,17 +238,21 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
   if (rc) return rc;
   hipStream_t st = b->stream;
   std::vector<PermDev> pd(2 * (size_t)nm);
-  long long max_elems = 0;
-  int max_rhs = 0, max_n = 0;
+  long long max_elems = 0, max_vals = 0;
+  int max_groups = 0, max_n = 0;
+  bool one = false, many = false;
   for (int m = 0; m < nm; m++) {
     const snumat *h = b->mats[m];
     const int n = h->P.n;
-    const long long base = b->h_vec[m].base;
+    const long long base = b->res_base[m];
     pd[m] = PermDev{h->d_order, d_b[m], d_x[m], (long long)ld[m], (long long)ld[m], n, m};
     pd[nm + m] = PermDev{h->d_order, b->r ? b->r + base : nullptr, b->dx ? b->dx + base : nullptr,
                          (long long)n, (long long)n, n, m};
-    max_elems = std::max(max_elems, (long long)n * nrhs[m]);
-    max_rhs = std::max(max_rhs, nrhs[m]);
+    max_elems = std::max(max_elems, (long long)n * vec_groups(nrhs[m]));
+    max_vals = std::max(max_vals, (long long)n * nrhs[m]);
+    max_groups = std::max(max_groups, vec_groups(nrhs[m]));
+    one |= nrhs[m] == 1;
+    many |= nrhs[m] > 1;
     max_n = std::max(max_n, n);
   }
   HIPCHK(hipMemcpyAsync(b->d_perm, pd.data(), sizeof(PermDev) * pd.size(), hipMemcpyHostToDevice, st));
@@ -241,16 +261,17 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
   ss.vec = b->d_vec;
   ss.nmat = nm;
   ss.max_elems = max_elems;
-  ss.max_rhs = max_rhs;
+  ss.max_groups = max_groups;
+  ss.one = one;
+  ss.many = many;
   ss.wd = &b->wd;
-  ss.cb_ld = b->wd.cb_total;
   HIPCHK(hipEventRecord(b->ev[6], st));
   if (b->prec == SNU_FP32) {
     std::vector<IrDev> ir(nm);
     std::vector<int> slot_mat;
     for (int m = 0; m < nm; m++) {
       const snumat *h = b->mats[m];
-      const long long base = b->h_vec[m].base;
+      const long long base = b->res_base[m];
       IrDev &e = ir[m];
       std::memset(&e, 0, sizeof(e));
       e.rowptr = h->d_arow;
@@ -276,7 +297,7 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
     rs.ir = b->d_ir;
     rs.nmat = nm;
     rs.max_n = max_n;
-    rs.max_elems = max_elems;
+    rs.max_elems = max_vals;
     rs.norms = b->norms;
     rs.nslots = (int)slot_mat.size();
     rs.slot_mat = &slot_mat;
@@ -286,7 +307,7 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
     rs.d_active = b->d_active;
     rs.max_steps = o.ir_max_steps > 0 ? o.ir_max_steps : o.ir_max_steps < 0 ? 0 : 10;
     rs.tol = o.ir_tol > 0 ? o.ir_tol : 1e-15;
-    rc = run_refined(rs, (float *)b->bp, (float *)b->cbuf, b->s32, st, &b->ir_steps, &b->berr);
+    rc = run_refined(rs, (float *)b->bp, (float *)b->wbuf, b->s32, st, &b->ir_steps, &b->berr);
     if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
     b->t[15] = 0;
     if (rc == SNU_ERR_NOT_CONVERGED) {
@@ -302,7 +323,7 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
       rc = SNU_OK;
     }
   } else {
-    run_sweep<double>(ss, (double *)b->bp, (double *)b->cbuf, b->s64, st);
+    run_sweep<double>(ss, (double *)b->bp, (double *)b->wbuf, b->s64, st);
     b->ir_steps = 0;
     b->berr.assign(nm, 0.0);
   }
@@ -348,39 +369,25 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   // concatenated leaves and work lists
   std::vector<LeafDev> leaves;
   WorkLists W;
-  W.tptr.assign(1, 0);
   W.tile_ptr.assign(1, 0);
-  int max_leaf = 0;
-  for (snumat *h : b->mats) max_leaf = std::max(max_leaf, h->wd.max_leaf);
-  int cb = 0;
   std::vector<PrepDev> prep;
   std::vector<IrDev> ira;
   for (int m = 0; m < count; m++) {
     snumat *h = b->mats[m];
-    const int lbase = (int)leaves.size(), sbase = (int)W.tsrc_leaf.size();
+    const int lbase = (int)leaves.size(), sbase = (int)W.tsrc.size();
     for (LeafDev L : h->h_leaves) {
-      L.cb_off += cb;
       L.vec = m;
       leaves.push_back(L);
     }
-    for (int r = 0; r < h->P.np; r++) {
-      const int nbr = h->P.leaves[r].nbr;
-      for (int f = 0; f < nbr; f += 4) W.fwg_leaf.push_back(lbase + r), W.fwg_first.push_back(f);
-    }
     const WorkLists &w = h->wl;
-    W.trow_blk.insert(W.trow_blk.end(), w.trow_blk.begin(), w.trow_blk.end());
-    W.trow_loc.insert(W.trow_loc.end(), w.trow_loc.begin(), w.trow_loc.end());
-    W.trow_glob.insert(W.trow_glob.end(), w.trow_glob.begin(), w.trow_glob.end());
-    for (size_t t = 1; t < w.tptr.size(); t++) W.tptr.push_back(sbase + w.tptr[t]);
-    for (int s : w.tsrc_leaf) W.tsrc_leaf.push_back(lbase + s);
-    W.tsrc_ri.insert(W.tsrc_ri.end(), w.tsrc_ri.begin(), w.tsrc_ri.end());
+    for (TargetDev t : w.targets) W.targets.push_back(TargetDev{t.row, sbase + t.s0, sbase + t.s1, m});
+    W.tsrc.insert(W.tsrc.end(), w.tsrc.begin(), w.tsrc.end());
     const int gbase = (int)W.seg_leaf.size();
     W.tile_blk.insert(W.tile_blk.end(), w.tile_blk.begin(), w.tile_blk.end());
     W.tile_row0.insert(W.tile_row0.end(), w.tile_row0.begin(), w.tile_row0.end());
     for (size_t t = 1; t < w.tile_ptr.size(); t++) W.tile_ptr.push_back(gbase + w.tile_ptr[t]);
     for (int s : w.seg_leaf) W.seg_leaf.push_back(lbase + s);
     W.seg_ri.insert(W.seg_ri.end(), w.seg_ri.begin(), w.seg_ri.end());
-    cb += h->wd.cb_total;
     PrepDev pd;
     pd.arena = b->prec == SNU_FP32 ? (void *)h->v32.arena : (void *)h->v64.arena;
     pd.inv = b->prec == SNU_FP32 ? (void *)h->v32.inv : (void *)h->v64.inv;
@@ -403,19 +410,11 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   }
   WorkDev &wd = b->wd;
   wd.nleaves = (int)leaves.size();
-  wd.nfwg = (int)W.fwg_leaf.size();
-  wd.ntarget = (int)W.trow_glob.size();
+  wd.ntarget = (int)W.targets.size();
   wd.ntile = (int)W.tile_blk.size();
-  wd.cb_total = cb;
-  wd.max_leaf = max_leaf;
-  wd.max_lev = 0;
-  for (snumat *h : b->mats) wd.max_lev = std::max(wd.max_lev, h->wd.max_lev);
   int rc;
-  if ((rc = bupload(b, &wd.leaves, leaves)) || (rc = bupload(b, &wd.fwg_leaf, W.fwg_leaf)) ||
-      (rc = bupload(b, &wd.fwg_first, W.fwg_first)) || (rc = bupload(b, &wd.trow_blk, W.trow_blk)) ||
-      (rc = bupload(b, &wd.trow_loc, W.trow_loc)) || (rc = bupload(b, &wd.trow_glob, W.trow_glob)) ||
-      (rc = bupload(b, &wd.tptr, W.tptr)) || (rc = bupload(b, &wd.tsrc_leaf, W.tsrc_leaf)) ||
-      (rc = bupload(b, &wd.tsrc_ri, W.tsrc_ri)) || (rc = bupload(b, &b->d_prep, prep)) ||
+  if ((rc = bupload(b, &wd.leaves, leaves)) || (rc = bupload(b, &wd.targets, W.targets)) ||
+      (rc = bupload(b, &wd.tsrc, W.tsrc)) || (rc = bupload(b, &b->d_prep, prep)) ||
       (rc = bupload(b, &wd.tile_blk, W.tile_blk)) || (rc = bupload(b, &wd.tile_row0, W.tile_row0)) ||
       (rc = bupload(b, &wd.tile_ptr, W.tile_ptr)) || (rc = bupload(b, &wd.seg_leaf, W.seg_leaf)) ||
       (rc = bupload(b, &wd.seg_ri, W.seg_ri)) ||
@@ -431,7 +430,7 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
       for (snumat *h : b->mats) parts.push_back(&vals<T>(h).fronts);
       merge_fronts(parts, fp);
       int r;
-      if ((r = upload_dense_plan(fp.dense)) || (r = bupload(b, &fp.d_small, fp.small)) ||
+      if ((r = upload_dense_plan(fp.dense)) || (r = bupload(b, &fp.d_iblk, fp.iblk)) || (r = bupload(b, &fp.d_small, fp.small)) ||
           (r = bupload(b, &fp.d_large, fp.large)) || (r = bupload(b, &fp.d_work, fp.work)) || (r = bupload(b, &fp.d_wrange, fp.wrange)) ||
           (r = bupload(b, &fp.d_ls, fp.ls)) || (r = bupload(b, &fp.d_tiles, fp.tiles)))
         return r;

@@ -29,11 +29,13 @@ struct Launch {
   int kind;  // 0 diag LU; GEMM (64 tile) 1: C = AB, 2: C -= AB, 6: C = -AB;
              // GEMM (128 tile) 5: C -= AB, 10: C = AB, 11: C = -AB; 3: copy
              // C = A (GEMM descriptors, 64 x 64 tiles); GEMV 7: y = Ax, 8: y -= Ax
+             // (one column), 17 / 18: the same on groups of 16 columns
   int p0, np, tiles;
   double flops;
   long long key;
-  int wgs = 0;          // GEMV: workgroups of the split-K partial pass (0: unsplit)
-  long long part = 0;   // GEMV: partial-sum values of the launch
+  int wgs = 0;          // GEMV: workgroups (one column: of the split-K partial pass, 0: unsplit)
+  long long part = 0;   // GEMV: partial-sum values of the launch (0: unsplit)
+  int gstep = 1, groups = 1;  // 16 columns: groups per workgroup, most groups of a problem
 };
 inline bool is_gemm(int kind) {
   return kind == 1 || kind == 2 || kind == 5 || kind == 6 || kind == 10 || kind == 11;
@@ -76,6 +78,7 @@ struct FrontLevel {
 template <typename T>
 struct FrontPlan {
   std::vector<FrontDev> small, large;
+  std::vector<int2> iblk;   // 16-pivot blocks of the small fronts: {front, first pivot}
   std::vector<int4> work;   // larger fronts: {front, first column, ranges offset, 0}
   std::vector<int> wrange;  // per work item: its owned-slot range, then per child its column range
   std::vector<FrontLevel> levels;
@@ -83,11 +86,18 @@ struct FrontPlan {
   std::vector<LeafSchurDev> ls;
   std::vector<int4> tiles;
   FrontDev *d_small = nullptr, *d_large = nullptr;
+  int2 *d_iblk = nullptr;
   int4 *d_work = nullptr;
   int *d_wrange = nullptr;
   LeafSchurDev *d_ls = nullptr;
   int4 *d_tiles = nullptr;
 };
+template <typename T>
+void list_inverse_blocks(FrontPlan<T> &fp) {
+  fp.iblk.clear();
+  for (size_t f = 0; f < fp.small.size(); f++)
+    for (int k = 0; k < fp.small[f].nk; k += 16) fp.iblk.push_back(make_int2((int)f, k));
+}
 inline long long front_key(int height, int step, int kind) {
   return (long long)height * 100000000LL + step * 8LL + kind;
 }
@@ -103,8 +113,9 @@ struct Values {
   T *farena = nullptr; // leaf fronts (each f x f; larger fronts then 2 x 64 x 64 of inverses)
   FrontPlan<T> fronts;
   DensePlan<T> fact;
-  // standalone solves
-  T *bp = nullptr, *ys = nullptr, *cbuf = nullptr;
+  // standalone solves: right-hand sides, dense-solve vectors, the fronts'
+  // update rows; w1: update rows of one column (allocation-free solves)
+  T *bp = nullptr, *ys = nullptr, *wbuf = nullptr, *w1 = nullptr;
   int plan_nrhs = -1;
   GemvPlan<T> sp;
   // allocation-free solves: the same plan over buffers in the library's
@@ -112,27 +123,24 @@ struct Values {
   // and are never freed)
   GemvPlan<T> sp_scratch;
   int scratch_nrhs = -1;
+  bool scratch_own_w = true;
 };
 
 // Host copies of the per-leaf work lists (kept for batching).
 struct WorkLists {
-  std::vector<int> fwg_leaf, fwg_first;  // forward boundary-row workgroups
-  std::vector<int> trow_blk, trow_loc, trow_glob, tptr, tsrc_leaf, tsrc_ri;  // targets
-  std::vector<int> tile_blk, tile_row0, tile_ptr, seg_leaf, seg_ri;          // assembly tiles
+  std::vector<TargetDev> targets;  // separator rows receiving leaf contributions
+  std::vector<int> tsrc;           // their sources: update rows of root fronts
+  std::vector<int> tile_blk, tile_row0, tile_ptr, seg_leaf, seg_ri;  // assembly tiles
 };
 
 // Device copies of the work lists of a launch set (one matrix or a batch).
 struct WorkDev {
   LeafDev *leaves = nullptr;
   int nleaves = 0;
-  int *fwg_leaf = nullptr, *fwg_first = nullptr, nfwg = 0;
-  int *trow_blk = nullptr, *trow_loc = nullptr, *trow_glob = nullptr, *tptr = nullptr;
-  int *tsrc_leaf = nullptr, *tsrc_ri = nullptr, ntarget = 0;
+  TargetDev *targets = nullptr;
+  int *tsrc = nullptr, ntarget = 0;
   int *tile_blk = nullptr, *tile_row0 = nullptr, *tile_ptr = nullptr;
   int *seg_leaf = nullptr, *seg_ri = nullptr, ntile = 0;
-  int cb_total = 0;
-  int max_leaf = 0;  // rows of the largest leaf
-  int max_lev = 0;   // most level sets of a leaf (forward or backward)
 };
 
 // A factorization's launch sequence captured once into a HIP graph and
@@ -160,10 +168,10 @@ struct snumat {
   int *d_arow = nullptr, *d_acol = nullptr;  // A's pattern (refinement residuals)
   int *d_order = nullptr;
   // leaves and work lists
-  std::vector<snu::LeafDev> h_leaves;  // vec = 0, cb_off local
+  std::vector<snu::LeafDev> h_leaves;  // vec = 0
   snu::WorkLists wl;
   snu::WorkDev wd;
-  int max_leaf_w = 0;  // widest leaf workspace (leaf_size + nbc)
+  int wrows = 0;       // update rows of the leaf fronts (solves)
   // dense tables
   snu::DenseDev *d_dd = nullptr;
   std::vector<long long> inv_off;
@@ -242,7 +250,7 @@ int add_gemm(std::vector<GemmProbT<T>> &gp, std::vector<GemmSegT<T>> &gs, int &t
              double &flops, int tb = 64);
 
 // GEMV plan of one matrix's dense solves into the packed vectors bp / ys at
-// this matrix's segment (ld = n, nrhs columns); keys order fwd / bwd.
+// this matrix's segment (VecDev form, nrhs columns); keys order fwd / bwd.
 template <typename T>
 void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &out);
 // Copy the plan's descriptors to the device on stream st, growing the
@@ -293,13 +301,13 @@ struct SolveSet {
   const PermDev *perm;
   const VecDev *vec;
   int nmat;
-  long long max_elems;
-  int max_rhs;
+  long long max_elems;  // largest n x groups of a matrix
+  int max_groups;
+  bool one, many;       // matrices with one / several columns present
   const WorkDev *wd;
-  int cb_ld;
 };
 template <typename T>
-void run_sweep(const SolveSet &ss, T *bp, T *cbuf, const GemvPlan<T> &plan, hipStream_t st);
+void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st);
 struct RefineSet {
   SolveSet sweep_b;  // permutation tables b -> x (the caller's vectors)
   SolveSet sweep_r;  // permutation tables r -> dx
@@ -314,15 +322,15 @@ struct RefineSet {
   int max_steps;
   double tol;
 };
-int run_refined(const RefineSet &rs, float *bp, float *cbuf, const GemvPlan<float> &plan,
+int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<float> &plan,
                 hipStream_t st, int *steps_out, std::vector<double> *berr_mat);
 
 // Buffers of one standalone solve: the permuted right-hand sides and the
-// boundary contributions (value type of the handle), the dense-solve launch
+// leaf fronts' update rows (value type of the handle), the dense-solve launch
 // plan with its device descriptors, and (SNU_FP32) the FP64 residual /
 // correction and the column norms of the refinement.
 struct SolveBuffers {
-  void *bp = nullptr, *cbuf = nullptr;
+  void *bp = nullptr, *wbuf = nullptr;
   const void *plan = nullptr;  // GemvPlan<T> of the handle's value type
   double *r = nullptr, *dx = nullptr;
   unsigned long long *colnorms = nullptr;

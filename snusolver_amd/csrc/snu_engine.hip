@@ -4,7 +4,7 @@
 //
 // Phase map (reference -> here):
 //   core_run (kernel_sparse.cu:1011-1037)        -> prepare (zero + scatter),
-//        k_leaf_rows, k_leaf_sep, k_assemble_schur
+//        the leaf fronts, k_front_schur, k_assemble_schur
 //   dense level loop (SnuMat_factorize.cu:258-284) -> per level: blocked
 //        getrf/trsm (k_diag_lu + k_gemm by the block inverses), then one
 //        grouped k_gemm for all Schur updates of the level (K-concatenated
@@ -269,7 +269,7 @@ struct GemvBatch {
   std::vector<GemvProbT<T>> p;
   int tiles = 0;
   double bytes = 0;
-  void add(std::vector<GemvSegT<T>> &vs, T *y, long long ldy, int M, int tri, int nrhs,
+  void add(std::vector<GemvSegT<T>> &vs, T *y, long long ldy, int M, int tri, int groups,
            const std::vector<GemvSegT<T>> &segs) {
     if (M <= 0) return;
     GemvProbT<T> q;
@@ -277,7 +277,7 @@ struct GemvBatch {
     q.ldy = ldy;
     q.M = M;
     q.tri = tri;
-    q.nrhs = nrhs;
+    q.groups = groups;
     q.seg0 = (int)vs.size();
     q.nseg = 0;
     for (const GemvSegT<T> &g : segs)
@@ -683,13 +683,16 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
   const Values<T> &VV = vals<T>(h);
   const Plan &P = h->P;
   T *dense = VV.arena + P.leaf_total;
-  const long long n = P.n;
+  // one column: groups 0, kinds 7 / 8; several: groups of 16, kinds 17 / 18
+  const int w = vec_width(nrhs), groups = nrhs == 1 ? 0 : vec_groups(nrhs);
+  const int kset = w == 1 ? 7 : 17, ksub = w == 1 ? 8 : 18;
+  const long long n = (long long)P.n * w;  // values per column (group)
   auto R = [&](int p) { return dense + P.offR[p]; };
   auto Lp = [&](int p) { return dense + P.offL[p]; };
   auto Li = [&](int p) { return VV.inv + h->inv_off[p]; };
   auto Ui = [&](int p) { return VV.inv + h->inv_off[p] + (long long)P.block_size[p] * P.block_size[p]; };
-  auto bseg = [&](int p) { return bp + P.block_start[p]; };
-  auto yseg = [&](int p) { return ys + P.block_start[p]; };
+  auto bseg = [&](int p) { return bp + (long long)P.block_start[p] * w; };
+  auto yseg = [&](int p) { return ys + (long long)P.block_start[p] * w; };
   S.vp.clear();
   S.vs.clear();
   S.fwd.clear();
@@ -700,9 +703,9 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
     int lo = 1 << l, hi = std::min((2 << l) - 1, P.np - 1);
     for (int i = lo; i <= hi; i++) {
       int s = P.block_size[i];
-      g.add(S.vs, yseg(i), n, s, 1, nrhs, {GemvSeg{Li(i), bseg(i), s, n, s}});
+      g.add(S.vs, yseg(i), n, s, 1, groups, {GemvSeg{Li(i), bseg(i), s, n, s}});
     }
-    g.flush(7, S.vp, S.fwd, height * 4LL + 0);
+    g.flush(kset, S.vp, S.fwd, height * 4LL + 0);
     for (int p = 1; p < lo; p++) {
       int lp = 31 - __builtin_clz(p);
       int first = p << (l - lp), last = ((p + 1) << (l - lp)) - 1;
@@ -715,10 +718,10 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
           if (r < 0) continue;
           segs.push_back(GemvSeg{Lp(i) + r, yseg(i), P.nL[i], n, P.block_size[i]});
         }
-        g.add(S.vs, bseg(p) + m0, n, mt, 0, nrhs, segs);
+        g.add(S.vs, bseg(p) + m0 * w, n, mt, 0, groups, segs);
       }
     }
-    g.flush(8, S.vp, S.fwd, height * 4LL + 1);
+    g.flush(ksub, S.vp, S.fwd, height * 4LL + 1);
   }
   for (int l = 0; l < P.max_level; l++) {
     const int height = P.max_level - l;
@@ -732,17 +735,17 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
         // stored column tiles of a, merged into runs (consecutive stored
         // tiles of one ancestor are consecutive columns of the panel)
         for (auto cr : nz_runs(P.block_size[a], [&](int x0, int x1) { return P.umap[i][off + x0] >= 0; }))
-          segs.push_back(GemvSeg{R(i) + (long long)(s + P.umap[i][off + cr.first]) * s, bseg(a) + cr.first, s, n,
+          segs.push_back(GemvSeg{R(i) + (long long)(s + P.umap[i][off + cr.first]) * s, bseg(a) + cr.first * w, s, n,
                                  cr.second - cr.first});
       }
-      g.add(S.vs, yseg(i), n, s, 0, nrhs, segs);
+      g.add(S.vs, yseg(i), n, s, 0, groups, segs);
     }
-    g.flush(8, S.vp, S.bwd, bkey + 0);
+    g.flush(ksub, S.vp, S.bwd, bkey + 0);
     for (int i = lo; i <= hi; i++) {
       int s = P.block_size[i];
-      g.add(S.vs, bseg(i), n, s, 2, nrhs, {GemvSeg{Ui(i), yseg(i), s, n, s}});
+      g.add(S.vs, bseg(i), n, s, 2, groups, {GemvSeg{Ui(i), yseg(i), s, n, s}});
     }
-    g.flush(7, S.vp, S.bwd, bkey + 1);
+    g.flush(kset, S.vp, S.bwd, bkey + 1);
   }
 }
 
@@ -755,21 +758,30 @@ size_t layout_gemv_plan(GemvPlan<T> &g) {
   size_t need_part = 0;
   for (std::vector<Launch> *ls : {&g.fwd, &g.bwd})
     for (Launch &L : *ls) {
-      int wgs = 0, split = 0;
+      const bool one = L.kind == 7 || L.kind == 8;
+      const int piece = one ? kGemvPiece : kGemvPiece16;
+      int wgs = 0, split = 0, mg = 1;
       long long off = 0;
+      for (int q = 0; q < L.np; q++) mg = std::max(mg, g.vp[L.p0 + q].groups);
+      L.groups = mg;
+      L.gstep = mg > 2 ? 4 : mg;
       for (int q = 0; q < L.np; q++) {
         GemvProbT<T> &p = g.vp[L.p0 + q];
         int kmax = 1;
         for (int j = 0; j < p.nseg; j++) kmax = std::max(kmax, g.vs[p.seg0 + j].K);
-        p.parts = (kmax + kGemvPiece - 1) / kGemvPiece;
+        p.parts = (kmax + piece - 1) / piece;
+        split |= p.parts > 1;
+      }
+      for (int q = 0; q < L.np; q++) {
+        GemvProbT<T> &p = g.vp[L.p0 + q];
+        if (!split) p.parts = 1;
         p.wg0 = wgs;
         p.poff = off;
         const int tiles = (p.M + 63) / 64;
-        wgs += tiles * p.parts;
-        off += (long long)tiles * p.parts * p.nrhs * 64;
-        split |= p.parts > 1;
+        wgs += tiles * p.parts * (one ? 1 : (p.groups + L.gstep - 1) / L.gstep);
+        off += (long long)tiles * p.parts * 64 * (one ? 1 : p.groups * kColGroup);
       }
-      L.wgs = split ? wgs : 0;
+      L.wgs = one && !split ? 0 : wgs;
       L.part = split ? off : 0;
       need_part = std::max(need_part, (size_t)L.part);
     }
@@ -937,9 +949,7 @@ int alloc_values(snumat *h, long long S_total) {
   if ((rc = upload_dense_plan(VV.fact))) return rc;
   // leaf descriptors point at this value type's arrays
   for (size_t r = 0; r < h->h_leaves.size(); r++) {
-    LeafDev &D = h->h_leaves[r];
-    D.vals = VV.arena + h->P.leaf_off[r];
-    D.dense = VV.arena + h->P.leaf_total;
+    h->h_leaves[r].dense = VV.arena + h->P.leaf_total;
   }
   return SNU_OK;
 }
@@ -952,6 +962,9 @@ int alloc_values(snumat *h, long long S_total) {
 // partial LU (per 64-column step: diagonal block LU with the pivot clamp,
 // both triangular solves by the block inverses, the trailing update of the
 // whole remaining front) and the boundary Schur tiles.
+static long long front_inv_size(int f, int nk, int fmax) {
+  return f > fmax ? (nk + 63) / 64 * 8192LL : (nk + 15) / 16 * 256LL;
+}
 template <typename T>
 int build_front_plan(snumat *h) {
   using GemmSeg = GemmSegT<T>;
@@ -983,7 +996,7 @@ int build_front_plan(snumat *h) {
     for (int f = 0; f < nf; f++) {
       foff[r][f] = ftotal;
       ftotal += (long long)L.ff[f] * L.ff[f];
-      if (L.ff[f] > fmax) ftotal += 2 * 64 * 64;  // inverses of the diagonal blocks
+      ftotal += front_inv_size(L.ff[f], L.fnk[f], fmax);
       if (L.fpar[f] >= 0) continue;
       std::vector<int> arow(L.nbr, -1), acol(L.nbc, -1);
       for (int q = L.fidx_ptr[f]; q < L.fidx_ptr[f + 1]; q++) {
@@ -1027,6 +1040,7 @@ int build_front_plan(snumat *h) {
     for (int f = 0; f < (int)L.ff.size(); f++) {
       FrontDev D;
       D.F = fa + foff[r][f];
+      D.inv = fa + foff[r][f] + (long long)L.ff[f] * L.ff[f];
       D.vals = VV.arena + P.leaf_off[r];
       D.slot = d_ints + o_slot[r] + L.fslot_ptr[f];
       D.pos = d_ints + o_pos[r] + L.fslot_ptr[f];
@@ -1088,7 +1102,7 @@ int build_front_plan(snumat *h) {
         if (D.nk <= k) continue;
         const int f = D.f, nb = std::min(64, D.nk - k), m = f - k - nb;
         T *F = (T *)D.F;
-        T *Li = F + (long long)f * f, *Ui = Li + 64 * 64;
+        T *Li = (T *)D.inv + (long long)step * 8192, *Ui = Li + 64 * 64;
         DiagProbT<T> dp{};
         dp.D = F + k + (long long)k * f;
         dp.ld = f;
@@ -1146,7 +1160,8 @@ int build_front_plan(snumat *h) {
   FrontRoot *d_roots = nullptr;
   if ((rc = dupload(h, &d_roots, roots))) return rc;
   for (LeafSchurDev &l : FP.ls) l.root = d_roots + (uintptr_t)l.root;
-  if ((rc = dupload(h, &FP.d_small, FP.small)) || (rc = dupload(h, &FP.d_large, FP.large)) ||
+  list_inverse_blocks(FP);
+  if ((rc = dupload(h, &FP.d_iblk, FP.iblk)) || (rc = dupload(h, &FP.d_small, FP.small)) || (rc = dupload(h, &FP.d_large, FP.large)) ||
       (rc = dupload(h, &FP.d_work, FP.work)) || (rc = dupload(h, &FP.d_wrange, FP.wrange)) ||
       (rc = dupload(h, &FP.d_ls, FP.ls)) ||
       (rc = dupload(h, &FP.d_tiles, FP.tiles)))
@@ -1203,6 +1218,7 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
     lv.nsmall = (int)out.small.size() - lv.small0;
     lv.nwork = (int)out.work.size() - lv.work0;
   }
+  list_inverse_blocks(out);
   std::vector<const DensePlan<T> *> dp;
   for (const FrontPlan<T> *p : in) dp.push_back(&p->dense);
   merge_dense(dp, out.dense);
@@ -1212,6 +1228,180 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
     for (int4 t : p->tiles) out.tiles.push_back(make_int4(base + t.x, t.y, t.z, t.w));
   }
 }
+// The leaf solves of one matrix: solve positions (leaf rows in front order, so
+// a front's pivots are consecutive), update rows, the children's
+// update rows each front row adds, the units of every phase (per height,
+// forward upwards: whole fronts and first pivot blocks, further pivot blocks
+// one phase each, boundary row tiles; backward downwards: boundary column
+// chunks and whole fronts, then the pivot blocks last to first) and the
+// separator rows' sources.
+template <typename T>
+static int build_leaf_solve(snumat *h) {
+  Values<T> &VV = vals<T>(h);
+  const Plan &P = h->P;
+  const int np = P.np, fmax = front_small_max<T>();
+  std::vector<int> pos(P.n), pull, plist, bidx, phase;
+  std::vector<std::pair<int, int>> more;
+  for (int i = 0; i < P.n; i++) pos[i] = i;
+  std::vector<SolveUnit> units;
+  struct Src { int R, row; };
+  std::vector<Src> src;
+  std::vector<std::array<size_t, 2>> o_phase(np);
+  long long ftotal = 0, wrows = 0;
+  for (int r = 0; r < np; r++) {
+    const LeafPlan &L = P.leaves[r];
+    LeafDev &D = h->h_leaves[r];
+    const int nf = (int)L.ff.size(), g0 = P.block_start[L.leaf], ls = L.leaf_size;
+    for (int q = 0; q < ls; q++) pos[g0 + L.fk[q]] = g0 + q;
+    // global solve position of a core index
+    auto gpos = [&](int x) {
+      if (x < ls) return pos[g0 + x];
+      int k = 1;
+      while (x >= L.cstart[k + 1]) k++;
+      return P.block_start[L.path[k]] + x - L.cstart[k];
+    };
+    std::vector<SolveUnit> base(nf);
+    std::vector<std::vector<int>> byh(nf ? L.fheight_max + 1 : 0);
+    for (int f = 0; f < nf; f++) {
+      SolveUnit &U = base[f];
+      std::memset(&U, 0, sizeof(U));
+      U.ld = L.ff[f];
+      U.nk = L.fnk[f];
+      U.nb = U.ld - U.nk;
+      U.F = VV.farena + ftotal;
+      U.inv = VV.farena + ftotal + (long long)U.ld * U.ld;
+      ftotal += (long long)U.ld * U.ld + front_inv_size(U.ld, U.nk, fmax);
+      U.kpos = g0 + L.fkp[f];
+      U.wrow = (int)wrows;
+      U.nq = U.ld > fmax ? (U.nb + 64 * ((U.nk + 63) / 64) - 1) / (64 * ((U.nk + 63) / 64)) : 0;
+      // the backward sweep's partial products share the update rows
+      wrows += std::max<long long>(U.nb, 64LL * ((U.nk + 63) / 64) * U.nq);
+      U.bidx = (int)bidx.size();
+      for (int q = L.fidx_ptr[f]; q < L.fidx_ptr[f + 1]; q++) bidx.push_back(gpos(L.fidx[q]));
+      U.pull = (int)(pull.size() / 2);
+      pull.resize(pull.size() + 2 * (size_t)U.ld, -1);
+      int *pf = pull.data() + 2 * (size_t)U.pull;
+      more.clear();
+      for (int k = L.fchild_ptr[f]; k < L.fchild_ptr[f + 1]; k++) {
+        const int c = L.fchild[k];
+        for (int q = L.fidx_ptr[c]; q < L.fidx_ptr[c + 1]; q++) {
+          const int row = base[c].wrow + q - L.fidx_ptr[c], i = L.frel[q];
+          if (pf[2 * i] < 0) pf[2 * i] = row;
+          else if (pf[2 * i + 1] == -1) pf[2 * i + 1] = row;
+          else more.push_back({i, row});
+        }
+      }
+      // rows with three or more sources: a list from the second on
+      std::stable_sort(more.begin(), more.end(),
+                       [](const std::pair<int, int> &a, const std::pair<int, int> &b) { return a.first < b.first; });
+      for (size_t q = 0; q < more.size();) {
+        const int i = more[q].first;
+        const size_t at = plist.size();
+        plist.push_back(0);
+        plist.push_back(pf[2 * i + 1]);
+        for (; q < more.size() && more[q].first == i; q++) plist.push_back(more[q].second);
+        plist[at] = (int)(plist.size() - at - 1);
+        pf[2 * i + 1] = -2 - (int)at;
+      }
+      if (L.fpar[f] < 0)
+        for (int q = L.fidx_ptr[f]; q < L.fidx_ptr[f + 1]; q++)
+          if (L.fsrow[q] >= 0) src.push_back({gpos(L.fidx[q]), U.wrow + q - L.fidx_ptr[f]});
+      byh[L.fheight[f]].push_back(f);
+    }
+    if (wrows > 2000000000LL || bidx.size() > 2000000000u || pull.size() > 2000000000u ||
+        plist.size() > 2000000000u)
+      return set_error(SNU_ERR_BAD_INPUT, "leaf fronts too large for 32-bit solve indices");
+    auto emit = [&](int f, int kind, int row0, int sblk, int q) {
+      SolveUnit U = base[f];
+      U.kind = kind;
+      U.row0 = row0;
+      U.s = sblk;
+      U.q = q;
+      units.push_back(U);
+    };
+    auto close = [&] {  // ends a phase unless it is empty
+      if ((size_t)phase.back() != units.size()) phase.push_back((int)units.size());
+    };
+    auto large = [&](int f) { return base[f].ld > fmax; };
+    auto blocks = [&](int f) { return (base[f].nk + 63) / 64; };
+    o_phase[r][0] = phase.size();
+    phase.push_back((int)units.size());
+    for (auto &fr : byh) {
+      int smax = 0;
+      for (int f : fr)
+        if (large(f)) emit(f, kFwdPivots, 0, 0, 0), smax = std::max(smax, blocks(f));
+      for (int f : fr)
+        if (!large(f)) emit(f, kFwdFront, 0, 0, 0);
+      close();
+      for (int k = 1; k < smax; k++) {
+        for (int f : fr)
+          if (large(f) && blocks(f) > k) emit(f, kFwdPivots, 0, k, 0);
+        close();
+      }
+      for (int f : fr)
+        if (large(f))
+          for (int t = 0; t < base[f].nb; t += 64) emit(f, kFwdRows, t, 0, 0);
+      close();
+    }
+    D.nfphase = (int)(phase.size() - o_phase[r][0]) - 1;
+    o_phase[r][1] = phase.size();
+    phase.push_back((int)units.size());
+    for (size_t hh = byh.size(); hh-- > 0;) {
+      const std::vector<int> &fr = byh[hh];
+      int smax = 0;
+      for (int f : fr)
+        if (large(f)) {
+          smax = std::max(smax, blocks(f));
+          for (int k = 0; k < blocks(f); k++)
+            for (int q = 0; q < base[f].nq; q++) emit(f, kBwdCols, 0, k, q);
+        }
+      for (int f : fr)
+        if (!large(f)) emit(f, kBwdFront, 0, 0, 0);
+      close();
+      for (int k = smax - 1; k >= 0; k--) {
+        for (int f : fr)
+          if (large(f) && blocks(f) > k) emit(f, kBwdPivots, 0, k, 0);
+        close();
+      }
+    }
+    D.nbphase = (int)(phase.size() - o_phase[r][1]) - 1;
+  }
+  h->wrows = (int)std::max(1LL, wrows);
+  // separator rows and their sources, ascending row, then leaf and front
+  std::stable_sort(src.begin(), src.end(), [](const Src &a, const Src &b) { return a.R < b.R; });
+  WorkLists &W = h->wl;
+  W.targets.clear();
+  W.tsrc.clear();
+  for (size_t q = 0; q < src.size(); q++) {
+    if (q == 0 || src[q].R != src[q - 1].R) W.targets.push_back(TargetDev{src[q].R, (int)q, (int)q, 0});
+    W.targets.back().s1 = (int)q + 1;
+    W.tsrc.push_back(src[q].row);
+  }
+  // solve order of the caller's rows
+  std::vector<int> order(P.n);
+  for (int i = 0; i < P.n; i++) order[i] = pos[P.order[i]];
+  int rc;
+  SolveUnit *d_units = nullptr;
+  int *d_phase = nullptr, *d_pull = nullptr, *d_plist = nullptr, *d_bidx = nullptr;
+  if ((rc = dupload(h, &d_units, units)) || (rc = dupload(h, &d_phase, phase)) ||
+      (rc = dupload(h, &d_pull, pull)) || (rc = dupload(h, &d_plist, plist)) ||
+      (rc = dupload(h, &d_bidx, bidx)) || (rc = dupload(h, &h->d_order, order)) ||
+      (rc = dupload(h, &h->wd.targets, W.targets)) || (rc = dupload(h, &h->wd.tsrc, W.tsrc)) ||
+      (rc = dalloc(h, &VV.w1, (size_t)h->wrows)))
+    return rc;
+  h->wd.ntarget = (int)W.targets.size();
+  for (int r = 0; r < np; r++) {
+    LeafDev &D = h->h_leaves[r];
+    D.units = d_units;
+    D.fphase = d_phase + o_phase[r][0];
+    D.bphase = d_phase + o_phase[r][1];
+    D.pull = d_pull;
+    D.pulllist = d_plist;
+    D.bidx = d_bidx;
+  }
+  return SNU_OK;
+}
+
 template void merge_fronts<double>(const std::vector<const FrontPlan<double> *> &, FrontPlan<double> &);
 template void merge_fronts<float>(const std::vector<const FrontPlan<float> *> &, FrontPlan<float> &);
 template int build_front_plan<double>(snumat *);
@@ -1225,91 +1415,30 @@ int upload(snumat *h) {
   else autotune_tiles<double>();
   const int np = P.np;
   // ---- leaf arrays (concatenated; descriptors hold pointers into them) ----
-  std::vector<int> rowptr, diag, levptr, levrows, ulevptr, ulevrows;
-  std::vector<int> brow, bcol_glob, bcol_blk, bcol_loc, wcol, ftask, btask, ubnd;
-  struct Off { size_t rp, idx, lev, levr, ulev, ulevr, brow, bcol, task, row; long long S; };
-  std::vector<Off> off(np);
+  std::vector<int> bcol_blk, bcol_loc;
+  std::vector<size_t> off_bcol(np);
+  std::vector<long long> off_S(np);
   long long S_total = 0;
   h->h_leaves.assign(np, LeafDev());
-  int maxw = 1, cb = 0;
   for (int r = 0; r < np; r++) {
     const LeafPlan &L = P.leaves[r];
     LeafDev &D = h->h_leaves[r];
-    Off &o = off[r];
-    o.rp = rowptr.size();
-    o.idx = wcol.size();
-    o.lev = levptr.size();
-    o.levr = levrows.size();
-    o.ulev = ulevptr.size();
-    o.ulevr = ulevrows.size();
-    o.brow = brow.size();
-    o.bcol = bcol_glob.size();
-    o.task = ftask.size();
-    o.row = ubnd.size();
-    o.S = S_total;
+    off_bcol[r] = bcol_blk.size();
+    off_S[r] = S_total;
     S_total += (long long)L.nbr * L.nbc;
-    rowptr.insert(rowptr.end(), L.lu_rowptr.begin(), L.lu_rowptr.end());
-    diag.insert(diag.end(), L.lu_diag.begin(), L.lu_diag.end());
-    diag.push_back(0);  // diag shares rowptr's offsets (core_n + 1 entries)
-    // level-ordered solve tasks {row, first entry, end, diagonal}: forward
-    // over the L part, backward over the U entries on leaf columns (they
-    // precede the boundary ones: columns ascend), then the boundary start
-    {
-      const int ls = L.leaf_size;
-      std::vector<int> pint(ls);
-      for (int i = 0; i < ls; i++) {
-        int q = L.lu_diag[i] + 1;
-        while (q < L.lu_rowptr[i + 1] && L.lu_colidx[q] < ls) q++;
-        pint[i] = q;
-        ubnd.push_back(q);
-      }
-      for (int k = 0; k < ls; k++) {
-        const int i = L.lev_rows[k];
-        ftask.insert(ftask.end(), {i, L.lu_rowptr[i], L.lu_diag[i], L.lu_diag[i]});
-        const int j = L.ulev_rows[k];
-        btask.insert(btask.end(), {j, L.lu_diag[j] + 1, pint[j], L.lu_diag[j]});
-      }
-    }
-    wcol.insert(wcol.end(), L.wcol.begin(), L.wcol.end());
-    levptr.insert(levptr.end(), L.lev_ptr.begin(), L.lev_ptr.end());
-    levrows.insert(levrows.end(), L.lev_rows.begin(), L.lev_rows.end());
-    ulevptr.insert(ulevptr.end(), L.ulev_ptr.begin(), L.ulev_ptr.end());
-    ulevrows.insert(ulevrows.end(), L.ulev_rows.begin(), L.ulev_rows.end());
-    brow.insert(brow.end(), L.brow.begin(), L.brow.end());
     for (int c : L.bcol) {
       int k = 1;
       while (c >= L.cstart[k + 1]) k++;
-      int b = L.path[k];
-      bcol_blk.push_back(b);
+      bcol_blk.push_back(L.path[k]);
       bcol_loc.push_back(c - L.cstart[k]);
-      bcol_glob.push_back(P.block_start[b] + c - L.cstart[k]);
     }
-    D.core_n = L.core_n;
-    D.leaf_size = L.leaf_size;
     D.nbr = L.nbr;
     D.nbc = L.nbc;
-    D.nlev = (int)L.lev_ptr.size() - 1;
-    D.nulev = (int)L.ulev_ptr.size() - 1;
-    D.gstart = P.block_start[L.leaf];
-    D.cb_off = cb;
     D.vec = 0;
-    cb += L.nbr;
-    maxw = std::max(maxw, L.leaf_size + L.nbc);
   }
-  h->max_leaf_w = maxw;
-  h->wd.cb_total = cb;
-  h->wd.max_leaf = 0;
-  for (int r = 0; r < np; r++) h->wd.max_leaf = std::max(h->wd.max_leaf, P.leaves[r].leaf_size);
-  h->wd.max_lev = 0;
-  for (int r = 0; r < np; r++)
-    h->wd.max_lev = std::max(h->wd.max_lev, (int)std::max(P.leaves[r].lev_ptr.size(), P.leaves[r].ulev_ptr.size()) - 1);
-  // work lists: forward boundary workgroups and boundary targets (separator
-  // rows receiving leaf contributions, each with its sources in ascending
-  // rank order)
+  // boundary rows of the leaves by separator row, ascending rank
   WorkLists &W = h->wl;
   W = WorkLists();
-  for (int r = 0; r < np; r++)
-    for (int f = 0; f < P.leaves[r].nbr; f += 4) W.fwg_leaf.push_back(r), W.fwg_first.push_back(f);
   struct Src { int R, leaf, ri; };
   std::vector<Src> src;
   for (int r = 0; r < np; r++) {
@@ -1326,18 +1455,6 @@ int upload(snumat *h) {
   std::vector<int> blk_of(P.n);
   for (int b = 1; b <= P.num_block; b++)
     for (int i = P.block_start[b]; i < P.block_start[b] + P.block_size[b]; i++) blk_of[i] = b;
-  W.tptr.assign(1, 0);
-  for (size_t s = 0; s < src.size(); s++) {
-    if (s == 0 || src[s].R != src[s - 1].R) {
-      if (s) W.tptr.push_back((int)s);
-      W.trow_glob.push_back(src[s].R);
-      W.trow_blk.push_back(blk_of[src[s].R]);
-      W.trow_loc.push_back(src[s].R - P.block_start[blk_of[src[s].R]]);
-    }
-    W.tsrc_leaf.push_back(src[s].leaf);
-    W.tsrc_ri.push_back(src[s].ri);
-  }
-  if (!src.empty()) W.tptr.push_back((int)src.size());
   // assembly tiles: 64 consecutive rows of one separator block; per tile the
   // contributing leaves in ascending rank, each with the boundary row (ri)
   // feeding every row of the tile (-1: none)
@@ -1383,29 +1500,14 @@ int upload(snumat *h) {
   h->tmp_total = inversion_tmp_size(P);
   h->arena_len = P.leaf_total + P.dense_total;
   // ---- structure uploads ----
-  int *d_rowptr, *d_diag, *d_wcol, *d_levptr, *d_levrows, *d_ulevptr, *d_ulevrows;
-  int *d_brow, *d_bcol_glob, *d_bcol_blk, *d_bcol_loc, *d_ftask, *d_btask, *d_ubnd;
+  int *d_bcol_blk, *d_bcol_loc;
   if ((rc = dalloc(h, &h->d_aval, (size_t)P.nnz))) return rc;
   if ((rc = dupload(h, &h->d_adest, std::vector<long long>(P.a_dest.begin(), P.a_dest.end())))) return rc;
-  if ((rc = dupload(h, &d_rowptr, rowptr)) || (rc = dupload(h, &d_diag, diag)) ||
-      (rc = dupload(h, &d_wcol, wcol)) || (rc = dupload(h, &d_levptr, levptr)) ||
-      (rc = dupload(h, &d_levrows, levrows)) || (rc = dupload(h, &d_ulevptr, ulevptr)) ||
-      (rc = dupload(h, &d_ulevrows, ulevrows)) || (rc = dupload(h, &d_brow, brow)) ||
-      (rc = dupload(h, &d_bcol_glob, bcol_glob)) || (rc = dupload(h, &d_bcol_blk, bcol_blk)) ||
-      (rc = dupload(h, &d_bcol_loc, bcol_loc)) || (rc = dupload(h, &h->d_order, P.order)) ||
-      (rc = dupload(h, &d_ftask, ftask)) || (rc = dupload(h, &d_btask, btask)) ||
-      (rc = dupload(h, &d_ubnd, ubnd)))
-    return rc;
+  if ((rc = dupload(h, &d_bcol_blk, bcol_blk)) || (rc = dupload(h, &d_bcol_loc, bcol_loc))) return rc;
   WorkDev &wd = h->wd;
   wd.nleaves = np;
-  wd.nfwg = (int)W.fwg_leaf.size();
-  wd.ntarget = (int)W.trow_glob.size();
   wd.ntile = (int)W.tile_blk.size();
-  if ((rc = dupload(h, &wd.fwg_leaf, W.fwg_leaf)) || (rc = dupload(h, &wd.fwg_first, W.fwg_first)) ||
-      (rc = dupload(h, &wd.trow_blk, W.trow_blk)) || (rc = dupload(h, &wd.trow_loc, W.trow_loc)) ||
-      (rc = dupload(h, &wd.trow_glob, W.trow_glob)) || (rc = dupload(h, &wd.tptr, W.tptr)) ||
-      (rc = dupload(h, &wd.tsrc_leaf, W.tsrc_leaf)) || (rc = dupload(h, &wd.tsrc_ri, W.tsrc_ri)) ||
-      (rc = dupload(h, &wd.tile_blk, W.tile_blk)) || (rc = dupload(h, &wd.tile_row0, W.tile_row0)) ||
+  if ((rc = dupload(h, &wd.tile_blk, W.tile_blk)) || (rc = dupload(h, &wd.tile_row0, W.tile_row0)) ||
       (rc = dupload(h, &wd.tile_ptr, W.tile_ptr)) || (rc = dupload(h, &wd.seg_leaf, W.seg_leaf)) ||
       (rc = dupload(h, &wd.seg_ri, W.seg_ri)))
     return rc;
@@ -1438,21 +1540,8 @@ int upload(snumat *h) {
   if ((rc = dupload(h, &h->d_dd, std::vector<DenseDev>{dd}))) return rc;
   for (int r = 0; r < np; r++) {
     LeafDev &D = h->h_leaves[r];
-    const Off &o = off[r];
-    D.rowptr = d_rowptr + o.rp;
-    D.diag = d_diag + o.rp;
-    D.wcol = d_wcol + o.idx;
-    D.levptr = d_levptr + o.lev;
-    D.levrows = d_levrows + o.levr;
-    D.ulevptr = d_ulevptr + o.ulev;
-    D.ulevrows = d_ulevrows + o.ulevr;
-    D.brow = d_brow + o.brow;
-    D.bcol_glob = d_bcol_glob + o.bcol;
-    D.bcol_blk = d_bcol_blk + o.bcol;
-    D.bcol_loc = d_bcol_loc + o.bcol;
-    D.ftask = d_ftask + o.task;
-    D.btask = d_btask + o.task;
-    D.ubnd = d_ubnd + o.row;
+    D.bcol_blk = d_bcol_blk + off_bcol[r];
+    D.bcol_loc = d_bcol_loc + off_bcol[r];
     D.dd = h->d_dd;
   }
   if ((rc = dalloc(h, &h->d_vec, 1)) || (rc = dalloc(h, &h->d_perm, 2)) ||
@@ -1464,14 +1553,16 @@ int upload(snumat *h) {
       return rc;
     rc = alloc_values<float>(h, S_total);
     if (!rc) {
-      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v32.S + off[r].S;
+      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v32.S + off_S[r];
       rc = build_front_plan<float>(h);
+      if (!rc) rc = build_leaf_solve<float>(h);
     }
   } else {
     rc = alloc_values<double>(h, S_total);
     if (!rc) {
-      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v64.S + off[r].S;
+      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v64.S + off_S[r];
       rc = build_front_plan<double>(h);
+      if (!rc) rc = build_leaf_solve<double>(h);
     }
   }
   if (rc) return rc;
@@ -1497,13 +1588,14 @@ size_t estimate_device_bytes(const snumat *h) {
   const int fmax = h->prec == SNU_FP32 ? front_small_max<float>() : front_small_max<double>();
   for (const LeafPlan &L : P.leaves) {
     S_total += (double)L.nbr * L.nbc;
-    idx += 2.0 * (L.core_n + 1) + L.lu_nnz + L.lev_ptr.size() + L.lev_rows.size() + L.ulev_ptr.size() +
-           L.ulev_rows.size() + L.brow.size() + 3.0 * L.bcol.size() + 2.0 * L.nbr / 4 + 4;
+    idx += 2.0 * L.bcol.size();
     // fronts: values (larger ones with their diagonal-block inverses), slot /
     // position / extend-add tables, root row / column maps, descriptors
     fronts += (double)L.fentries;
-    for (int f : L.ff) fronts += f > fmax ? 2.0 * 64 * 64 : 0.0;
+    for (size_t f = 0; f < L.ff.size(); f++) fronts += (double)front_inv_size(L.ff[f], L.fnk[f], fmax);
     idx += 2.0 * L.fslot.size() + L.frel.size() + (double)(L.nbr + L.nbc) + 16.0 * L.ff.size();
+    // solve units, children's update rows, positions of the B entries
+    idx += 34.0 * L.ff.size() + 4.0 * L.fidx.size() + L.leaf_size;
   }
   S_total += fronts;
   for (int p = 1; p < P.np; p++) inv += 2.0 * P.block_size[p] * P.block_size[p];
@@ -1573,6 +1665,11 @@ void run_launch(const Launch &L, const GemmProbT<T> *gp, const GemmSegT<T> *gs,
       if (L.wgs > 0) launch_gemv_split(vp + L.p0, L.np, vs, L.tiles, L.wgs, L.kind == 7 ? 1 : 0, part, st);
       else launch_gemv(vp + L.p0, L.np, vs, L.tiles, L.kind == 7 ? 1 : 0, st);
       break;
+    case 17:
+    case 18:
+      launch_gemv16(vp + L.p0, L.np, vs, L.tiles, L.wgs, L.gstep, L.groups, L.kind == 17 ? 1 : 0,
+                    L.part ? part : nullptr, st);
+      break;
   }
 }
 }  // namespace
@@ -1632,6 +1729,7 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
     }
     launch_front_writeback<T>(fp.d_large, fp.d_work + lv.work0, fp.d_wrange, lv.nwork, st);
   }
+  launch_front_inverse<T>(fp.d_small, fp.d_iblk, (int)fp.iblk.size(), st);
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[2], st));
   launch_front_schur<T>(fp.d_ls, fp.d_tiles, (int)fp.tiles.size(), st);
@@ -1708,26 +1806,23 @@ int run_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st,
 }
 
 template <typename T>
-void run_sweep(const SolveSet &ss, T *bp, T *cbuf, const GemvPlan<T> &plan, hipStream_t st) {
+void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st) {
   const WorkDev &wd = *ss.wd;
   launch_permute_in(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
-  launch_leaf_solve(wd.leaves, wd.nleaves, ss.vec, bp, wd.max_leaf, wd.max_lev, ss.max_rhs, false, st);
-  launch_leaf_fwd_sep(wd.leaves, wd.fwg_leaf, wd.fwg_first, wd.nfwg, 4, ss.vec, bp, cbuf, ss.cb_ld,
-                      st);
-  launch_assemble_rhs(wd.ntarget, wd.trow_glob, wd.tptr, wd.tsrc_leaf, wd.tsrc_ri, wd.leaves,
-                      ss.vec, cbuf, ss.cb_ld, bp, ss.max_rhs, st);
+  launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, false, st);
+  launch_assemble_rhs(wd.targets, wd.ntarget, wd.tsrc, ss.vec, wbuf, bp, ss.max_groups, ss.one, ss.many, st);
   for (const Launch &L : plan.fwd)
     run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, st);
   for (const Launch &L : plan.bwd)
     run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, st);
-  launch_leaf_solve(wd.leaves, wd.nleaves, ss.vec, bp, wd.max_leaf, wd.max_lev, ss.max_rhs, true, st);
+  launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, true, st);
   launch_permute_out(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
 }
 
 // FP32 factors, FP64 refinement over a set of matrices: x = sweep(b), then
 // x += sweep(b - A x) for the matrices whose backward error is above tol and
 // still at least halving per step, at most max_steps corrections each.
-int run_refined(const RefineSet &rs, float *bp, float *cbuf, const GemvPlan<float> &plan,
+int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<float> &plan,
                 hipStream_t st, int *steps_out, std::vector<double> *berr_mat) {
   const int nm = rs.nmat, ns = rs.nslots;
   std::vector<unsigned long long> u(3 * (size_t)ns);
@@ -1742,7 +1837,7 @@ int run_refined(const RefineSet &rs, float *bp, float *cbuf, const GemvPlan<floa
   int rc;
   launch_colmax(rs.ir, nm, rs.max_n, 0, rs.norms, ns, st);
   if ((rc = fetch(0, bn))) return rc;
-  run_sweep<float>(rs.sweep_b, bp, cbuf, plan, st);
+  run_sweep<float>(rs.sweep_b, bp, wbuf, plan, st);
   std::vector<double> prev(nm, INFINITY), berr(nm, INFINITY);
   std::vector<int> active(nm, 0), steps(nm, 0);
   int max_steps_taken = 0;
@@ -1769,7 +1864,7 @@ int run_refined(const RefineSet &rs, float *bp, float *cbuf, const GemvPlan<floa
     for (int m = 0; m < nm; m++)
       if (active[m]) prev[m] = berr[m], steps[m]++, max_steps_taken = std::max(max_steps_taken, steps[m]);
     HIPCHK(hipMemcpyAsync(rs.d_active, active.data(), sizeof(int) * nm, hipMemcpyHostToDevice, st));
-    run_sweep<float>(rs.sweep_r, bp, cbuf, plan, st);
+    run_sweep<float>(rs.sweep_r, bp, wbuf, plan, st);
     launch_update(rs.ir, nm, rs.max_elems, rs.d_active, st);
     HIPCHK(hipGetLastError());
   }

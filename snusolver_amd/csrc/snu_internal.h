@@ -24,12 +24,9 @@ struct LeafPlan {
   int lu_nnz = 0;
   std::vector<int> lu_rowptr, lu_colidx, lu_diag, lu_bias;
   // GPU-side views
-  std::vector<int> wcol;    // workspace column of each LU entry
   int nbr = 0, nbc = 0;     // boundary rows (non-empty L_SL) / cols (U_LS)
   std::vector<int> brow;    // core rows of the boundary rows
   std::vector<int> bcol;    // core cols of the boundary cols
-  std::vector<int> lev_ptr, lev_rows;    // factor / forward level sets
-  std::vector<int> ulev_ptr, ulev_rows;  // backward level sets
   double flops = 0;         // structural leaf flops (LU + Schur)
   // multifrontal form of the leaf factorization (build_fronts), fronts
   // ordered by their largest pivot (children before parents):

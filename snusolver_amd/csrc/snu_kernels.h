@@ -22,24 +22,39 @@ struct DenseDev {
   int nk;
 };
 
+// Solve work of the leaf fronts.  A unit is what one wave does between two
+// barriers: a whole front (orders the LDS factor kernel takes), or of a larger
+// front one 64-pivot block (forward or backward), one 64-row tile of its
+// boundary rows (forward) or one 64-pivot block's product with a chunk of its
+// boundary columns (backward).
+enum SolveUnitKind { kFwdFront = 0, kFwdPivots, kFwdRows, kBwdFront, kBwdCols, kBwdPivots };
+struct SolveUnit {
+  const void *F, *inv;       // the front (column-major), its diagonal blocks' inverses
+  int ld, nk, nb;            // front order, pivots, boundary entries B
+  int kpos;                  // solve position of the first pivot (pivots are consecutive)
+  int wrow;                  // first row of the front's update vector
+  int pull;                  // first entry of the front's rows in pull
+  int bidx;                  // first entry of B in bidx
+  int kind;
+  int row0;                  // kFwdRows: first row of the tile
+  int s, q, nq;              // pivot block; column chunk and chunks per block (kBwdCols, kBwdPivots)
+};
 // One leaf (one reference rank) of one matrix: device pointers into the
 // owning matrix's arrays, so that leaves of several matrices can share a
 // launch.
 struct LeafDev {
-  const int *rowptr, *diag, *wcol;       // LU rowptr (core_n + 1), diag, workspace column per slot
-  const int *levptr, *levrows;           // factor / forward level sets
-  const int *ulevptr, *ulevrows;         // backward level sets
-  const int *ftask, *btask;              // level-ordered row tasks {row, p0, p1, diag}, fwd / bwd
-  const int *ubnd;                       // per leaf row: first U entry on a boundary column
-  const int *brow;                       // boundary rows (core-local)
-  const int *bcol_glob, *bcol_blk, *bcol_loc;  // boundary columns: permuted index, block, offset
-  void *vals;                            // leaf LU values (value type of the launch)
+  const int *bcol_blk, *bcol_loc;        // boundary columns: block, offset
   void *S;                               // boundary Schur block, nbr x nbc row-major
   void *dense;                           // the matrix's dense separator arena
   const DenseDev *dd;                    // the matrix's separator tables
-  int core_n, leaf_size, nbr, nbc, nlev, nulev;
-  int gstart;                            // permuted index of the first leaf row
-  int cb_off;                            // rows of the rhs contribution buffer
+  const SolveUnit *units;                // the leaf's solve units, by phase
+  const int *fphase, *bphase;            // bounds of the forward / backward phases in units
+  // per front row {s0, s1}: the children's update rows to add, in order (-1:
+  // none; s1 <= -2: the list at pulllist[-2 - s1], its length first)
+  const int *pull, *pulllist;
+  const int *bidx;                       // solve positions of the fronts' B entries
+  int nfphase, nbphase;
+  int nbr, nbc;
   int vec;                               // the matrix's slot in the launch's VecDev table
   int pad;
 };
@@ -54,6 +69,9 @@ struct FrontChild {
 struct FrontDev {
   void *F;                  // the front's values (f x f, column-major)
   void *vals;               // the leaf's LU values (owned slots are read, then written)
+  void *inv;                // inverses of the pivot blocks' triangles (small: 16 x 16 blocks,
+                            // L^-1 below the diagonal, U^-1 on and above it; larger: per
+                            // 64-pivot block L^-1, then U^-1, 64 x 64 each)
   const int *slot, *pos;    // owned LU slots and their positions in F (ascending positions)
   const FrontChild *child;  // children in ascending order (their updates are added in it)
   int f, nk, nslot, nchild;
@@ -72,11 +90,24 @@ struct LeafSchurDev {
   int nbr, nbc, nroot;
 };
 
-// Segment of a packed right-hand-side buffer: columns of length n at
-// base + c ld, c < nrhs.
+// A matrix's right-hand sides in the packed solve vectors.  One column: n
+// consecutive values at base.  Several: groups of 16 columns (the last one
+// padded with zeros), each n x 16 with the columns of a row adjacent, so that
+// a row is one cache line and an MFMA operand is one contiguous load.  Update
+// vectors of the leaf fronts: wrows rows at wbase in the same form.
 struct VecDev {
-  long long base;
-  int ld, nrhs;
+  long long base, wbase;
+  int n, nrhs, wrows, pad;
+};
+constexpr int kColGroup = 16;
+__host__ __device__ inline int vec_groups(int nrhs) {
+  return nrhs <= 1 ? (nrhs > 0 ? 1 : 0) : (nrhs + kColGroup - 1) / kColGroup;
+}
+__host__ __device__ inline int vec_width(int nrhs) { return nrhs == 1 ? 1 : kColGroup; }
+// Separator row receiving leaf contributions: the update rows [s0, s1) of
+// tsrc, added in order; vec: its matrix.
+struct TargetDev {
+  int row, s0, s1, vec;
 };
 // Caller-side vectors of one matrix for the (un)permutation.
 struct PermDev {
@@ -129,8 +160,10 @@ struct DiagProbT {
   long long ldi;
   T eps;           // pivots of magnitude below eps become +-eps (0: none)
 };
-// y (M x nrhs) = / -= sum_seg A_seg (M x K) x_seg (K x nrhs); tri: 0 dense,
-// 1 lower triangular single segment (columns k <= row), 2 upper (k >= row).
+// y = / -= sum_seg A_seg (M x K) x_seg; tri: 0 dense, 1 lower triangular
+// single segment (columns k <= row), 2 upper (k >= row).  One column
+// (groups 0), or `groups` groups of 16 columns: x and y rows hold 16 adjacent
+// values, consecutive groups are ldx / ldy values apart.
 template <typename T>
 struct GemvSegT {
   const T *A, *x;
@@ -141,14 +174,14 @@ template <typename T>
 struct GemvProbT {
   T *y;
   long long ldy;
-  int M, seg0, nseg, tri, tile0, nrhs;
-  // split K: each segment in pieces of kGemvPiece columns, one workgroup per
-  // (64-row tile, piece) writing partial sums at poff; wg0 numbers the
-  // problem's first workgroup in its launch
+  int M, seg0, nseg, tri, tile0, groups;
+  // split K: each segment in pieces of kGemvPiece (16 columns: kGemvPiece16)
+  // columns of A, one workgroup per (64-row tile, piece) writing partial sums
+  // at poff; wg0 numbers the problem's first workgroup in its launch
   int parts, wg0;
   long long poff;
 };
-constexpr int kGemvPiece = 128;
+constexpr int kGemvPiece = 128, kGemvPiece16 = 256;
 using GemmSeg = GemmSegT<double>;
 using GemmProb = GemmProbT<double>;
 using DiagProb = DiagProbT<double>;
@@ -201,39 +234,39 @@ void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *
 template <typename T>
 void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
                  int total_tiles, int mode, hipStream_t st);
+// 16-column groups on MFMA; gstep groups per workgroup (1, 2 or 4); part
+// non-null: split K, max_groups the most groups of a problem.
+template <typename T>
+void launch_gemv16(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_tiles,
+                   int total_wgs, int gstep, int max_groups, int mode, T *part, hipStream_t st);
 template <typename T>
 void launch_diag_lu(const DiagProbT<T> *probs, int nprob, hipStream_t st);
-// max_elems: the largest n x nrhs of the matrices
+// Right-hand sides into / solutions out of the packed vectors; max_elems: the
+// largest n x groups of the matrices.
 template <typename T>
 void launch_permute_in(const PermDev *pd, int nmat, const VecDev *vd, T *bp,
                        long long max_elems, hipStream_t st);
 template <typename T>
 void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *bp,
                         long long max_elems, hipStream_t st);
+// Separator rows += the root fronts' update rows.
 template <typename T>
-void launch_leaf_fwd(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, hipStream_t st);
+void launch_assemble_rhs(const TargetDev *targets, int ntarget, const int *tsrc, const VecDev *vd,
+                         const T *wbuf, T *bp, int max_groups, bool one, bool many, hipStream_t st);
+// Forward / backward solve with the leaf fronts.  one / many: whether matrices
+// with one / several columns are in the launch set.
 template <typename T>
-void launch_leaf_fwd_sep(const LeafDev *leaves, const int *wg_leaf, const int *wg_first, int nwg,
-                         int waves, const VecDev *vd, const T *bp, T *cbuf, int cb_ld,
-                         hipStream_t st);
-template <typename T>
-void launch_assemble_rhs(int ntarget, const int *trow_glob, const int *tptr,
-                         const int *tsrc_leaf, const int *tsrc_ri, const LeafDev *leaves,
-                         const VecDev *vd, const T *cbuf, int cb_ld, T *bp, int max_rhs,
-                         hipStream_t st);
-template <typename T>
-void launch_leaf_bwd(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, hipStream_t st);
-// Leaf forward (bwd false) or backward solve with the solution in LDS;
-// leaves beyond the LDS fall back to launch_leaf_fwd / launch_leaf_bwd.
-template <typename T>
-void launch_leaf_solve(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, int max_leaf,
-                       int max_lev, int max_rhs, bool bwd, hipStream_t st);
+void launch_leaf_sweep(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, T *wbuf,
+                       int max_groups, bool one, bool many, bool bwd, hipStream_t st);
 
 // ---- multifrontal leaf factorization ----
 // Fronts held whole in LDS (f <= max_f): assembly, partial LU with the
 // pivot clamp, write-back of the owned slots, update block to global memory.
 template <typename T>
 void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st);
+// Inverses of their 16 x 16 diagonal blocks; blk: {front, first pivot}.
+template <typename T>
+void launch_front_inverse(const FrontDev *fr, const int2 *blk, int nblk, hipStream_t st);
 // Largest front order the LDS kernel takes for this value type.
 template <typename T>
 int front_small_max();

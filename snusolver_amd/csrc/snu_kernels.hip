@@ -1,63 +1,18 @@
-// HIP kernels for gfx950 (MI355X): leaf sparse LU, boundary Schur assembly,
-// blocked no-pivot dense LU on MFMA, and the level-scheduled solves.
+// HIP kernels for gfx950 (MI355X): boundary Schur assembly, blocked no-pivot
+// dense LU on MFMA, FP64 refinement and the factor set-up.
 //
-// Wave size 64 throughout.  The leaf kernels are bit-exact with the
-// reference's core_numfact_v2 (kernel_sparse.cu:740-781): every LU entry
-// receives the same sequence of `a - l*u` updates (ascending pivot order, no
-// FMA contraction) and the same correctly rounded divisions; the reference's
-// right-looking column sweep is evaluated here row by row (up-looking), which
-// applies the identical per-entry sequence.
+// Wave size 64 throughout.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <type_traits>
 
+#include "snu_device.h"
 #include "snu_kernels.h"
 
 #include <utility>
 
 namespace snu {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-// Pointers read from launch descriptors are generic; casting them to the
-// global address space makes the compiler emit global_load/global_store
-// (flat accesses also count against lgkmcnt, which would make every LDS wait
-// drain the global prefetch as well).
-typedef __attribute__((address_space(1))) const double gcdouble;
-typedef __attribute__((address_space(1))) double gdouble;
-__device__ __forceinline__ gcdouble *gptr(const double *p) { return (gcdouble *)p; }
-__device__ __forceinline__ gdouble *gptr(double *p) { return (gdouble *)p; }
-typedef __attribute__((address_space(1))) const float gcfloat;
-typedef __attribute__((address_space(1))) float gfloat;
-__device__ __forceinline__ gcfloat *gptr(const float *p) { return (gcfloat *)p; }
-__device__ __forceinline__ gfloat *gptr(float *p) { return (gfloat *)p; }
-
-__device__ __forceinline__ int rl(int v, int l) {
-  return __builtin_amdgcn_readlane(v, l);
-}
-__device__ __forceinline__ double rld(double v, int l) {
-  long long x = __double_as_longlong(v);
-  int lo = rl((int)(x & 0xffffffffLL), l);
-  int hi = rl((int)(x >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ float rld(float v, int l) {
-  return __int_as_float(rl(__float_as_int(v), l));
-}
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-}
-// Workgroup barrier for LDS-only communication: waits for this wave's LDS
-// (and scalar) operations, not for its global loads, which stay in flight
-// across the barrier (a __syncthreads would drain them).
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // ---------------------------------------------------------------------------
 // elementwise
@@ -192,17 +147,6 @@ __device__ __forceinline__ int xcd_remap(int bid, int nb) {
   const int x = bid & 7, i = bid >> 3;
   return ((i / kXcdChunk) * 8 + x) * kXcdChunk + (i % kXcdChunk);
 }
-// row_ror within rows of 16 lanes reads a valid lane for every lane, so the
-// destination's old value is never kept (no zeroing needed)
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  int lo = __double2loint(v), hi = __double2hiint(v);
-  lo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, false);
-  hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef double d4 __attribute__((ext_vector_type(4)));
 // DEPTH: chunks of A and B in flight in registers ahead of the chunk being
 // multiplied (1: the next chunk's loads overlap one MFMA block; 2: loads are
 // issued two chunks ahead, alternating two register stages).
@@ -795,223 +739,6 @@ void launch_gemm_variant(const GemmProbT<T> *probs, int nprob, const GemmSegT<T>
 }
 
 // ---------------------------------------------------------------------------
-// dense: grouped GEMV (the dense solves)
-// ---------------------------------------------------------------------------
-// One workgroup per 64 rows of a problem; lane = row, the 4 waves take
-// interleaved columns and are combined in LDS (fixed order: deterministic).
-// A is read once, coalesced down its columns; x through scalar loads.
-// nrhs columns are processed in groups of 16 (A is re-read per group).
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_gemv(const GemvProbT<T> *__restrict__ probs,
-                                              int nprob,
-                                              const GemvSegT<T> *__restrict__ segs) {
-  constexpr int CG = 16;  // right-hand-side columns per pass over A
-  __shared__ T red[4][CG][64];
-  const int tile = blockIdx.x;
-  int lo = 0, hi = nprob - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (probs[mid].tile0 <= tile) lo = mid;
-    else hi = mid - 1;
-  }
-  const GemvProbT<T> P = probs[lo];
-  const int nrhs = P.nrhs;
-  const int m0 = (tile - P.tile0) * 64;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m = m0 + lane, mc = min(m, P.M - 1);
-  for (int c0 = 0; c0 < nrhs; c0 += CG) {
-    const int nc = min(CG, nrhs - c0);
-    T acc[CG];
-#pragma unroll
-    for (int c = 0; c < CG; c++) acc[c] = T(0);
-    for (int sg = 0; sg < P.nseg; sg++) {
-      const GemvSegT<T> S = segs[P.seg0 + sg];
-      int kb = 0, ke = S.K;
-      if (P.tri == 1) ke = min(S.K, m0 + 64);
-      if (P.tri == 2) kb = m0;
-      auto A = gptr(S.A) + mc;
-      auto X = gptr(S.x) + (long long)c0 * S.ldx;
-      int k = kb + w;
-      // NF columns of A in flight per wave (the loads are independent of the
-      // accumulation), added in groups of four: 8 in FP64, 16 in FP32 (the
-      // same bytes in flight)
-      constexpr int NF = sizeof(T) == 4 ? 16 : 8;
-      for (; k + 4 * (NF - 1) < ke; k += 4 * NF) {
-        T a[NF];
-#pragma unroll
-        for (int j = 0; j < NF; j++) a[j] = A[(long long)(k + 4 * j) * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) {
-            auto xc = X + (long long)c * S.ldx + k;
-#pragma unroll
-            for (int j = 0; j < NF; j += 4)
-              acc[c] += a[j] * xc[4 * j] + a[j + 1] * xc[4 * j + 4] + a[j + 2] * xc[4 * j + 8] +
-                        a[j + 3] * xc[4 * j + 12];
-          }
-      }
-      for (; k + 12 < ke; k += 16) {
-        T a0 = A[(long long)k * S.lda], a1 = A[(long long)(k + 4) * S.lda];
-        T a2 = A[(long long)(k + 8) * S.lda], a3 = A[(long long)(k + 12) * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) {
-            auto xc = X + (long long)c * S.ldx;
-            acc[c] += a0 * xc[k] + a1 * xc[k + 4] + a2 * xc[k + 8] + a3 * xc[k + 12];
-          }
-      }
-      for (; k < ke; k += 4) {
-        T a0 = A[(long long)k * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) acc[c] += a0 * X[(long long)c * S.ldx + k];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CG; c++) red[w][c][lane] = acc[c];
-    __syncthreads();
-    if (w == 0 && m < P.M) {
-      for (int c = 0; c < nc; c++) {
-        T v = red[0][c][lane] + red[1][c][lane] + red[2][c][lane] + red[3][c][lane];
-        auto y = gptr(P.y) + m + (long long)(c0 + c) * P.ldy;
-        if (MODE == 1) *y = v;
-        else *y = *y - v;
-      }
-    }
-    __syncthreads();
-  }
-}
-// Split-K GEMV, pass 1: workgroup (problem, tile lt, piece) sums
-// A[rows of lt][k] x[k] over k in [piece * kGemvPiece, (piece + 1) *
-// kGemvPiece) of every segment (within the triangle for tri problems), in
-// the order of the unsplit kernel, and stores the 64 x nrhs partial block.
-// Pass 2 adds the pieces in ascending order.  The decomposition depends on
-// the problem alone, so a problem gives the same bits in any launch.
-template <typename T>
-__global__ __launch_bounds__(256) void k_gemv_part(const GemvProbT<T> *__restrict__ probs,
-                                                   int nprob,
-                                                   const GemvSegT<T> *__restrict__ segs,
-                                                   T *__restrict__ part) {
-  constexpr int CG = 16;
-  __shared__ T red[4][CG][64];
-  const int b = blockIdx.x;
-  int lo = 0, hi = nprob - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (probs[mid].wg0 <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  const GemvProbT<T> P = probs[lo];
-  const int local = b - P.wg0, lt = local / P.parts, pc = local % P.parts;
-  const int nrhs = P.nrhs;
-  const int m0 = lt * 64;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m = m0 + lane, mc = min(m, P.M - 1);
-  T *out = part + P.poff + (long long)(lt * P.parts + pc) * nrhs * 64;
-  for (int c0 = 0; c0 < nrhs; c0 += CG) {
-    const int nc = min(CG, nrhs - c0);
-    T acc[CG];
-#pragma unroll
-    for (int c = 0; c < CG; c++) acc[c] = T(0);
-    for (int sg = 0; sg < P.nseg; sg++) {
-      const GemvSegT<T> S = segs[P.seg0 + sg];
-      int kb = 0, ke = S.K;
-      if (P.tri == 1) ke = min(S.K, m0 + 64);
-      if (P.tri == 2) kb = m0;
-      kb = max(kb, pc * kGemvPiece);
-      ke = min(ke, (pc + 1) * kGemvPiece);
-      auto A = gptr(S.A) + mc;
-      auto X = gptr(S.x) + (long long)c0 * S.ldx;
-      int k = kb + w;
-      // NF columns of A in flight per wave (the loads are independent of the
-      // accumulation), added in groups of four: 8 in FP64, 16 in FP32 (the
-      // same bytes in flight)
-      constexpr int NF = sizeof(T) == 4 ? 16 : 8;
-      for (; k + 4 * (NF - 1) < ke; k += 4 * NF) {
-        T a[NF];
-#pragma unroll
-        for (int j = 0; j < NF; j++) a[j] = A[(long long)(k + 4 * j) * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) {
-            auto xc = X + (long long)c * S.ldx + k;
-#pragma unroll
-            for (int j = 0; j < NF; j += 4)
-              acc[c] += a[j] * xc[4 * j] + a[j + 1] * xc[4 * j + 4] + a[j + 2] * xc[4 * j + 8] +
-                        a[j + 3] * xc[4 * j + 12];
-          }
-      }
-      for (; k + 12 < ke; k += 16) {
-        T a0 = A[(long long)k * S.lda], a1 = A[(long long)(k + 4) * S.lda];
-        T a2 = A[(long long)(k + 8) * S.lda], a3 = A[(long long)(k + 12) * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) {
-            auto xc = X + (long long)c * S.ldx;
-            acc[c] += a0 * xc[k] + a1 * xc[k + 4] + a2 * xc[k + 8] + a3 * xc[k + 12];
-          }
-      }
-      for (; k < ke; k += 4) {
-        T a0 = A[(long long)k * S.lda];
-#pragma unroll
-        for (int c = 0; c < CG; c++)
-          if (c < nc) acc[c] += a0 * X[(long long)c * S.ldx + k];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CG; c++) red[w][c][lane] = acc[c];
-    __syncthreads();
-    if (w == 0)
-      for (int c = 0; c < nc; c++)
-        out[(c0 + c) * 64 + lane] = red[0][c][lane] + red[1][c][lane] + red[2][c][lane] + red[3][c][lane];
-    __syncthreads();
-  }
-}
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_gemv_sum(const GemvProbT<T> *__restrict__ probs, int nprob,
-                                                  const T *__restrict__ part) {
-  const int tile = blockIdx.x;
-  int lo = 0, hi = nprob - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (probs[mid].tile0 <= tile) lo = mid;
-    else hi = mid - 1;
-  }
-  const GemvProbT<T> P = probs[lo];
-  const int lt = tile - P.tile0, m = lt * 64 + (threadIdx.x & 63);
-  if (m >= P.M) return;
-  const T *in = part + P.poff + (long long)lt * P.parts * P.nrhs * 64 + (threadIdx.x & 63);
-  for (int c = threadIdx.x >> 6; c < P.nrhs; c += 4) {
-    T v = in[c * 64];
-    for (int pc = 1; pc < P.parts; pc++) v += in[((long long)pc * P.nrhs + c) * 64];
-    auto y = gptr(P.y) + m + (long long)c * P.ldy;
-    if (MODE == 1) *y = v;
-    else *y = *y - v;
-  }
-}
-template <typename T>
-void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
-                       int total_tiles, int total_wgs, int mode, T *part, hipStream_t st) {
-  if (total_tiles <= 0 || nprob <= 0) return;
-  hipLaunchKernelGGL(k_gemv_part<T>, dim3(total_wgs), dim3(256), 0, st, probs, nprob, segs, part);
-  if (mode == 1)
-    hipLaunchKernelGGL((k_gemv_sum<T, 1>), dim3(total_tiles), dim3(256), 0, st, probs, nprob, part);
-  else
-    hipLaunchKernelGGL((k_gemv_sum<T, 0>), dim3(total_tiles), dim3(256), 0, st, probs, nprob, part);
-}
-template <typename T>
-void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
-                 int total_tiles, int mode, hipStream_t st) {
-  if (total_tiles <= 0 || nprob <= 0) return;
-  if (mode == 1)
-    hipLaunchKernelGGL((k_gemv<T, 1>), dim3(total_tiles), dim3(256), 0, st, probs, nprob, segs);
-  else
-    hipLaunchKernelGGL((k_gemv<T, 0>), dim3(total_tiles), dim3(256), 0, st, probs, nprob, segs);
-}
-
-// ---------------------------------------------------------------------------
 // dense: diagonal block LU (no pivoting, as cusolverDnDgetrf with a null
 // ipiv / LAPACKE_mkl_dgetrfnp) and the inverses of its triangular factors.
 // ---------------------------------------------------------------------------
@@ -1034,16 +761,6 @@ void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
 // of, at or right of J is a compile-time fact for most (J, q) and a uniform
 // select for the rest; runtime steps make the compiler shuffle the register
 // arrays between branches).
-template <typename T>
-__device__ __forceinline__ T lane_value(T v, int lane) {
-  if constexpr (std::is_same<T, double>::value) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-    return __hiloint2double(hi, lo);
-  } else {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-  }
-}
 template <typename T, int J>
 __device__ __forceinline__ void diag_step(T (&x)[8], T (&xl)[8], T (&xu)[8], int r, int g,
                                           T (*lb)[64], T (*yb)[64], T eps) {
@@ -1056,8 +773,8 @@ __device__ __forceinline__ void diag_step(T (&x)[8], T (&xl)[8], T (&xu)[8], int
   T uq[8], xq[8];
 #pragma unroll
   for (int q = 0; q < 8; q++) {
-    if (8 * q + 7 > J) uq[q] = lane_value(x[q], J);
-    if (8 * q <= J) xq[q] = lane_value(xl[q], J);
+    if (8 * q + 7 > J) uq[q] = rld(x[q], J);
+    if (8 * q <= J) xq[q] = rld(xl[q], J);
   }
   __syncthreads();
   // keep the scheduler from interleaving steps (register pressure)
@@ -1136,402 +853,6 @@ template <typename T>
 void launch_diag_lu(const DiagProbT<T> *probs, int nprob, hipStream_t st) {
   if (nprob <= 0) return;
   hipLaunchKernelGGL(k_diag_lu<T>, dim3(nprob), dim3(512), 0, st, probs);
-}
-
-// ---------------------------------------------------------------------------
-// solve: permutation, leaf triangular solves, boundary rhs assembly
-// ---------------------------------------------------------------------------
-// One matrix per blockIdx.y: bp[vbase + order[r] + col ld] = b[r + col ldb].
-template <typename T>
-__global__ void k_permute_in(const PermDev *__restrict__ pd, const VecDev *__restrict__ vd,
-                             T *bp) {
-  const PermDev P = pd[blockIdx.y];
-  const VecDev V = vd[P.vec];
-  const long long tot = (long long)P.n * V.nrhs;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int col = (int)(i / P.n), r = (int)(i % P.n);
-    bp[V.base + P.order[r] + (long long)col * V.ld] = (T)P.b[r + col * P.ldb];
-  }
-}
-template <typename T>
-__global__ void k_permute_out(const PermDev *__restrict__ pd, const VecDev *__restrict__ vd,
-                              const T *bp) {
-  const PermDev P = pd[blockIdx.y];
-  const VecDev V = vd[P.vec];
-  const long long tot = (long long)P.n * V.nrhs;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int col = (int)(i / P.n), r = (int)(i % P.n);
-    P.x[r + col * P.ldx] = (double)bp[V.base + P.order[r] + (long long)col * V.ld];
-  }
-}
-static unsigned perm_blocks(long long max_elems) {
-  long long b = (max_elems + 255) / 256;
-  return (unsigned)std::max(1LL, std::min(b, 2048LL));
-}
-template <typename T>
-void launch_permute_in(const PermDev *pd, int nmat, const VecDev *vd, T *bp,
-                       long long max_elems, hipStream_t st) {
-  if (nmat <= 0 || max_elems <= 0) return;
-  hipLaunchKernelGGL(k_permute_in<T>, dim3(perm_blocks(max_elems), nmat), dim3(256), 0, st, pd,
-                     vd, bp);
-}
-template <typename T>
-void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *bp,
-                        long long max_elems, hipStream_t st) {
-  if (nmat <= 0 || max_elems <= 0) return;
-  hipLaunchKernelGGL(k_permute_out<T>, dim3(perm_blocks(max_elems), nmat), dim3(256), 0, st,
-                     pd, vd, bp);
-}
-
-// Sparse dot products of the leaf solves with several right-hand sides: a
-// wave serves CW = the largest power of two <= min(nrhs, 16) columns at once,
-// KL = 64 / CW lanes per column striding over the row's entries, partial
-// sums combined within the KL lanes.  CW = 1 (one rhs) is the plain wave
-// reduction.  The rounding of a column's sum depends on CW, i.e. on nrhs.
-__device__ __forceinline__ int col_width(int nrhs) {
-  const int m = min(nrhs, 16);
-  return 1 << (31 - __clz(max(m, 1)));
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-template <int CTRL, typename T>
-__device__ __forceinline__ T dpp_v(T v) {
-  if constexpr (sizeof(T) == 8) return dpp_d<CTRL>(v);
-  else return dpp_f<CTRL>(v);
-}
-// Sum over each group of kl consecutive lanes (kl a power of two <= 64),
-// valid in the group's first lane: DPP within rows of 16 lanes (quad
-// butterflies, then rotations that bring lanes +4 and +8 of a row to its
-// front), read-lane sums across rows.
-template <typename T>
-__device__ __forceinline__ T group_sum(T v, int kl) {
-  if (kl >= 2) v += dpp_v<0xB1>(v);   // quad_perm 1,0,3,2
-  if (kl >= 4) v += dpp_v<0x4E>(v);   // quad_perm 2,3,0,1
-  if (kl >= 8) v += dpp_v<0x12C>(v);  // row_ror:12: lane i <- lane i + 4
-  if (kl >= 16) v += dpp_v<0x128>(v); // row_ror:8: lane i <- lane i + 8
-  if (kl == 32) {
-    const T lo = rld(v, 0) + rld(v, 16), hi = rld(v, 32) + rld(v, 48);
-    v = (threadIdx.x & 63) < 32 ? lo : hi;
-  } else if (kl == 64) {
-    v = (rld(v, 0) + rld(v, 16)) + (rld(v, 32) + rld(v, 48));
-  }
-  return v;
-}
-
-// y_L = L_LL^-1 b_L (unit lower), level by level; the (row, column group)
-// pairs of a level are spread over the waves.
-template <typename T>
-__global__ __launch_bounds__(256) void k_leaf_fwd(const LeafDev *__restrict__ leaves,
-                                                  const VecDev *__restrict__ vd, T *bp) {
-  const LeafDev L = leaves[blockIdx.x];
-  const VecDev V = vd[L.vec];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int W = blockDim.x >> 6;
-  const int *rp = L.rowptr, *dg = L.diag, *wc = L.wcol;
-  const T *v = (const T *)L.vals;
-  const int *lp = L.levptr, *lr = L.levrows;
-  const int cw = col_width(V.nrhs), kl = 64 / cw, ng = (V.nrhs + cw - 1) / cw;
-  const int sub = lane % kl, cl = lane / kl;
-  for (int lev = 0; lev < L.nlev; lev++) {
-    const int r0 = lp[lev], nr = lp[lev + 1] - r0;
-    for (int t = wave; t < nr * ng; t += W) {
-      const int i = lr[r0 + t % nr], col = (t / nr) * cw + cl;
-      const bool on = col < V.nrhs;
-      T *b = bp + V.base + (long long)min(col, V.nrhs - 1) * V.ld + L.gstart;
-      T s = T(0);
-      for (int p = rp[i] + sub; p < dg[i]; p += kl) s += v[p] * b[wc[p]];
-      s = group_sum(s, kl);
-      if (on && sub == 0) b[i] -= s;
-    }
-    __syncthreads();
-  }
-}
-template <typename T>
-void launch_leaf_fwd(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, hipStream_t st) {
-  if (nleaves <= 0) return;
-  hipLaunchKernelGGL(k_leaf_fwd<T>, dim3(nleaves), dim3(256), 0, st, leaves, vd, bp);
-}
-
-// Boundary rows: cbuf[ri] = sum_k L_SL(r, k) y_k (kernel_sparse.cu:935-944).
-template <typename T>
-__global__ __launch_bounds__(256) void k_leaf_fwd_sep(const LeafDev *__restrict__ leaves,
-                                                      const int *__restrict__ wg_leaf,
-                                                      const int *__restrict__ wg_first,
-                                                      const VecDev *__restrict__ vd,
-                                                      const T *__restrict__ bp,
-                                                      T *__restrict__ cbuf, int cb_ld) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const LeafDev L = leaves[wg_leaf[blockIdx.x]];
-  const VecDev V = vd[L.vec];
-  const int ri = wg_first[blockIdx.x] + wave;
-  if (ri >= L.nbr) return;
-  const int r = L.brow[ri];
-  const int *rp = L.rowptr, *wc = L.wcol;
-  const T *v = (const T *)L.vals;
-  const int cw = col_width(V.nrhs), kl = 64 / cw;
-  const int sub = lane % kl, cl = lane / kl;
-  for (int c0 = 0; c0 < V.nrhs; c0 += cw) {
-    const int col = c0 + cl;
-    const bool on = col < V.nrhs;
-    const T *b = bp + V.base + (long long)min(col, V.nrhs - 1) * V.ld + L.gstart;
-    T s = T(0);
-    for (int p = rp[r] + sub; p < rp[r + 1]; p += kl) s += v[p] * b[wc[p]];
-    s = group_sum(s, kl);
-    if (on && sub == 0) cbuf[L.cb_off + ri + (long long)col * cb_ld] = s;
-  }
-}
-template <typename T>
-void launch_leaf_fwd_sep(const LeafDev *leaves, const int *wg_leaf, const int *wg_first, int nwg,
-                         int waves, const VecDev *vd, const T *bp, T *cbuf, int cb_ld,
-                         hipStream_t st) {
-  if (nwg <= 0) return;
-  hipLaunchKernelGGL(k_leaf_fwd_sep<T>, dim3(nwg), dim3(64 * waves), 0, st, leaves, wg_leaf,
-                     wg_first, vd, bp, cbuf, cb_ld);
-}
-
-// b_R -= contributions of the leaves touching row R, in ascending rank
-// (one thread per target row and rhs column; the target's matrix is that of
-// its sources).
-template <typename T>
-__global__ void k_assemble_rhs(int ntarget, const int *__restrict__ trow_glob,
-                               const int *__restrict__ tptr,
-                               const int *__restrict__ tsrc_leaf,
-                               const int *__restrict__ tsrc_ri,
-                               const LeafDev *__restrict__ leaves,
-                               const VecDev *__restrict__ vd,
-                               const T *__restrict__ cbuf, int cb_ld, T *bp, int max_rhs) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)ntarget * max_rhs) return;
-  const int t = (int)(i % ntarget), col = (int)(i / ntarget);
-  const VecDev V = vd[leaves[tsrc_leaf[tptr[t]]].vec];
-  if (col >= V.nrhs) return;
-  T *b = bp + V.base + (long long)col * V.ld + trow_glob[t];
-  T acc = *b;
-  for (int s = tptr[t]; s < tptr[t + 1]; s++)
-    acc -= cbuf[leaves[tsrc_leaf[s]].cb_off + tsrc_ri[s] + (long long)col * cb_ld];
-  *b = acc;
-}
-template <typename T>
-void launch_assemble_rhs(int ntarget, const int *trow_glob, const int *tptr,
-                         const int *tsrc_leaf, const int *tsrc_ri, const LeafDev *leaves,
-                         const VecDev *vd, const T *cbuf, int cb_ld, T *bp, int max_rhs,
-                         hipStream_t st) {
-  long long tot = (long long)ntarget * max_rhs;
-  if (tot <= 0) return;
-  hipLaunchKernelGGL(k_assemble_rhs<T>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st,
-                     ntarget, trow_glob, tptr, tsrc_leaf, tsrc_ri, leaves, vd, cbuf, cb_ld, bp,
-                     max_rhs);
-}
-
-// x_L = U_LL^-1 (y_L - U_LS x_S), level by level (SnuMat_factorize.cu:331-344);
-// the (row, rhs column) pairs of a level are spread over the waves.
-template <typename T>
-__global__ __launch_bounds__(256) void k_leaf_bwd(const LeafDev *__restrict__ leaves,
-                                                  const VecDev *__restrict__ vd, T *bp) {
-  const LeafDev L = leaves[blockIdx.x];
-  const VecDev V = vd[L.vec];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int W = blockDim.x >> 6;
-  const int ls = L.leaf_size;
-  const int *rp = L.rowptr, *dg = L.diag, *wc = L.wcol, *bg = L.bcol_glob;
-  const T *v = (const T *)L.vals;
-  const int *lp = L.ulevptr, *lr = L.ulevrows;
-  const int cw = col_width(V.nrhs), kl = 64 / cw, ng = (V.nrhs + cw - 1) / cw;
-  const int sub = lane % kl, cl = lane / kl;
-  for (int lev = 0; lev < L.nulev; lev++) {
-    const int r0 = lp[lev], nr = lp[lev + 1] - r0;
-    for (int t = wave; t < nr * ng; t += W) {
-      const int i = lr[r0 + t % nr], col = (t / nr) * cw + cl;
-      const bool on = col < V.nrhs;
-      T *b = bp + V.base + (long long)min(col, V.nrhs - 1) * V.ld;
-      T s = T(0);
-      for (int p = dg[i] + 1 + sub; p < rp[i + 1]; p += kl) {
-        int c = wc[p];
-        long long g = c < ls ? (long long)L.gstart + c : (long long)bg[c - ls];
-        s += v[p] * b[g];
-      }
-      s = group_sum(s, kl);
-      if (on && sub == 0) b[L.gstart + i] = (b[L.gstart + i] - s) / v[dg[i]];
-    }
-    __syncthreads();
-  }
-}
-template <typename T>
-void launch_leaf_bwd(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, hipStream_t st) {
-  if (nleaves <= 0) return;
-  hipLaunchKernelGGL(k_leaf_bwd<T>, dim3(nleaves), dim3(256), 0, st, leaves, vd, bp);
-}
-
-// Leaf triangular solves with the leaf's solution segment in LDS (used when
-// every leaf of the launch is resident at once): the
-// level offsets and the level-ordered row tasks {row, first entry, end,
-// diagonal} are staged in LDS once, then per level every (row, column) task
-// gathers from LDS, so a level costs one round of entry loads instead of a
-// dependent chain of index, entry and vector loads.  Backward: the boundary
-// part of every U row (entries on separator columns, whose x is final) is
-// subtracted for all rows at once before the sweep, which then reads only
-// leaf columns.  Columns go in batches of cmax.
-// LDS: [level offsets | tasks at task_off | cmax x ls values at xs_off].
-// Threads per leaf: the waves take a level's rows in turn.
-extern __shared__ __align__(16) char lds_raw[];
-constexpr int kLeafSolveThreads = 1024;
-template <typename T, bool BWD>
-__global__ __launch_bounds__(kLeafSolveThreads) void k_leaf_solve(const LeafDev *__restrict__ leaves,
-                                                    const VecDev *__restrict__ vd, T *bp,
-                                                    int cmax, int task_off, int xs_off) {
-  const LeafDev L = leaves[blockIdx.x];
-  const VecDev V = vd[L.vec];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, W = blockDim.x >> 6;
-  const int ls = L.leaf_size, nlev = BWD ? L.nulev : L.nlev;
-  int *lps = (int *)lds_raw;
-  int4 *tq = (int4 *)(lds_raw + task_off);
-  T *xs = (T *)(lds_raw + xs_off);
-  const int *lp = BWD ? L.ulevptr : L.levptr;
-  const int4 *tk = (const int4 *)(BWD ? L.btask : L.ftask);
-  for (int e = tid; e <= nlev; e += blockDim.x) lps[e] = lp[e];
-  for (int e = tid; e < ls; e += blockDim.x) tq[e] = tk[e];
-  const T *v = (const T *)L.vals;
-  const int *wc = L.wcol;
-  for (int c0 = 0; c0 < V.nrhs; c0 += cmax) {
-    const int nc = min(cmax, V.nrhs - c0);
-    __syncthreads();
-    for (int e = tid; e < nc * ls; e += blockDim.x) {
-      const int c = e / ls, i = e - c * ls;
-      xs[e] = bp[V.base + (long long)(c0 + c) * V.ld + L.gstart + i];
-    }
-    __syncthreads();
-    const int cw = col_width(nc), kl = 64 / cw, ng = (nc + cw - 1) / cw;
-    const int sub = lane % kl, cl = lane / kl;
-    if (BWD) {
-      for (int t = wave; t < ls * ng; t += W) {
-        const int i = t % ls, col = (t / ls) * cw + cl, cc = min(col, nc - 1);
-        const T *b = bp + V.base + (long long)(c0 + cc) * V.ld;
-        T s = T(0);
-        const int pe = L.rowptr[i + 1];
-        for (int p = L.ubnd[i] + sub; p < pe; p += 8 * kl) {
-          // eight chunks of loads in flight (clamped addresses, masked use)
-          T vv[8];
-          int gg[8];
-#pragma unroll
-          for (int j = 0; j < 8; j++) {
-            const int pc = min(p + j * kl, pe - 1);
-            vv[j] = v[pc];
-            gg[j] = L.bcol_glob[wc[pc] - ls];
-          }
-#pragma unroll
-          for (int j = 0; j < 8; j++)
-            if (p + j * kl < pe) s += vv[j] * b[gg[j]];
-        }
-        s = group_sum(s, kl);
-        if (col < nc && sub == 0) xs[cc * ls + i] -= s;
-      }
-      __syncthreads();
-    }
-    // the first chunk of each wave's first task of the next level is loaded
-    // while the current level is solved
-    auto first_chunk = [&](int lev, T &pv, int &pw) {
-      pv = T(0);
-      pw = 0;
-      if (lev >= nlev) return;
-      const int r0 = lps[lev], nr = lps[lev + 1] - r0;
-      if (wave >= nr * ng) return;
-      const int4 q = tq[r0 + wave % nr];
-      const int p = q.y + sub;
-      if (p < q.z) pv = v[p], pw = wc[p];
-    };
-    // one level; (cv, cwi) hold this level's first chunk, (nv, nw) receive
-    // the next level's (two register sets alternate: no copy waits on loads)
-    auto level = [&](int lev, T cv, int cwi, T &nv, int &nw) {
-      const int r0 = lps[lev], nr = lps[lev + 1] - r0;
-      first_chunk(lev + 1, nv, nw);
-      for (int t = wave; t < nr * ng; t += W) {
-        const int4 q = tq[r0 + t % nr];
-        const int col = (t / nr) * cw + cl, cc = min(col, nc - 1);
-        const T *x = xs + cc * ls;
-        T s = T(0);
-        int p = q.y + sub;
-        if (t == wave) {  // first chunk already in registers
-          if (p < q.z) s = cv * x[cwi];
-          p += kl;
-        }
-        for (; p < q.z; p += 8 * kl) {
-          // eight chunks of loads in flight (clamped addresses, masked use)
-          T vv[8];
-          int ww[8];
-#pragma unroll
-          for (int j = 0; j < 8; j++) {
-            const int pc = min(p + j * kl, q.z - 1);
-            vv[j] = v[pc];
-            ww[j] = wc[pc];
-          }
-#pragma unroll
-          for (int j = 0; j < 8; j++)
-            if (p + j * kl < q.z) s += vv[j] * x[ww[j]];
-        }
-        s = group_sum(s, kl);
-        if (col < nc && sub == 0) {
-          T *xi = xs + cc * ls + q.x;
-          if (BWD) *xi = (*xi - s) / v[q.w];
-          else *xi -= s;
-        }
-      }
-      lds_barrier();
-    };
-    T va, vb;
-    int wa, wb;
-    first_chunk(0, va, wa);
-    for (int lev = 0; lev < nlev; lev += 2) {
-      level(lev, va, wa, vb, wb);
-      if (lev + 1 < nlev) level(lev + 1, vb, wb, va, wa);
-    }
-    for (int e = tid; e < nc * ls; e += blockDim.x) {
-      const int c = e / ls, i = e - c * ls;
-      bp[V.base + (long long)(c0 + c) * V.ld + L.gstart + i] = xs[e];
-    }
-  }
-}
-template <typename T>
-void launch_leaf_solve(const LeafDev *leaves, int nleaves, const VecDev *vd, T *bp, int max_leaf,
-                       int max_lev, int max_rhs, bool bwd, hipStream_t st) {
-  if (nleaves <= 0) return;
-  constexpr int kLds = 160 * 1024;
-  const int task_off = ((max_lev + 1) * 4 + 15) & ~15;
-  const int xs_off = task_off + max_leaf * 16;
-  const int col_bytes = max_leaf * (int)sizeof(T);
-  if (xs_off + col_bytes > kLds || max_rhs < 1) {  // leaves too large for LDS
-    if (bwd) launch_leaf_bwd(leaves, nleaves, vd, bp, st);
-    else launch_leaf_fwd(leaves, nleaves, vd, bp, st);
-    return;
-  }
-  const int cmax = std::max(1, std::min(std::min(max_rhs, 16), (kLds - xs_off) / std::max(col_bytes, 1)));
-  const size_t lds = (size_t)xs_off + (size_t)cmax * col_bytes;
-  // many leaves (batches): the LDS sized for the largest would leave most
-  // of them waiting for a CU; the global-memory kernels keep them resident.
-  // That pays for single-column FP64 sweeps only (512-matrix batch: 4.50 ms
-  // against 4.67 with the LDS kernel); FP32 sweeps (13.5 against 14.2 ms)
-  // and several columns (96^3 over 512 leaves, 16 columns: 34.7 against 55.2
-  // ms) are faster queued on the LDS kernel
-  const void *kern = bwd ? (const void *)k_leaf_solve<T, true> : (const void *)k_leaf_solve<T, false>;
-  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  int dev = 0, cus = 0, per_cu = 0;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kLeafSolveThreads, lds);
-  if (sizeof(T) == 8 && max_rhs == 1 && (long long)nleaves > (long long)cus * std::max(per_cu, 1)) {
-    if (bwd) launch_leaf_bwd(leaves, nleaves, vd, bp, st);
-    else launch_leaf_fwd(leaves, nleaves, vd, bp, st);
-    return;
-  }
-  if (bwd)
-    hipLaunchKernelGGL((k_leaf_solve<T, true>), dim3(nleaves), dim3(kLeafSolveThreads), lds, st, leaves, vd, bp,
-                       cmax, task_off, xs_off);
-  else
-    hipLaunchKernelGGL((k_leaf_solve<T, false>), dim3(nleaves), dim3(kLeafSolveThreads), lds, st, leaves, vd, bp,
-                       cmax, task_off, xs_off);
 }
 
 // ---------------------------------------------------------------------------
@@ -1717,24 +1038,7 @@ int device_lds_limit() {
                                   hipStream_t);                                               \
   template void launch_gemm_variant<T>(const GemmProbT<T> *, int, const GemmSegT<T> *, int,  \
                                        int, int, int, hipStream_t);                           \
-  template void launch_gemv_split<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int,  \
-                                     int, T *, hipStream_t);                                    \
-  template void launch_gemv<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int,     \
-                               hipStream_t);                                                  \
-  template void launch_diag_lu<T>(const DiagProbT<T> *, int, hipStream_t);                   \
-  template void launch_permute_in<T>(const PermDev *, int, const VecDev *, T *, long long,    \
-                                     hipStream_t);                                            \
-  template void launch_permute_out<T>(const PermDev *, int, const VecDev *, const T *,        \
-                                      long long, hipStream_t);                                \
-  template void launch_leaf_fwd<T>(const LeafDev *, int, const VecDev *, T *, hipStream_t);   \
-  template void launch_leaf_fwd_sep<T>(const LeafDev *, const int *, const int *, int, int,   \
-                                       const VecDev *, const T *, T *, int, hipStream_t);     \
-  template void launch_assemble_rhs<T>(int, const int *, const int *, const int *,            \
-                                       const int *, const LeafDev *, const VecDev *,          \
-                                       const T *, int, T *, int, hipStream_t);                \
-  template void launch_leaf_bwd<T>(const LeafDev *, int, const VecDev *, T *, hipStream_t);   \
-  template void launch_leaf_solve<T>(const LeafDev *, int, const VecDev *, T *, int, int, int,  \
-                                     bool, hipStream_t);
+  template void launch_diag_lu<T>(const DiagProbT<T> *, int, hipStream_t);
 SNU_INSTANTIATE(double)
 SNU_INSTANTIATE(float)
 #undef SNU_INSTANTIATE

@@ -1,0 +1,90 @@
+"""The solve sweeps over the leaf fronts and the 16-column dense products
+against a dense FP64 solve (numpy), through the C-ABI.
+
+Column counts sit at the edges of the column groups (1; 2, 15, 16, 17; 33, 64,
+65).  The matrices put fronts on both sides of the LDS order, with pivot counts
+around multiples of 16 and 64 (a one-leaf 27-point cube has pivot blocks beyond
+64; a one-leaf 2D grid has only small fronts), one leaf and several, and
+separators of a few rows.  Bars: those of the path, x within 1e-9 and backward
+error <= 1e-12.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [((9, 9, 9), 27, 1), ((13, 7, 5), 7, 2), ((31, 23, 1), 9, 4), ((17, 16, 1), 5, 1), ((11, 10, 8), 27, 8)]
+DIAG = {5: 4.1, 9: 8.1, 7: 6.1, 27: 0.0}
+
+
+def _matrix(S, dims, stencil, seed):
+    return S.gen_grid(*dims, stencil, 1 if stencil == 27 else 0, DIAG[stencil], seed)
+
+
+def _dense(A):
+    D = np.zeros((A.n, A.n))
+    D[np.repeat(np.arange(A.n), np.diff(A.rowptr)), A.colidx] = A.data
+    return D
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims,stencil,np_", GRIDS)
+def test_column_counts_vs_dense(S, precision, dims, stencil, np_):
+    A = _matrix(S, dims, stencil, 3)
+    rng = np.random.default_rng(5)
+    B = np.asfortranarray(rng.standard_normal((A.n, 65)))
+    X = np.linalg.solve(_dense(A), B)
+    with S.SnuMat(A, np_, grid=dims, device=0, precision=precision, ir_tol=1e-12) as M:
+        M.factorize()
+        for k in (1, 2, 15, 16, 17, 33, 64, 65, 1):
+            print("case", precision, dims, "columns", k, flush=True)
+            x = M.solve(B[:, :k])
+            assert np.max(np.abs(x - X[:, :k])) <= 1e-9 * np.max(np.abs(X[:, :k]))
+            assert S.backward_error(A, x, B[:, :k]) <= 1e-12
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_batch_of_uneven_columns_bitwise(S, precision):
+    """One launch set with one-column, many-column and skipped members: each
+    answer equals the member's own solve bit for bit."""
+    mats, bs = [], []
+    rng = np.random.default_rng(6)
+    for (dims, stencil, np_), k in zip(GRIDS, (1, 17, 0, 16, 3)):
+        A = _matrix(S, dims, stencil, 4)
+        mats.append(S.SnuMat(A, np_, grid=dims, device=0, precision=precision, ir_tol=1e-12))
+        bs.append(rng.standard_normal((A.n, k)) if k else None)
+    with S.Batch(mats) as batch:
+        batch.factorize()
+        for M, b, x in zip(mats, bs, batch.solve(bs)):
+            if b is not None:
+                print("case", precision, M.A.n, "columns", b.shape[1], flush=True)
+                assert np.array_equal(x, M.solve(b))
+    for M in mats:
+        M.close()
+
+
+def test_scratch_solve_column_by_column(S):
+    """A scratch call whose padded column groups do not fit runs its columns
+    one at a time: same answers as the allocating solve's single columns, and
+    the same size refused as before (16 n nrhs bytes)."""
+    A = S.gen_grid(1024, 1024, 1, 5, 0, 4.1, 2)
+    k = 2  # two columns pad to 16: 2 x 8 B x 16 n = 256 MiB and the update rows
+    rng = np.random.default_rng(7)
+    B = np.asfortranarray(rng.standard_normal((A.n, k)))
+    with S.SnuMat(A, 512, grid=(1024, 1024, 1), device=0) as M:
+        M.factorize()
+        d_b, d_x = S.DeviceBuffer(8 * A.n * k), S.DeviceBuffer(8 * A.n * k)
+        try:
+            d_b.upload(B)
+            M.solve_device_scratch_ptr(d_b.ptr.value, d_x.ptr.value, k)
+            x = np.zeros((A.n, k), order="F")
+            d_x.download(x)
+            for c in range(k):
+                assert np.array_equal(x[:, c], M.solve(B[:, c]))
+            rc = S.lib().snumat_solve_device_scratch(M._h, d_b.ptr, d_x.ptr, 17, A.n)
+            assert rc == -1 and b"scratch" in S.lib().snu_last_error()
+        finally:
+            d_b.free()
+            d_x.free()
