@@ -73,17 +73,12 @@ int ensure_rhs(snumat *h, int nrhs) {
     return SNU_OK;
   };
   drop_alloc(h, h->d_bx);
-  drop_alloc(h, h->d_r);
-  drop_alloc(h, h->d_dx);
   drop_alloc(h, h->d_colnorms);
-  h->d_bx = h->d_r = h->d_dx = nullptr;
+  h->d_bx = nullptr;
   h->d_colnorms = nullptr;
   if ((rc = h->prec == SNU_FP32 ? vec(h->v32) : vec(h->v64))) return rc;
   if ((rc = halloc(h, &h->d_bx, n * nrhs * 2))) return rc;
-  if (h->prec == SNU_FP32 &&
-      ((rc = halloc(h, &h->d_r, n * nrhs)) || (rc = halloc(h, &h->d_dx, n * nrhs)) ||
-       (rc = halloc(h, &h->d_colnorms, 3 * (size_t)nrhs))))
-    return rc;
+  if (h->prec == SNU_FP32 && (rc = halloc(h, &h->d_colnorms, norm_values(1, h->P.n, nrhs)))) return rc;
   h->nrhs_cap = nrhs;
   return SNU_OK;
 }
@@ -107,12 +102,9 @@ IrDev ir_entry(snumat *h, const double *b, long long ldb, double *x, long long l
   e.val = h->d_aval;
   e.b = b;
   e.x = x;
-  e.r = h->d_r;
-  e.dx = h->d_dx;
+  e.order = h->d_order;
   e.ldb = ldb;
   e.ldx = ldx;
-  e.ldr = h->P.n;
-  e.lddx = h->P.n;
   e.n = h->P.n;
   e.nrhs = nrhs;
   e.norm0 = 0;
@@ -411,12 +403,9 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
   h->t[15] = 0;
   const int n = h->P.n;
   VecDev vd{0, 0, n, nrhs, h->wrows, 0};
-  PermDev pd[2];
-  std::memset(pd, 0, sizeof(pd));
-  pd[0] = PermDev{h->d_order, d_b, d_x, ldb, ldx, n, 0};
-  pd[1] = PermDev{h->d_order, B.r, B.dx, (long long)n, (long long)n, n, 0};
+  const PermDev pd{h->d_order, d_b, d_x, ldb, ldx, n, 0};
   HIPCHK(hipMemcpyAsync(h->d_vec, &vd, sizeof(vd), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(h->d_perm, pd, sizeof(pd), hipMemcpyHostToDevice, st));
+  HIPCHK(hipMemcpyAsync(h->d_perm, &pd, sizeof(pd), hipMemcpyHostToDevice, st));
   SolveSet ss;
   ss.perm = h->d_perm;
   ss.vec = h->d_vec;
@@ -432,17 +421,12 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
     std::vector<int> slot_mat(nrhs, 0);
     std::vector<double> anorm{h->anorm};
     IrDev e = ir_entry(h, d_b, ldb, d_x, ldx, nrhs);
-    e.r = B.r;
-    e.dx = B.dx;
     HIPCHK(hipMemcpyAsync(h->d_ir, &e, sizeof(e), hipMemcpyHostToDevice, st));
     RefineSet rs;
-    rs.sweep_b = ss;
-    rs.sweep_r = ss;
-    rs.sweep_r.perm = h->d_perm + 1;
+    rs.sweep = ss;
     rs.ir = h->d_ir;
     rs.nmat = 1;
     rs.max_n = n;
-    rs.max_elems = (long long)n * nrhs;
     rs.norms = B.colnorms;
     rs.nslots = nrhs;
     rs.slot_mat = &slot_mat;
@@ -464,7 +448,7 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
     }
     if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
   } else {
-    run_sweep<double>(ss, (double *)B.bp, (double *)B.wbuf, *(const GemvPlan<double> *)B.plan, st);
+    run_solve<double>(ss, (double *)B.bp, (double *)B.wbuf, *(const GemvPlan<double> *)B.plan, st);
     h->ir_steps = 0;
     h->ir_berr = 0;
   }
@@ -495,8 +479,6 @@ int solve_dev(snumat *h, const double *d_b, long long ldb, double *d_x, long lon
     B.wbuf = h->v64.wbuf;
     B.plan = &h->v64.sp;
   }
-  B.r = h->d_r;
-  B.dx = h->d_dx;
   B.colnorms = h->d_colnorms;
   return solve_core(h, d_b, ldb, d_x, ldx, nrhs, B, true);
 }
@@ -529,8 +511,8 @@ extern "C" int snumat_solve_device(snumat_t *h, const double *d_b, double *d_x,
 namespace {
 // The solve of snumat_solve_device over buffers carved from the device's
 // scratch: permuted right-hand sides, dense-solve vectors, the leaf fronts'
-// update rows, (SNU_FP32) residual, correction and column norms, then the
-// dense-solve descriptors and split-K partial sums.  Every buffer is written
+// update rows, (SNU_FP32) column norms, then the dense-solve descriptors and
+// split-K partial sums.  Every buffer is written
 // before it is read within the call (the column norms are zeroed by their
 // own kernel), so no clearing is needed; the descriptors are copied in on
 // every call, as another handle's call may have overwritten them.  A call
@@ -568,11 +550,7 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
     T *bp = (T *)carve(sizeof(T) * n * cols), *ys = (T *)carve(sizeof(T) * n * cols);
     B.bp = bp;
     B.wbuf = own_w ? (void *)carve(sizeof(T) * (size_t)h->wrows * cols) : (void *)VV.w1;
-    if (h->prec == SNU_FP32) {
-      B.r = (double *)carve(sizeof(double) * n * k);
-      B.dx = (double *)carve(sizeof(double) * n * k);
-      B.colnorms = (unsigned long long *)carve(sizeof(double) * 3 * (size_t)k);
-    }
+    if (h->prec == SNU_FP32) B.colnorms = (double *)carve(sizeof(double) * norm_values(1, (int)n, k));
     if (off > kScratchBytes) return false;
     if (VV.scratch_nrhs != k || VV.scratch_own_w != own_w) {
       VV.scratch_nrhs = -1;

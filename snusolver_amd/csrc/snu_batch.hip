@@ -39,19 +39,17 @@ struct snubatch {
   FrontPlan<float> fr32;
   // solves (sized for the last right-hand-side pattern)
   std::vector<int> pattern;  // nrhs per matrix of the current solve plan
-  long long vec_cap = 0, res_cap = 0, w_cap = 0;
+  long long vec_cap = 0, w_cap = 0;
   int slot_cap = 0;
   void *bp = nullptr, *ys = nullptr, *wbuf = nullptr;
-  double *r = nullptr, *dx = nullptr;
-  unsigned long long *norms = nullptr;
+  double *norms = nullptr;
   int *d_active = nullptr;
   VecDev *d_vec = nullptr;
-  PermDev *d_perm = nullptr;  // 2 x nmat: b -> x, then r -> dx
+  PermDev *d_perm = nullptr;
   IrDev *d_ir = nullptr;
   GemvPlan<double> s64;
   GemvPlan<float> s32;
   std::vector<VecDev> h_vec;
-  std::vector<long long> res_base;  // FP64 residual segment of each matrix
   std::vector<double> anorm;
   int ir_steps = 0;
   std::vector<double> berr;
@@ -120,14 +118,13 @@ template <typename T>
 int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   if (b->pattern == nrhs) return SNU_OK;
   const int nm = (int)b->mats.size();
-  // packed vectors (padded column groups), update rows, FP64 residuals
-  long long tot = 0, wtot = 0, rtot = 0;
+  // packed vectors (padded column groups), update rows
+  long long tot = 0, wtot = 0;
   int slots = 0;
   for (int m = 0; m < nm; m++) {
     const long long cols = (long long)vec_groups(nrhs[m]) * vec_width(nrhs[m]);
     tot += (long long)b->mats[m]->P.n * cols;
     wtot += (long long)b->mats[m]->wrows * cols;
-    rtot += (long long)b->mats[m]->P.n * nrhs[m];
     slots += nrhs[m];
   }
   int rc;
@@ -141,16 +138,6 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
       return rc;
     b->vec_cap = tot;
   }
-  if (b->prec == SNU_FP32 && rtot > b->res_cap) {
-    bfree(b, b->r);
-    bfree(b, b->dx);
-    b->r = b->dx = nullptr;
-    b->res_cap = 0;
-    if ((rc = balloc(b, (void **)&b->r, sizeof(double) * rtot)) ||
-        (rc = balloc(b, (void **)&b->dx, sizeof(double) * rtot)))
-      return rc;
-    b->res_cap = rtot;
-  }
   if (wtot > b->w_cap) {
     bfree(b, b->wbuf);
     b->wbuf = nullptr;
@@ -161,20 +148,17 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   if (slots > b->slot_cap) {
     bfree(b, b->norms);
     b->norms = nullptr;
-    if ((rc = balloc(b, (void **)&b->norms, sizeof(unsigned long long) * 3 * (size_t)slots))) return rc;
+    if ((rc = balloc(b, (void **)&b->norms, sizeof(double) * norm_values(nm, b->max_n, slots)))) return rc;
     b->slot_cap = slots;
   }
   b->h_vec.assign(nm, VecDev());
-  b->res_base.assign(nm, 0);
-  long long base = 0, wbase = 0, rbase = 0;
+  long long base = 0, wbase = 0;
   for (int m = 0; m < nm; m++) {
     const snumat *h = b->mats[m];
     const long long cols = (long long)vec_groups(nrhs[m]) * vec_width(nrhs[m]);
     b->h_vec[m] = VecDev{base, wbase, h->P.n, nrhs[m], h->wrows, 0};
-    b->res_base[m] = rbase;
     base += (long long)h->P.n * cols;
     wbase += (long long)h->wrows * cols;
-    rbase += (long long)h->P.n * nrhs[m];
   }
   HIPCHK(hipMemcpyAsync(b->d_vec, b->h_vec.data(), sizeof(VecDev) * nm, hipMemcpyHostToDevice, b->stream));
   GemvPlan<T> &out = std::is_same<T, double>::value ? (GemvPlan<T> &)b->s64 : (GemvPlan<T> &)b->s32;
@@ -237,19 +221,15 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
   int rc = ensure_pattern<T>(b, pat);
   if (rc) return rc;
   hipStream_t st = b->stream;
-  std::vector<PermDev> pd(2 * (size_t)nm);
-  long long max_elems = 0, max_vals = 0;
+  std::vector<PermDev> pd(nm);
+  long long max_elems = 0;
   int max_groups = 0, max_n = 0;
   bool one = false, many = false;
   for (int m = 0; m < nm; m++) {
     const snumat *h = b->mats[m];
     const int n = h->P.n;
-    const long long base = b->res_base[m];
     pd[m] = PermDev{h->d_order, d_b[m], d_x[m], (long long)ld[m], (long long)ld[m], n, m};
-    pd[nm + m] = PermDev{h->d_order, b->r ? b->r + base : nullptr, b->dx ? b->dx + base : nullptr,
-                         (long long)n, (long long)n, n, m};
     max_elems = std::max(max_elems, (long long)n * vec_groups(nrhs[m]));
-    max_vals = std::max(max_vals, (long long)n * nrhs[m]);
     max_groups = std::max(max_groups, vec_groups(nrhs[m]));
     one |= nrhs[m] == 1;
     many |= nrhs[m] > 1;
@@ -271,7 +251,6 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
     std::vector<int> slot_mat;
     for (int m = 0; m < nm; m++) {
       const snumat *h = b->mats[m];
-      const long long base = b->res_base[m];
       IrDev &e = ir[m];
       std::memset(&e, 0, sizeof(e));
       e.rowptr = h->d_arow;
@@ -279,10 +258,9 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
       e.val = h->d_aval;
       e.b = d_b[m];
       e.x = d_x[m];
-      e.r = b->r + base;
-      e.dx = b->dx + base;
+      e.order = h->d_order;
+      e.vec = m;
       e.ldb = e.ldx = ld[m];
-      e.ldr = e.lddx = h->P.n;
       e.n = h->P.n;
       e.nrhs = nrhs[m];
       e.norm0 = (int)slot_mat.size();
@@ -291,13 +269,10 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
     HIPCHK(hipMemcpyAsync(b->d_ir, ir.data(), sizeof(IrDev) * nm, hipMemcpyHostToDevice, st));
     const snu_opts_t &o = b->mats[0]->opts;
     RefineSet rs;
-    rs.sweep_b = ss;
-    rs.sweep_r = ss;
-    rs.sweep_r.perm = b->d_perm + nm;
+    rs.sweep = ss;
     rs.ir = b->d_ir;
     rs.nmat = nm;
     rs.max_n = max_n;
-    rs.max_elems = max_vals;
     rs.norms = b->norms;
     rs.nslots = (int)slot_mat.size();
     rs.slot_mat = &slot_mat;
@@ -323,7 +298,7 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
       rc = SNU_OK;
     }
   } else {
-    run_sweep<double>(ss, (double *)b->bp, (double *)b->wbuf, b->s64, st);
+    run_solve<double>(ss, (double *)b->bp, (double *)b->wbuf, b->s64, st);
     b->ir_steps = 0;
     b->berr.assign(nm, 0.0);
   }
@@ -441,7 +416,7 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   if ((rc = balloc(b, (void **)&b->d_anorm, sizeof(unsigned long long) * count)) ||
       (rc = balloc(b, (void **)&b->d_active, sizeof(int) * count)) ||
       (rc = balloc(b, (void **)&b->d_vec, sizeof(VecDev) * count)) ||
-      (rc = balloc(b, (void **)&b->d_perm, sizeof(PermDev) * 2 * count)) ||
+      (rc = balloc(b, (void **)&b->d_perm, sizeof(PermDev) * count)) ||
       (rc = balloc(b, (void **)&b->d_ir, sizeof(IrDev) * count)))
     return fail(rc);
   *out = b;

@@ -16,6 +16,8 @@ __device__ __forceinline__ gcdouble *gptr(const double *p) { return (gcdouble *)
 __device__ __forceinline__ gdouble *gptr(double *p) { return (gdouble *)p; }
 typedef __attribute__((address_space(1))) const float gcfloat;
 typedef __attribute__((address_space(1))) float gfloat;
+typedef __attribute__((address_space(1))) const long long gcint64;
+__device__ __forceinline__ gcint64 *gptr(const long long *p) { return (gcint64 *)p; }
 typedef __attribute__((address_space(1))) const int gcint;
 __device__ __forceinline__ gcint *gptr(const int *p) { return (gcint *)p; }
 __device__ __forceinline__ gcfloat *gptr(const float *p) { return (gcfloat *)p; }

@@ -180,9 +180,8 @@ struct snumat {
   snu::Values<float> v32;
   // standalone solves
   double *d_bx = nullptr;  // staging for host-pointer solves
-  double *d_r = nullptr, *d_dx = nullptr;  // refinement residual / correction
   unsigned long long *d_norms = nullptr;     // |A|inf (bits of a double)
-  unsigned long long *d_colnorms = nullptr;  // refinement column norms (3 x nrhs)
+  double *d_colnorms = nullptr;              // refinement column norms (norm_values)
   int *d_active = nullptr;
   snu::VecDev *d_vec = nullptr;
   snu::PermDev *d_perm = nullptr;
@@ -306,15 +305,17 @@ struct SolveSet {
   bool one, many;       // matrices with one / several columns present
   const WorkDev *wd;
 };
+// Forward and backward sweep over the packed vectors.
 template <typename T>
 void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st);
+// b into the packed vectors, the sweep, x out of them.
+template <typename T>
+void run_solve(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st);
 struct RefineSet {
-  SolveSet sweep_b;  // permutation tables b -> x (the caller's vectors)
-  SolveSet sweep_r;  // permutation tables r -> dx
+  SolveSet sweep;
   const IrDev *ir;
   int nmat, max_n;
-  long long max_elems;
-  unsigned long long *norms;  // 3 areas (b, r, x) of nslots
+  double *norms;  // norm_values(): column maxima of |b|, |r|, |x|, then workgroups' maxima
   int nslots;
   const std::vector<int> *slot_mat;   // matrix of each column slot
   const std::vector<double> *anorm;   // |A|inf per matrix
@@ -327,13 +328,12 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
 
 // Buffers of one standalone solve: the permuted right-hand sides and the
 // leaf fronts' update rows (value type of the handle), the dense-solve launch
-// plan with its device descriptors, and (SNU_FP32) the FP64 residual /
-// correction and the column norms of the refinement.
+// plan with its device descriptors, and (SNU_FP32) the column norms of the
+// refinement.
 struct SolveBuffers {
   void *bp = nullptr, *wbuf = nullptr;
   const void *plan = nullptr;  // GemvPlan<T> of the handle's value type
-  double *r = nullptr, *dx = nullptr;
-  unsigned long long *colnorms = nullptr;
+  double *colnorms = nullptr;
 };
 // Solve with device pointers (caller's b / x, column-major) on the given
 // buffers, on the handle's stream; returns when the work is done.  fallback:

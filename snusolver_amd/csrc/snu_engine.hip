@@ -1544,7 +1544,7 @@ int upload(snumat *h) {
     D.bcol_loc = d_bcol_loc + off_bcol[r];
     D.dd = h->d_dd;
   }
-  if ((rc = dalloc(h, &h->d_vec, 1)) || (rc = dalloc(h, &h->d_perm, 2)) ||
+  if ((rc = dalloc(h, &h->d_vec, 1)) || (rc = dalloc(h, &h->d_perm, 1)) ||
       (rc = dalloc(h, &h->d_prep, 1)) || (rc = dalloc(h, &h->d_ir, 1)) ||
       (rc = dalloc(h, &h->d_active, 1)) || (rc = dalloc(h, &h->d_norms, 1)))
     return rc;
@@ -1603,7 +1603,7 @@ size_t estimate_device_bytes(const snumat *h) {
                        (double)inversion_tmp_size(P));
   bytes += 16.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block;
   if (h->prec == SNU_FP32) bytes += 4.0 * (P.n + 1 + P.nnz);
-  bytes += 2 * vs * P.n + 16.0 * P.n + (h->prec == SNU_FP32 ? 16.0 * P.n : 0.0);
+  bytes += 2 * vs * P.n + 16.0 * P.n;
   return (size_t)bytes;
 }
 
@@ -1808,7 +1808,6 @@ int run_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st,
 template <typename T>
 void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st) {
   const WorkDev &wd = *ss.wd;
-  launch_permute_in(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
   launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, false, st);
   launch_assemble_rhs(wd.targets, wd.ntarget, wd.tsrc, ss.vec, wbuf, bp, ss.max_groups, ss.one, ss.many, st);
   for (const Launch &L : plan.fwd)
@@ -1816,7 +1815,12 @@ void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipS
   for (const Launch &L : plan.bwd)
     run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, st);
   launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, true, st);
-  launch_permute_out(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
+}
+template <typename T>
+void run_solve(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipStream_t st) {
+  launch_permute_in(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
+  run_sweep<T>(ss, bp, wbuf, plan, st);
+  launch_permute_out(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, false, nullptr, st);
 }
 
 // FP32 factors, FP64 refinement over a set of matrices: x = sweep(b), then
@@ -1825,28 +1829,20 @@ void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipS
 int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<float> &plan,
                 hipStream_t st, int *steps_out, std::vector<double> *berr_mat) {
   const int nm = rs.nmat, ns = rs.nslots;
-  std::vector<unsigned long long> u(3 * (size_t)ns);
-  std::vector<double> bn(ns), rn(ns), xn(ns);
-  auto fetch = [&](int area, std::vector<double> &out) -> int {
-    HIPCHK(hipMemcpyAsync(u.data(), rs.norms + (size_t)area * ns, sizeof(unsigned long long) * ns,
-                          hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    for (int i = 0; i < ns; i++) std::memcpy(&out[i], &u[i], sizeof(double));
-    return SNU_OK;
-  };
-  int rc;
-  launch_colmax(rs.ir, nm, rs.max_n, 0, rs.norms, ns, st);
-  if ((rc = fetch(0, bn))) return rc;
-  run_sweep<float>(rs.sweep_b, bp, wbuf, plan, st);
+  const SolveSet &ss = rs.sweep;
+  std::vector<double> u(3 * (size_t)ns);  // |b|, |r|, |x| per column
+  const double *bn = u.data(), *rn = bn + ns, *xn = rn + ns;
+  launch_permute_in(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, st);
+  run_sweep<float>(ss, bp, wbuf, plan, st);
+  launch_permute_out(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, false, nullptr, st);
   std::vector<double> prev(nm, INFINITY), berr(nm, INFINITY);
   std::vector<int> active(nm, 0), steps(nm, 0);
   int max_steps_taken = 0;
   for (;;) {
-    launch_residual(rs.ir, nm, rs.max_n, st);
-    launch_colmax(rs.ir, nm, rs.max_n, 1, rs.norms + ns, ns, st);
-    launch_colmax(rs.ir, nm, rs.max_n, 2, rs.norms + 2 * (size_t)ns, ns, st);
+    launch_residual(rs.ir, ss.vec, nm, rs.max_n, bp, rs.norms, ns, st);
     HIPCHK(hipGetLastError());
-    if ((rc = fetch(1, rn)) || (rc = fetch(2, xn))) return rc;
+    HIPCHK(hipMemcpyAsync(u.data(), rs.norms, sizeof(double) * u.size(), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
     std::fill(berr.begin(), berr.end(), 0.0);
     for (int i = 0; i < ns; i++) {
       const int m = (*rs.slot_mat)[i];
@@ -1863,9 +1859,10 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
     if (!nact) break;
     for (int m = 0; m < nm; m++)
       if (active[m]) prev[m] = berr[m], steps[m]++, max_steps_taken = std::max(max_steps_taken, steps[m]);
-    HIPCHK(hipMemcpyAsync(rs.d_active, active.data(), sizeof(int) * nm, hipMemcpyHostToDevice, st));
-    run_sweep<float>(rs.sweep_r, bp, wbuf, plan, st);
-    launch_update(rs.ir, nm, rs.max_elems, rs.d_active, st);
+    if (nact < nm)
+      HIPCHK(hipMemcpyAsync(rs.d_active, active.data(), sizeof(int) * nm, hipMemcpyHostToDevice, st));
+    run_sweep<float>(ss, bp, wbuf, plan, st);
+    launch_permute_out(ss.perm, ss.nmat, ss.vec, bp, ss.max_elems, true, nact < nm ? rs.d_active : nullptr, st);
     HIPCHK(hipGetLastError());
   }
   if (steps_out) *steps_out = max_steps_taken;
@@ -1891,7 +1888,7 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
   template int run_factor<T>(const FactorSet &, const DensePlan<T> &, hipStream_t,            \
                              const std::vector<hipEvent_t> *, bool, std::vector<hipEvent_t> *, \
                              double *, FactorGraph *);                                        \
-  template void run_sweep<T>(const SolveSet &, T *, T *, const GemvPlan<T> &, hipStream_t);
+  template void run_solve<T>(const SolveSet &, T *, T *, const GemvPlan<T> &, hipStream_t);
 SNU_ENGINE_INST(double)
 SNU_ENGINE_INST(float)
 #undef SNU_ENGINE_INST

@@ -129,12 +129,13 @@ struct PrepDev {
 struct IrDev {
   const int *rowptr, *colidx;
   const double *val;
+  const int *order;  // solve position of each row
   const double *b;
-  double *x, *r, *dx;
-  long long ldb, ldx, ldr, lddx;
+  const double *x;
+  long long ldb, ldx;
   int n, nrhs;
   int norm0;  // first slot of this matrix's columns in the norm arrays
-  int pad;
+  int vec;    // its slot in the VecDev table
 };
 
 template <typename T>
@@ -196,7 +197,6 @@ void launch_fill(T *p, long long n, hipStream_t st);
 template <typename T>
 void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long max_nnz,
                     hipStream_t st);
-void launch_zero_i32(int *p, int n, hipStream_t st);
 // dst = src, bytes a multiple of 16
 void launch_copy(const void *src, void *dst, long long bytes, hipStream_t st);
 // boundary Schur rows into the dense blocks, per tile of 64 separator rows
@@ -242,13 +242,14 @@ void launch_gemv16(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs
 template <typename T>
 void launch_diag_lu(const DiagProbT<T> *probs, int nprob, hipStream_t st);
 // Right-hand sides into / solutions out of the packed vectors; max_elems: the
-// largest n x groups of the matrices.
+// largest n x groups of the matrices.  Out: add: x += instead of x =, for the
+// matrices whose active flag is set (null: all).
 template <typename T>
 void launch_permute_in(const PermDev *pd, int nmat, const VecDev *vd, T *bp,
                        long long max_elems, hipStream_t st);
 template <typename T>
 void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *bp,
-                        long long max_elems, hipStream_t st);
+                        long long max_elems, bool add, const int *active, hipStream_t st);
 // Separator rows += the root fronts' update rows.
 template <typename T>
 void launch_assemble_rhs(const TargetDev *targets, int ntarget, const int *tsrc, const VecDev *vd,
@@ -283,14 +284,16 @@ template <typename T>
 void launch_front_schur(const LeafSchurDev *ls, const int4 *tiles, int ntile, hipStream_t st);
 
 // ---- FP64 iterative refinement (one matrix per table entry) ----
-void launch_residual(const IrDev *tab, int nmat, int max_n, hipStream_t st);
-// which: 0 b, 1 r, 2 x; out (nout slots) is zeroed first
-void launch_colmax(const IrDev *tab, int nmat, int max_n, int which, unsigned long long *out,
-                   int nout, hipStream_t st);
+// r = b - A x into the packed vectors and max |b|, |r|, |x| per column into
+// the three areas of norms (nslots each; the workgroups' maxima after them)
+constexpr int kResidualBlocks = 2048;
+int residual_blocks(int nmat, int max_n);
+inline size_t norm_values(int nmat, int max_n, int nslots) {
+  return 3 * (size_t)nslots * (1 + residual_blocks(nmat, max_n));
+}
+template <typename T>
+void launch_residual(const IrDev *tab, const VecDev *vd, int nmat, int max_n, T *bp, double *norms, int nslots,
+                     hipStream_t st);
 void launch_rowabs_max(const IrDev *tab, int nmat, int max_n, unsigned long long *out,
                        hipStream_t st);
-// x += dx where active[matrix] != 0
-void launch_update(const IrDev *tab, int nmat, long long max_elems, const int *active,
-                   hipStream_t st);
-
 }  // namespace snu

@@ -859,33 +859,10 @@ void launch_diag_lu(const DiagProbT<T> *probs, int nprob, hipStream_t st) {
 // FP64 iterative refinement around the FP32 factors (original CSR order)
 // ---------------------------------------------------------------------------
 // One matrix per blockIdx.y throughout; FP64 arithmetic.
-// r = b - A x with 8 lanes per row.
-__global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab) {
-  const IrDev M = tab[blockIdx.y];
-  const int sub = threadIdx.x & 7;
-  for (long long row = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 3; row < M.n;
-       row += ((long long)gridDim.x * blockDim.x) >> 3) {
-    const int p0 = M.rowptr[row], p1 = M.rowptr[row + 1];
-    for (int c = 0; c < M.nrhs; c++) {
-      const double *xc = M.x + (long long)c * M.ldx;
-      double s = 0.0;
-      for (int p = p0 + sub; p < p1; p += 8) s += M.val[p] * xc[M.colidx[p]];
-      s += __shfl_xor(s, 1, 8);
-      s += __shfl_xor(s, 2, 8);
-      s += __shfl_xor(s, 4, 8);
-      if (sub == 0) M.r[row + (long long)c * M.ldr] = M.b[row + (long long)c * M.ldb] - s;
-    }
-  }
-}
 static unsigned ir_blocks(long long rows_x_lanes) {
   long long b = (rows_x_lanes + 255) / 256;
   return (unsigned)std::max(1LL, std::min(b, 1024LL));
 }
-void launch_residual(const IrDev *tab, int nmat, int max_n, hipStream_t st) {
-  if (nmat <= 0 || max_n <= 0) return;
-  hipLaunchKernelGGL(k_residual, dim3(ir_blocks(8LL * max_n), nmat), dim3(256), 0, st, tab);
-}
-
 __device__ __forceinline__ double block_max(double v, double *red) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -896,24 +873,142 @@ __device__ __forceinline__ double block_max(double v, double *red) {
   for (int i = 1; i < (int)(blockDim.x >> 6); i++) v = fmax(v, red[i]);
   return v;
 }
-// out[norm0 + c] = max_i |v[i + c ld]| for v = b (which 0), r (1) or x (2).
-// Nonnegative doubles order like their bit patterns, so an integer atomic
-// max on the bits is exact.
-__global__ __launch_bounds__(256) void k_colmax(const IrDev *__restrict__ tab, int which,
-                                                unsigned long long *out) {
-  __shared__ double red[4];
+// Nonnegative doubles order like their bit patterns, so an integer atomic max
+// on the bits is exact.
+__device__ __forceinline__ void atomic_max_bits(unsigned long long *p, double v) {
+  atomicMax(p, (unsigned long long)__double_as_longlong(v));
+}
+// r = b - A x, rounded to T straight into the packed vectors (the next
+// sweep's right-hand sides, so no FP64 residual goes through memory), and the
+// column maxima of |b|, |r| and |x| in the same pass: each workgroup stores its
+// own, k_norm_max combines them (atomic maxima from all workgroups queue up on
+// a few cache lines: six packed matrices 230 -> 184 us).  One column: 8 lanes
+// per row.  Several: a lane is a row, 8 columns at a time, so every load covers
+// 512 contiguous bytes of one column and A's entries are read once per 8
+// columns (16 rows x 4 columns per load: 1.18 ms against 0.84 for 1000^2
+// 5-point with 64 columns).  As separate passes, column by column, the same
+// work took 2.58 ms for the residual and 2 x 0.39 ms for the norms; the
+// vectors alone (1.3 GB) take 0.25 ms.
+template <typename T>
+__global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab, const VecDev *__restrict__ vd,
+                                                  T *__restrict__ bp, double *__restrict__ part, int nslots) {
+  __shared__ double red[3][4][kColGroup];
   const IrDev M = tab[blockIdx.y];
-  const double *v = which == 0 ? M.b : which == 1 ? M.r : M.x;
-  const long long ld = which == 0 ? M.ldb : which == 1 ? M.ldr : M.ldx;
-  for (int c = 0; c < M.nrhs; c++) {
-    double m = 0.0;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.n;
-         i += (long long)gridDim.x * blockDim.x)
-      m = fmax(m, fabs(v[i + c * ld]));
-    m = block_max(m, red);
-    if (threadIdx.x == 0) atomicMax(out + M.norm0 + c, (unsigned long long)__double_as_longlong(m));
+  const VecDev V = vd[M.vec];
+  const int nblk = gridDim.x;
+  T *out = bp + V.base;
+  const auto rowptr = gptr(M.rowptr), colidx = gptr(M.colidx), order = gptr(M.order);
+  const auto val = gptr(M.val), x = gptr(M.x), rhs = gptr(M.b);
+  const int sub = threadIdx.x & 7, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long long first = ((long long)blockIdx.x * 256 + threadIdx.x) >> 3, step = ((long long)gridDim.x * 256) >> 3;
+  if (M.nrhs == 1) {
+    double mb = 0.0, mr = 0.0, mx = 0.0;
+    for (long long row = first; row < M.n; row += step) {
+      const int p0 = rowptr[row], p1 = rowptr[row + 1];
+      double s = 0.0;
+      for (int p = p0 + sub; p < p1; p += 8) s += val[p] * x[colidx[p]];
+      s += __shfl_xor(s, 1, 8);
+      s += __shfl_xor(s, 2, 8);
+      s += __shfl_xor(s, 4, 8);
+      if (sub == 0) {
+        const double b = rhs[row], r = b - s;
+        out[order[row]] = (T)r;
+        mb = fmax(mb, fabs(b));
+        mr = fmax(mr, fabs(r));
+        mx = fmax(mx, fabs(x[row]));
+      }
+    }
+    double *rd = &red[0][0][0];
+    mb = block_max(mb, rd);
+    mr = block_max(mr, rd);
+    mx = block_max(mx, rd);
+    if (threadIdx.x == 0) {
+      part[(long long)M.norm0 * nblk + blockIdx.x] = mb;
+      part[((long long)nslots + M.norm0) * nblk + blockIdx.x] = mr;
+      part[(2LL * nslots + M.norm0) * nblk + blockIdx.x] = mx;
+    }
+    return;
+  }
+  // consecutive rows per workgroup, and consecutive workgroups of one XCD (ids
+  // go round-robin over the 8) on consecutive rows: neighbouring rows share
+  // their x entries in that XCD's L2
+  constexpr int NC = 8;
+  const int nw = gridDim.x & ~7, wg = (int)blockIdx.x < nw ? (blockIdx.x & 7) * (nw >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int chunk = (M.n + gridDim.x - 1) / gridDim.x;
+  const int row_end = min((long long)M.n, (long long)(wg + 1) * chunk);
+  for (int c0 = 0; c0 < M.nrhs; c0 += NC) {
+    T *oc = out + (long long)(c0 / kColGroup) * V.n * kColGroup + c0 % kColGroup;
+    double m[3][NC];
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int c = 0; c < NC; c++) m[q][c] = 0.0;
+    for (int row = wg * chunk + threadIdx.x; row < row_end; row += 256) {
+      const int p0 = rowptr[row], p1 = rowptr[row + 1];
+      T *o = oc + (long long)order[row] * kColGroup;
+      double b[NC], xr[NC], s[NC];
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        const long long cc = min(c0 + c, M.nrhs - 1);
+        b[c] = rhs[row + cc * M.ldb];
+        xr[c] = x[row + cc * M.ldx];
+        s[c] = 0.0;
+      }
+      for (int p = p0; p < p1; p++) {
+        const double v = val[p];
+        const auto xi = x + colidx[p];
+#pragma unroll
+        for (int c = 0; c < NC; c++) s[c] += v * xi[min(c0 + c, M.nrhs - 1) * M.ldx];
+      }
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        const double r = b[c] - s[c];
+        o[c] = c0 + c < M.nrhs ? (T)r : T(0);
+        m[0][c] = fmax(m[0][c], fabs(b[c]));
+        m[1][c] = fmax(m[1][c], fabs(r));
+        m[2][c] = fmax(m[2][c], fabs(xr[c]));
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        for (int o = 1; o < 64; o <<= 1) m[q][c] = fmax(m[q][c], __shfl_xor(m[q][c], o, 64));
+        if (lane == 0) red[q][wave][c] = m[q][c];
+      }
+    __syncthreads();
+    if (threadIdx.x < 3 * NC) {
+      const int c = threadIdx.x % NC, q = threadIdx.x / NC;
+      if (c0 + c < M.nrhs)
+        part[((long long)q * nslots + M.norm0 + c0 + c) * nblk + blockIdx.x] =
+            fmax(fmax(red[q][0][c], red[q][1][c]), fmax(red[q][2][c], red[q][3][c]));
+    }
   }
 }
+// norms[s] = max of the workgroups' values part[s nblk ...]
+__global__ __launch_bounds__(256) void k_norm_max(const double *__restrict__ part, int nblk,
+                                                  double *__restrict__ norms) {
+  __shared__ double red[4];
+  double m = 0.0;
+  for (int i = threadIdx.x; i < nblk; i += 256) m = fmax(m, part[(long long)blockIdx.x * nblk + i]);
+  m = block_max(m, red);
+  if (threadIdx.x == 0) norms[blockIdx.x] = m;
+}
+int residual_blocks(int nmat, int max_n) {
+  const long long want = (8LL * max_n + 255) / 256;
+  return (int)std::max(1LL, std::min(want, (long long)std::max(16, kResidualBlocks / std::max(1, nmat))));
+}
+template <typename T>
+void launch_residual(const IrDev *tab, const VecDev *vd, int nmat, int max_n, T *bp, double *norms, int nslots,
+                     hipStream_t st) {
+  if (nmat <= 0 || max_n <= 0 || nslots <= 0) return;
+  const int nblk = residual_blocks(nmat, max_n);
+  double *part = norms + 3LL * nslots;
+  hipLaunchKernelGGL(k_residual<T>, dim3(nblk, nmat), dim3(256), 0, st, tab, vd, bp, part, nslots);
+  hipLaunchKernelGGL(k_norm_max, dim3(3 * nslots), dim3(256), 0, st, part, nblk, norms);
+}
+template void launch_residual<float>(const IrDev *, const VecDev *, int, int, float *, double *, int, hipStream_t);
 // Plain streaming copy (16 B per lane per iteration): the reference kernel
 // for scaling the HBM byte counters.
 __global__ __launch_bounds__(256) void k_copy(const double2 *__restrict__ src,
@@ -927,34 +1022,22 @@ void launch_copy(const void *src, void *dst, long long bytes, hipStream_t st) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_copy, dim3(4096), dim3(256), 0, st, (const double2 *)src, (double2 *)dst, n);
 }
-__global__ void k_zero_i32(int *p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-void launch_zero_i32(int *p, int n, hipStream_t st) {
-  if (n > 0) hipLaunchKernelGGL(k_zero_i32, dim3((n + 255) / 256), dim3(256), 0, st, p, n);
-}
 __global__ void k_zero_u64(unsigned long long *p, int n) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
-}
-void launch_colmax(const IrDev *tab, int nmat, int max_n, int which, unsigned long long *out,
-                   int nout, hipStream_t st) {
-  if (nout > 0)
-    hipLaunchKernelGGL(k_zero_u64, dim3((nout + 255) / 256), dim3(256), 0, st, out, nout);
-  if (nmat <= 0 || max_n <= 0) return;
-  hipLaunchKernelGGL(k_colmax, dim3(ir_blocks(max_n), nmat), dim3(256), 0, st, tab, which, out);
 }
 // out[matrix] = max_i sum_j |A_ij|
 __global__ __launch_bounds__(256) void k_rowabs_max(const IrDev *__restrict__ tab,
                                                     unsigned long long *out) {
   __shared__ double red[4];
   const IrDev M = tab[blockIdx.y];
+  const auto rowptr = gptr(M.rowptr);
+  const auto val = gptr(M.val);
   double m = 0.0;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.n;
        i += (long long)gridDim.x * blockDim.x) {
     double s = 0.0;
-    for (int p = M.rowptr[i]; p < M.rowptr[i + 1]; p++) s += fabs(M.val[p]);
+    for (int p = rowptr[i]; p < rowptr[i + 1]; p++) s += fabs(val[p]);
     m = fmax(m, s);
   }
   m = block_max(m, red);
@@ -967,29 +1050,12 @@ void launch_rowabs_max(const IrDev *tab, int nmat, int max_n, unsigned long long
   if (max_n <= 0) return;
   hipLaunchKernelGGL(k_rowabs_max, dim3(ir_blocks(max_n), nmat), dim3(256), 0, st, tab, out);
 }
-// x += dx for the matrices whose flag is set
-__global__ void k_update(const IrDev *__restrict__ tab, const int *__restrict__ active) {
-  const IrDev M = tab[blockIdx.y];
-  if (!active[blockIdx.y]) return;
-  const long long tot = (long long)M.n * M.nrhs;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
-       i += (long long)gridDim.x * blockDim.x) {
-    const long long c = i / M.n, r = i % M.n;
-    M.x[r + c * M.ldx] += M.dx[r + c * M.lddx];
-  }
-}
-void launch_update(const IrDev *tab, int nmat, long long max_elems, const int *active,
-                   hipStream_t st) {
-  if (nmat <= 0 || max_elems <= 0) return;
-  hipLaunchKernelGGL(k_update, dim3(ir_blocks(max_elems), nmat), dim3(256), 0, st, tab, active);
-}
-
 // Factor set-up for a set of matrices (one per blockIdx.y): zero the value
 // arena and the inverse blocks, then scatter A's values into their slots.
 template <typename T>
 __global__ void k_prep_fill(const PrepDev *__restrict__ tab) {
   const PrepDev M = tab[blockIdx.y];
-  T *a = (T *)M.arena, *v = (T *)M.inv;
+  const auto a = gptr((T *)M.arena), v = gptr((T *)M.inv);
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.arena_len; i += stride)
     a[i] = T(0);
@@ -999,10 +1065,12 @@ __global__ void k_prep_fill(const PrepDev *__restrict__ tab) {
 template <typename T>
 __global__ void k_prep_scatter(const PrepDev *__restrict__ tab) {
   const PrepDev M = tab[blockIdx.y];
-  T *a = (T *)M.arena;
+  const auto a = gptr((T *)M.arena);
+  const auto dest = gptr(M.adest);
+  const auto aval = gptr(M.aval);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.nnz;
        i += (long long)gridDim.x * blockDim.x)
-    a[M.adest[i]] = (T)M.aval[i];
+    a[dest[i]] = (T)aval[i];
 }
 template <typename T>
 void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long max_nnz,

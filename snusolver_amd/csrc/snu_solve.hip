@@ -26,15 +26,17 @@ __global__ void k_permute_in(const PermDev *__restrict__ pd, const VecDev *__res
   const VecDev V = vd[P.vec];
   const long long tot = (long long)P.n * vec_groups(V.nrhs);
   T *x = bp + V.base;
+  const auto order = gptr(P.order);
+  const auto rhs = gptr(P.b);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
        i += (long long)gridDim.x * blockDim.x) {
     if (V.nrhs == 1) {
-      x[P.order[i]] = (T)P.b[i];
+      x[order[i]] = (T)rhs[i];
       continue;
     }
     const int g = (int)(i / P.n), r = (int)(i % P.n);
-    T *d = x + ((long long)g * P.n + P.order[r]) * kColGroup;
-    const double *b = P.b + r + (long long)g * kColGroup * P.ldb;
+    T *d = x + ((long long)g * P.n + order[r]) * kColGroup;
+    const auto b = rhs + r + (long long)g * kColGroup * P.ldb;
     T v[kColGroup];
 #pragma unroll
     for (int c = 0; c < kColGroup; c++)
@@ -43,27 +45,37 @@ __global__ void k_permute_in(const PermDev *__restrict__ pd, const VecDev *__res
     for (int c = 0; c < kColGroup; c++) d[c] = v[c];
   }
 }
-template <typename T>
-__global__ void k_permute_out(const PermDev *__restrict__ pd, const VecDev *__restrict__ vd, const T *bp) {
+template <typename T, bool ADD>
+__global__ void k_permute_out(const PermDev *__restrict__ pd, const VecDev *__restrict__ vd, const T *bp,
+                              const int *__restrict__ active) {
+  const long long first = (long long)blockIdx.x * blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+  if (ADD && active && !active[blockIdx.y]) return;
   const PermDev P = pd[blockIdx.y];
   const VecDev V = vd[P.vec];
   const long long tot = (long long)P.n * vec_groups(V.nrhs);
   const T *x = bp + V.base;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot;
-       i += (long long)gridDim.x * blockDim.x) {
+  const auto order = gptr(P.order);
+  const auto sol = gptr(P.x);
+  for (long long i = first; i < tot; i += step) {
     if (V.nrhs == 1) {
-      P.x[i] = (double)x[P.order[i]];
+      const double v = (double)x[order[i]];
+      sol[i] = ADD ? sol[i] + v : v;
       continue;
     }
     const int g = (int)(i / P.n), r = (int)(i % P.n);
-    const T *s = x + ((long long)g * P.n + P.order[r]) * kColGroup;
-    double *d = P.x + r + (long long)g * kColGroup * P.ldx;
+    const T *s = x + ((long long)g * P.n + order[r]) * kColGroup;
+    const auto d = sol + r + (long long)g * kColGroup * P.ldx;
+    const int nc = V.nrhs - g * kColGroup;
     T v[kColGroup];
+    double o[kColGroup];
 #pragma unroll
-    for (int c = 0; c < kColGroup; c++) v[c] = s[c];
+    for (int c = 0; c < kColGroup; c++) {
+      v[c] = s[c];
+      o[c] = ADD && c < nc ? d[c * P.ldx] : 0.0;
+    }
 #pragma unroll
     for (int c = 0; c < kColGroup; c++)
-      if (g * kColGroup + c < V.nrhs) d[c * P.ldx] = (double)v[c];
+      if (c < nc) d[c * P.ldx] = ADD ? o[c] + (double)v[c] : (double)v[c];
   }
 }
 static unsigned perm_blocks(long long max_elems) {
@@ -77,10 +89,14 @@ void launch_permute_in(const PermDev *pd, int nmat, const VecDev *vd, T *bp, lon
   hipLaunchKernelGGL(k_permute_in<T>, dim3(perm_blocks(max_elems), nmat), dim3(256), 0, st, pd, vd, bp);
 }
 template <typename T>
-void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *bp, long long max_elems,
-                        hipStream_t st) {
+void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *bp, long long max_elems, bool add,
+                        const int *active, hipStream_t st) {
   if (nmat <= 0 || max_elems <= 0) return;
-  hipLaunchKernelGGL(k_permute_out<T>, dim3(perm_blocks(max_elems), nmat), dim3(256), 0, st, pd, vd, bp);
+  const dim3 g(perm_blocks(max_elems), nmat);
+  if (add)
+    hipLaunchKernelGGL((k_permute_out<T, true>), g, dim3(256), 0, st, pd, vd, bp, active);
+  else
+    hipLaunchKernelGGL((k_permute_out<T, false>), g, dim3(256), 0, st, pd, vd, bp, active);
 }
 
 // ---------------------------------------------------------------------------
@@ -991,7 +1007,7 @@ void launch_gemv16(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs
 #define SNU_SOLVE_INST(T)                                                                            \
   template void launch_permute_in<T>(const PermDev *, int, const VecDev *, T *, long long, hipStream_t); \
   template void launch_permute_out<T>(const PermDev *, int, const VecDev *, const T *, long long,   \
-                                      hipStream_t);                                                 \
+                                      bool, const int *, hipStream_t);                              \
   template void launch_assemble_rhs<T>(const TargetDev *, int, const int *, const VecDev *, const T *, T *, int, \
                                        bool, bool, hipStream_t);                                    \
   template void launch_leaf_sweep<T>(const LeafDev *, int, const VecDev *, T *, T *, int, bool, bool, bool, \
