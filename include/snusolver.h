@@ -276,7 +276,7 @@ int snumat_leaf_fronts(const snumat_t *h, int rank, int *front5, int *idx_ptr,
 /* the pivots K of each front (ascending within a front; k_ptr has
  * fronts + 1 entries, k the leaf size). */
 int snumat_leaf_front_pivots(const snumat_t *h, int rank, int *k_ptr, int *k);
-/* leaf LU values after factorize (copied back from the device); after
+/* leaf LU values after factorize (gathered from the leaf's fronts); after
  * snumat_factorize_stage(h, 0), A's leaf values in the LU layout. */
 int snumat_leaf_values(const snumat_t *h, int rank, double *lu_data);
 /* dense diagonal block of separator e (1 <= e < np), s_e x s_e col-major. */
@@ -288,8 +288,9 @@ int snumat_sep_diag(const snumat_t *h, int e, double *out);
 int snumat_factorize_stage(snumat_t *h, int stage);
 int snumat_sep_block(const snumat_t *h, int i, int j, double *out);
 /* phase timings of the last factorize / solve in ms (GPU events):
- * t[0] scatter, t[1] leaf fronts (the leaves' LU), t[2] the leaves'
- * boundary Schur blocks gathered from their root fronts, t[3] Schur assembly, t[4] dense levels, t[5] factorize total,
+ * t[0] scatter, t[1] leaf fronts (the leaves' LU), t[2] 0 (kept for the
+ * layout), t[3] the root fronts' updates added into the separator blocks,
+ * t[4] dense levels, t[5] factorize total,
  * t[6] solve total; dense GEMM launches of the factorization:
  * t[7] C -= AB kernel time (sum over launches, needs snumat_set_profiling),
  * t[8] its launches, t[9] its algorithmic GFLOP (2 M N K per problem);

@@ -293,7 +293,7 @@ int factorize_values(snumat *h, int stage) {
   fs.prep = h->d_prep;
   fs.nmat = 1;
   fs.max_len = std::max(h->arena_len, h->inv_total);
-  fs.max_nnz = h->P.nnz;
+  fs.max_nnz = h->nsep_ent;
   fs.ir = h->prec == SNU_FP32 ? h->d_ir : nullptr;
   fs.anorm_out = h->d_norms;
   fs.max_n = h->P.n;
@@ -348,6 +348,7 @@ int factorize_values(snumat *h, int stage) {
   }
   h->factored = stage >= 2;
   h->staged = true;
+  h->scattered = stage == 0;
   return SNU_OK;
 }
 
@@ -682,6 +683,21 @@ static int read_values(const snumat_t *h, long long off, size_t count, double *o
   }
   return SNU_OK;
 }
+// The factors of one leaf in its LU layout, gathered from its fronts.
+template <typename T>
+static int gather_leaf(const snumat_t *h, int rank, double *out) {
+  const LeafPlan &L = h->P.leaves[rank];
+  const int fmax = front_small_max<T>();
+  std::vector<T> F((size_t)(h->leaf_foff[rank + 1] - h->leaf_foff[rank]));
+  if (F.empty()) return SNU_OK;
+  HIPCHK(hipMemcpy(F.data(), vals<T>(h).farena + h->leaf_foff[rank], sizeof(T) * F.size(), hipMemcpyDeviceToHost));
+  long long off = 0;
+  for (size_t f = 0; f < L.ff.size(); f++) {
+    for (int q = L.fslot_ptr[f]; q < L.fslot_ptr[f + 1]; q++) out[L.fslot[q]] = (double)F[off + L.fpos[q]];
+    off += (long long)L.ff[f] * L.ff[f] + front_inv_size(L.ff[f], L.fnk[f], fmax);
+  }
+  return SNU_OK;
+}
 extern "C" int snumat_info(const snumat_t *h, int64_t *info) {
   if (!h || !info) return set_error(SNU_ERR_BAD_INPUT, "null");
   const Plan &P = h->P;
@@ -796,13 +812,24 @@ extern "C" int snumat_leaf_values(const snumat_t *h, int rank, double *out) {
   if (!h || rank < 0 || rank >= h->P.np) return set_error(SNU_ERR_BAD_INPUT, "bad rank");
   if (!h->factored && !h->staged) return set_error(SNU_ERR_NOT_FACTORED, "not factored");
   const LeafPlan &L = h->P.leaves[rank];
-  return read_values(h, h->P.leaf_off[rank], (size_t)L.lu_nnz, out);
+  HIPCHK(hipSetDevice(h->device));
+  std::fill(out, out + L.lu_nnz, 0.0);
+  if (h->scattered) {  // stage 0: A's values in the LU layout
+    std::vector<double> a((size_t)h->P.nnz);
+    if (!a.empty()) HIPCHK(hipMemcpy(a.data(), h->d_aval, sizeof(double) * a.size(), hipMemcpyDeviceToHost));
+    for (int q = 0; q < h->P.nnz; q++) {
+      const int64_t d = h->P.a_dest[q] - h->P.leaf_off[rank];
+      if (d >= 0 && d < L.lu_nnz) out[d] = h->prec == SNU_FP32 ? (double)(float)a[q] : a[q];
+    }
+    return SNU_OK;
+  }
+  return h->prec == SNU_FP32 ? gather_leaf<float>(h, rank, out) : gather_leaf<double>(h, rank, out);
 }
 extern "C" int snumat_sep_diag(const snumat_t *h, int e, double *out) {
   if (!h || e < 1 || e >= h->P.np) return set_error(SNU_ERR_BAD_INPUT, "bad separator");
   if (!h->factored) return set_error(SNU_ERR_NOT_FACTORED, "not factored");
   int s = h->P.block_size[e];
-  return read_values(h, h->P.leaf_total + h->P.offR[e], (size_t)s * s, out);
+  return read_values(h, h->P.offR[e], (size_t)s * s, out);
 }
 extern "C" int snumat_sep_block(const snumat_t *h, int i, int j, double *out) {
   if (!h || !out) return set_error(SNU_ERR_BAD_INPUT, "null handle or output");
@@ -822,12 +849,12 @@ extern "C" int snumat_sep_block(const snumat_t *h, int i, int j, double *out) {
   auto copy = [&](long long src, long long ld, int rows, int cols, double *dst) -> int {
     if (h->prec == SNU_FP32) {
       std::vector<float> tmp((size_t)rows * cols);
-      HIPCHK(hipMemcpy2D(tmp.data(), sizeof(float) * rows, h->v32.arena + P.leaf_total + src, sizeof(float) * ld,
+      HIPCHK(hipMemcpy2D(tmp.data(), sizeof(float) * rows, h->v32.arena + src, sizeof(float) * ld,
                          sizeof(float) * rows, cols, hipMemcpyDeviceToHost));
       for (int c = 0; c < cols; c++)
         for (int r = 0; r < rows; r++) dst[r + (size_t)c * si] = tmp[r + (size_t)c * rows];
     } else {
-      HIPCHK(hipMemcpy2D(dst, sizeof(double) * si, h->v64.arena + P.leaf_total + src, sizeof(double) * ld,
+      HIPCHK(hipMemcpy2D(dst, sizeof(double) * si, h->v64.arena + src, sizeof(double) * ld,
                          sizeof(double) * rows, cols, hipMemcpyDeviceToHost));
     }
     return SNU_OK;

@@ -207,6 +207,7 @@ int batch_factorize(snubatch *b) {
   }
   for (int m = 0; m < nm; m++) {
     b->mats[m]->factored = true;
+    b->mats[m]->scattered = false;
     b->mats[m]->fb64_current = false;  // an FP64 twin refactorizes on its next use
     b->mats[m]->anorm = b->anorm[m];
   }
@@ -344,12 +345,11 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   // concatenated leaves and work lists
   std::vector<LeafDev> leaves;
   WorkLists W;
-  W.tile_ptr.assign(1, 0);
   std::vector<PrepDev> prep;
   std::vector<IrDev> ira;
   for (int m = 0; m < count; m++) {
     snumat *h = b->mats[m];
-    const int lbase = (int)leaves.size(), sbase = (int)W.tsrc.size();
+    const int sbase = (int)W.tsrc.size();
     for (LeafDev L : h->h_leaves) {
       L.vec = m;
       leaves.push_back(L);
@@ -357,12 +357,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
     const WorkLists &w = h->wl;
     for (TargetDev t : w.targets) W.targets.push_back(TargetDev{t.row, sbase + t.s0, sbase + t.s1, m});
     W.tsrc.insert(W.tsrc.end(), w.tsrc.begin(), w.tsrc.end());
-    const int gbase = (int)W.seg_leaf.size();
-    W.tile_blk.insert(W.tile_blk.end(), w.tile_blk.begin(), w.tile_blk.end());
-    W.tile_row0.insert(W.tile_row0.end(), w.tile_row0.begin(), w.tile_row0.end());
-    for (size_t t = 1; t < w.tile_ptr.size(); t++) W.tile_ptr.push_back(gbase + w.tile_ptr[t]);
-    for (int s : w.seg_leaf) W.seg_leaf.push_back(lbase + s);
-    W.seg_ri.insert(W.seg_ri.end(), w.seg_ri.begin(), w.seg_ri.end());
     PrepDev pd;
     pd.arena = b->prec == SNU_FP32 ? (void *)h->v32.arena : (void *)h->v64.arena;
     pd.inv = b->prec == SNU_FP32 ? (void *)h->v32.inv : (void *)h->v64.inv;
@@ -370,7 +364,8 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
     pd.inv_len = h->inv_total;
     pd.aval = h->d_aval;
     pd.adest = h->d_adest;
-    pd.nnz = h->P.nnz;
+    pd.asrc = h->d_asrc;
+    pd.nnz = h->nsep_ent;
     prep.push_back(pd);
     IrDev e;
     std::memset(&e, 0, sizeof(e));
@@ -380,19 +375,15 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
     e.n = h->P.n;
     ira.push_back(e);
     b->max_len = std::max(b->max_len, std::max(h->arena_len, h->inv_total));
-    b->max_nnz = std::max(b->max_nnz, (long long)h->P.nnz);
+    b->max_nnz = std::max(b->max_nnz, h->nsep_ent);
     b->max_n = std::max(b->max_n, h->P.n);
   }
   WorkDev &wd = b->wd;
   wd.nleaves = (int)leaves.size();
   wd.ntarget = (int)W.targets.size();
-  wd.ntile = (int)W.tile_blk.size();
   int rc;
   if ((rc = bupload(b, &wd.leaves, leaves)) || (rc = bupload(b, &wd.targets, W.targets)) ||
       (rc = bupload(b, &wd.tsrc, W.tsrc)) || (rc = bupload(b, &b->d_prep, prep)) ||
-      (rc = bupload(b, &wd.tile_blk, W.tile_blk)) || (rc = bupload(b, &wd.tile_row0, W.tile_row0)) ||
-      (rc = bupload(b, &wd.tile_ptr, W.tile_ptr)) || (rc = bupload(b, &wd.seg_leaf, W.seg_leaf)) ||
-      (rc = bupload(b, &wd.seg_ri, W.seg_ri)) ||
       (rc = bupload(b, &b->d_ir_a, ira)))
     return fail(rc);
   // the members' leaf fronts, merged per height (descriptors point into the
@@ -406,8 +397,7 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
       merge_fronts(parts, fp);
       int r;
       if ((r = upload_dense_plan(fp.dense)) || (r = bupload(b, &fp.d_iblk, fp.iblk)) || (r = bupload(b, &fp.d_small, fp.small)) ||
-          (r = bupload(b, &fp.d_large, fp.large)) || (r = bupload(b, &fp.d_work, fp.work)) || (r = bupload(b, &fp.d_wrange, fp.wrange)) ||
-          (r = bupload(b, &fp.d_ls, fp.ls)) || (r = bupload(b, &fp.d_tiles, fp.tiles)))
+          (r = bupload(b, &fp.d_tiles, fp.tiles)) || (r = bupload(b, &fp.d_src, fp.src)))
         return r;
       return SNU_OK;
     };

@@ -67,31 +67,32 @@ struct GemvPlan {
 
 // Multifrontal leaf factorization of a launch set (one matrix, or a batch
 // merged): per height of the leaves' front trees, the fronts the LDS kernel
-// takes whole and the larger fronts' 64-column work items (front index into
-// `large`); the larger fronts' blocked partial LU as a keyed launch list
-// (key: height, step within it); the tiles of the boundary Schur blocks.
+// takes whole and the larger fronts' extend-add tiles; the larger fronts'
+// blocked partial LU as a keyed launch list (key: height, step within it);
+// the extend-add tiles of the separator blocks (after the last height).
 struct FrontLevel {
   int small0 = 0, nsmall = 0, max_f = 0;
   int nsmall_lo = 0, max_f_lo = 0;  // the first nsmall_lo small fronts have order <= kFrontLo
-  int work0 = 0, nwork = 0;
+  int tile0 = 0, ntile = 0;
 };
 template <typename T>
 struct FrontPlan {
-  std::vector<FrontDev> small, large;
+  std::vector<FrontDev> small;
   std::vector<int2> iblk;   // 16-pivot blocks of the small fronts: {front, first pivot}
-  std::vector<int4> work;   // larger fronts: {front, first column, ranges offset, 0}
-  std::vector<int> wrange;  // per work item: its owned-slot range, then per child its column range
+  std::vector<AddTile> tiles;  // by height, then the separator tiles
+  std::vector<AddSrc> src;
+  int sep0 = 0;             // first separator tile
   std::vector<FrontLevel> levels;
   DensePlan<T> dense;
-  std::vector<LeafSchurDev> ls;
-  std::vector<int4> tiles;
-  FrontDev *d_small = nullptr, *d_large = nullptr;
+  FrontDev *d_small = nullptr;
   int2 *d_iblk = nullptr;
-  int4 *d_work = nullptr;
-  int *d_wrange = nullptr;
-  LeafSchurDev *d_ls = nullptr;
-  int4 *d_tiles = nullptr;
+  AddTile *d_tiles = nullptr;
+  AddSrc *d_src = nullptr;
 };
+// Values of the inverses kept behind a front (FrontDev::inv).
+inline long long front_inv_size(int f, int nk, int fmax) {
+  return f > fmax ? (nk + 63) / 64 * 8192LL : (nk + 15) / 16 * 256LL;
+}
 template <typename T>
 void list_inverse_blocks(FrontPlan<T> &fp) {
   fp.iblk.clear();
@@ -106,11 +107,10 @@ inline int front_key_height(long long key) { return (int)(key / 100000000LL); }
 // Value-typed device state of one matrix (FP64, or FP32 refined in FP64).
 template <typename T>
 struct Values {
-  T *arena = nullptr;  // leaf LU values, then dense blocks
-  T *S = nullptr;      // boundary Schur blocks
+  T *arena = nullptr;  // the separators' dense blocks
   T *inv = nullptr;    // per separator: full L^-1 then U^-1 (s x s each)
   T *tmp = nullptr;    // products of the triangular inversion
-  T *farena = nullptr; // leaf fronts (each f x f; larger fronts then 2 x 64 x 64 of inverses)
+  T *farena = nullptr; // leaf fronts (each f x f, then the inverses of its pivot blocks)
   FrontPlan<T> fronts;
   DensePlan<T> fact;
   // standalone solves: right-hand sides, dense-solve vectors, the fronts'
@@ -130,7 +130,6 @@ struct Values {
 struct WorkLists {
   std::vector<TargetDev> targets;  // separator rows receiving leaf contributions
   std::vector<int> tsrc;           // their sources: update rows of root fronts
-  std::vector<int> tile_blk, tile_row0, tile_ptr, seg_leaf, seg_ri;  // assembly tiles
 };
 
 // Device copies of the work lists of a launch set (one matrix or a batch).
@@ -139,8 +138,6 @@ struct WorkDev {
   int nleaves = 0;
   TargetDev *targets = nullptr;
   int *tsrc = nullptr, ntarget = 0;
-  int *tile_blk = nullptr, *tile_row0 = nullptr, *tile_ptr = nullptr;
-  int *seg_leaf = nullptr, *seg_ri = nullptr, ntile = 0;
 };
 
 // A factorization's launch sequence captured once into a HIP graph and
@@ -158,13 +155,17 @@ struct snumat {
   bool on_device = false;
   bool factored = false;
   bool staged = false;  // a factorize_stage ran on the current values
+  bool scattered = false;  // and it was stage 0: the fronts hold no factors
   int device = -1;
   hipStream_t stream = nullptr;
   std::vector<void *> allocs;
   size_t dev_bytes = 0;
   long long arena_len = 0;
   double *d_aval = nullptr;  // A's values in the caller's CSR order (FP64)
-  long long *d_adest = nullptr;
+  long long *d_adest = nullptr;  // A's separator entries: place in the arena,
+  int *d_asrc = nullptr;         // index in A's values
+  long long nsep_ent = 0;
+  std::vector<long long> leaf_foff;  // first front value of each leaf (np + 1)
   int *d_arow = nullptr, *d_acol = nullptr;  // A's pattern (refinement residuals)
   int *d_order = nullptr;
   // leaves and work lists
@@ -173,7 +174,6 @@ struct snumat {
   snu::WorkDev wd;
   int wrows = 0;       // update rows of the leaf fronts (solves)
   // dense tables
-  snu::DenseDev *d_dd = nullptr;
   std::vector<long long> inv_off;
   long long inv_total = 0, tmp_total = 0;
   snu::Values<double> v64;

@@ -346,7 +346,7 @@ void build_dense_plan(snumat *h) {
   const Plan &P = h->P;
   const TileRule rule = tile_rule<T>(h);
   Values<T> &VV = vals<T>(h);
-  T *dense = VV.arena + P.leaf_total;
+  T *dense = VV.arena;
   auto R = [&](int p) { return dense + P.offR[p]; };
   auto Lp = [&](int p) { return dense + P.offL[p]; };
   auto Li = [&](int p) { return VV.inv + h->inv_off[p]; };
@@ -682,7 +682,7 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
   using GemvSeg = GemvSegT<T>;
   const Values<T> &VV = vals<T>(h);
   const Plan &P = h->P;
-  T *dense = VV.arena + P.leaf_total;
+  T *dense = VV.arena;
   // one column: groups 0, kinds 7 / 8; several: groups of 16, kinds 17 / 18
   const int w = vec_width(nrhs), groups = nrhs == 1 ? 0 : vec_groups(nrhs);
   const int kset = w == 1 ? 7 : 17, ksub = w == 1 ? 8 : 18;
@@ -938,33 +938,23 @@ void merge_gemv(const std::vector<const GemvPlan<T> *> &in, GemvPlan<T> &out) {
 // ---------------------------------------------------------------------------
 namespace {
 template <typename T>
-int alloc_values(snumat *h, long long S_total) {
+int alloc_values(snumat *h) {
   Values<T> &VV = vals<T>(h);
   int rc;
-  if ((rc = dalloc(h, &VV.arena, (size_t)h->arena_len)) || (rc = dalloc(h, &VV.S, (size_t)S_total)) ||
-      (rc = dalloc(h, &VV.inv, (size_t)h->inv_total)) ||
+  if ((rc = dalloc(h, &VV.arena, (size_t)h->arena_len)) || (rc = dalloc(h, &VV.inv, (size_t)h->inv_total)) ||
       (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_total))))
     return rc;
   build_dense_plan<T>(h);
-  if ((rc = upload_dense_plan(VV.fact))) return rc;
-  // leaf descriptors point at this value type's arrays
-  for (size_t r = 0; r < h->h_leaves.size(); r++) {
-    h->h_leaves[r].dense = VV.arena + h->P.leaf_total;
-  }
-  return SNU_OK;
+  return upload_dense_plan(VV.fact);
 }
 }  // namespace
 
-// Multifrontal plan of one matrix's leaves (value arrays allocated): the
-// front value arena, the integer tables (owned slots and positions,
-// extend-add indices, the root fronts' boundary rows / columns), child and
-// root descriptors, per-height front tables, the larger fronts' blocked
-// partial LU (per 64-column step: diagonal block LU with the pivot clamp,
-// both triangular solves by the block inverses, the trailing update of the
-// whole remaining front) and the boundary Schur tiles.
-static long long front_inv_size(int f, int nk, int fmax) {
-  return f > fmax ? (nk + 63) / 64 * 8192LL : (nk + 15) / 16 * 256LL;
-}
+// Multifrontal plan of one matrix's leaves (value arrays allocated): the front
+// value arena, the fronts' entries of A, extend-add positions and child
+// tables, per-height front tables and extend-add tiles, the larger fronts'
+// blocked partial LU (per 64-column step: diagonal block LU with the pivot
+// clamp, both triangular solves by the block inverses, the trailing update of
+// the whole remaining front) and the extend-add tiles of the separator blocks.
 template <typename T>
 int build_front_plan(snumat *h) {
   using GemmSeg = GemmSegT<T>;
@@ -976,45 +966,90 @@ int build_front_plan(snumat *h) {
   free_dense_plan(FP.dense);
   FP = FrontPlan<T>();
   int rc;
-  // integer tables and front value offsets
-  std::vector<int> ints;
-  std::vector<size_t> o_slot(np), o_pos(np), o_rel(np);
+  // front value offsets; per B entry its index in the target: the parent
+  // front, or (root fronts) the separator block it belongs to
+  std::vector<int> rel;
+  std::vector<size_t> o_rel(np);
   std::vector<std::vector<long long>> foff(np);
-  std::vector<std::vector<std::pair<size_t, size_t>>> o_root(np);  // per root: arow, acol offsets
+  h->leaf_foff.assign(np + 1, 0);
   long long ftotal = 0;
   int levels = 0;
   for (int r = 0; r < np; r++) {
     const LeafPlan &L = P.leaves[r];
-    o_slot[r] = ints.size();
-    ints.insert(ints.end(), L.fslot.begin(), L.fslot.end());
-    o_pos[r] = ints.size();
-    ints.insert(ints.end(), L.fpos.begin(), L.fpos.end());
-    o_rel[r] = ints.size();
-    ints.insert(ints.end(), L.frel.begin(), L.frel.end());
     const int nf = (int)L.ff.size();
+    o_rel[r] = rel.size();
+    rel.insert(rel.end(), L.frel.begin(), L.frel.end());
     foff[r].resize(nf);
     for (int f = 0; f < nf; f++) {
       foff[r][f] = ftotal;
-      ftotal += (long long)L.ff[f] * L.ff[f];
-      ftotal += front_inv_size(L.ff[f], L.fnk[f], fmax);
+      ftotal += (long long)L.ff[f] * L.ff[f] + front_inv_size(L.ff[f], L.fnk[f], fmax);
       if (L.fpar[f] >= 0) continue;
-      std::vector<int> arow(L.nbr, -1), acol(L.nbc, -1);
+      int k = 1;
       for (int q = L.fidx_ptr[f]; q < L.fidx_ptr[f + 1]; q++) {
-        if (L.fsrow[q] >= 0) arow[L.fsrow[q]] = q - L.fidx_ptr[f];
-        if (L.fscol[q] >= 0) acol[L.fscol[q]] = q - L.fidx_ptr[f];
+        while (L.fidx[q] >= L.cstart[k + 1]) k++;
+        rel[o_rel[r] + q] = L.fidx[q] - L.cstart[k];
       }
-      const size_t oa = ints.size();
-      ints.insert(ints.end(), arow.begin(), arow.end());
-      const size_t oc = ints.size();
-      ints.insert(ints.end(), acol.begin(), acol.end());
-      o_root[r].push_back({oa, oc});
     }
+    h->leaf_foff[r + 1] = ftotal;
     if (nf) levels = std::max(levels, L.fheight_max + 1);
   }
-  int *d_ints = nullptr;
-  if ((rc = dupload(h, &d_ints, ints)) || (rc = dalloc(h, &VV.farena, (size_t)std::max(1LL, ftotal)))) return rc;
+  int *d_rel = nullptr;
+  if ((rc = dupload(h, &d_rel, rel)) || (rc = dalloc(h, &VV.farena, (size_t)std::max(1LL, ftotal)))) return rc;
   T *fa = VV.farena;
-  // children
+  // A's entries by front (small fronts: column-major position; larger ones:
+  // by tile, position from the tile's first value); the rest go to the
+  // separators
+  std::vector<std::vector<int>> ent0(np);      // per front: first entry (nf + 1)
+  std::vector<std::vector<int>> tile_ent(np);  // per leaf, larger fronts in turn: entries per tile
+  std::vector<AEntry> ent;
+  {
+    auto leaf_of = [&](int q) {  // leaf of A's entry q, -1: a separator entry
+      if (P.a_dest[q] >= P.leaf_total) return -1;
+      return (int)(std::upper_bound(P.leaf_off.begin(), P.leaf_off.end(), P.a_dest[q]) - P.leaf_off.begin()) - 1;
+    };
+    std::vector<int> leaf(P.nnz);
+    for (int r = 0; r < np; r++) ent0[r].assign(P.leaves[r].ff.size() + 1, 0);
+    for (int q = 0; q < P.nnz; q++) {
+      const int r = leaf[q] = leaf_of(q);
+      if (r >= 0) ent0[r][P.leaves[r].afront[P.perm_map[q] - P.leaves[r].coo_off] + 1]++;
+    }
+    int total = 0;
+    for (int r = 0; r < np; r++)
+      for (int &e : ent0[r]) e = total += e;
+    ent.resize(total);
+    std::vector<std::vector<int>> at = ent0;
+    for (int q = 0; q < P.nnz; q++) {
+      const int r = leaf[q];
+      if (r < 0) continue;
+      const LeafPlan &L = P.leaves[r];
+      const int k = P.perm_map[q] - L.coo_off;
+      ent[at[r][L.afront[k]]++] = AEntry{L.apos[k], q};
+    }
+    // larger fronts: by tile
+    std::vector<std::pair<int, AEntry>> tmp;
+    for (int r = 0; r < np; r++) {
+      const LeafPlan &L = P.leaves[r];
+      for (int f = 0; f < (int)L.ff.size(); f++) {
+        const int ff = L.ff[f], nt = (ff + 63) / 64;
+        if (ff <= fmax) continue;
+        const size_t tbase = tile_ent[r].size();
+        tile_ent[r].resize(tbase + (size_t)nt * nt, 0);
+        tmp.clear();
+        for (int e = ent0[r][f]; e < ent0[r][f + 1]; e++) {
+          const int row = ent[e].pos % ff, col = ent[e].pos / ff, t = (col / 64) * nt + row / 64;
+          tile_ent[r][tbase + t]++;
+          tmp.push_back({t, AEntry{row % 64 + (col % 64) * ff, ent[e].idx}});
+        }
+        std::sort(tmp.begin(), tmp.end(), [](const std::pair<int, AEntry> &x, const std::pair<int, AEntry> &y) {
+          return x.first != y.first ? x.first < y.first : x.second.pos < y.second.pos;
+        });
+        for (size_t e = 0; e < tmp.size(); e++) ent[ent0[r][f] + e] = tmp[e].second;
+      }
+    }
+  }
+  AEntry *d_ent = nullptr;
+  if ((rc = dupload(h, &d_ent, ent))) return rc;
+  // children (of the fronts factored in LDS)
   std::vector<FrontChild> ch;
   std::vector<std::vector<int>> ch0(np);
   for (int r = 0; r < np; r++) {
@@ -1023,34 +1058,42 @@ int build_front_plan(snumat *h) {
     ch0[r].resize(nf);
     for (int f = 0; f < nf; f++) {
       ch0[r][f] = (int)ch.size();
+      if (L.ff[f] > fmax) continue;
       for (int q = L.fchild_ptr[f]; q < L.fchild_ptr[f + 1]; q++) {
         const int c = L.fchild[q], fc = L.ff[c], nkc = L.fnk[c];
         ch.push_back(FrontChild{fa + foff[r][c] + nkc + (long long)nkc * fc,
-                                d_ints + o_rel[r] + L.fidx_ptr[c], fc, fc - nkc});
+                                d_rel + o_rel[r] + L.fidx_ptr[c], fc, fc - nkc});
       }
     }
   }
   FrontChild *d_ch = nullptr;
   if ((rc = dupload(h, &d_ch, ch))) return rc;
   // fronts by height
-  std::vector<std::vector<FrontDev>> sm(levels), lg(levels);
-  std::vector<std::vector<std::pair<int, int>>> lgid(levels);  // (leaf, front) of each larger front
+  std::vector<std::vector<FrontDev>> sm(levels);
+  struct Large { T *F, *inv; int f, nk, leaf, front, tile_ent; };
+  std::vector<std::vector<Large>> lg(levels);
   for (int r = 0; r < np; r++) {
     const LeafPlan &L = P.leaves[r];
+    int te = 0;
     for (int f = 0; f < (int)L.ff.size(); f++) {
+      const int ff = L.ff[f];
+      T *F = fa + foff[r][f], *inv = F + (long long)ff * ff;
+      if (ff > fmax) {
+        lg[L.fheight[f]].push_back(Large{F, inv, ff, L.fnk[f], r, f, te});
+        te += ((ff + 63) / 64) * ((ff + 63) / 64);
+        continue;
+      }
       FrontDev D;
-      D.F = fa + foff[r][f];
-      D.inv = fa + foff[r][f] + (long long)L.ff[f] * L.ff[f];
-      D.vals = VV.arena + P.leaf_off[r];
-      D.slot = d_ints + o_slot[r] + L.fslot_ptr[f];
-      D.pos = d_ints + o_pos[r] + L.fslot_ptr[f];
+      D.F = F;
+      D.inv = inv;
+      D.aval = h->d_aval;
+      D.ent = d_ent + ent0[r][f];
       D.child = d_ch + ch0[r][f];
-      D.f = L.ff[f];
+      D.f = ff;
       D.nk = L.fnk[f];
-      D.nslot = L.fslot_ptr[f + 1] - L.fslot_ptr[f];
+      D.nent = ent0[r][f + 1] - ent0[r][f];
       D.nchild = L.fchild_ptr[f + 1] - L.fchild_ptr[f];
-      (D.f <= fmax ? sm : lg)[L.fheight[f]].push_back(D);
-      if (D.f > fmax) lgid[L.fheight[f]].push_back({r, f});
+      sm[L.fheight[f]].push_back(D);
     }
   }
   FP.levels.assign(levels, FrontLevel());
@@ -1067,30 +1110,52 @@ int build_front_plan(snumat *h) {
       lv.max_f = std::max(lv.max_f, D.f);
     }
     FP.small.insert(FP.small.end(), sm[hh].begin(), sm[hh].end());
-    lv.work0 = (int)FP.work.size();
-    const int lbase = (int)FP.large.size();
+    // extend-add tiles of the larger fronts, column by column: each child's
+    // entries per 64-index chunk of the front, every pair of chunks a source
+    lv.tile0 = (int)FP.tiles.size();
     int kmax = 0;
-    for (size_t q = 0; q < lg[hh].size(); q++) {
-      const FrontDev &D = lg[hh][q];
-      const LeafPlan &L = P.leaves[lgid[hh][q].first];
-      const int fr = lgid[hh][q].second;
-      const int *pos = L.fpos.data() + L.fslot_ptr[fr];
-      for (int c0 = 0; c0 < D.f; c0 += 64) {
-        const int c1 = std::min(D.f, c0 + 64);
-        FP.work.push_back(make_int4(lbase + (int)q, c0, (int)FP.wrange.size(), 0));
-        FP.wrange.push_back((int)(std::lower_bound(pos, pos + D.nslot, c0 * D.f) - pos));
-        FP.wrange.push_back((int)(std::lower_bound(pos, pos + D.nslot, c1 * D.f) - pos));
-        for (int k = L.fchild_ptr[fr]; k < L.fchild_ptr[fr + 1]; k++) {
-          const int c = L.fchild[k];
-          const int *rel = L.frel.data() + L.fidx_ptr[c], nb = L.fidx_ptr[c + 1] - L.fidx_ptr[c];
-          FP.wrange.push_back((int)(std::lower_bound(rel, rel + nb, c0) - rel));
-          FP.wrange.push_back((int)(std::lower_bound(rel, rel + nb, c1) - rel));
+    std::vector<int> bound;  // per child: first entry of each chunk (nt + 1)
+    for (const Large &D : lg[hh]) {
+      const LeafPlan &L = P.leaves[D.leaf];
+      const int f = D.f, nt = (f + 63) / 64, nc = L.fchild_ptr[D.front + 1] - L.fchild_ptr[D.front];
+      bound.resize((size_t)nc * (nt + 1));
+      for (int k = 0; k < nc; k++) {
+        const int c = L.fchild[L.fchild_ptr[D.front] + k];
+        const int *rc0 = L.frel.data() + L.fidx_ptr[c], nb = L.fidx_ptr[c + 1] - L.fidx_ptr[c];
+        int q = 0;
+        for (int t = 0; t <= nt; t++) {
+          while (q < nb && rc0[q] < 64 * t) q++;
+          bound[(size_t)k * (nt + 1) + t] = q;
         }
       }
+      int e = ent0[D.leaf][D.front];
+      for (int ct = 0; ct < nt; ct++)
+        for (int rt = 0; rt < nt; rt++) {
+          AddTile t;
+          t.C = D.F + 64 * rt + (long long)64 * ct * f;
+          t.aval = h->d_aval;
+          t.ent = d_ent + e;
+          t.nent = tile_ent[D.leaf][D.tile_ent + ct * nt + rt];
+          e += t.nent;
+          t.ldc = f;
+          t.nr = std::min(64, f - 64 * rt);
+          t.nc = std::min(64, f - 64 * ct);
+          t.keep = 0;
+          t.s0 = (int)FP.src.size();
+          for (int k = 0; k < nc; k++) {
+            const int *bk = bound.data() + (size_t)k * (nt + 1);
+            if (bk[rt] == bk[rt + 1] || bk[ct] == bk[ct + 1]) continue;
+            const int c = L.fchild[L.fchild_ptr[D.front] + k], fc = L.ff[c], nkc = L.fnk[c];
+            FP.src.push_back(AddSrc{fa + foff[D.leaf][c] + nkc + (long long)nkc * fc,
+                                    d_rel + o_rel[D.leaf] + L.fidx_ptr[c], fc, bk[rt], bk[rt + 1] - bk[rt], bk[ct],
+                                    bk[ct + 1] - bk[ct], 64 * rt, 64 * ct, 0});
+          }
+          t.s1 = (int)FP.src.size();
+          FP.tiles.push_back(t);
+        }
       kmax = std::max(kmax, D.nk);
     }
-    lv.nwork = (int)FP.work.size() - lv.work0;
-    FP.large.insert(FP.large.end(), lg[hh].begin(), lg[hh].end());
+    lv.ntile = (int)FP.tiles.size() - lv.tile0;
     // blocked partial LU of this height's larger fronts, grouped per step
     for (int k = 0; k < kmax; k += 64) {
       const int step = k / 64;
@@ -1098,11 +1163,11 @@ int build_front_plan(snumat *h) {
       Launch tr{1, (int)DP.gp.size(), 0, 0, 0, front_key(hh, step, 1)};
       GemmBatch<T> tu;
       tu.rule = tile_rule<T>(h);
-      for (const FrontDev &D : lg[hh]) {
+      for (const Large &D : lg[hh]) {
         if (D.nk <= k) continue;
         const int f = D.f, nb = std::min(64, D.nk - k), m = f - k - nb;
-        T *F = (T *)D.F;
-        T *Li = (T *)D.inv + (long long)step * 8192, *Ui = Li + 64 * 64;
+        T *F = D.F;
+        T *Li = D.inv + (long long)step * 8192, *Ui = Li + 64 * 64;
         DiagProbT<T> dp{};
         dp.D = F + k + (long long)k * f;
         dp.ld = f;
@@ -1136,35 +1201,82 @@ int build_front_plan(snumat *h) {
     }
   }
   if ((rc = upload_dense_plan(DP))) return rc;
-  // boundary Schur blocks from the root fronts
-  std::vector<FrontRoot> roots;
+  // extend-add tiles of the separator blocks: the root fronts' update blocks,
+  // per pair of 64-index tiles of the blocks their B entries belong to (pairs
+  // whose panel tile is not stored are structurally zero)
+  FP.sep0 = (int)FP.tiles.size();
+  struct Piece { long long key; T *C; long long ldc; int nr, nc; AddSrc s; };
+  std::vector<Piece> pieces;
+  struct Group { int blk, t, b0, b1; };
+  std::vector<Group> gr;
+  std::vector<long long> tbase(P.num_block + 2, 0);  // tiles of the blocks before each block
+  for (int b = 1; b <= P.num_block; b++) tbase[b + 1] = tbase[b] + (P.block_size[b] + 63) / 64;
   for (int r = 0; r < np; r++) {
     const LeafPlan &L = P.leaves[r];
-    const int root0 = (int)roots.size();
-    int k = 0;
     for (int f = 0; f < (int)L.ff.size(); f++) {
       if (L.fpar[f] >= 0) continue;
-      const int ff = L.ff[f], nk = L.fnk[f];
-      roots.push_back(FrontRoot{fa + foff[r][f] + nk + (long long)nk * ff, d_ints + o_root[r][k].first,
-                                d_ints + o_root[r][k].second, ff});
-      k++;
-    }
-    if (L.nbr > 0 && L.nbc > 0) {
-      const int li = (int)FP.ls.size();
-      FP.ls.push_back(LeafSchurDev{h->h_leaves[r].S, nullptr, L.nbr, L.nbc, (int)roots.size() - root0});
-      FP.ls.back().root = (const FrontRoot *)(uintptr_t)root0;  // index until the table is uploaded
-      for (int r0 = 0; r0 < L.nbr; r0 += 64)
-        for (int c0 = 0; c0 < L.nbc; c0 += 64) FP.tiles.push_back(make_int4(li, r0, c0, 0));
+      const int fc = L.ff[f], nkc = L.fnk[f], i0 = L.fidx_ptr[f], nb = L.fidx_ptr[f + 1] - i0;
+      const T *U = fa + foff[r][f] + nkc + (long long)nkc * fc;
+      gr.clear();
+      int k = 1;
+      for (int q = 0; q < nb; q++) {
+        while (L.fidx[i0 + q] >= L.cstart[k + 1]) k++;
+        const int t = (L.fidx[i0 + q] - L.cstart[k]) / 64;
+        if (gr.empty() || gr.back().blk != L.path[k] || gr.back().t != t) gr.push_back(Group{L.path[k], t, q, q});
+        gr.back().b1 = q + 1;
+      }
+      for (const Group &a : gr)
+        for (const Group &c : gr) {
+          const int p = a.blk, q = c.blk, sp = P.block_size[p], sq = P.block_size[q];
+          T *C;
+          long long ldc;
+          if (p == q) {
+            C = VV.arena + P.offR[p] + 64 * a.t + (long long)64 * c.t * sp;
+            ldc = sp;
+          } else if (p > q) {  // row block deeper: its U panel
+            const int u = P.umap[p][P.anc_off(p, q) + 64 * c.t];
+            if (u < 0) continue;
+            C = VV.arena + P.offR[p] + 64 * a.t + (long long)(sp + u) * sp;
+            ldc = sp;
+          } else {
+            const int l = P.lmap[q][P.anc_off(q, p) + 64 * a.t];
+            if (l < 0) continue;
+            C = VV.arena + P.offL[q] + l + (long long)64 * c.t * P.nL[q];
+            ldc = P.nL[q];
+          }
+          pieces.push_back(Piece{(tbase[p] + a.t) * tbase[P.num_block + 1] + tbase[q] + c.t, C, ldc,
+                                 std::min(64, sp - 64 * a.t), std::min(64, sq - 64 * c.t),
+                                 AddSrc{U, d_rel + o_rel[r] + i0, fc, a.b0, a.b1 - a.b0, c.b0, c.b1 - c.b0,
+                                        64 * a.t, 64 * c.t, 0}});
+        }
     }
   }
-  FrontRoot *d_roots = nullptr;
-  if ((rc = dupload(h, &d_roots, roots))) return rc;
-  for (LeafSchurDev &l : FP.ls) l.root = d_roots + (uintptr_t)l.root;
+  std::vector<int> po(pieces.size());
+  for (size_t q = 0; q < po.size(); q++) po[q] = (int)q;
+  std::sort(po.begin(), po.end(), [&](int a, int b) {
+    return pieces[a].key != pieces[b].key ? pieces[a].key < pieces[b].key : a < b;  // leaves in ascending order
+  });
+  for (size_t q = 0; q < po.size(); q++) {
+    const Piece &x = pieces[po[q]];
+    if (q == 0 || x.key != pieces[po[q - 1]].key) {
+      AddTile t;
+      t.C = x.C;
+      t.aval = nullptr;
+      t.ent = nullptr;
+      t.ldc = x.ldc;
+      t.nr = x.nr;
+      t.nc = x.nc;
+      t.s0 = t.s1 = (int)FP.src.size();
+      t.nent = 0;
+      t.keep = 1;
+      FP.tiles.push_back(t);
+    }
+    FP.src.push_back(x.s);
+    FP.tiles.back().s1 = (int)FP.src.size();
+  }
   list_inverse_blocks(FP);
-  if ((rc = dupload(h, &FP.d_iblk, FP.iblk)) || (rc = dupload(h, &FP.d_small, FP.small)) || (rc = dupload(h, &FP.d_large, FP.large)) ||
-      (rc = dupload(h, &FP.d_work, FP.work)) || (rc = dupload(h, &FP.d_wrange, FP.wrange)) ||
-      (rc = dupload(h, &FP.d_ls, FP.ls)) ||
-      (rc = dupload(h, &FP.d_tiles, FP.tiles)))
+  if ((rc = dupload(h, &FP.d_iblk, FP.iblk)) || (rc = dupload(h, &FP.d_small, FP.small)) ||
+      (rc = dupload(h, &FP.d_tiles, FP.tiles)) || (rc = dupload(h, &FP.d_src, FP.src)))
     return rc;
   return SNU_OK;
 }
@@ -1172,23 +1284,28 @@ int build_front_plan(snumat *h) {
 template <typename T>
 void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out) {
   out.small.clear();
-  out.large.clear();
-  out.work.clear();
-  out.wrange.clear();
-  std::vector<int> rbase;
-  for (const FrontPlan<T> *p : in) {
-    rbase.push_back((int)out.wrange.size());
-    out.wrange.insert(out.wrange.end(), p->wrange.begin(), p->wrange.end());
-  }
-  out.ls.clear();
   out.tiles.clear();
+  out.src.clear();
+  std::vector<int> sbase;
   size_t levels = 0;
-  for (const FrontPlan<T> *p : in) levels = std::max(levels, p->levels.size());
+  for (const FrontPlan<T> *p : in) {
+    sbase.push_back((int)out.src.size());
+    out.src.insert(out.src.end(), p->src.begin(), p->src.end());
+    levels = std::max(levels, p->levels.size());
+  }
+  auto add_tiles = [&](size_t pi, int first, int count) {
+    for (int q = first; q < first + count; q++) {
+      AddTile t = in[pi]->tiles[q];
+      t.s0 += sbase[pi];
+      t.s1 += sbase[pi];
+      out.tiles.push_back(t);
+    }
+  };
   out.levels.assign(levels, FrontLevel());
   for (size_t hh = 0; hh < levels; hh++) {
     FrontLevel &lv = out.levels[hh];
     lv.small0 = (int)out.small.size();
-    lv.work0 = (int)out.work.size();
+    lv.tile0 = (int)out.tiles.size();
     for (size_t pi = 0; pi < in.size(); pi++) {
       const FrontPlan<T> *p = in[pi];
       if (hh >= p->levels.size()) continue;
@@ -1196,17 +1313,7 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
       out.small.insert(out.small.end(), p->small.begin() + pl.small0, p->small.begin() + pl.small0 + pl.nsmall_lo);
       lv.max_f = std::max(lv.max_f, pl.max_f);
       lv.max_f_lo = std::max(lv.max_f_lo, pl.max_f_lo);
-      // this matrix's larger fronts of the height, in the order its work items name them
-      int first = -1, last = -1;
-      for (int q = pl.work0; q < pl.work0 + pl.nwork; q++) {
-        if (first < 0) first = p->work[q].x;
-        last = p->work[q].x;
-      }
-      if (first < 0) continue;
-      const int base = (int)out.large.size();
-      out.large.insert(out.large.end(), p->large.begin() + first, p->large.begin() + last + 1);
-      for (int q = pl.work0; q < pl.work0 + pl.nwork; q++)
-        out.work.push_back(make_int4(base + p->work[q].x - first, p->work[q].y, rbase[pi] + p->work[q].z, 0));
+      add_tiles(pi, pl.tile0, pl.ntile);
     }
     lv.nsmall_lo = (int)out.small.size() - lv.small0;
     for (const FrontPlan<T> *p : in)  // then every matrix's larger small fronts
@@ -1216,17 +1323,14 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
                          p->small.begin() + pl.small0 + pl.nsmall);
       }
     lv.nsmall = (int)out.small.size() - lv.small0;
-    lv.nwork = (int)out.work.size() - lv.work0;
+    lv.ntile = (int)out.tiles.size() - lv.tile0;
   }
+  out.sep0 = (int)out.tiles.size();
+  for (size_t pi = 0; pi < in.size(); pi++) add_tiles(pi, in[pi]->sep0, (int)in[pi]->tiles.size() - in[pi]->sep0);
   list_inverse_blocks(out);
   std::vector<const DensePlan<T> *> dp;
   for (const FrontPlan<T> *p : in) dp.push_back(&p->dense);
   merge_dense(dp, out.dense);
-  for (const FrontPlan<T> *p : in) {
-    const int base = (int)out.ls.size();
-    out.ls.insert(out.ls.end(), p->ls.begin(), p->ls.end());
-    for (int4 t : p->tiles) out.tiles.push_back(make_int4(base + t.x, t.y, t.z, t.w));
-  }
 }
 // The leaf solves of one matrix: solve positions (leaf rows in front order, so
 // a front's pivots are consecutive), update rows, the children's
@@ -1414,82 +1518,9 @@ int upload(snumat *h) {
   if (h->prec == SNU_FP32) autotune_tiles<float>();
   else autotune_tiles<double>();
   const int np = P.np;
-  // ---- leaf arrays (concatenated; descriptors hold pointers into them) ----
-  std::vector<int> bcol_blk, bcol_loc;
-  std::vector<size_t> off_bcol(np);
-  std::vector<long long> off_S(np);
-  long long S_total = 0;
   h->h_leaves.assign(np, LeafDev());
-  for (int r = 0; r < np; r++) {
-    const LeafPlan &L = P.leaves[r];
-    LeafDev &D = h->h_leaves[r];
-    off_bcol[r] = bcol_blk.size();
-    off_S[r] = S_total;
-    S_total += (long long)L.nbr * L.nbc;
-    for (int c : L.bcol) {
-      int k = 1;
-      while (c >= L.cstart[k + 1]) k++;
-      bcol_blk.push_back(L.path[k]);
-      bcol_loc.push_back(c - L.cstart[k]);
-    }
-    D.nbr = L.nbr;
-    D.nbc = L.nbc;
-    D.vec = 0;
-  }
-  // boundary rows of the leaves by separator row, ascending rank
-  WorkLists &W = h->wl;
-  W = WorkLists();
-  struct Src { int R, leaf, ri; };
-  std::vector<Src> src;
-  for (int r = 0; r < np; r++) {
-    const LeafPlan &L = P.leaves[r];
-    for (int ri = 0; ri < L.nbr; ri++) {
-      int c = L.brow[ri], k = 1;
-      while (c >= L.cstart[k + 1]) k++;
-      src.push_back({P.block_start[L.path[k]] + c - L.cstart[k], r, ri});
-    }
-  }
-  std::sort(src.begin(), src.end(), [](const Src &a, const Src &b) {
-    return a.R != b.R ? a.R < b.R : a.leaf < b.leaf;
-  });
-  std::vector<int> blk_of(P.n);
-  for (int b = 1; b <= P.num_block; b++)
-    for (int i = P.block_start[b]; i < P.block_start[b] + P.block_size[b]; i++) blk_of[i] = b;
-  // assembly tiles: 64 consecutive rows of one separator block; per tile the
-  // contributing leaves in ascending rank, each with the boundary row (ri)
-  // feeding every row of the tile (-1: none)
-  W.tile_blk.clear();
-  W.tile_row0.clear();
-  W.tile_ptr.assign(1, 0);
-  W.seg_leaf.clear();
-  W.seg_ri.clear();
-  {
-    size_t s0 = 0;
-    while (s0 < src.size()) {
-      const int b = blk_of[src[s0].R];
-      const int row0 = ((src[s0].R - P.block_start[b]) / 64) * 64;
-      const int R0 = P.block_start[b] + row0, R1 = std::min(R0 + 64, P.block_start[b] + P.block_size[b]);
-      size_t s1 = s0;
-      while (s1 < src.size() && src[s1].R < R1) s1++;
-      std::vector<Src> part(src.begin() + s0, src.begin() + s1);
-      std::stable_sort(part.begin(), part.end(), [](const Src &a, const Src &c) { return a.leaf < c.leaf; });
-      for (size_t q = 0; q < part.size(); q++) {
-        if (q == 0 || part[q].leaf != part[q - 1].leaf) {
-          W.seg_leaf.push_back(part[q].leaf);
-          W.seg_ri.insert(W.seg_ri.end(), 64, -1);
-        }
-        W.seg_ri[W.seg_ri.size() - 64 + (part[q].R - R0)] = part[q].ri;
-      }
-      W.tile_blk.push_back(b);
-      W.tile_row0.push_back(row0);
-      W.tile_ptr.push_back((int)W.seg_leaf.size());
-      s0 = s1;
-    }
-  }
+  h->wl = WorkLists();
   // ---- dense tables ----
-  std::vector<int> aoff((P.num_block + 1) * P.nk, 0);
-  for (int p = 1; p <= P.num_block; p++)
-    for (int d = 1; (p >> d) >= 1; d++) aoff[p * P.nk + d] = P.anc_off(p, p >> d);
   h->inv_off.assign(P.num_block + 1, 0);
   long long inv_total = 0;
   for (int p = 1; p < np; p++) {
@@ -1498,52 +1529,18 @@ int upload(snumat *h) {
   }
   h->inv_total = inv_total;
   h->tmp_total = inversion_tmp_size(P);
-  h->arena_len = P.leaf_total + P.dense_total;
+  h->arena_len = P.dense_total;
   // ---- structure uploads ----
-  int *d_bcol_blk, *d_bcol_loc;
-  if ((rc = dalloc(h, &h->d_aval, (size_t)P.nnz))) return rc;
-  if ((rc = dupload(h, &h->d_adest, std::vector<long long>(P.a_dest.begin(), P.a_dest.end())))) return rc;
-  if ((rc = dupload(h, &d_bcol_blk, bcol_blk)) || (rc = dupload(h, &d_bcol_loc, bcol_loc))) return rc;
+  std::vector<long long> adest;
+  std::vector<int> asrc;
+  for (int q = 0; q < P.nnz; q++)
+    if (P.a_dest[q] >= P.leaf_total) adest.push_back(P.a_dest[q] - P.leaf_total), asrc.push_back(q);
+  h->nsep_ent = (long long)asrc.size();
+  if ((rc = dalloc(h, &h->d_aval, (size_t)P.nnz)) || (rc = dupload(h, &h->d_adest, adest)) ||
+      (rc = dupload(h, &h->d_asrc, asrc)))
+    return rc;
   WorkDev &wd = h->wd;
   wd.nleaves = np;
-  wd.ntile = (int)W.tile_blk.size();
-  if ((rc = dupload(h, &wd.tile_blk, W.tile_blk)) || (rc = dupload(h, &wd.tile_row0, W.tile_row0)) ||
-      (rc = dupload(h, &wd.tile_ptr, W.tile_ptr)) || (rc = dupload(h, &wd.seg_leaf, W.seg_leaf)) ||
-      (rc = dupload(h, &wd.seg_ri, W.seg_ri)))
-    return rc;
-  long long *d_offR, *d_offL, *d_mapoff;
-  int *d_bsize, *d_nL, *d_lmap, *d_umap, *d_aoff;
-  std::vector<long long> offR(P.offR.begin(), P.offR.end()), offL(P.offL.begin(), P.offL.end());
-  std::vector<long long> mapoff(P.num_block + 1, 0);
-  std::vector<int> lmap, umap;
-  for (int p = 1; p < np; p++) {
-    mapoff[p] = (long long)lmap.size();
-    lmap.insert(lmap.end(), P.lmap[p].begin(), P.lmap[p].end());
-    umap.insert(umap.end(), P.umap[p].begin(), P.umap[p].end());
-  }
-  if (lmap.empty()) lmap.push_back(-1), umap.push_back(-1);
-  if ((rc = dupload(h, &d_offR, offR)) || (rc = dupload(h, &d_offL, offL)) ||
-      (rc = dupload(h, &d_mapoff, mapoff)) || (rc = dupload(h, &d_bsize, P.block_size)) ||
-      (rc = dupload(h, &d_nL, P.nL)) || (rc = dupload(h, &d_lmap, lmap)) || (rc = dupload(h, &d_umap, umap)) ||
-      (rc = dupload(h, &d_aoff, aoff)))
-    return rc;
-  DenseDev dd;
-  dd.offR = d_offR;
-  dd.offL = d_offL;
-  dd.mapoff = d_mapoff;
-  dd.bsize = d_bsize;
-  dd.nL = d_nL;
-  dd.lmap = d_lmap;
-  dd.umap = d_umap;
-  dd.aoff = d_aoff;
-  dd.nk = P.nk;
-  if ((rc = dupload(h, &h->d_dd, std::vector<DenseDev>{dd}))) return rc;
-  for (int r = 0; r < np; r++) {
-    LeafDev &D = h->h_leaves[r];
-    D.bcol_blk = d_bcol_blk + off_bcol[r];
-    D.bcol_loc = d_bcol_loc + off_bcol[r];
-    D.dd = h->d_dd;
-  }
   if ((rc = dalloc(h, &h->d_vec, 1)) || (rc = dalloc(h, &h->d_perm, 1)) ||
       (rc = dalloc(h, &h->d_prep, 1)) || (rc = dalloc(h, &h->d_ir, 1)) ||
       (rc = dalloc(h, &h->d_active, 1)) || (rc = dalloc(h, &h->d_norms, 1)))
@@ -1551,19 +1548,13 @@ int upload(snumat *h) {
   if (h->prec == SNU_FP32) {
     if ((rc = dupload(h, &h->d_arow, P.a_rowptr)) || (rc = dupload(h, &h->d_acol, P.a_colidx)))
       return rc;
-    rc = alloc_values<float>(h, S_total);
-    if (!rc) {
-      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v32.S + off_S[r];
-      rc = build_front_plan<float>(h);
-      if (!rc) rc = build_leaf_solve<float>(h);
-    }
+    rc = alloc_values<float>(h);
+    if (!rc) rc = build_front_plan<float>(h);
+    if (!rc) rc = build_leaf_solve<float>(h);
   } else {
-    rc = alloc_values<double>(h, S_total);
-    if (!rc) {
-      for (int r = 0; r < np; r++) h->h_leaves[r].S = h->v64.S + off_S[r];
-      rc = build_front_plan<double>(h);
-      if (!rc) rc = build_leaf_solve<double>(h);
-    }
+    rc = alloc_values<double>(h);
+    if (!rc) rc = build_front_plan<double>(h);
+    if (!rc) rc = build_leaf_solve<double>(h);
   }
   if (rc) return rc;
   if ((rc = dupload(h, &wd.leaves, h->h_leaves))) return rc;
@@ -1574,7 +1565,8 @@ int upload(snumat *h) {
   pd.inv_len = h->inv_total;
   pd.aval = h->d_aval;
   pd.adest = h->d_adest;
-  pd.nnz = P.nnz;
+  pd.asrc = h->d_asrc;
+  pd.nnz = h->nsep_ent;
   HIPCHK(hipMemcpy(h->d_prep, &pd, sizeof(pd), hipMemcpyHostToDevice));
   return SNU_OK;
 }
@@ -1584,22 +1576,22 @@ int upload(snumat *h) {
 size_t estimate_device_bytes(const snumat *h) {
   const Plan &P = h->P;
   const double vs = h->prec == SNU_FP32 ? 4.0 : 8.0;
-  double S_total = 0, idx = 0, inv = 0, fronts = 0;
+  double idx = 0, inv = 0, fronts = 0;
   const int fmax = h->prec == SNU_FP32 ? front_small_max<float>() : front_small_max<double>();
   for (const LeafPlan &L : P.leaves) {
-    S_total += (double)L.nbr * L.nbc;
-    idx += 2.0 * L.bcol.size();
-    // fronts: values (larger ones with their diagonal-block inverses), slot /
-    // position / extend-add tables, root row / column maps, descriptors
+    // fronts: values with the inverses of their pivot blocks; solve units,
+    // children's update rows, positions of the B entries; extend-add tiles
+    // and their sources
     fronts += (double)L.fentries;
-    for (size_t f = 0; f < L.ff.size(); f++) fronts += (double)front_inv_size(L.ff[f], L.fnk[f], fmax);
-    idx += 2.0 * L.fslot.size() + L.frel.size() + (double)(L.nbr + L.nbc) + 16.0 * L.ff.size();
-    // solve units, children's update rows, positions of the B entries
-    idx += 34.0 * L.ff.size() + 4.0 * L.fidx.size() + L.leaf_size;
+    for (size_t f = 0; f < L.ff.size(); f++) {
+      fronts += (double)front_inv_size(L.ff[f], L.fnk[f], fmax);
+      const double nt = (L.ff[f] + 63) / 64;
+      idx += L.ff[f] > fmax ? 14.0 * nt * nt + 12.0 * nt * nt : 18.0;
+    }
+    idx += 34.0 * L.ff.size() + 5.0 * L.fidx.size() + 3.0 * L.leaf_size;
   }
-  S_total += fronts;
   for (int p = 1; p < P.np; p++) inv += 2.0 * P.block_size[p] * P.block_size[p];
-  double bytes = vs * ((double)P.leaf_total + (double)P.dense_total + S_total + inv +
+  double bytes = vs * ((double)P.dense_total + fronts + inv +
                        (double)inversion_tmp_size(P));
   bytes += 16.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block;
   if (h->prec == SNU_FP32) bytes += 4.0 * (P.n + 1 + P.nnz);
@@ -1697,7 +1689,7 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
     return SNU_OK;
   }
   // leaf fronts, height by height: whole fronts in LDS; larger fronts
-  // assembled, factored by the dense launches of their height, written back
+  // assembled and factored by the dense launches of their height
   const FrontPlan<T> &fp = *(const FrontPlan<T> *)fs.fronts;
   int ngemm = 0;
   for (const Launch &L : fp.dense.launches) ngemm += is_gemm(L.kind);
@@ -1722,21 +1714,19 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
     const FrontLevel &lv = fp.levels[hh];
     launch_front_small<T>(fp.d_small + lv.small0, lv.nsmall_lo, lv.max_f_lo, fs.eps, st);
     launch_front_small<T>(fp.d_small + lv.small0 + lv.nsmall_lo, lv.nsmall - lv.nsmall_lo, lv.max_f, fs.eps, st);
-    launch_front_assemble<T>(fp.d_large, fp.d_work + lv.work0, fp.d_wrange, lv.nwork, st);
+    launch_extend_add<T>(fp.d_tiles + lv.tile0, lv.ntile, fp.d_src, st);
     for (; li < nl && front_key_height(fp.dense.launches[li].key) == hh; li++) {
       int rc = run_timed(fp.dense.launches[li], fp.dense);
       if (rc) return rc;
     }
-    launch_front_writeback<T>(fp.d_large, fp.d_work + lv.work0, fp.d_wrange, lv.nwork, st);
   }
   launch_front_inverse<T>(fp.d_small, fp.d_iblk, (int)fp.iblk.size(), st);
   HIPCHK(hipGetLastError());
-  if (ev) HIPCHK(hipEventRecord((*ev)[2], st));
-  launch_front_schur<T>(fp.d_ls, fp.d_tiles, (int)fp.tiles.size(), st);
-  HIPCHK(hipGetLastError());
-  if (ev) HIPCHK(hipEventRecord((*ev)[3], st));
-  launch_assemble_schur<T>(wd.ntile, wd.tile_blk, wd.tile_row0, wd.tile_ptr, wd.seg_leaf, wd.seg_ri,
-                           wd.leaves, st);
+  if (ev) {
+    HIPCHK(hipEventRecord((*ev)[2], st));
+    HIPCHK(hipEventRecord((*ev)[3], st));
+  }
+  launch_extend_add<T>(fp.d_tiles + fp.sep0, (int)fp.tiles.size() - fp.sep0, fp.d_src, st);
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[4], st));
   for (const Launch &L : plan.launches) {

@@ -208,8 +208,13 @@ int build_fronts(LeafPlan &L) {
       if (L.frel[q] < 0) return set_error(SNU_ERR_STRUCTURE, "leaf front extend-add index missing (internal error)");
     }
   }
-  // owned LU slots with their front positions (column-major), by position
+  // owned LU slots with their front positions (column-major), by position;
+  // and for each of A's entries in the core its front and position
   std::vector<std::vector<std::pair<int, int>>> own(nf);
+  std::vector<int> entry_of(L.lu_nnz, -1);
+  for (size_t k = 0; k < L.core_map.size(); k++) entry_of[L.core_map[k]] = (int)k;
+  L.afront.assign(L.core_map.size(), -1);
+  L.apos.assign(L.core_map.size(), -1);
   for (int i = 0; i < cn; i++)
     for (int q = L.lu_rowptr[i]; q < L.lu_rowptr[i + 1]; q++) {
       const int j = L.lu_colidx[q], m = std::min(i, j);
@@ -218,6 +223,7 @@ int build_fronts(LeafPlan &L) {
       const int r = loc(f, i), c = loc(f, j);
       if (r < 0 || c < 0) return set_error(SNU_ERR_STRUCTURE, "LU entry outside its front (internal error)");
       own[f].push_back({c * L.ff[f] + r, q});
+      if (entry_of[q] >= 0) L.afront[entry_of[q]] = f, L.apos[entry_of[q]] = c * L.ff[f] + r;
     }
   for (int f = 0; f < nf; f++) {
     std::sort(own[f].begin(), own[f].end());

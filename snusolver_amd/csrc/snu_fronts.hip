@@ -6,19 +6,19 @@
 // of every matrix of a launch set sharing each launch:
 //   small fronts (the whole front fits the LDS): k_front_small does
 //     everything in one workgroup per front;
-//   larger fronts live in global memory: k_front_assemble, then the blocked
-//     partial LU on the dense kernels (k_diag_lu with the pivot clamp, the
-//     triangular solves and the update on the MFMA k_gemm), then
-//     k_front_writeback;
-//   k_front_schur gathers the root fronts' updates into each leaf's boundary
-//     Schur block S, which k_assemble_schur adds into the separator blocks.
-// Every front position receives its contributions in a fixed order (owned
-// slots, then the children in ascending order), so results do not depend on
-// scheduling.
+//   larger fronts live in global memory: k_extend_add builds them, then the
+//     blocked partial LU on the dense kernels (k_diag_lu with the pivot clamp,
+//     the triangular solves and the update on the MFMA k_gemm);
+//   k_extend_add then adds the root fronts' updates into the separator blocks
+//     (the reference's boundary Schur assembly).
+// The factors stay in the fronts, where the solves read them.
+// Every position receives its contributions in a fixed order, so results do
+// not depend on scheduling.
 #include <hip/hip_runtime.h>
 
 #include <utility>
 
+#include "snu_device.h"
 #include "snu_kernels.h"
 
 namespace snu {
@@ -33,19 +33,22 @@ __global__ __launch_bounds__(256) void k_front_small(const FrontDev *__restrict_
   const int f = D.f, nk = D.nk, n2 = f * f, tid = threadIdx.x, nt = blockDim.x;
   for (int i = tid; i < n2; i += nt) F[i] = T(0);
   __syncthreads();
-  const T *vin = (const T *)D.vals;
-  for (int q = tid; q < D.nslot; q += nt) F[D.pos[q]] = vin[D.slot[q]];
+  for (int q = tid; q < D.nent; q += nt) {
+    const AEntry e = D.ent[q];
+    F[e.pos] = (T)D.aval[e.idx];
+  }
   __syncthreads();
   // children's updates, one child after another (fixed summation order)
   // (lane = row within 64-row groups, wave = column modulo the waves)
   const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
   for (int c = 0; c < D.nchild; c++) {
     const FrontChild C = D.child[c];
-    const T *U = (const T *)C.U;
+    const auto U = gptr((const T *)C.U);
+    const auto rel = gptr(C.rel);
     const int nb = C.nb;
     for (int b = wv; b < nb; b += nw) {
-      const int cb = C.rel[b] * f;
-      for (int a = lane; a < nb; a += 64) F[C.rel[a] + cb] += U[a + (long long)b * C.ld];
+      const int cb = rel[b] * f;
+      for (int a = lane; a < nb; a += 64) F[rel[a] + cb] += U[a + (long long)b * C.ld];
     }
     __syncthreads();
   }
@@ -66,11 +69,9 @@ __global__ __launch_bounds__(256) void k_front_small(const FrontDev *__restrict_
     }
     __syncthreads();
   }
-  // factors into the owned slots; the whole front (the solves read its
-  // factors, its parent the update block) to global memory
-  T *vout = (T *)D.vals;
-  for (int q = tid; q < D.nslot; q += nt) vout[D.slot[q]] = F[D.pos[q]];
-  T *G = (T *)D.F;
+  // the whole front to global memory: the solves read its factors, its
+  // parent the update block
+  const auto G = gptr((T *)D.F);
   for (int i = tid; i < n2; i += nt) G[i] = F[i];
 }
 
@@ -158,112 +159,76 @@ void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, h
   hipLaunchKernelGGL(k_front_small<T>, dim3(nfront), dim3(256), lds, st, fr, (T)eps);
 }
 
-// Columns [c0, c0 + 64) of one front in global memory: zeroed, the owned
-// slots placed, the children's update columns that land there added (child
-// after child).  Within one workgroup the phases are separated by barriers;
-// different work items touch different columns.  The work item's ranges
-// (its owned slots, each child's columns in the chunk) come from the host.
+// One 64 x 64 tile of a target per workgroup, wave w its columns 16 w ..
+// 16 w + 15, lane = row, summed in registers and written once: every source
+// that lands in the tile (the host lists them, in order) is read through the
+// maps tile row -> its row, tile column -> its column, which each wave builds
+// in LDS from the source's ascending positions.  Bound by the update blocks
+// read and the target written; 64^3 7-point FP64, all heights and the
+// separator blocks together 1.6 ms.  (Fronts zeroed, filled from CSR factor
+// slots and added to child by child in memory took 3.5 ms, boundary Schur
+// blocks gathered and then added 2.1 ms, the factors' write-back into CSR
+// slots 1.5 ms.)
 template <typename T>
-__global__ __launch_bounds__(256) void k_front_assemble(const FrontDev *__restrict__ fr,
-                                                        const int4 *__restrict__ work,
-                                                        const int *__restrict__ wrange) {
-  const int4 w = work[blockIdx.x];
-  const FrontDev D = fr[w.x];
-  const int *rg = wrange + w.z;
-  const int f = D.f, c0 = w.y, c1 = min(f, c0 + 64), tid = threadIdx.x, nt = blockDim.x;
-  T *F = (T *)D.F;
-  const long long base = (long long)c0 * f, cnt = (long long)(c1 - c0) * f;
-  for (long long i = tid; i < cnt; i += nt) F[base + i] = T(0);
+__global__ __launch_bounds__(256) void k_extend_add(const AddTile *__restrict__ tiles,
+                                                    const AddSrc *__restrict__ src) {
+  __shared__ int rmap[4][64], cmap[4][64];
+  const AddTile t = tiles[blockIdx.x];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c0 = 16 * wave;
+  const auto C = gptr((T *)t.C) + min(lane, t.nr - 1);
+  T v[16];
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j] = T(0);
+  if (t.keep) {
+#pragma unroll
+    for (int j = 0; j < 16; j++) v[j] = C[min(c0 + j, t.nc - 1) * t.ldc];
+  }
+  for (int s = t.s0; s < t.s1; s++) {
+    const AddSrc S = src[s];
+    const auto pos = gptr(S.pos);
+    // (the fences keep the compiler from carrying a lane's own value over
+    // another lane's store; the wave's LDS accesses run in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    rmap[wave][lane] = -1;
+    cmap[wave][lane] = -1;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < S.rn) rmap[wave][pos[S.rb + lane] - S.r0] = S.rb + lane;
+    if (lane < S.cn) cmap[wave][pos[S.cb + lane] - S.c0] = S.cb + lane;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int rr = rmap[wave][lane], cc = cmap[wave][lane];
+    if (!__any(lane >= c0 && lane < c0 + 16 && cc >= 0)) continue;
+    const auto U = gptr((const T *)S.U) + max(rr, 0);
+    T u[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) u[j] = U[(long long)max(rl(cc, c0 + j), S.cb) * S.ld];
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+      if (rr >= 0 && rl(cc, c0 + j) >= 0) v[j] += u[j];
+  }
+  if (lane < t.nr) {
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+      if (c0 + j < t.nc) C[(c0 + j) * t.ldc] = v[j];
+  }
+  if (t.nent == 0) return;  // uniform
   __syncthreads();
-  const T *vin = (const T *)D.vals;
-  const int q0 = rg[0], q1 = rg[1];
-  for (int q = q0 + tid; q < q1; q += nt) F[D.pos[q]] = vin[D.slot[q]];
-  __syncthreads();
-  // children: wave w takes the child's columns b0 + w, b0 + w + 4, ...,
-  // its lanes the rows (reads of U run down its columns)
-  const int lane = tid & 63, wv = tid >> 6, nw = nt >> 6;
-  for (int c = 0; c < D.nchild; c++) {
-    const int b0 = rg[2 + 2 * c], b1 = rg[3 + 2 * c];
-    if (b0 == b1) continue;  // uniform: no column of this child lands here
-    const FrontChild C = D.child[c];
-    const T *U = (const T *)C.U;
-    const int nb = C.nb;
-    for (int b = b0 + wv; b < b1; b += nw) {
-      T *Fc = F + (long long)C.rel[b] * f;
-      const T *Ub = U + (long long)b * C.ld;
-      for (int a = lane; a < nb; a += 64) Fc[C.rel[a]] += Ub[a];
-    }
-    __syncthreads();
+  const auto base = gptr((T *)t.C);
+  for (int q = threadIdx.x; q < t.nent; q += 256) {
+    const AEntry e = t.ent[q];
+    base[e.pos] += (T)gptr(t.aval)[e.idx];
   }
 }
-
 template <typename T>
-__global__ __launch_bounds__(256) void k_front_writeback(const FrontDev *__restrict__ fr,
-                                                         const int4 *__restrict__ work,
-                                                         const int *__restrict__ wrange) {
-  const int4 w = work[blockIdx.x];
-  const FrontDev D = fr[w.x];
-  const T *F = (const T *)D.F;
-  T *vout = (T *)D.vals;
-  const int q0 = wrange[w.z], q1 = wrange[w.z + 1];
-  for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x) vout[D.slot[q]] = F[D.pos[q]];
-}
-
-template <typename T>
-void launch_front_assemble(const FrontDev *fr, const int4 *work, const int *wrange, int nwork, hipStream_t st) {
-  if (nwork <= 0) return;
-  hipLaunchKernelGGL(k_front_assemble<T>, dim3(nwork), dim3(256), 0, st, fr, work, wrange);
-}
-template <typename T>
-void launch_front_writeback(const FrontDev *fr, const int4 *work, const int *wrange, int nwork, hipStream_t st) {
-  if (nwork <= 0) return;
-  hipLaunchKernelGGL(k_front_writeback<T>, dim3(nwork), dim3(256), 0, st, fr, work, wrange);
-}
-
-// One 64 x 64 tile of a leaf's S per workgroup: accumulated column by column
-// (reads of the roots' updates run down their columns), then written row by
-// row through LDS (S is row-major).
-template <typename T>
-__global__ __launch_bounds__(256) void k_front_schur(const LeafSchurDev *__restrict__ ls,
-                                                     const int4 *__restrict__ tiles) {
-  __shared__ T t[64][65];
-  const int4 w = tiles[blockIdx.x];
-  const LeafSchurDev L = ls[w.x];
-  const int r0 = w.y, c0 = w.z, tid = threadIdx.x;
-  const int nr = min(64, L.nbr - r0), nc = min(64, L.nbc - c0);
-  for (int i = tid; i < 64 * 64; i += 256) t[i & 63][i >> 6] = T(0);
-  for (int k = 0; k < L.nroot; k++) {
-    const FrontRoot R = L.root[k];
-    const T *U = (const T *)R.U;
-    for (int i = tid; i < 64 * 64; i += 256) {
-      const int r = i & 63, c = i >> 6;
-      if (r < nr && c < nc) {
-        const int a = R.arow[r0 + r], b = R.acol[c0 + c];
-        if (a >= 0 && b >= 0) t[r][c] += U[a + (long long)b * R.ld];
-      }
-    }
-  }
-  __syncthreads();
-  T *S = (T *)L.S;
-  for (int i = tid; i < 64 * 64; i += 256) {
-    const int r = i >> 6, c = i & 63;
-    if (r < nr && c < nc) S[(long long)(r0 + r) * L.nbc + c0 + c] = t[r][c];
-  }
-}
-
-template <typename T>
-void launch_front_schur(const LeafSchurDev *ls, const int4 *tiles, int ntile, hipStream_t st) {
+void launch_extend_add(const AddTile *tiles, int ntile, const AddSrc *src, hipStream_t st) {
   if (ntile <= 0) return;
-  hipLaunchKernelGGL(k_front_schur<T>, dim3(ntile), dim3(256), 0, st, ls, tiles);
+  hipLaunchKernelGGL(k_extend_add<T>, dim3(ntile), dim3(256), 0, st, tiles, src);
 }
 
 #define SNU_FRONT_INST(T)                                                                      \
   template int front_small_max<T>();                                                           \
   template void launch_front_small<T>(const FrontDev *, int, int, double, hipStream_t);        \
   template void launch_front_inverse<T>(const FrontDev *, const int2 *, int, hipStream_t);     \
-  template void launch_front_assemble<T>(const FrontDev *, const int4 *, const int *, int, hipStream_t);  \
-  template void launch_front_writeback<T>(const FrontDev *, const int4 *, const int *, int, hipStream_t); \
-  template void launch_front_schur<T>(const LeafSchurDev *, const int4 *, int, hipStream_t);
+  template void launch_extend_add<T>(const AddTile *, int, const AddSrc *, hipStream_t);
 SNU_FRONT_INST(double)
 SNU_FRONT_INST(float)
 #undef SNU_FRONT_INST

@@ -36,6 +36,7 @@ struct LeafPlan {
   std::vector<int> fidx_ptr, fidx;       // B of each front: core indices beyond K
   std::vector<int> frel;                 // per B entry: local index in the parent
   std::vector<int> fslot_ptr, fslot, fpos;  // owned LU slots, front position (col-major)
+  std::vector<int> afront, apos;         // per entry of core_map: front, position in it
   std::vector<int> fchild_ptr, fchild;   // children, ascending
   std::vector<int> fsrow, fscol;         // root fronts: per B entry, boundary row / col (-1)
   long long fentries = 0;                // sum of front order squared

@@ -9,19 +9,6 @@
 
 namespace snu {
 
-// Single-copy separator storage, panels tile-compressed:
-//   R_p = [D_p | Up_p] : s_p x (s_p + nU_p), ld s_p
-//   Lp_p              : nL_p x s_p, ld nL_p
-// lmap / umap (from mapoff[p], A_p entries, ancestors bottom-up): stored row
-// of Lp_p / stored column of Up_p of each ancestor index, -1 if not stored.
-struct DenseDev {
-  const long long *offR, *offL, *mapoff;  // per heap block
-  const int *bsize, *nL;                  // per heap block
-  const int *lmap, *umap;
-  const int *aoff;                        // (block * nk + distance) -> ancestor offset
-  int nk;
-};
-
 // Solve work of the leaf fronts.  A unit is what one wave does between two
 // barriers: a whole front (orders the LDS factor kernel takes), or of a larger
 // front one 64-pivot block (forward or backward), one 64-row tile of its
@@ -43,10 +30,6 @@ struct SolveUnit {
 // owning matrix's arrays, so that leaves of several matrices can share a
 // launch.
 struct LeafDev {
-  const int *bcol_blk, *bcol_loc;        // boundary columns: block, offset
-  void *S;                               // boundary Schur block, nbr x nbc row-major
-  void *dense;                           // the matrix's dense separator arena
-  const DenseDev *dd;                    // the matrix's separator tables
   const SolveUnit *units;                // the leaf's solve units, by phase
   const int *fphase, *bphase;            // bounds of the forward / backward phases in units
   // per front row {s0, s1}: the children's update rows to add, in order (-1:
@@ -54,7 +37,6 @@ struct LeafDev {
   const int *pull, *pulllist;
   const int *bidx;                       // solve positions of the fronts' B entries
   int nfphase, nbphase;
-  int nbr, nbc;
   int vec;                               // the matrix's slot in the launch's VecDev table
   int pad;
 };
@@ -66,28 +48,41 @@ struct FrontChild {
   const int *rel;    // per entry of the child's B: index in this front (ascending)
   int ld, nb;        // the child's front order, |B| of the child
 };
+// One entry of A in a front or tile: position (from its first value), index in
+// A's values.
+struct AEntry {
+  int pos, idx;
+};
+// A front factored whole in LDS.
 struct FrontDev {
   void *F;                  // the front's values (f x f, column-major)
-  void *vals;               // the leaf's LU values (owned slots are read, then written)
-  void *inv;                // inverses of the pivot blocks' triangles (small: 16 x 16 blocks,
-                            // L^-1 below the diagonal, U^-1 on and above it; larger: per
-                            // 64-pivot block L^-1, then U^-1, 64 x 64 each)
-  const int *slot, *pos;    // owned LU slots and their positions in F (ascending positions)
+  void *inv;                // inverses of the pivot blocks' triangles: 16 x 16 blocks, L^-1 below
+                            // the diagonal, U^-1 on and above it (larger fronts: per 64-pivot
+                            // block L^-1, then U^-1, 64 x 64 each)
+  const double *aval;       // A's values
+  const AEntry *ent;        // its entries of A
   const FrontChild *child;  // children in ascending order (their updates are added in it)
-  int f, nk, nslot, nchild;
+  int f, nk, nent, nchild;
 };
-// Boundary Schur block of one leaf from the updates of its root fronts: S
-// (nbr x nbc, row-major) = sum over roots of U[arow[r], acol[c]] (entries
-// whose row or column the root lacks, -1, add nothing).
-struct FrontRoot {
+// Extend-add: one 64 x 64 tile of a target (a larger front, or a separator's
+// dense block) and the pieces of update blocks that land in it, added in
+// order.  pos: per entry of the update block's B, its index in the target;
+// entries [rb, rb + rn) are the tile's rows at pos - r0, [cb, cb + cn) its
+// columns at pos - c0.
+struct AddSrc {
   const void *U;
-  const int *arow, *acol;   // per S row / column: index in the root's B (-1)
-  int ld;
+  const int *pos;
+  int ld, rb, rn, cb, cn, r0, c0, pad;
 };
-struct LeafSchurDev {
-  void *S;
-  const FrontRoot *root;
-  int nbr, nbc, nroot;
+struct AddTile {
+  void *C;
+  const double *aval;
+  const AEntry *ent;
+  long long ldc;
+  int nr, nc;               // rows, columns of the tile
+  int s0, s1;               // its sources
+  int nent;                 // entries of A added after them
+  int keep;                 // 1: onto the values there, 0: onto zero
 };
 
 // A matrix's right-hand sides in the packed solve vectors.  One column: n
@@ -117,12 +112,14 @@ struct PermDev {
   long long ldb, ldx;
   int n, vec;
 };
-// Factor set-up of one matrix.
+// Factor set-up of one matrix: the separators' dense blocks and inverses are
+// zeroed, then A's separator entries put into place.
 struct PrepDev {
   void *arena, *inv;
   long long arena_len, inv_len;
   const double *aval;
-  const long long *adest;
+  const long long *adest;   // per separator entry: place in the arena
+  const int *asrc;          // and index in A's values
   long long nnz;
 };
 // FP64 refinement of one matrix: A in its CSR order, column-major vectors.
@@ -199,11 +196,6 @@ void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long m
                     hipStream_t st);
 // dst = src, bytes a multiple of 16
 void launch_copy(const void *src, void *dst, long long bytes, hipStream_t st);
-// boundary Schur rows into the dense blocks, per tile of 64 separator rows
-template <typename T>
-void launch_assemble_schur(int ntile, const int *tile_blk, const int *tile_row0,
-                           const int *tile_ptr, const int *seg_leaf, const int *seg_ri,
-                           const LeafDev *leaves, hipStream_t st);
 // mode 0: C -= sum A B; 1: C = A B; 2: C = -A B
 // C = A (first segment) per problem, 64 x 64 tiles numbered as the GEMM's
 template <typename T>
@@ -271,17 +263,10 @@ void launch_front_inverse(const FrontDev *fr, const int2 *blk, int nblk, hipStre
 // Largest front order the LDS kernel takes for this value type.
 template <typename T>
 int front_small_max();
-// Larger fronts, in global memory: assembly (zero, owned slots, children's
-// updates) and write-back of the owned slots after the dense partial LU, one
-// workgroup per (front, 64-column chunk) work item.
+// Extend-add of update blocks into target tiles (larger fronts before their
+// partial LU on the dense kernels; separator blocks), one workgroup per tile.
 template <typename T>
-void launch_front_assemble(const FrontDev *fr, const int4 *work, const int *wrange, int nwork, hipStream_t st);
-template <typename T>
-void launch_front_writeback(const FrontDev *fr, const int4 *work, const int *wrange, int nwork, hipStream_t st);
-// Boundary Schur blocks from the root fronts, one workgroup per 64 x 64 S
-// tile (leaf, first row, first column).
-template <typename T>
-void launch_front_schur(const LeafSchurDev *ls, const int4 *tiles, int ntile, hipStream_t st);
+void launch_extend_add(const AddTile *tiles, int ntile, const AddSrc *src, hipStream_t st);
 
 // ---- FP64 iterative refinement (one matrix per table entry) ----
 // r = b - A x into the packed vectors and max |b|, |r|, |x| per column into

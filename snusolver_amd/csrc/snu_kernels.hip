@@ -1,5 +1,5 @@
-// HIP kernels for gfx950 (MI355X): boundary Schur assembly, blocked no-pivot
-// dense LU on MFMA, FP64 refinement and the factor set-up.
+// HIP kernels for gfx950 (MI355X): blocked no-pivot dense LU on MFMA, FP64
+// refinement and the factor set-up.
 //
 // Wave size 64 throughout.
 #include <hip/hip_runtime.h>
@@ -31,88 +31,6 @@ void launch_fill(T *p, long long n, hipStream_t st) {
   hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)blocks), dim3(256), 0, st, p, n);
 }
 
-
-// Slot of separator entry (bi, lr) x (bj, lc) in the dense arena, -1 when
-// it lies in a panel tile that is not stored.
-__device__ __forceinline__ long long sep_index(const DenseDev &d, int bi,
-                                               int lr, int bj, int lc) {
-  if (bi == bj) return d.offR[bi] + lr + (long long)lc * d.bsize[bi];
-  if (bi > bj) {  // row block deeper: U panel of bi
-    int dist = (31 - __clz(bi)) - (31 - __clz(bj));
-    int c = d.umap[d.mapoff[bi] + d.aoff[bi * d.nk + dist] + lc];
-    return c < 0 ? -1 : d.offR[bi] + lr + (long long)(d.bsize[bi] + c) * d.bsize[bi];
-  }
-  int dist = (31 - __clz(bj)) - (31 - __clz(bi));
-  int r = d.lmap[d.mapoff[bj] + d.aoff[bj * d.nk + dist] + lr];
-  return r < 0 ? -1 : d.offL[bj] + r + (long long)lc * d.nL[bj];
-}
-
-// One workgroup per assembly tile: 64 consecutive rows of one separator
-// block.  For each contributing leaf (ascending rank) and each chunk of 64 of
-// its boundary columns, the S block is staged through LDS (rows read along
-// S's rows) and added into the dense block down its columns, where the 64
-// rows of the tile are contiguous: both sides coalesced.  Every element
-// receives its leaves' contributions in ascending rank order from one thread
-// (deterministic; no atomics); zero contributions are skipped.
-constexpr int kAsmWaves = 16;  // waves of an assembly workgroup
-template <typename T>
-__global__ __launch_bounds__(64 * kAsmWaves) void k_assemble_schur(
-    int ntile, const int *__restrict__ tile_blk, const int *__restrict__ tile_row0,
-    const int *__restrict__ tile_ptr, const int *__restrict__ seg_leaf,
-    const int *__restrict__ seg_ri, const LeafDev *__restrict__ leaves) {
-  __shared__ T st[64][65];
-  const int tile = blockIdx.x;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int bi = tile_blk[tile], row0 = tile_row0[tile];
-  for (int sg = tile_ptr[tile]; sg < tile_ptr[tile + 1]; sg++) {
-    const LeafDev L = leaves[seg_leaf[sg]];
-    const DenseDev dd = *L.dd;
-    T *dense = (T *)L.dense;
-    const T *S = (const T *)L.S;
-    const int *ri = seg_ri + (long long)sg * 64;
-    for (int c0 = 0; c0 < L.nbc; c0 += 64) {
-      // stage: wave w reads tile rows w, w + kAsmWaves, ... (64 columns each)
-      for (int rr = wave; rr < 64; rr += kAsmWaves) {
-        const int r = ri[rr];
-        T v = T(0);
-        if (r >= 0 && c0 + lane < L.nbc) v = S[(long long)r * L.nbc + c0 + lane];
-        st[rr][lane] = v;
-      }
-      __syncthreads();
-      // add: wave w takes columns w, w + kAsmWaves, ...; lane = tile row.
-      // The columns of one leaf go to distinct dense columns, so all targets
-      // of a lane are read before any is written (one round trip)
-      const int nc = min(64, L.nbc - c0);
-      constexpr int NJ = 64 / kAsmWaves;
-      // (every structurally nonzero entry of S lies in a stored tile; an
-      // index outside them, which the analysis rules out, is skipped)
-      T v[NJ], old[NJ];
-      long long idx[NJ];
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const int cc = wave + kAsmWaves * j;
-        v[j] = cc < nc ? st[lane][cc] : T(0);
-        idx[j] = -1;
-        if (v[j] != T(0)) {
-          idx[j] = sep_index(dd, bi, row0 + lane, L.bcol_blk[c0 + cc], L.bcol_loc[c0 + cc]);
-          if (idx[j] >= 0) old[j] = dense[idx[j]];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < NJ; j++)
-        if (idx[j] >= 0) dense[idx[j]] = old[j] + v[j];
-      __syncthreads();
-    }
-  }
-}
-template <typename T>
-void launch_assemble_schur(int ntile, const int *tile_blk, const int *tile_row0,
-                           const int *tile_ptr, const int *seg_leaf, const int *seg_ri,
-                           const LeafDev *leaves, hipStream_t st) {
-  if (ntile <= 0) return;
-  hipLaunchKernelGGL(k_assemble_schur<T>, dim3(ntile), dim3(64 * kAsmWaves), 0, st, ntile, tile_blk,
-                     tile_row0, tile_ptr, seg_leaf, seg_ri, leaves);
-}
 
 // ---------------------------------------------------------------------------
 // dense: grouped GEMM on MFMA (FP64 v_mfma_f64_16x16x4f64, FP32
@@ -1050,8 +968,8 @@ void launch_rowabs_max(const IrDev *tab, int nmat, int max_n, unsigned long long
   if (max_n <= 0) return;
   hipLaunchKernelGGL(k_rowabs_max, dim3(ir_blocks(max_n), nmat), dim3(256), 0, st, tab, out);
 }
-// Factor set-up for a set of matrices (one per blockIdx.y): zero the value
-// arena and the inverse blocks, then scatter A's values into their slots.
+// Factor set-up for a set of matrices (one per blockIdx.y): zero the
+// separators' blocks and inverses, then put A's separator entries into place.
 template <typename T>
 __global__ void k_prep_fill(const PrepDev *__restrict__ tab) {
   const PrepDev M = tab[blockIdx.y];
@@ -1067,10 +985,11 @@ __global__ void k_prep_scatter(const PrepDev *__restrict__ tab) {
   const PrepDev M = tab[blockIdx.y];
   const auto a = gptr((T *)M.arena);
   const auto dest = gptr(M.adest);
+  const auto src = gptr(M.asrc);
   const auto aval = gptr(M.aval);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.nnz;
        i += (long long)gridDim.x * blockDim.x)
-    a[dest[i]] = (T)aval[i];
+    a[dest[i]] = (T)aval[src[i]];
 }
 template <typename T>
 void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long max_nnz,
@@ -1096,9 +1015,6 @@ int device_lds_limit() {
 #define SNU_INSTANTIATE(T)                                                                    \
   template void launch_fill<T>(T *, long long, hipStream_t);                                  \
   template void launch_prepare<T>(const PrepDev *, int, long long, long long, hipStream_t);   \
-  template void launch_assemble_schur<T>(int, const int *, const int *, const int *,          \
-                                         const int *, const int *, const LeafDev *,           \
-                                         hipStream_t);                                        \
   template void launch_copy2d<T>(const GemmProbT<T> *, int, const GemmSegT<T> *, int, hipStream_t); \
   template void launch_gemm<T>(const GemmProbT<T> *, int, const GemmSegT<T> *, int, int,     \
                                hipStream_t);                                                  \

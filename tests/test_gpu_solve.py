@@ -88,3 +88,29 @@ def test_scratch_solve_column_by_column(S):
         finally:
             d_b.free()
             d_x.free()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 96, 97, 128, 129, 200])
+def test_dense_leaf_front_orders(S, precision, n):
+    """One full matrix as one front, at the orders where the front kernels and
+    the 64 x 64 extend-add tiles change: factors against a no-pivot LU in FP64
+    (FP32: within n u32 of the largest entry, the diagonally dominant LU's
+    rounding bound), solution at the path's bars."""
+    rng = np.random.default_rng(n)
+    D = rng.uniform(-1, 1, (n, n)) + 2.0 * n * np.eye(n)
+    rp = np.arange(0, n * n + 1, n)
+    A = S.CSR(n, rp, np.tile(np.arange(n), n), D.reshape(-1))
+    LU = D.copy()
+    for k in range(n):
+        LU[k + 1:, k] /= LU[k, k]
+        LU[k + 1:, k + 1:] -= np.outer(LU[k + 1:, k], LU[k, k + 1:])
+    tol = 1e-12 if precision == "fp64" else max(n, 8) * 2.0 ** -24
+    b = rng.standard_normal((n, 3))
+    with S.SnuMat(A, 1, order=np.arange(n), sizes=[n], device=0, precision=precision, ir_tol=1e-12) as M:
+        M.factorize()
+        v = M.leaf_values(0).reshape(n, n)
+        assert np.max(np.abs(v - LU)) <= tol * np.max(np.abs(LU))
+        x = np.linalg.solve(D, b)
+        for k in (1, 3):
+            assert np.max(np.abs(M.solve(b[:, :k]) - x[:, :k])) <= 1e-9 * np.max(np.abs(x))
