@@ -693,6 +693,14 @@ static int gather_leaf(const snumat_t *h, int rank, double *out) {
   HIPCHK(hipMemcpy(F.data(), vals<T>(h).farena + h->leaf_foff[rank], sizeof(T) * F.size(), hipMemcpyDeviceToHost));
   long long off = 0;
   for (size_t f = 0; f < L.ff.size(); f++) {
+    const int ff = L.ff[f];
+    if (ff > fmax)  // a larger front's diagonal blocks are factored behind it
+      for (int k = 0; k < L.fnk[f]; k += 64) {
+        const T *lu = F.data() + off + (long long)ff * ff + (long long)(k / 64) * kFrontInv + 8192;
+        const int nb = std::min(64, L.fnk[f] - k);
+        for (int c = 0; c < nb; c++)
+          for (int r = 0; r < nb; r++) F[off + k + r + (long long)(k + c) * ff] = lu[r + 64 * c];
+      }
     for (int q = L.fslot_ptr[f]; q < L.fslot_ptr[f + 1]; q++) out[L.fslot[q]] = (double)F[off + L.fpos[q]];
     off += (long long)L.ff[f] * L.ff[f] + front_inv_size(L.ff[f], L.fnk[f], fmax);
   }
@@ -825,11 +833,25 @@ extern "C" int snumat_leaf_values(const snumat_t *h, int rank, double *out) {
   }
   return h->prec == SNU_FP32 ? gather_leaf<float>(h, rank, out) : gather_leaf<double>(h, rank, out);
 }
+// The factored 64 x 64 diagonal blocks of separator e over its s x s block.
+template <typename T>
+static int overlay_diag(const snumat_t *h, int e, double *out) {
+  const int s = h->P.block_size[e];
+  std::vector<T> lu((size_t)(s + 63) / 64 * 4096);
+  if (lu.empty()) return SNU_OK;
+  HIPCHK(hipMemcpy(lu.data(), vals<T>(h).lu + h->lu_off[e], sizeof(T) * lu.size(), hipMemcpyDeviceToHost));
+  for (int k = 0; k < s; k += 64)
+    for (int c = k; c < std::min(s, k + 64); c++)
+      for (int r = k; r < std::min(s, k + 64); r++)
+        out[r + (size_t)c * s] = (double)lu[(size_t)(k / 64) * 4096 + (r - k) + 64 * (c - k)];
+  return SNU_OK;
+}
 extern "C" int snumat_sep_diag(const snumat_t *h, int e, double *out) {
   if (!h || e < 1 || e >= h->P.np) return set_error(SNU_ERR_BAD_INPUT, "bad separator");
   if (!h->factored) return set_error(SNU_ERR_NOT_FACTORED, "not factored");
   int s = h->P.block_size[e];
-  return read_values(h, h->P.offR[e], (size_t)s * s, out);
+  int rc = read_values(h, h->P.offR[e], (size_t)s * s, out);
+  return rc ? rc : h->prec == SNU_FP32 ? overlay_diag<float>(h, e, out) : overlay_diag<double>(h, e, out);
 }
 extern "C" int snumat_sep_block(const snumat_t *h, int i, int j, double *out) {
   if (!h || !out) return set_error(SNU_ERR_BAD_INPUT, "null handle or output");
@@ -860,7 +882,10 @@ extern "C" int snumat_sep_block(const snumat_t *h, int i, int j, double *out) {
     return SNU_OK;
   };
   int rc;
-  if (i == j) return copy(P.offR[i], si, si, si, out);
+  if (i == j) {
+    if ((rc = copy(P.offR[i], si, si, si, out)) || !h->factored) return rc;
+    return h->prec == SNU_FP32 ? overlay_diag<float>(h, i, out) : overlay_diag<double>(h, i, out);
+  }
   if (i > j) {  // columns of the U panel of i: runs of stored columns
     const int o = P.anc_off(i, j);
     for (int c = 0; c < sj;) {
@@ -917,6 +942,7 @@ void executed_work(const snumat *h, double *w) {
         const double nb = VV.fact.dp[L.p0 + q].nb;
         fl += 4.0 / 3.0 * nb * nb * nb;  // LU (2/3 nb^3) + both triangular inverses
       }
+      fl += L.flops;  // the panels
     } else if (is_gemm(L.kind)) {
       fl += L.flops;
     }
@@ -1006,11 +1032,17 @@ int test_diag_lu(int nb, T *D, int ld, T *Linv, T *Uinv) {
   HIPCHK(hipMalloc((void **)&dD, sizeof(T) * ld * nb));
   HIPCHK(hipMalloc((void **)&dI, sizeof(T) * 8192));
   HIPCHK(hipMemcpy(dD, D, sizeof(T) * ld * nb, hipMemcpyHostToDevice));
-  DiagProbT<T> p{dD, ld, nb, dI, dI + 4096, 64};
+  DiagProbT<T> p{};
+  p.D = p.LU = dD;  // one workgroup: the factors can replace the block
+  p.ld = p.ldlu = ld;
+  p.nb = nb;
+  p.Linv = dI;
+  p.Uinv = dI + 4096;
+  p.ldi = 64;
   DiagProbT<T> *dp;
   HIPCHK(hipMalloc((void **)&dp, sizeof(p)));
   HIPCHK(hipMemcpy(dp, &p, sizeof(p), hipMemcpyHostToDevice));
-  launch_diag_lu<T>(dp, 1, nullptr);
+  launch_diag_lu<T>(dp, 1, 0, nullptr);
   HIPCHK(hipGetLastError());
   HIPCHK(hipDeviceSynchronize());
   HIPCHK(hipMemcpy(D, dD, sizeof(T) * ld * nb, hipMemcpyDeviceToHost));

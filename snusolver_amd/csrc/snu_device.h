@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace snu {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -34,6 +36,40 @@ __device__ __forceinline__ double rld(double v, int l) {
 }
 __device__ __forceinline__ float rld(float v, int l) {
   return __int_as_float(rl(__float_as_int(v), l));
+}
+
+// lane K's value in each group of 16 lanes
+template <int K>
+__device__ __forceinline__ float bcast16(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + K, 0xf, 0xf, false));
+}
+template <int K>
+__device__ __forceinline__ double bcast16(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + K, 0xf, 0xf, false),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + K, 0xf, 0xf, false));
+}
+
+// MFMA fragments, 16x16x4 products.  A 16 x 16 block of a vector group (16 rows, 16 columns)
+// is one fragment: register r of lane l holds row frag_row(r), column l % 16,
+// which is both the layout the product leaves its result in and, taking the
+// four rows of register r as one K step, the layout of its second operand.  So
+// results feed the next product without passing through LDS; the first
+// operand's K columns follow the same frag_row order.
+template <typename T>
+using Frag = T __attribute__((ext_vector_type(4)));
+template <typename T>
+__device__ __forceinline__ int frag_row(int r, int lk) {
+  return std::is_same<T, double>::value ? 4 * r + lk : 4 * lk + r;
+}
+__device__ __forceinline__ Frag<double> mfma4(double a, double b, Frag<double> c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ Frag<float> mfma4(float a, float b, Frag<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ Frag<T> frag_zero() {
+  return Frag<T>{T(0), T(0), T(0), T(0)};
 }
 
 }  // namespace snu

@@ -26,7 +26,7 @@ namespace snu {
 // several matrices with equal (key, kind) are independent and are merged
 // into one launch.
 struct Launch {
-  int kind;  // 0 diag LU; GEMM (64 tile) 1: C = AB, 2: C -= AB, 6: C = -AB;
+  int kind;  // 0 diagonal blocks and their panels (tiles: panel workgroups); GEMM (64 tile) 1: C = AB, 2: C -= AB, 6: C = -AB;
              // GEMM (128 tile) 5: C -= AB, 10: C = AB, 11: C = -AB; 3: copy
              // C = A (GEMM descriptors, 64 x 64 tiles); GEMV 7: y = Ax, 8: y -= Ax
              // (one column), 17 / 18: the same on groups of 16 columns
@@ -91,7 +91,7 @@ struct FrontPlan {
 };
 // Values of the inverses kept behind a front (FrontDev::inv).
 inline long long front_inv_size(int f, int nk, int fmax) {
-  return f > fmax ? (nk + 63) / 64 * 8192LL : (nk + 15) / 16 * 256LL;
+  return f > fmax ? (nk + 63) / 64 * (long long)kFrontInv : (nk + 15) / 16 * 256LL;
 }
 template <typename T>
 void list_inverse_blocks(FrontPlan<T> &fp) {
@@ -109,6 +109,7 @@ template <typename T>
 struct Values {
   T *arena = nullptr;  // the separators' dense blocks
   T *inv = nullptr;    // per separator: full L^-1 then U^-1 (s x s each)
+  T *lu = nullptr;     // per separator: LU of its 64 x 64 diagonal blocks
   T *tmp = nullptr;    // products of the triangular inversion
   T *farena = nullptr; // leaf fronts (each f x f, then the inverses of its pivot blocks)
   FrontPlan<T> fronts;
@@ -174,7 +175,7 @@ struct snumat {
   snu::WorkDev wd;
   int wrows = 0;       // update rows of the leaf fronts (solves)
   // dense tables
-  std::vector<long long> inv_off;
+  std::vector<long long> inv_off, lu_off;
   long long inv_total = 0, tmp_total = 0;
   snu::Values<double> v64;
   snu::Values<float> v32;

@@ -327,10 +327,10 @@ inline long long fkey(int height, long long step) { return (long long)height * 1
 
 // Host-built launch descriptors of the dense factorization of one matrix.
 // Per tree level, bottom-up:
-//   for each 64-column step k of the diagonal blocks D: k_diag_lu (LU of the
-//   diagonal block and the inverses of its triangles, written into the
-//   separator's full L^-1 / U^-1), L21 <- L21 U11^-1 and U12 <- L11^-1 U12
-//   inside D (GEMM by the block inverses), trailing update of D (GEMM);
+//   for each 64-column step k of the diagonal blocks D: LU of the diagonal
+//   block and the inverses of its triangles (written into the separator's full
+//   L^-1 / U^-1), L21 <- L21 U11^-1 and U12 <- L11^-1 U12 inside D by the
+//   block inverses, trailing update of D (GEMM);
 //   then the full inverses L^-1, U^-1 of every separator of the level by
 //   recursive doubling (two grouped GEMMs per doubling step);
 //   then the panels in one pass each, Lp <- Lp U^-1 and Up <- L^-1 Up (GEMM
@@ -379,28 +379,18 @@ void build_dense_plan(snumat *h) {
         dp.Linv = Li(i) + k + (long long)k * s;
         dp.Uinv = Ui(i) + k + (long long)k * s;
         dp.ldi = s;
+        dp.LU = VV.lu + h->lu_off[i] + (long long)(k / 64) * 4096;
+        dp.ldlu = 64;
+        // L21 <- L21 U11^-1 (rows of D below the block) and U12 <- L11^-1 U12
+        // (row block of D right of it)
+        dp.m = s - k - nb;
+        dp.tile0 = d.tiles;
+        d.tiles += panel_tiles(dp.m);
+        d.flops += 4.0 * dp.m * nb * nb;
         h_dp.push_back(dp);
         d.np++;
       }
       if (d.np) out.push_back(d);
-      // L21 <- L21 U11^-1 (rows of D below the block) and U12 <- L11^-1 U12
-      // (row block of D right of the diagonal block): independent products,
-      // one grouped launch
-      Launch tr{1, (int)h_gp.size(), 0, 0, 0, fkey(height, ks + 1)};
-      for (int i = lo; i <= hi; i++) {
-        int s = P.block_size[i];
-        if (s <= k) continue;
-        int nb = std::min(64, s - k);
-        const T *U11i = Ui(i) + k + (long long)k * s;
-        T *X1 = R(i) + (k + nb) + (long long)k * s;
-        tr.np += add_gemm(h_gp, h_gs, tr.tiles, X1, s, s - k - nb, nb,
-                          {GemmSeg{X1, U11i, s, s, nb}}, tr.flops);
-        const T *L11i = Li(i) + k + (long long)k * s;
-        T *X = R(i) + k + (long long)(k + nb) * s;
-        tr.np += add_gemm(h_gp, h_gs, tr.tiles, X, s, nb, s - k - nb,
-                          {GemmSeg{L11i, X, s, s, nb}}, tr.flops);
-      }
-      if (tr.np) out.push_back(tr);
       // trailing update of D, outer-blocked by kPanel columns: inside a
       // panel [K0, K1) a step updates only the L-shaped rest of the panel
       // (its columns below the step, its rows right of the panel); the last
@@ -876,8 +866,13 @@ void merge_dense(const std::vector<const DensePlan<T> *> &in, DensePlan<T> &out)
       for (const Ref &r : g) {
         const DensePlan<T> &D = *in[r.src];
         const Launch &L = D.launches[r.idx];
-        out.dp.insert(out.dp.end(), D.dp.begin() + L.p0, D.dp.begin() + L.p0 + L.np);
+        for (int q = 0; q < L.np; q++) {
+          out.dp.push_back(D.dp[L.p0 + q]);
+          out.dp.back().tile0 += M.tiles;
+        }
         M.np += L.np;
+        M.tiles += L.tiles;
+        M.flops += L.flops;
       }
     } else {
       M.p0 = (int)out.gp.size();
@@ -942,7 +937,8 @@ int alloc_values(snumat *h) {
   Values<T> &VV = vals<T>(h);
   int rc;
   if ((rc = dalloc(h, &VV.arena, (size_t)h->arena_len)) || (rc = dalloc(h, &VV.inv, (size_t)h->inv_total)) ||
-      (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_total))))
+      (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_total))) ||
+      (rc = dalloc(h, &VV.lu, (size_t)std::max(1LL, h->lu_off[h->P.np]))))
     return rc;
   build_dense_plan<T>(h);
   return upload_dense_plan(VV.fact);
@@ -1160,14 +1156,13 @@ int build_front_plan(snumat *h) {
     for (int k = 0; k < kmax; k += 64) {
       const int step = k / 64;
       Launch d{0, (int)DP.dp.size(), 0, 0, 0, front_key(hh, step, 0)};
-      Launch tr{1, (int)DP.gp.size(), 0, 0, 0, front_key(hh, step, 1)};
       GemmBatch<T> tu;
       tu.rule = tile_rule<T>(h);
       for (const Large &D : lg[hh]) {
         if (D.nk <= k) continue;
         const int f = D.f, nb = std::min(64, D.nk - k), m = f - k - nb;
         T *F = D.F;
-        T *Li = D.inv + (long long)step * 8192, *Ui = Li + 64 * 64;
+        T *Li = D.inv + (long long)step * kFrontInv, *Ui = Li + 4096;
         DiagProbT<T> dp{};
         dp.D = F + k + (long long)k * f;
         dp.ld = f;
@@ -1175,14 +1170,17 @@ int build_front_plan(snumat *h) {
         dp.Linv = Li;
         dp.Uinv = Ui;
         dp.ldi = 64;
+        dp.LU = Ui + 4096;
+        dp.ldlu = 64;
         dp.eps = eps;
+        // L21 <- L21 U11^-1 (rows below), U12 <- L11^-1 U12 (columns right)
+        dp.m = m;
+        dp.tile0 = d.tiles;
+        d.tiles += panel_tiles(m);
+        d.flops += 4.0 * m * nb * nb;
         DP.dp.push_back(dp);
         d.np++;
-        // L21 <- L21 U11^-1 (rows below), U12 <- L11^-1 U12 (columns right)
-        T *X1 = F + (k + nb) + (long long)k * f;
-        tr.np += add_gemm(DP.gp, DP.gs, tr.tiles, X1, f, m, nb, {GemmSeg{X1, Ui, f, 64, nb}}, tr.flops);
-        T *X = F + k + (long long)(k + nb) * f;
-        tr.np += add_gemm(DP.gp, DP.gs, tr.tiles, X, f, nb, m, {GemmSeg{Li, X, 64, f, nb}}, tr.flops);
+        T *X1 = F + (k + nb) + (long long)k * f, *X = F + k + (long long)(k + nb) * f;
         // trailing update of the remaining front, outer-blocked by kPanel
         // pivots as for the separators (the last step of a panel applies
         // its rank-64 updates to F[K1:, K1:] at once)
@@ -1196,7 +1194,6 @@ int build_front_plan(snumat *h) {
         }
       }
       if (d.np) DP.launches.push_back(d);
-      if (tr.np) DP.launches.push_back(tr);
       tu.flush(DP.gp, DP.gs, DP.launches, front_key(hh, step, 3));
     }
   }
@@ -1522,6 +1519,8 @@ int upload(snumat *h) {
   h->wl = WorkLists();
   // ---- dense tables ----
   h->inv_off.assign(P.num_block + 1, 0);
+  h->lu_off.assign(np + 1, 0);
+  for (int p = 1; p < np; p++) h->lu_off[p + 1] = h->lu_off[p] + (P.block_size[p] + 63) / 64 * 4096LL;
   long long inv_total = 0;
   for (int p = 1; p < np; p++) {
     h->inv_off[p] = inv_total;
@@ -1590,7 +1589,8 @@ size_t estimate_device_bytes(const snumat *h) {
     }
     idx += 34.0 * L.ff.size() + 5.0 * L.fidx.size() + 3.0 * L.leaf_size;
   }
-  for (int p = 1; p < P.np; p++) inv += 2.0 * P.block_size[p] * P.block_size[p];
+  for (int p = 1; p < P.np; p++)
+    inv += 2.0 * P.block_size[p] * P.block_size[p] + (P.block_size[p] + 63) / 64 * 4096.0;
   double bytes = vs * ((double)P.dense_total + fronts + inv +
                        (double)inversion_tmp_size(P));
   bytes += 16.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block;
@@ -1644,7 +1644,7 @@ void run_launch(const Launch &L, const GemmProbT<T> *gp, const GemmSegT<T> *gs,
     }
   }
   switch (L.kind) {
-    case 0: launch_diag_lu(dp + L.p0, L.np, st); break;
+    case 0: launch_diag_lu(dp + L.p0, L.np, L.tiles, st); break;
     case 1: launch_gemm(gp + L.p0, L.np, gs, L.tiles, 1, st); break;
     case 2: launch_gemm(gp + L.p0, L.np, gs, L.tiles, 0, st); break;
     case 3: launch_copy2d(gp + L.p0, L.np, gs, L.tiles, st); break;

@@ -82,15 +82,6 @@ __global__ __launch_bounds__(256) void k_front_small(const FrontDev *__restrict_
 // own: inside k_front_small the unrolled substitution took its registers from
 // 30 to 256 and its workgroups per CU with them (batch of 96 2D matrices: 6.2
 // -> 9.2 ms per factorize + solve).
-template <int K>
-__device__ __forceinline__ float bcast16(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + K, 0xf, 0xf, false));
-}
-template <int K>
-__device__ __forceinline__ double bcast16(double v) {
-  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + K, 0xf, 0xf, false),
-                          __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + K, 0xf, 0xf, false));
-}
 template <typename T, int K>
 __device__ __forceinline__ void inv_step_l(T (&a)[16], T (&x)[16]) {
 #pragma unroll

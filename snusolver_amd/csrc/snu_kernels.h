@@ -58,7 +58,7 @@ struct FrontDev {
   void *F;                  // the front's values (f x f, column-major)
   void *inv;                // inverses of the pivot blocks' triangles: 16 x 16 blocks, L^-1 below
                             // the diagonal, U^-1 on and above it (larger fronts: per 64-pivot
-                            // block L^-1, then U^-1, 64 x 64 each)
+                            // block L^-1, U^-1 and LU, 64 x 64 each)
   const double *aval;       // A's values
   const AEntry *ent;        // its entries of A
   const FrontChild *child;  // children in ascending order (their updates are added in it)
@@ -149,15 +149,26 @@ struct GemmProbT {
   int seg0, nseg;
   int tiles_n, tile0;
 };
+// One 64-column step of a blocked LU: the diagonal block D (nb x nb), whose
+// factors go to LU (D itself keeps its values: several workgroups read it) and
+// whose triangles' inverses to Linv / Uinv; and the panels beside it, in place:
+// the m rows below D (D + nb) times U^-1, L^-1 times the m columns right of it
+// (D + nb ld), 64 rows / columns per workgroup from tile0 on.
 template <typename T>
 struct DiagProbT {
   T *D;
   long long ld;
-  int nb;
+  int nb, m;
   T *Linv, *Uinv;  // nb x nb diagonal blocks of the full inverses
   long long ldi;
+  T *LU;
+  long long ldlu;
+  int tile0;
   T eps;           // pivots of magnitude below eps become +-eps (0: none)
 };
+// Its panel workgroups (one also for a block without panels).
+inline int panel_tiles(int m) { return m > 0 ? 2 * ((m + 63) / 64) : 1; }
+constexpr int kFrontInv = 3 * 4096;  // values per 64-pivot block of a larger front: L^-1, U^-1, LU
 // y = / -= sum_seg A_seg (M x K) x_seg; tri: 0 dense, 1 lower triangular
 // single segment (columns k <= row), 2 upper (k >= row).  One column
 // (groups 0), or `groups` groups of 16 columns: x and y rows hold 16 adjacent
@@ -231,8 +242,9 @@ void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
 template <typename T>
 void launch_gemv16(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_tiles,
                    int total_wgs, int gstep, int max_groups, int mode, T *part, hipStream_t st);
+// Diagonal blocks and their panels (tiles: panel workgroups of all problems).
 template <typename T>
-void launch_diag_lu(const DiagProbT<T> *probs, int nprob, hipStream_t st);
+void launch_diag_lu(const DiagProbT<T> *probs, int nprob, int tiles, hipStream_t st);
 // Right-hand sides into / solutions out of the packed vectors; max_elems: the
 // largest n x groups of the matrices.  Out: add: x += instead of x =, for the
 // matrices whose active flag is set (null: all).

@@ -100,32 +100,6 @@ void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *
 }
 
 // ---------------------------------------------------------------------------
-// MFMA fragments of 16 columns
-// ---------------------------------------------------------------------------
-// 16x16x4 products.  A 16 x 16 block of a vector group (16 rows, 16 columns)
-// is one fragment: register r of lane l holds row frag_row(r), column l % 16,
-// which is both the layout the product leaves its result in and, taking the
-// four rows of register r as one K step, the layout of its second operand.  So
-// results feed the next product without passing through LDS; the first
-// operand's K columns follow the same frag_row order.
-template <typename T>
-using Frag = T __attribute__((ext_vector_type(4)));
-template <typename T>
-__device__ __forceinline__ int frag_row(int r, int lk) {
-  return std::is_same<T, double>::value ? 4 * r + lk : 4 * lk + r;
-}
-__device__ __forceinline__ Frag<double> mfma4(double a, double b, Frag<double> c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ Frag<float> mfma4(float a, float b, Frag<float> c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-template <typename T>
-__device__ __forceinline__ Frag<T> frag_zero() {
-  return Frag<T>{T(0), T(0), T(0), T(0)};
-}
-
-// ---------------------------------------------------------------------------
 // leaf fronts
 // ---------------------------------------------------------------------------
 // Forward, per front: w = (b of its pivots, 0) + the children's updates; y =
@@ -314,7 +288,7 @@ __device__ __forceinline__ T block_inverse1(const T *inv, int nbk, T v, int lane
 template <typename T, bool BWD>
 __device__ __forceinline__ void unit1(const LeafDev &L, const SolveUnit &U, T *x, T *W, int lane) {
   constexpr int RPL = sizeof(T) == 8 ? 1 : 2;
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * 8192;
+  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * kFrontInv;
   const int f = U.ld, nk = U.nk, r0 = 64 * U.s, nbk = min(64, nk - r0), r = r0 + min(lane, nbk - 1);
   if constexpr (!BWD) switch (U.kind) {
     case kFwdFront: fwd_front1<T, RPL>(L, U, x, W, lane); break;
@@ -598,7 +572,7 @@ __device__ __forceinline__ void block_inverse16(Frag<T> (&y)[4], const T *inv, i
 }
 template <typename T, bool BWD>
 __device__ __forceinline__ void unit16(const LeafDev &L, const SolveUnit &U, T *x, T *W, const SweepCtx &c) {
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * 8192;
+  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * kFrontInv;
   const int f = U.ld, nk = U.nk, r0 = 64 * U.s, nbk = min(64, nk - r0);
   T *xk = x + (long long)U.kpos * kColGroup, *wf = W + (long long)U.wrow * kColGroup;
   Frag<T> acc[4];
