@@ -1030,14 +1030,15 @@ int test_diag_lu(int nb, T *D, int ld, T *Linv, T *Uinv) {
   if (nb < 1 || nb > 64 || ld < nb) return set_error(SNU_ERR_BAD_INPUT, "bad block");
   T *dD, *dI;
   HIPCHK(hipMalloc((void **)&dD, sizeof(T) * ld * nb));
-  HIPCHK(hipMalloc((void **)&dI, sizeof(T) * 8192));
+  HIPCHK(hipMalloc((void **)&dI, sizeof(T) * 3 * 4096));
   HIPCHK(hipMemcpy(dD, D, sizeof(T) * ld * nb, hipMemcpyHostToDevice));
   DiagProbT<T> p{};
-  p.D = p.LU = dD;  // one workgroup: the factors can replace the block
-  p.ld = p.ldlu = ld;
+  p.D = dD;
+  p.ld = ld;
   p.nb = nb;
   p.Linv = dI;
   p.Uinv = dI + 4096;
+  p.LU = dI + 8192;
   p.ldi = 64;
   DiagProbT<T> *dp;
   HIPCHK(hipMalloc((void **)&dp, sizeof(p)));
@@ -1045,7 +1046,7 @@ int test_diag_lu(int nb, T *D, int ld, T *Linv, T *Uinv) {
   launch_diag_lu<T>(dp, 1, 0, nullptr);
   HIPCHK(hipGetLastError());
   HIPCHK(hipDeviceSynchronize());
-  HIPCHK(hipMemcpy(D, dD, sizeof(T) * ld * nb, hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy2D(D, sizeof(T) * ld, p.LU, sizeof(T) * 64, sizeof(T) * nb, nb, hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpy(Linv, dI, sizeof(T) * 4096, hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpy(Uinv, dI + 4096, sizeof(T) * 4096, hipMemcpyDeviceToHost));
   (void)hipFree(dD);

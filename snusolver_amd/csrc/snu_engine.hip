@@ -380,7 +380,6 @@ void build_dense_plan(snumat *h) {
         dp.Uinv = Ui(i) + k + (long long)k * s;
         dp.ldi = s;
         dp.LU = VV.lu + h->lu_off[i] + (long long)(k / 64) * 4096;
-        dp.ldlu = 64;
         // L21 <- L21 U11^-1 (rows of D below the block) and U12 <- L11^-1 U12
         // (row block of D right of it)
         dp.m = s - k - nb;
@@ -1171,7 +1170,6 @@ int build_front_plan(snumat *h) {
         dp.Uinv = Ui;
         dp.ldi = 64;
         dp.LU = Ui + 4096;
-        dp.ldlu = 64;
         dp.eps = eps;
         // L21 <- L21 U11^-1 (rows below), U12 <- L11^-1 U12 (columns right)
         dp.m = m;

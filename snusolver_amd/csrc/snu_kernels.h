@@ -161,8 +161,7 @@ struct DiagProbT {
   int nb, m;
   T *Linv, *Uinv;  // nb x nb diagonal blocks of the full inverses
   long long ldi;
-  T *LU;
-  long long ldlu;
+  T *LU;           // 64 x 64
   int tile0;
   T eps;           // pivots of magnitude below eps become +-eps (0: none)
 };

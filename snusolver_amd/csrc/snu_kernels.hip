@@ -660,177 +660,250 @@ void launch_gemm_variant(const GemmProbT<T> *probs, int nprob, const GemmSegT<T>
 // dense: diagonal block LU (no pivoting, as cusolverDnDgetrf with a null
 // ipiv / LAPACKE_mkl_dgetrfnp) and the inverses of its triangular factors.
 // ---------------------------------------------------------------------------
-// One workgroup of 8 waves per block (padded to 64 x 64 with a unit diagonal),
+// One workgroup of 4 waves per block (padded to 64 x 64 with a unit diagonal),
 // in LDS, blocked by 16 columns.  Per block column kb:
-//   (1) three waves, each factoring the 16 x 16 diagonal block for itself in
-//       registers (every group of 16 lanes holds it, row per lane, and reads a
+//   (1) two waves, each factoring the 16 x 16 diagonal block for itself in
+//       registers (every group of 16 lanes holds it, row per lane, and takes a
 //       pivot row by DPP broadcast: no barrier, no scalar registers), carry it
-//       over to
-//         the panel's 64 rows, lane = row (L21);
-//         the 64 columns that need L11^-1, lane = column: U12 right of the
-//         panel, X = L^-1 up to it;
-//         the rows of Y = U^-1 above the panel that need U11^-1, lane = row;
+//       over to what needs the inverse of its factors:
+//         lane = row: U11^-1 for the rows below the block (L21) and, of
+//         Y = U^-1, the rows above it; the block's own rows start from the
+//         identity and become Y's diagonal block;
+//         lane = column: L11^-1 for the columns right of the block (U12) and,
+//         of X = L^-1, those left of it; the block's own become X's;
 //   (2) all waves: the rank-16 updates A22 -= L21 U12, X -= L21 X_kb,
 //       Y -= Y_kb U12 on MFMA tiles.
-// Bound by the pivot chain of (1): 64 dependent broadcast, division and update
-// steps of about 0.23 us.  One block 20.6 us FP64, 17.0 FP32 (27.8 and 22.2 as
-// 64 barrier-separated steps over register tiles of 8 waves).
-// X's blocks below the diagonal and Y's above share one array; their diagonal
-// blocks have their own.  [column][row]; odd leading dimension: accesses along
-// rows are conflict-free too.
+// X and Y replace the factors in place: L21 and U12 are read by (2) of their
+// own block column alone, which leaves X's and Y's blocks there (all tiles are
+// computed before any is written).  [column][row]; odd leading dimension:
+// accesses along rows are conflict-free too.  42 KB FP64: three blocks share a
+// CU (84 KB and 8 waves, with X and Y beside the factors, kept it to one).
+// Bound by the pivot chain of (1): of one block's 45,000 cycles (18.6 us,
+// FP64) 19,000 are its 64 dependent broadcast, division and update steps,
+// 14,000 the tiles of (2), 7,000 reading the block and storing the results.
+// Broadcast inside the FMA (DPP), one reciprocal for the two quotients of a
+// step and tiles loaded together brought a step's launch with panels from 26.1
+// to 22.4 us FP64 and from 21.4 to 18.6 us FP32.
 template <typename T>
 struct DiagLds {
-  T A[64][65], XY[64][65], Xd[4][16][17], Yd[4][16][17];
+  T A[64][65], Xd[4][16][17];
 };
-// Column J of the diagonal block d (entry l16 of its columns per lane) and of
-// what a wave carries along in v.  rows: lanes with rows > J are below the
-// pivot, rows == J at it (64: a wave whose lanes are all below); keep: v[J]
-// stays as it is instead of being divided by the pivot.  One code path for the
-// three waves: the unrolled steps of a block are 10 KB of instructions, and
-// fetching three variants of them cost more than the arithmetic.
+// d[c] -= md u, v[c] -= mv u, u: lane J's d[c], for N columns from C on.
+// (s_nop: a DPP source must not have been written by the two instructions
+// before; the compiler's own hazard check does not see into the block.)
+#define SNU_RANK1(type, op)                                                                                        \
+  template <int J, int C, int N>                                                                                  \
+  __device__ __forceinline__ void rank1_block(type(&d)[16], type(&v)[16], type md, type mv) {                     \
+    static_assert(N == 1 || N == 2 || N == 4, "columns");                                                         \
+    if constexpr (N == 4)                                                                                         \
+      asm volatile("s_nop 1\n\t" op " %4, %0, -%9 row_newbcast:%10\n\t" op " %0, %0, -%8 row_newbcast:%10\n\t"     \
+                   op " %5, %1, -%9 row_newbcast:%10\n\t" op " %1, %1, -%8 row_newbcast:%10\n\t"                   \
+                   op " %6, %2, -%9 row_newbcast:%10\n\t" op " %2, %2, -%8 row_newbcast:%10\n\t"                   \
+                   op " %7, %3, -%9 row_newbcast:%10\n\t" op " %3, %3, -%8 row_newbcast:%10"                       \
+                   : "+v"(d[C]), "+v"(d[C + 1]), "+v"(d[C + 2]), "+v"(d[C + 3]), "+v"(v[C]), "+v"(v[C + 1]),       \
+                     "+v"(v[C + 2]), "+v"(v[C + 3])                                                               \
+                   : "v"(md), "v"(mv), "n"(J));                                                                   \
+    else if constexpr (N == 2)                                                                                    \
+      asm volatile("s_nop 1\n\t" op " %2, %0, -%5 row_newbcast:%6\n\t" op " %0, %0, -%4 row_newbcast:%6\n\t"       \
+                   op " %3, %1, -%5 row_newbcast:%6\n\t" op " %1, %1, -%4 row_newbcast:%6"                         \
+                   : "+v"(d[C]), "+v"(d[C + 1]), "+v"(v[C]), "+v"(v[C + 1])                                       \
+                   : "v"(md), "v"(mv), "n"(J));                                                                   \
+    else                                                                                                          \
+      asm volatile("s_nop 1\n\t" op " %1, %0, -%3 row_newbcast:%4\n\t" op " %0, %0, -%2 row_newbcast:%4\n\ts_nop 1" \
+                   : "+v"(d[C]), "+v"(v[C])                                                                       \
+                   : "v"(md), "v"(mv), "n"(J));                                                                   \
+  }
+SNU_RANK1(double, "v_fmac_f64_dpp")
+SNU_RANK1(float, "v_fmac_f32_dpp")
+#undef SNU_RANK1
+template <typename T, int J, int C>
+__device__ __forceinline__ void rank1(T (&d)[16], T (&v)[16], T md, T mv) {
+  // (two columns at least in a step's first block: the next step broadcasts
+  // its first column)
+  if constexpr (C < 16) {
+    constexpr int N = 16 - C >= 4 ? 4 : 16 - C >= 2 ? 2 : 1;
+    rank1_block<J, C, N>(d, v, md, mv);
+    rank1<T, J, C + N>(d, v, md, mv);
+  }
+}
+// frexp, reciprocal, fixup and ldexp in both precisions
+__device__ __forceinline__ double frexp_m(double x) { return __builtin_amdgcn_frexp_mant(x); }
+__device__ __forceinline__ float frexp_m(float x) { return __builtin_amdgcn_frexp_mantf(x); }
+__device__ __forceinline__ int frexp_e(double x) { return __builtin_amdgcn_frexp_exp(x); }
+__device__ __forceinline__ int frexp_e(float x) { return __builtin_amdgcn_frexp_expf(x); }
+__device__ __forceinline__ double recip(double x) { return __builtin_amdgcn_rcp(x); }
+__device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double div_end(double z, int e, double p, double a) {
+  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_ldexp(z, e), p, a);
+}
+__device__ __forceinline__ float div_end(float z, int e, float p, float a) {
+  return __builtin_amdgcn_div_fixupf(__builtin_amdgcn_ldexpf(z, e), p, a);
+}
+// Column J of the diagonal block d (entry l16 of its columns per lane; becomes
+// its LU factors) and of what a wave carries along in v.  keep: v[J] stays as
+// it is instead of being divided by the pivot.  One code path for both waves:
+// fetching variants of the unrolled steps cost more than the arithmetic.
+// d[J] / pivot and v[J] / pivot are rounded as by two divisions, with one
+// reciprocal (Newton steps and a last correction by the exact remainder, in
+// FMA, on the pivot's mantissa: Markstein's division).
 template <typename T, int J>
-__device__ __forceinline__ void diag_step(T (&d)[16], T (&v)[16], int rows, bool keep, T eps) {
+__device__ __forceinline__ void diag_step(T (&d)[16], T (&v)[16], int l16, bool keep, T eps) {
   // pivots of magnitude below eps become +-eps (the leaf pivots' rule; eps = 0
   // leaves them)
   T piv = bcast16<J>(d[J]);
   const T cl = piv < T(0) ? -eps : eps;
   piv = fabs(piv) < eps ? cl : piv;
-  // (rows of d up to the pivot are not read again: no mask)
-  const T md = d[J] / piv;
-  const T q = v[J] / piv, mv = rows > J ? q : T(0);
-  const T vk = keep ? v[J] : q, vj = rows == J ? piv : v[J];
-  v[J] = rows > J ? vk : vj;
-#pragma unroll
-  for (int c = J + 1; c < 16; c++) {
-    const T u = bcast16<J>(d[c]);
-    d[c] -= md * u;
-    v[c] -= mv * u;
-  }
-  // (opaque between steps: keeps later steps' values out of registers)
-#pragma unroll
-  for (int c = 0; c < 16; c++) asm volatile("" : "+v"(d[c]), "+v"(v[c]));
+  const T m = frexp_m(piv);
+  const int e = -frexp_e(piv);
+  T r = recip(m);
+  r = fma(fma(-m, r, T(1)), r, r);
+  if constexpr (std::is_same<T, double>::value) r = fma(fma(-m, r, T(1)), r, r);
+  T a = d[J] * r, b = v[J] * r;
+  a = fma(fma(-m, a, d[J]), r, a), b = fma(fma(-m, b, v[J]), r, b);
+  if constexpr (std::is_same<T, float>::value) a = fma(fma(-m, a, d[J]), r, a), b = fma(fma(-m, b, v[J]), r, b);
+  a = div_end(a, e, piv, d[J]), b = div_end(b, e, piv, v[J]);
+  const T md = l16 > J ? a : T(0);
+  d[J] = l16 > J ? a : l16 == J ? piv : d[J];
+  v[J] = keep ? v[J] : b;
+  asm volatile("" : "+v"(d[J]), "+v"(v[J]));  // (not left, with its inputs, for the end)
+  rank1<T, J, J + 1>(d, v, md, b);
 }
 template <typename T, int... J>
-__device__ __forceinline__ void diag_block(std::integer_sequence<int, J...>, T (&d)[16], T (&v)[16], int rows,
+__device__ __forceinline__ void diag_block(std::integer_sequence<int, J...>, T (&d)[16], T (&v)[16], int l16,
                                            bool keep, T eps) {
-  (diag_step<T, J>(d, v, rows, keep, eps), ...);
+  (diag_step<T, J>(d, v, l16, keep, eps), ...);
 }
+// store: this workgroup writes the block's factors to LU.
 template <typename T>
-__device__ __forceinline__ void factor_block(DiagLds<T> &S, const DiagProbT<T> &P, int lane, int wave) {
-  const int nb = P.nb, l16 = lane & 15, lk = lane >> 4;
+__device__ __forceinline__ void factor_block(DiagLds<T> &S, const DiagProbT<T> &P, int lane, int wave, bool store) {
+  const int nb = P.nb;
   {
     const auto D = gptr((const T *)P.D);
-    T v[8];
+    T v[16];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int c = wave + 8 * q;
+    for (int q = 0; q < 16; q++) {
+      const int c = wave + 4 * q;
       v[q] = D[min(lane, nb - 1) + (long long)min(c, nb - 1) * P.ld];
     }
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int c = wave + 8 * q;
+    for (int q = 0; q < 16; q++) {
+      const int c = wave + 4 * q;
       S.A[c][lane] = lane < nb && c < nb ? v[q] : (lane == c ? T(1) : T(0));
-      S.XY[c][lane] = T(0);
     }
   }
   __syncthreads();
+  const auto LU = gptr(P.LU);
+#pragma unroll 1
   for (int kb = 0; kb < 4; kb++) {
-    const int k0 = 16 * kb;
-    if (wave < 3) {
-      // wave 0: lane = row; the block and the panel by rows.  Wave 1: lane =
-      // column, all transposed (the scaled pivot row then plays the part of
-      // the multipliers).  Wave 2: rows of Y.  Strides of entry j and lane in
-      // d and v:
-      const int b16 = lane >> 4;
-      const bool tr = wave == 1, one = wave > 0 && b16 == kb;
+    asm volatile("" : "+v"(lane));  // (addresses and masks by lane are not kept from one pass to the next)
+    const int k0 = 16 * kb, l16 = lane & 15, lk = lane >> 4;
+    if (wave < 2) {
+      // wave 0: lane = row.  Wave 1: lane = column, all transposed (the scaled
+      // pivot row then plays the part of the multipliers).
+      const bool tr = wave == 1, own = lk == kb;
       const T *ds = &S.A[0][0] + (tr ? (k0 + l16) * 65 + k0 : k0 * 65 + k0 + l16);
-      const T *base = wave == 0 || (tr && b16 > kb) ? &S.A[0][0] : &S.XY[0][0];
-      const T *vs = base + (tr ? lane * 65 + k0 : k0 * 65 + lane);
-      const int sj = tr ? 1 : 65;
+      T *vs = &S.A[0][0] + (tr ? lane * 65 + k0 : k0 * 65 + lane);
       T d[16], v[16];
+      if (tr) {
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        d[j] = ds[j * sj];
-        v[j] = vs[j * sj];
+        for (int j = 0; j < 16; j++) d[j] = ds[j], v[j] = vs[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; j++) d[j] = ds[j * 65], v[j] = vs[j * 65];
       }
 #pragma unroll
-      for (int j = 0; j < 16; j++) asm volatile("" : "+v"(v[j]));  // loads not predicated one by one
-#pragma unroll
-      for (int j = 0; j < 16; j++) v[j] = one ? (j == l16 ? T(1) : T(0)) : v[j];
-      diag_block<T>(std::make_integer_sequence<int, 16>{}, d, v, wave == 0 ? lane - k0 : 64, tr, P.eps);
-      // (the diagonal block is read by all three before wave 0 writes it)
+      for (int j = 0; j < 16; j++) v[j] = own ? (j == l16 ? T(1) : T(0)) : v[j];
+      diag_block<T>(std::make_integer_sequence<int, 16>{}, d, v, l16, tr, P.eps);
+      // (the diagonal block is read by both before wave 0 writes it)
       __builtin_amdgcn_s_barrier();
-      T *out = wave == 0 || (tr && b16 > kb) ? &S.A[0][0] : &S.XY[0][0];
-      out += tr ? lane * 65 + k0 : k0 * 65 + lane;
-      int so = sj;
-      if (one) out = tr ? &S.Xd[kb][l16][0] : &S.Yd[kb][0][l16], so = tr ? 1 : 17;
-      if (wave < 2 || b16 <= kb) {
+      if (tr) {
+        if (own) vs = &S.Xd[kb][l16][0];
 #pragma unroll
-        for (int j = 0; j < 16; j++) out[j * so] = v[j];
+        for (int j = 0; j < 16; j++) vs[j] = v[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; j++) vs[j * 65] = v[j];
+        if (store && lane < 16) {
+#pragma unroll
+          for (int j = 0; j < 16; j++) LU[k0 * 65 + lane + j * 64] = d[j];
+        }
       }
     } else {
       __builtin_amdgcn_s_barrier();
     }
     __syncthreads();
-    const int n1 = 3 - kb, nA = n1 * n1, nX = n1 * (kb + 1);
-    for (int t = wave; t < nA + 2 * nX; t += 8) {
-      // C (16 x 16) -= A B: pointers to the blocks' first entries, leading
-      // dimensions of A and B
-      T *C;
-      const T *a, *b;
-      int lda = 65, ldb = 65;
-      if (t < nA) {
-        const int i = kb + 1 + t / n1, j = kb + 1 + t % n1;
-        C = &S.A[16 * j][16 * i];
-        a = &S.A[k0][16 * i];
-        b = &S.A[16 * j][k0];
-      } else if (t < nA + nX) {
-        const int i = kb + 1 + (t - nA) / (kb + 1), j = (t - nA) % (kb + 1);
-        C = &S.XY[16 * j][16 * i];
-        a = &S.A[k0][16 * i];
-        b = j < kb ? &S.XY[16 * j][k0] : &S.Xd[kb][0][0];
-        if (j == kb) ldb = 17;
-      } else {
-        const int i = (t - nA - nX) % (kb + 1), j = kb + 1 + (t - nA - nX) / (kb + 1);
-        C = &S.XY[16 * j][16 * i];
-        a = i < kb ? &S.XY[k0][16 * i] : &S.Yd[kb][0][0];
-        if (i == kb) lda = 17;
-        b = &S.A[16 * j][k0];
-      }
-      Frag<T> acc;
-      T av[4], bv[4];
+    // tile (i, j) (16 x 16 blocks) -= (i, kb) (kb, j) for i > kb (column
+    // j = wave), then for i <= kb, j > kb; X's and Y's first contribution
+    // (j == kb, i == kb) replaces L21 and U12.  A wave's tiles are loaded
+    // together, those past the last one as copies of it.
+    if (kb == 3) break;
+    // (i, j) of tile t: the digits of 4 i + j in base 16
+    const int nt = kb == 0 ? 15 : kb == 1 ? 12 : 7;
+    const unsigned long long list = kb == 0 ? 0x3321FEDCBA987654ull : kb == 1 ? 0x77777632FEDCBA98ull : 0xBBBBBBBBBB73FEDCull;
+    Frag<T> acc[4];
+    T av[4][4], bv[4][4];
+    int at[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int ij = (int)(list >> (4 * (wave + 4 * q))) & 15, i = ij >> 2, j = ij & 3;
+      at[q] = 16 * j * 65 + 16 * i;
+      const T *a = &S.A[k0][16 * i], *b = j == kb ? &S.Xd[kb][0][0] : &S.A[16 * j][k0], *c = &S.A[0][0] + at[q];
+      const int ldb = j == kb ? 17 : 65;
+      const bool first = i == kb || j == kb;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int k = frag_row<T>(r, lk);
-        acc[r] = C[l16 * 65 + k];
-        av[r] = -a[k * lda + l16];
-        bv[r] = b[l16 * ldb + k];
+        const T x = c[l16 * 65 + k];
+        acc[q][r] = first ? T(0) : x;
+        av[q][r] = a[k * 65 + l16];
+        bv[q][r] = b[l16 * ldb + k];
       }
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc = mfma4(av[r], bv[r], acc);
-#pragma unroll
-      for (int r = 0; r < 4; r++) C[l16 * 65 + frag_row<T>(r, lk)] = acc[r];
     }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) acc[q] = mfma4(-av[q][r], bv[q][r], acc[q]);
+    if (store) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int ij = (int)(list >> (4 * (wave + 4 * q))) & 15, i = ij >> 2, j = ij & 3;
+        if (i != kb && j != kb) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int k = k0 + frag_row<T>(r, lk);
+          LU[i == kb ? k + (16 * j + l16) * 64 : 16 * i + l16 + k * 64] = i == kb ? bv[q][r] : av[q][r];
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (wave + 4 * q < nt) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) (&S.A[0][0])[at[q] + l16 * 65 + frag_row<T>(r, lk)] = acc[q][r];
+      }
     __syncthreads();
   }
 }
+// The inverses (lower: L^-1, upper: U^-1) into their places.
 template <typename T>
-__device__ __forceinline__ void store_block(const DiagLds<T> &S, const DiagProbT<T> &P, int lane, int wave) {
+__device__ __forceinline__ void store_block(const DiagLds<T> &S, const DiagProbT<T> &P, int lane, int wave, bool lower,
+                                            bool upper) {
   const int rb = lane >> 4, l16 = lane & 15;
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int c = wave + 8 * q, cb = c >> 4;
+  for (int q = 0; q < 16; q++) {
+    const int c = wave + 4 * q, cb = q >> 2;
+    const T a = S.A[c][lane], xd = S.Xd[cb][c & 15][l16];
     if (lane < P.nb && c < P.nb) {
-      gptr(P.LU)[lane + (long long)c * P.ldlu] = S.A[c][lane];
-      gptr(P.Linv)[lane + (long long)c * P.ldi] = rb > cb ? S.XY[c][lane] : rb == cb ? S.Xd[cb][c & 15][l16] : T(0);
-      gptr(P.Uinv)[lane + (long long)c * P.ldi] = rb < cb ? S.XY[c][lane] : rb == cb ? S.Yd[cb][c & 15][l16] : T(0);
+      if (lower) gptr(P.Linv)[lane + c * P.ldi] = rb > cb ? a : rb == cb ? xd : T(0);
+      if (upper) gptr(P.Uinv)[lane + c * P.ldi] = rb <= cb ? a : T(0);
     }
   }
 }
 // Panel tile q of a problem: rows 64 q .. below the block times U^-1, or (from
-// the middle on) L^-1 times the columns right of it.  Waves 0-3 and 4-7 share
-// the 16-row (column) blocks of the tile, two 16 x 16 results each; a wave's
-// operand from the panel is loaded in MFMA layout before the block is factored.
+// the middle on) L^-1 times the columns right of it.  A wave takes 16 rows
+// (columns) of the tile; its operand from the panel is loaded in MFMA layout
+// before the block is factored.
 template <typename T>
 struct PanelTile {
   bool rows;     // below the block (else right of it)
@@ -841,7 +914,7 @@ template <typename T>
 __device__ __forceinline__ void load_panel(PanelTile<T> &t, const DiagProbT<T> &P, int q, int lane, int wave) {
   const int mt = (P.m + 63) >> 6, l16 = lane & 15, lk = lane >> 4;
   t.rows = q < mt;
-  const int base = 64 * (t.rows ? q : q - mt) + 16 * (wave & 3);
+  const int base = 64 * (t.rows ? q : q - mt) + 16 * wave;
   t.at = base;
   t.left = P.m - base;
   if (P.m == 0) return;  // a block without panels
@@ -857,35 +930,40 @@ __device__ __forceinline__ void load_panel(PanelTile<T> &t, const DiagProbT<T> &
     if (16 * (j >> 2) + frag_row<T>(j & 3, lk) >= P.nb) t.v[j] = T(0);
 }
 // inv(kb, o, k): entry (16 kb + k, 16 o + l16) of U^-1 (rows), or (16 o + l16,
-// 16 kb + k) of L^-1
+// 16 kb + k) of L^-1.  The operand order leaves consecutive rows of C in
+// consecutive lanes.
 template <typename T, class Inv>
-__device__ __forceinline__ void panel_product(const DiagProbT<T> &P, const PanelTile<T> &t, int lane, int wave, Inv inv) {
+__device__ __forceinline__ void panel_product(const DiagProbT<T> &P, const PanelTile<T> &t, int lane, Inv inv) {
   const int l16 = lane & 15, lk = lane >> 4;
   if (t.left <= 0) return;
-  T *C = P.D + (t.rows ? P.nb + t.at : (P.nb + (long long)t.at) * P.ld);
+  const auto C = gptr(P.D + (t.rows ? P.nb + t.at : (P.nb + (long long)t.at) * P.ld));
+  Frag<T> acc[4];
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const int o = 2 * (wave >> 2) + h;  // block of the inverse's columns (rows)
-    Frag<T> acc = frag_zero<T>();
+  for (int o = 0; o < 4; o++) acc[o] = frag_zero<T>();
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-      if (kb > o) continue;  // the inverse is triangular
+  for (int kb = 0; kb < 4; kb++) {
+    T w[4][4];  // (the inverse is triangular: blocks o >= kb)
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const T w = inv(kb, o, frag_row<T>(r, lk));
-        acc = t.rows ? mfma4(t.v[4 * kb + r], w, acc) : mfma4(w, t.v[4 * kb + r], acc);
-      }
-    }
+    for (int o = kb; o < 4; o++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) w[o][r] = inv(kb, o, frag_row<T>(r, lk));
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int o = kb; o < 4; o++)
+        acc[o] = t.rows ? mfma4(w[o][r], t.v[4 * kb + r], acc[o]) : mfma4(t.v[4 * kb + r], w[o][r], acc[o]);
+  }
+#pragma unroll
+  for (int o = 0; o < 4; o++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int a = frag_row<T>(r, lk);
-      if (t.rows) {  // rows at + a, column 16 o + l16
-        if (a < t.left && 16 * o + l16 < P.nb) gptr(C)[a + (long long)(16 * o + l16) * P.ld] = acc[r];
-      } else {  // row 16 o + a, column at + l16
-        if (l16 < t.left && 16 * o + a < P.nb) gptr(C)[16 * o + a + (long long)l16 * P.ld] = acc[r];
+      if (t.rows) {  // row at + l16, column 16 o + a
+        if (l16 < t.left && 16 * o + a < P.nb) C[l16 + (16 * o + a) * P.ld] = acc[o][r];
+      } else {  // row 16 o + l16, column at + a
+        if (a < t.left && 16 * o + l16 < P.nb) C[16 * o + l16 + a * P.ld] = acc[o][r];
       }
     }
-  }
 }
 template <typename T>
 __device__ __forceinline__ int find_tile(const DiagProbT<T> *__restrict__ probs, int nprob, int tile) {
@@ -899,39 +977,38 @@ __device__ __forceinline__ int find_tile(const DiagProbT<T> *__restrict__ probs,
 }
 // One block per workgroup.
 template <typename T>
-__global__ __launch_bounds__(512) void k_diag_lu(const DiagProbT<T> *__restrict__ probs) {
-  extern __shared__ __align__(16) char diag_raw[];
-  DiagLds<T> &S = *(DiagLds<T> *)diag_raw;
+__global__ __launch_bounds__(256, 3) void k_diag_lu(const DiagProbT<T> *__restrict__ probs) {
+  __shared__ DiagLds<T> S;
   const DiagProbT<T> P = probs[blockIdx.x];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  factor_block(S, P, lane, wave);
-  store_block(S, P, lane, wave);
+  factor_block(S, P, lane, wave, true);
+  store_block(S, P, lane, wave, true, true);
 }
 // One panel tile per workgroup, which factors the block for itself first (the
-// problem's first one stores it).
+// problem's first ones store it).
 template <typename T>
-__global__ __launch_bounds__(512) void k_diag_panel(const DiagProbT<T> *__restrict__ probs, int nprob) {
-  extern __shared__ __align__(16) char diag_raw[];
-  DiagLds<T> &S = *(DiagLds<T> *)diag_raw;
+__global__ __launch_bounds__(256, 3) void k_diag_panel(const DiagProbT<T> *__restrict__ probs, int nprob) {
+  __shared__ DiagLds<T> S;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const DiagProbT<T> P = probs[find_tile(probs, nprob, blockIdx.x)];
   const int q = blockIdx.x - P.tile0, l16 = lane & 15;
   PanelTile<T> t = {};
   load_panel(t, P, q, lane, wave);
-  factor_block(S, P, lane, wave);
+  factor_block(S, P, lane, wave, q == 0);
   // every wave holds its part of the tile before any overwrites it
 #pragma unroll
   for (int j = 0; j < 16; j++) asm volatile("" : "+v"(t.v[j]));
   __syncthreads();
-  panel_product(P, t, lane, wave, [&](int kb, int o, int k) {
-    if (t.rows) return kb == o ? S.Yd[o][l16][k] : S.XY[16 * o + l16][16 * kb + k];
-    return kb == o ? S.Xd[o][k][l16] : S.XY[16 * kb + k][16 * o + l16];
-  });
-  if (q == 0) store_block(S, P, lane, wave);
+  if (t.rows)
+    panel_product(P, t, lane, [&](int kb, int o, int k) { return S.A[16 * o + l16][16 * kb + k]; });
+  else
+    panel_product(P, t, lane, [&](int kb, int o, int k) { return kb == o ? S.Xd[o][k][l16] : S.A[16 * kb + k][16 * o + l16]; });
+  // (L^-1 by the first, U^-1 by the second if there are panels)
+  if (q <= (P.m > 0)) store_block(S, P, lane, wave, q == 0, q == 1 || P.m == 0);
 }
 // One panel tile per workgroup, by the stored inverse.
 template <typename T>
-__global__ __launch_bounds__(512) void k_panel(const DiagProbT<T> *__restrict__ probs, int nprob) {
+__global__ __launch_bounds__(256) void k_panel(const DiagProbT<T> *__restrict__ probs, int nprob) {
   __shared__ T W[64][65];  // the inverse that the tile takes, [column][row]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const DiagProbT<T> P = probs[find_tile(probs, nprob, blockIdx.x)];
@@ -940,43 +1017,39 @@ __global__ __launch_bounds__(512) void k_panel(const DiagProbT<T> *__restrict__ 
   PanelTile<T> t = {};
   load_panel(t, P, blockIdx.x - P.tile0, lane, wave);
   const auto inv = gptr((const T *)(t.rows ? P.Uinv : P.Linv));
-  T w[8];
+  T w[16];
 #pragma unroll
-  for (int q = 0; q < 8; q++) w[q] = inv[min(lane, P.nb - 1) + min(wave + 8 * q, P.nb - 1) * P.ldi];
+  for (int q = 0; q < 16; q++) w[q] = inv[min(lane, P.nb - 1) + min(wave + 4 * q, P.nb - 1) * P.ldi];
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int c = wave + 8 * q;
+  for (int q = 0; q < 16; q++) {
+    const int c = wave + 4 * q;
     W[c][lane] = lane < P.nb && c < P.nb ? w[q] : (lane == c ? T(1) : T(0));
   }
 #pragma unroll
   for (int j = 0; j < 16; j++) asm volatile("" : "+v"(t.v[j]));
   __syncthreads();
-  panel_product(P, t, lane, wave, [&](int kb, int o, int k) {
-    return t.rows ? W[16 * o + l16][16 * kb + k] : W[16 * kb + k][16 * o + l16];
-  });
+  if (t.rows)
+    panel_product(P, t, lane, [&](int kb, int o, int k) { return W[16 * o + l16][16 * kb + k]; });
+  else
+    panel_product(P, t, lane, [&](int kb, int o, int k) { return W[16 * kb + k][16 * o + l16]; });
 }
 // A step's blocks and panels as one launch, every panel workgroup factoring
-// its block for itself, while the launch fits the device in one round of
-// workgroups (256: one per CU in FP64).  The chain of a factorization's upper
-// levels is a sequence of such steps: 25 to 28 us FP64 and 20 to 24 us FP32
-// each, against 20.6 / 17.0 for the blocks and 8 to 10 more for a launch of
-// the panels.  With more panel tiles the blocks are factored once each first.
-// The product is the same code on the same values either way.
+// its block for itself, while the launch has at most one workgroup per CU (256).
+// The chain of a factorization's upper levels is a sequence of such steps: 22
+// us FP64 and 18.5 us FP32 each, against 19 / 16 for the blocks and 8 to 10
+// more for a launch of the panels.  With more panel tiles the blocks are
+// factored once each first.  The product is the same code on the same values
+// either way.
 template <typename T>
 void launch_diag_lu(const DiagProbT<T> *probs, int nprob, int tiles, hipStream_t st) {
   if (nprob <= 0) return;
-  constexpr int lds = (int)sizeof(DiagLds<T>), kFused = 256;
-  auto allow = [](const void *f) {
-    (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  };
+  constexpr int kFused = 256;
   if (tiles > 0 && tiles <= kFused) {
-    allow((const void *)k_diag_panel<T>);
-    hipLaunchKernelGGL(k_diag_panel<T>, dim3(tiles), dim3(512), lds, st, probs, nprob);
+    hipLaunchKernelGGL(k_diag_panel<T>, dim3(tiles), dim3(256), 0, st, probs, nprob);
     return;
   }
-  allow((const void *)k_diag_lu<T>);
-  hipLaunchKernelGGL(k_diag_lu<T>, dim3(nprob), dim3(512), lds, st, probs);
-  if (tiles > 0) hipLaunchKernelGGL(k_panel<T>, dim3(tiles), dim3(512), 0, st, probs, nprob);
+  hipLaunchKernelGGL(k_diag_lu<T>, dim3(nprob), dim3(256), 0, st, probs);
+  if (tiles > 0) hipLaunchKernelGGL(k_panel<T>, dim3(tiles), dim3(256), 0, st, probs, nprob);
 }
 
 // ---------------------------------------------------------------------------

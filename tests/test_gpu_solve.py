@@ -114,3 +114,28 @@ def test_dense_leaf_front_orders(S, precision, n):
         x = np.linalg.solve(D, b)
         for k in (1, 3):
             assert np.max(np.abs(M.solve(b[:, :k]) - x[:, :k])) <= 1e-9 * np.max(np.abs(x))
+
+
+@pytest.mark.parametrize("prec,power", [("fp64", 600), ("fp64", -600), ("fp32", 60), ("fp32", -60)])
+@pytest.mark.parametrize("nb", [1, 15, 16, 31, 33, 48, 49, 63, 64])
+def test_diagonal_block_scales_exactly(S, nb, prec, power):
+    """Factors of 2^power A are those of A scaled, bit for bit (the pivot
+    division keeps its rounding far from 1), and A = L U within the
+    elimination's bound nb u |L||U|, elementwise."""
+    import ctypes as C
+    f64 = prec == "fp64"
+    t, u = (np.float64, 2.0 ** -53) if f64 else (np.float32, 2.0 ** -24)
+    A = np.random.default_rng(nb).standard_normal((nb, nb)) + 2 * nb * np.eye(nb)
+    out = []
+    for p in (0, power):
+        D = np.asfortranarray((A.astype(t) * t(2.0 ** p)).astype(t))
+        Li, Ui = np.zeros(4096, t), np.zeros(4096, t)
+        f = S.lib().snu_test_diag_lu if f64 else S.lib().snu_test_diag_lu_f32
+        assert f(nb, *(x.ctypes.data_as(C.c_void_p) if i != 1 else nb for i, x in enumerate((D, None, Li, Ui)))) == 0
+        out.append((D, Li.reshape(64, 64)[:nb, :nb], Ui.reshape(64, 64)[:nb, :nb]))
+    (D, Li, Ui), (Ds, Lis, Uis) = out
+    sc = t(2.0 ** power)
+    assert np.array_equal(np.tril(D, -1), np.tril(Ds, -1)) and np.array_equal(np.triu(D) * sc, np.triu(Ds))
+    assert np.array_equal(Li, Lis) and np.array_equal(Ui, Uis * sc)
+    L, U = np.tril(D, -1).astype(np.float64) + np.eye(nb), np.triu(D).astype(np.float64)
+    assert np.all(np.abs(L @ U - A.astype(t)) <= (nb + 2) * u * (np.abs(L) @ np.abs(U)))
