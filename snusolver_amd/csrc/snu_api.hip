@@ -34,7 +34,11 @@ namespace {
 // The handle's stream and events, created on its first standalone use
 // (members of a batch run on the batch's stream).
 int ensure_stream(snumat *h) {
-  if (!h->stream) HIPCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
+  if (!h->stream) {
+    HIPCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
+    int rc = h->prec == SNU_FP32 ? make_side<float>({&h->v32.fact}, h->side) : make_side<double>({&h->v64.fact}, h->side);
+    if (rc) return rc;
+  }
   if (h->ev.empty()) {
     h->ev.resize(8);
     for (auto &e : h->ev) HIPCHK(hipEventCreate(&e));
@@ -290,6 +294,7 @@ template <typename T>
 int factorize_values(snumat *h, int stage) {
   Values<T> &VV = vals<T>(h);
   FactorSet fs;
+  fs.side = &h->side;
   fs.prep = h->d_prep;
   fs.nmat = 1;
   fs.max_len = std::max(h->arena_len, h->inv_total);

@@ -58,6 +58,7 @@ struct snubatch {
   bool factor_plan = false;  // merged dense plan built (on first factorize)
   bool use_graph = false;
   FactorGraph graph;
+  SideStream side;
   std::vector<hipEvent_t> ev;
   double t[16] = {0};
 };
@@ -99,6 +100,7 @@ void free_batch(snubatch *b) {
   b->allocs.clear();
   for (hipEvent_t e : b->ev) (void)hipEventDestroy(e);
   b->ev.clear();
+  free_side(b->side);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   b->stream = nullptr;
 }
@@ -179,6 +181,7 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
 template <typename T>
 int batch_factorize(snubatch *b) {
   FactorSet fs;
+  fs.side = &b->side;
   fs.prep = b->d_prep;
   fs.nmat = (int)b->mats.size();
   fs.max_len = b->max_len;
@@ -339,6 +342,13 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   hipError_t he = hipSetDevice(b->device);
   if (he == hipSuccess) he = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (he != hipSuccess) return fail(set_error(SNU_ERR_HIP, hipGetErrorString(he)));
+  {
+    std::vector<const DensePlan<double> *> d64;
+    std::vector<const DensePlan<float> *> d32;
+    for (const snumat *h : b->mats) d64.push_back(&h->v64.fact), d32.push_back(&h->v32.fact);
+    int rc = b->prec == SNU_FP32 ? make_side<float>(d32, b->side) : make_side<double>(d64, b->side);
+    if (rc) return fail(rc);
+  }
   b->ev.resize(8);
   for (auto &e : b->ev)
     if (hipEventCreate(&e) != hipSuccess) return fail(set_error(SNU_ERR_HIP, "event creation failed"));

@@ -141,6 +141,16 @@ struct WorkDev {
   int *tsrc = nullptr, ntarget = 0;
 };
 
+// Second stream of a factorization: the next height's diagonal blocks while the
+// Schur updates that they do not need run.  One per matrix or batch that has
+// work for it (make_side), made right after the owner's first stream: streams
+// made one after the other get different hardware queues (made at the first
+// factorization, with several handles alive, it shared its owner's, and
+// nothing overlapped).
+struct SideStream {
+  hipStream_t st = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
+};
 // A factorization's launch sequence captured once into a HIP graph and
 // replayed (no memset nodes: buffers are cleared by kernels).
 struct FactorGraph {
@@ -196,6 +206,7 @@ struct snumat {
   bool profile = false;
   bool use_graph = false;
   snu::FactorGraph graph;
+  snu::SideStream side;
   std::vector<hipEvent_t> ev, pev;
   double t[16] = {0};
   // C -= AB launches by tile: 64 x 64 (time ms, launches, GFLOP), then 128 x 128
@@ -278,6 +289,7 @@ void merge_gemv(const std::vector<const GemvPlan<T> *> &in, GemvPlan<T> &out);
 
 // Executors over a launch set.
 struct FactorSet {
+  SideStream *side = nullptr;  // (null: one stream)
   const PrepDev *prep;
   int nmat;
   long long max_len, max_nnz;
@@ -297,6 +309,10 @@ int run_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st,
                const std::vector<hipEvent_t> *ev, bool profile, std::vector<hipEvent_t> *pev,
                double *gemm_ms, FactorGraph *graph = nullptr);
 void free_graph(FactorGraph &g);
+// (no stream if no height of the plans, taken together, has work for it)
+template <typename T>
+int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s);
+void free_side(SideStream &s);
 struct SolveSet {
   const PermDev *perm;
   const VecDev *vec;

@@ -323,7 +323,8 @@ constexpr int kFrontLo = 64;
 
 // Launch keys: tree height (1 = parents of the leaves) major, then the step
 // inside the level.  Matrices of different depths align at equal height.
-inline long long fkey(int height, long long step) { return (long long)height * 100000000LL + step; }
+constexpr long long kHeight = 100000000LL, kPanels = 60000000LL, kNextD = 90000000LL;
+inline long long fkey(int height, long long step) { return height * kHeight + step; }
 
 // Host-built launch descriptors of the dense factorization of one matrix.
 // Per tree level, bottom-up:
@@ -337,8 +338,10 @@ inline long long fkey(int height, long long step) { return (long long)height * 1
 //   into scratch over the structurally nonzero rows / columns, K limited by
 //   the triangle, then copied back): the panels are read and written once
 //   instead of once per 64-column step;
-//   then one grouped GEMM for all Schur updates of the ancestors,
-//   K-concatenated over the level's separators below each of them.
+//   then the Schur updates of the ancestors, K-concatenated over the level's
+//   separators below each of them: one grouped GEMM for the diagonal blocks of
+//   the next level (step kNextD), which that level starts from, and one for
+//   all others (kNextD + 1).
 template <typename T>
 void build_dense_plan(snumat *h) {
   using GemmSeg = GemmSegT<T>;
@@ -501,9 +504,9 @@ void build_dense_plan(snumat *h) {
         if (nu && rule.pick(s, nu) == 128) big += (long long)((s + 127) / 128) * ((nu + 127) / 128);
       }
       const int W = big >= rule.min128() ? 128 : 64;
-      Launch pm{W == 128 ? 10 : 1, (int)h_gp.size(), 0, 0, 0, fkey(height, 60000000LL)};
+      Launch pm{W == 128 ? 10 : 1, (int)h_gp.size(), 0, 0, 0, fkey(height, kPanels)};
       std::vector<GemmProbT<T>> cp;
-      Launch cl{3, 0, 0, 0, 0, fkey(height, 60000001LL)};
+      Launch cl{3, 0, 0, 0, 0, fkey(height, kPanels + 1)};
       double cfl = 0;
       long long toff = 0;
       for (int i = lo; i <= hi; i++) {
@@ -539,13 +542,13 @@ void build_dense_plan(snumat *h) {
       }
     }
     // Schur updates of every ancestor, K-concatenated over the level's
-    // separators below it (one grouped launch per level).  Emitted per
+    // separators below it (the next level's diagonal blocks first).  Emitted per
     // target tile (64 rows / columns aligned to the first index of the block
     // they belong to, the tiles of the compressed storage), with only the
     // contributors that store both the L-panel rows and the U-panel columns
     // of that tile (the other products are exactly zero).
-    GemmBatch<T> sc;
-    sc.rule = rule;
+    GemmBatch<T> sc, sn;
+    sc.rule = sn.rule = rule;
     for (int p = 1; p < lo; p++) {
       int lp = 31 - __builtin_clz(p);
       int first = p << (l - lp), last = ((p + 1) << (l - lp)) - 1;
@@ -563,13 +566,15 @@ void build_dense_plan(snumat *h) {
           if (P.umap[p][o + t] >= 0) anU.push_back({sp + P.umap[p][o + t], w, o + t});
         }
       }
-      for (int pass = 0; pass < 2; pass++) {  // 0: R_p = [D_p | Up_p], 1: Lp_p
-        std::vector<std::array<int, 3>> rows = pass == 0 ? own : anL, cols = own;
-        if (pass == 0) cols.insert(cols.end(), anU.begin(), anU.end());
+      for (int pass = 0; pass < 3; pass++) {  // 0: D_p (not a parent's: R_p = [D_p | Up_p]), 1: Up_p, 2: Lp_p
+        const bool parent = lp == l - 1;
+        std::vector<std::array<int, 3>> rows = pass == 2 ? anL : own, cols = pass == 1 ? anU : own;
+        if (pass == 0 && !parent) cols.insert(cols.end(), anU.begin(), anU.end());
+        if (pass == 1 && !parent) continue;
         const int tm = (int)rows.size(), tn = (int)cols.size();
         if (!tm || !tn) continue;
-        T *Cb = pass == 0 ? R(p) : Lp(p);
-        const int ldc = pass == 0 ? sp : P.nL[p];
+        T *Cb = pass == 2 ? Lp(p) : R(p);
+        const int ldc = pass == 2 ? P.nL[p] : sp;
         // index of a tile in contributor i's ancestor space
         auto ix = [&](int i, const std::array<int, 3> &t) {
           return P.anc_off(i, p) + (t[2] < 0 ? -1 - t[2] : sp + t[2]);
@@ -595,7 +600,7 @@ void build_dense_plan(snumat *h) {
           int mt = 0, nt = 0;
           for (int x = 0; x < ta; x++) mt += rows[a + x][1];
           for (int y = 0; y < tb; y++) nt += cols[b + y][1];
-          sc.add(Cb + rows[a][0] + (long long)cols[b][0] * ldc, ldc, mt, nt, segs_of(w, a, b));
+          (parent && pass == 0 ? sn : sc).add(Cb + rows[a][0] + (long long)cols[b][0] * ldc, ldc, mt, nt, segs_of(w, a, b));
         };
         auto nonempty = [&](int a, int b) { return a < tm && b < tn && !who[(size_t)a * tn + b].empty(); };
         // tiles a, a + 1 (rows) are consecutive in every contributor's L
@@ -632,7 +637,8 @@ void build_dense_plan(snumat *h) {
             }
       }
     }
-    sc.flush(h_gp, h_gs, out, fkey(height, 90000000LL));
+    sn.flush(h_gp, h_gs, out, fkey(height, kNextD));
+    sc.flush(h_gp, h_gs, out, fkey(height, kNextD + 1));
   }
 }
 
@@ -1602,8 +1608,15 @@ void free_graph(FactorGraph &g) {
   g.exec = nullptr;
 }
 
+void free_side(SideStream &s) {
+  if (s.fork) (void)hipEventDestroy(s.fork);
+  if (s.join) (void)hipEventDestroy(s.join);
+  if (s.st) (void)hipStreamDestroy(s.st);
+  s = SideStream();
+}
 void free_device(snumat *h) {
   free_graph(h->graph);
+  free_side(h->side);
   free_gemv_plan(h->v64.sp);
   free_gemv_plan(h->v32.sp);
   free_dense_plan(h->v64.fact);
@@ -1664,6 +1677,37 @@ void run_launch(const Launch &L, const GemmProbT<T> *gp, const GemmSegT<T> *gs,
 }
 }  // namespace
 
+// Whether the launches from i on, the Schur updates of a height that its
+// parents' diagonal blocks do not need, are work enough to run those beside.  A
+// chain of diagonal blocks leaves most CUs idle (a step: 22 us, at most 256
+// workgroups), so its time goes where the updates take longer: 64^3 FP64 26.2
+// -> 24.9 ms, 56^3 27-point FP32 15.2 -> 13.8, 45x37x29 4.37 -> 4.29.  Below
+// about 20 us of updates a fork and its join cost what they give (a batch of 96
+// 2D matrices: 3.55 ms from 1 GFLOP on, 3.60 from 0.2).
+constexpr double kBesideFlops = 1e9;
+inline bool beside(double flops) { return flops >= kBesideFlops; }
+template <typename T>
+bool beside(const DensePlan<T> &plan, size_t i) {
+  const long long key = plan.launches[i].key;
+  if (key % kHeight != kNextD + 1) return false;
+  double flops = 0;
+  for (; i < plan.launches.size() && plan.launches[i].key == key; i++) flops += plan.launches[i].flops;
+  return beside(flops);
+}
+template <typename T>
+int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s) {
+  std::map<long long, double> flops;
+  for (const DensePlan<T> *p : in)
+    for (const Launch &L : p->launches)
+      if (L.key % kHeight == kNextD + 1) flops[L.key] += L.flops;
+  if (std::none_of(flops.begin(), flops.end(), [](const auto &f) { return beside(f.second); })) return SNU_OK;
+  hipError_t e = hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&s.fork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&s.join, hipEventDisableTiming);
+  if (e == hipSuccess) return SNU_OK;
+  free_side(s);
+  return set_error(SNU_ERR_HIP, std::string("second stream: ") + hipGetErrorString(e));
+}
 // ev (optional): 6 events marking prepare / leaf fronts / leaf Schur /
 // assembly / dense; pev (optional, with profile): a begin/end pair per GEMM
 // launch (the leaf fronts' launches, then the dense ones), their times summed
@@ -1699,10 +1743,10 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
     for (auto &e : *pev) HIPCHK(hipEventCreate(&e));
   }
   int g = 0;
-  auto run_timed = [&](const Launch &L, const DensePlan<T> &dp) -> int {
+  auto run_timed = [&](const Launch &L, const DensePlan<T> &dp, hipStream_t on) -> int {
     const bool gm = prof && is_gemm(L.kind);
     if (gm) HIPCHK(hipEventRecord((*pev)[2 * g], st));
-    run_launch<T>(L, dp.d_gp, dp.d_gs, dp.d_dp, nullptr, nullptr, nullptr, st, fs.split);
+    run_launch<T>(L, dp.d_gp, dp.d_gs, dp.d_dp, nullptr, nullptr, nullptr, on, fs.split);
     if (gm) HIPCHK(hipEventRecord((*pev)[2 * g++ + 1], st));
     return SNU_OK;
   };
@@ -1714,7 +1758,7 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
     launch_front_small<T>(fp.d_small + lv.small0 + lv.nsmall_lo, lv.nsmall - lv.nsmall_lo, lv.max_f, fs.eps, st);
     launch_extend_add<T>(fp.d_tiles + lv.tile0, lv.ntile, fp.d_src, st);
     for (; li < nl && front_key_height(fp.dense.launches[li].key) == hh; li++) {
-      int rc = run_timed(fp.dense.launches[li], fp.dense);
+      int rc = run_timed(fp.dense.launches[li], fp.dense, st);
       if (rc) return rc;
     }
   }
@@ -1727,10 +1771,31 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   launch_extend_add<T>(fp.d_tiles + fp.sep0, (int)fp.tiles.size() - fp.sep0, fp.d_src, st);
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[4], st));
-  for (const Launch &L : plan.launches) {
-    int rc = run_timed(L, plan);
-    if (rc) return rc;
+  // the diagonal blocks of the height above and their inverses on the second
+  // stream, from the updates of those blocks until its panels need them, beside
+  // the other Schur updates of the height (one stream when profiled: launches
+  // are timed one by one)
+  SideStream *side = prof ? nullptr : fs.side;
+  bool forked = false;
+  auto join = [&]() -> int {
+    HIPCHK(hipEventRecord(side->join, side->st));
+    HIPCHK(hipStreamWaitEvent(st, side->join, 0));
+    forked = false;
+    return SNU_OK;
+  };
+  int rc;
+  for (size_t i = 0; i < plan.launches.size(); i++) {
+    const Launch &L = plan.launches[i];
+    const long long step = L.key % kHeight;
+    if (side && side->st && !forked && beside(plan, i)) {
+      HIPCHK(hipEventRecord(side->fork, st));
+      HIPCHK(hipStreamWaitEvent(side->st, side->fork, 0));
+      forked = true;
+    }
+    if (forked && step >= kPanels && step < kNextD && (rc = join())) return rc;
+    if ((rc = run_timed(L, plan, forked && step < kPanels ? side->st : st))) return rc;
   }
+  if (forked && (rc = join())) return rc;
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[5], st));
   return SNU_OK;
@@ -1740,7 +1805,6 @@ template <typename T>
 int run_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st,
                const std::vector<hipEvent_t> *ev, bool profile, std::vector<hipEvent_t> *pev,
                double *gemm_ms, FactorGraph *graph) {
-  const WorkDev &wd = *fs.wd;
   int rc;
   if (graph && !profile) {
     // replay the captured launch sequence (captured on first use)
@@ -1873,6 +1937,7 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
   template void free_dense_plan<T>(DensePlan<T> &);                                           \
   template void merge_dense<T>(const std::vector<const DensePlan<T> *> &, DensePlan<T> &);    \
   template void merge_gemv<T>(const std::vector<const GemvPlan<T> *> &, GemvPlan<T> &);       \
+  template int make_side<T>(const std::vector<const DensePlan<T> *> &, SideStream &);           \
   template int run_factor<T>(const FactorSet &, const DensePlan<T> &, hipStream_t,            \
                              const std::vector<hipEvent_t> *, bool, std::vector<hipEvent_t> *, \
                              double *, FactorGraph *);                                        \

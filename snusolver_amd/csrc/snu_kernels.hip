@@ -979,6 +979,7 @@ __device__ __forceinline__ int find_tile(const DiagProbT<T> *__restrict__ probs,
 template <typename T>
 __global__ __launch_bounds__(256, 3) void k_diag_lu(const DiagProbT<T> *__restrict__ probs) {
   __shared__ DiagLds<T> S;
+  __builtin_amdgcn_s_setprio(3);  // (before waves of Schur updates on the same CU: 14.0 -> 13.8 ms, 56^3 FP32)
   const DiagProbT<T> P = probs[blockIdx.x];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   factor_block(S, P, lane, wave, true);
@@ -989,6 +990,7 @@ __global__ __launch_bounds__(256, 3) void k_diag_lu(const DiagProbT<T> *__restri
 template <typename T>
 __global__ __launch_bounds__(256, 3) void k_diag_panel(const DiagProbT<T> *__restrict__ probs, int nprob) {
   __shared__ DiagLds<T> S;
+  __builtin_amdgcn_s_setprio(3);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const DiagProbT<T> P = probs[find_tile(probs, nprob, blockIdx.x)];
   const int q = blockIdx.x - P.tile0, l16 = lane & 15;

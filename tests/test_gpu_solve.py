@@ -139,3 +139,21 @@ def test_diagonal_block_scales_exactly(S, nb, prec, power):
     assert np.array_equal(Li, Lis) and np.array_equal(Ui, Uis * sc)
     L, U = np.tril(D, -1).astype(np.float64) + np.eye(nb), np.triu(D).astype(np.float64)
     assert np.all(np.abs(L @ U - A.astype(t)) <= (nb + 2) * u * (np.abs(L) @ np.abs(U)))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_diagonal_blocks_beside_schur_updates(S, prec):
+    """Diagonal blocks on the second stream beside the Schur updates leave the
+    bits of one stream (profiled factorizations run on one), factorization
+    after factorization and as replays of a graph."""
+    A = S.gen_grid(45, 37, 29, 7, 0, 6.1, 4)
+    order, sizes = S.order_grid(45, 37, 29, 32)
+    b = S.gen_rhs(A, 1, 1)[1][:, 0]
+    with S.SnuMat(A, 32, order=order, sizes=sizes, device=0, precision=prec) as M:
+        S._check(S.lib().snumat_set_profiling(M._h, 1))
+        x = M.factorize().solve(b)
+        S._check(S.lib().snumat_set_profiling(M._h, 0))
+        assert S.backward_error(A, x, b) <= 1e-12
+        for graph in (0, 0, 1, 1, 0, 1):
+            S._check(S.lib().snumat_use_graph(M._h, graph))
+            assert np.array_equal(M.factorize().solve(b), x)
