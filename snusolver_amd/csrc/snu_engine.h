@@ -71,8 +71,9 @@ struct GemvPlan {
 // blocked partial LU as a keyed launch list (key: height, step within it);
 // the extend-add tiles of the separator blocks (after the last height).
 struct FrontLevel {
-  int small0 = 0, nsmall = 0, max_f = 0;
-  int nsmall_lo = 0, max_f_lo = 0;  // the first nsmall_lo small fronts have order <= kFrontLo
+  // small fronts from small0 on, by class: orders up to kFrontWave, up to
+  // kFrontLo, above; the largest order of each
+  int small0 = 0, nsmall[3] = {0, 0, 0}, max_f[3] = {0, 0, 0};
   int tile0 = 0, ntile = 0;
 };
 template <typename T>

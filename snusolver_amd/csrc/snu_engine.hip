@@ -318,8 +318,10 @@ std::vector<std::pair<int, int>> nz_runs(int len, F any) {
 // Outer panel width of the blocked LU of the separators' diagonal blocks.
 constexpr int kPanel = 512;
 
-// Small fronts up to this order run in their own launch per height.
+// Small fronts by order, a launch per height each: one wave per front, one
+// workgroup per front up to kFrontLo, and above it.
 constexpr int kFrontLo = 64;
+inline int front_class(int f) { return f <= kFrontWave ? 0 : f <= kFrontLo ? 1 : 2; }
 
 // Launch keys: tree height (1 = parents of the leaves) major, then the step
 // inside the level.  Matrices of different depths align at equal height.
@@ -1102,13 +1104,13 @@ int build_front_plan(snumat *h) {
   for (int hh = 0; hh < levels; hh++) {
     FrontLevel &lv = FP.levels[hh];
     lv.small0 = (int)FP.small.size();
-    lv.nsmall = (int)sm[hh].size();
-    // fronts of order <= kFrontLo first: their launch needs a quarter of the
-    // LDS or less, so more of them share a CU
-    std::stable_partition(sm[hh].begin(), sm[hh].end(), [](const FrontDev &D) { return D.f <= kFrontLo; });
+    // by class: more workgroups of smaller fronts share a CU's LDS
+    std::stable_sort(sm[hh].begin(), sm[hh].end(),
+                     [](const FrontDev &x, const FrontDev &y) { return front_class(x.f) < front_class(y.f); });
     for (const FrontDev &D : sm[hh]) {
-      if (D.f <= kFrontLo) lv.nsmall_lo++, lv.max_f_lo = std::max(lv.max_f_lo, D.f);
-      lv.max_f = std::max(lv.max_f, D.f);
+      const int k = front_class(D.f);
+      lv.nsmall[k]++;
+      lv.max_f[k] = std::max(lv.max_f[k], D.f);
     }
     FP.small.insert(FP.small.end(), sm[hh].begin(), sm[hh].end());
     // extend-add tiles of the larger fronts, column by column: each child's
@@ -1307,23 +1309,18 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
     FrontLevel &lv = out.levels[hh];
     lv.small0 = (int)out.small.size();
     lv.tile0 = (int)out.tiles.size();
-    for (size_t pi = 0; pi < in.size(); pi++) {
-      const FrontPlan<T> *p = in[pi];
-      if (hh >= p->levels.size()) continue;
-      const FrontLevel &pl = p->levels[hh];
-      out.small.insert(out.small.end(), p->small.begin() + pl.small0, p->small.begin() + pl.small0 + pl.nsmall_lo);
-      lv.max_f = std::max(lv.max_f, pl.max_f);
-      lv.max_f_lo = std::max(lv.max_f_lo, pl.max_f_lo);
-      add_tiles(pi, pl.tile0, pl.ntile);
-    }
-    lv.nsmall_lo = (int)out.small.size() - lv.small0;
-    for (const FrontPlan<T> *p : in)  // then every matrix's larger small fronts
-      if (hh < p->levels.size()) {
+    for (int k = 0; k < 3; k++)  // every matrix's fronts of a class side by side
+      for (const FrontPlan<T> *p : in) {
+        if (hh >= p->levels.size()) continue;
         const FrontLevel &pl = p->levels[hh];
-        out.small.insert(out.small.end(), p->small.begin() + pl.small0 + pl.nsmall_lo,
-                         p->small.begin() + pl.small0 + pl.nsmall);
+        int first = pl.small0;
+        for (int j = 0; j < k; j++) first += pl.nsmall[j];
+        out.small.insert(out.small.end(), p->small.begin() + first, p->small.begin() + first + pl.nsmall[k]);
+        lv.nsmall[k] += pl.nsmall[k];
+        lv.max_f[k] = std::max(lv.max_f[k], pl.max_f[k]);
       }
-    lv.nsmall = (int)out.small.size() - lv.small0;
+    for (size_t pi = 0; pi < in.size(); pi++)
+      if (hh < in[pi]->levels.size()) add_tiles(pi, in[pi]->levels[hh].tile0, in[pi]->levels[hh].ntile);
     lv.ntile = (int)out.tiles.size() - lv.tile0;
   }
   out.sep0 = (int)out.tiles.size();
@@ -1754,8 +1751,9 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   const size_t nl = fp.dense.launches.size();
   for (int hh = 0; hh < (int)fp.levels.size(); hh++) {
     const FrontLevel &lv = fp.levels[hh];
-    launch_front_small<T>(fp.d_small + lv.small0, lv.nsmall_lo, lv.max_f_lo, fs.eps, st);
-    launch_front_small<T>(fp.d_small + lv.small0 + lv.nsmall_lo, lv.nsmall - lv.nsmall_lo, lv.max_f, fs.eps, st);
+    const FrontDev *fr = fp.d_small + lv.small0;
+    for (int k = 0; k < 3; fr += lv.nsmall[k++])
+      (k == 0 ? launch_front_wave<T> : launch_front_small<T>)(fr, lv.nsmall[k], lv.max_f[k], fs.eps, st);
     launch_extend_add<T>(fp.d_tiles + lv.tile0, lv.ntile, fp.d_src, st);
     for (; li < nl && front_key_height(fp.dense.launches[li].key) == hh; li++) {
       int rc = run_timed(fp.dense.launches[li], fp.dense, st);

@@ -75,6 +75,88 @@ __global__ __launch_bounds__(256) void k_front_small(const FrontDev *__restrict_
   for (int i = tid; i < n2; i += nt) G[i] = F[i];
 }
 
+// One wave per front of order <= kFrontWave: assembled in LDS (f^2 values), then
+// lane = row with the columns in registers; the pivot row by v_readlane, so no
+// barrier anywhere.  A front's columns come in chunks of 8 (those past f are
+// skipped), its arithmetic is k_front_small's, operation for operation.
+// Bound by instruction issue (three per column and pivot) and, where a launch
+// fills the device, by the fronts written; k_front_small's two barriers per
+// pivot left its waves waiting: 8190 fronts of order 31 with 15 pivots 123 -> 65
+// us FP64, 32,898 of order 28 with 10 pivots 430 -> 252, 16 fronts 24 -> 13.
+// Orders above 48 would take more than 128 registers.
+constexpr int kFrontCol = 8;
+template <typename T, int P, int C>
+__device__ __forceinline__ void wave_update(T (&a)[kFrontWave], T q, int f) {
+  if constexpr (C < kFrontWave) {
+    if (C < f) {
+#pragma unroll
+      for (int c = C; c < C + kFrontCol; c++)
+        if (c > P) a[c] -= q * rld(a[c], P);
+      wave_update<T, P, C + kFrontCol>(a, q, f);
+    }
+  }
+}
+template <typename T, int P>
+__device__ __forceinline__ void wave_step(T (&a)[kFrontWave], int f, int nk, int lane, T eps) {
+  if (P >= nk) return;
+  T d = rld(a[P], P);
+  if (d < eps && d > -eps) d = d < T(0) ? -eps : eps;
+  const T q = a[P] / d;
+  a[P] = lane > P ? q : lane == P ? d : a[P];
+  if (lane > P) wave_update<T, P, (P + 1) / kFrontCol * kFrontCol>(a, q, f);
+}
+template <typename T, int... P>
+__device__ __forceinline__ void wave_steps(std::integer_sequence<int, P...>, T (&a)[kFrontWave], int f, int nk,
+                                           int lane, T eps) {
+  (wave_step<T, P>(a, f, nk, lane, eps), ...);
+}
+template <typename T>
+__global__ __launch_bounds__(64) void k_front_wave(const FrontDev *__restrict__ fr, T eps) {
+  T *F = (T *)front_lds;
+  const FrontDev D = fr[blockIdx.x];
+  const int f = D.f, n2 = f * f, lane = threadIdx.x;
+  for (int i = lane; i < n2; i += 64) F[i] = T(0);
+  __syncthreads();  // (one wave: orders its LDS accesses)
+  for (int q = lane; q < D.nent; q += 64) {
+    const AEntry e = D.ent[q];
+    F[e.pos] = (T)gptr(D.aval)[e.idx];
+  }
+  __syncthreads();
+  // children's updates, one child after another (fixed summation order); lane
+  // = row, 8 columns' loads in flight
+  for (int c = 0; c < D.nchild; c++) {
+    const FrontChild C = D.child[c];
+    if (C.nb == 0) continue;
+    const auto U = gptr((const T *)C.U) + min(lane, C.nb - 1);
+    const auto rel = gptr(C.rel);
+    const int row = rel[min(lane, C.nb - 1)];
+    for (int b = 0; b < C.nb; b += 8) {
+      T u[8];
+      int col[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int bj = min(b + j, C.nb - 1);
+        col[j] = rel[bj] * f;
+        u[j] = U[(long long)bj * C.ld];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (lane < C.nb && b + j < C.nb) F[row + col[j]] += u[j];
+    }
+    __syncthreads();
+  }
+  T a[kFrontWave];
+#pragma unroll
+  for (int c = 0; c < kFrontWave; c++) a[c] = c < f ? F[min(lane, f - 1) + c * f] : T(0);
+  wave_steps<T>(std::make_integer_sequence<int, kFrontWave>{}, a, f, D.nk, lane, eps);
+  const auto G = gptr((T *)D.F) + lane;
+  if (lane < f) {
+#pragma unroll
+    for (int c = 0; c < kFrontWave; c++)
+      if (c < f) G[c * f] = a[c];
+  }
+}
+
 // Inverses of the 16 x 16 diagonal blocks of L11 and U11 of the fronts factored
 // in LDS (the solves multiply by them): a group of 16 lanes per block, lane =
 // column, by substitution in registers; the multipliers come from the lane
@@ -210,6 +292,12 @@ __global__ __launch_bounds__(256) void k_extend_add(const AddTile *__restrict__ 
   }
 }
 template <typename T>
+void launch_front_wave(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st) {
+  if (nfront <= 0) return;
+  const size_t lds = (size_t)max_f * max_f * sizeof(T);
+  hipLaunchKernelGGL(k_front_wave<T>, dim3(nfront), dim3(64), lds, st, fr, (T)eps);
+}
+template <typename T>
 void launch_extend_add(const AddTile *tiles, int ntile, const AddSrc *src, hipStream_t st) {
   if (ntile <= 0) return;
   hipLaunchKernelGGL(k_extend_add<T>, dim3(ntile), dim3(256), 0, st, tiles, src);
@@ -218,6 +306,7 @@ void launch_extend_add(const AddTile *tiles, int ntile, const AddSrc *src, hipSt
 #define SNU_FRONT_INST(T)                                                                      \
   template int front_small_max<T>();                                                           \
   template void launch_front_small<T>(const FrontDev *, int, int, double, hipStream_t);        \
+  template void launch_front_wave<T>(const FrontDev *, int, int, double, hipStream_t);         \
   template void launch_front_inverse<T>(const FrontDev *, const int2 *, int, hipStream_t);     \
   template void launch_extend_add<T>(const AddTile *, int, const AddSrc *, hipStream_t);
 SNU_FRONT_INST(double)

@@ -268,6 +268,10 @@ void launch_leaf_sweep(const LeafDev *leaves, int nleaves, const VecDev *vd, T *
 // pivot clamp, write-back of the owned slots, update block to global memory.
 template <typename T>
 void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st);
+// The same, one wave per front, for orders up to kFrontWave.
+constexpr int kFrontWave = 48;
+template <typename T>
+void launch_front_wave(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st);
 // Inverses of their 16 x 16 diagonal blocks; blk: {front, first pivot}.
 template <typename T>
 void launch_front_inverse(const FrontDev *fr, const int2 *blk, int nblk, hipStream_t st);

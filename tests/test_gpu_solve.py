@@ -157,3 +157,31 @@ def test_diagonal_blocks_beside_schur_updates(S, prec):
         for graph in (0, 0, 1, 1, 0, 1):
             S._check(S.lib().snumat_use_graph(M._h, graph))
             assert np.array_equal(M.factorize().solve(b), x)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [7, 8, 9, 32, 47, 48, 49])
+def test_one_wave_front_orders(S, precision, n):
+    """The same at the orders around the one-wave front kernel's column chunks
+    and its largest order."""
+    test_dense_leaf_front_orders(S, precision, n)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_one_wave_fronts_with_children(S, precision):
+    """Chains of fronts of every order up to the one-wave kernel's largest and
+    beyond, each with children: banded matrices as one leaf against a dense
+    solve."""
+    for n, band in ((180, 23), (181, 24), (182, 25), (150, 46), (151, 47), (153, 48)):
+        rng = np.random.default_rng(n)
+        D = np.where(np.abs(np.subtract.outer(np.arange(n), np.arange(n))) <= band, rng.uniform(-1, 1, (n, n)), 0.0)
+        D += 2.0 * (band + 1) * np.eye(n)
+        r, c = np.nonzero(D)
+        A = S.CSR(n, np.searchsorted(r, np.arange(n + 1)), c, D[r, c])
+        order = rng.permutation(4).repeat((n + 3) // 4)[:n].argsort(kind="stable")
+        b = rng.standard_normal((n, 2))
+        x = np.linalg.solve(D, b)
+        for o in (np.arange(n), order):
+            with S.SnuMat(A, 1, order=o, sizes=[n], device=0, precision=precision, ir_tol=1e-12) as M:
+                M.factorize()
+                assert np.max(np.abs(M.solve(b) - x)) <= 1e-9 * np.max(np.abs(x))
