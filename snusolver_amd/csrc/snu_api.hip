@@ -143,8 +143,13 @@ namespace {
 constexpr size_t kScratchBytes = size_t(256) << 20;  // 256 MiB per device
 constexpr int kMaxDevices = 64;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// Arrival counters of the split products over it (0 between launches; one per
+// 64 rows of a vector, of which two fit it: 2^19 at most)
+constexpr size_t kScratchDone = size_t(1) << 19;
+__device__ int scratch_done[kScratchDone];
 std::mutex g_scratch_mu;
 void *g_scratch_base[kMaxDevices] = {};
+int *g_scratch_done[kMaxDevices] = {};
 
 // Address of this device's scratch (looked up once per device, with that
 // device current); the caller has made `device` current.
@@ -158,7 +163,12 @@ int scratch_base(int device, unsigned char **out) {
     if (e != hipSuccess || !p)
       return set_error(SNU_ERR_HIP, std::string("hipGetSymbolAddress(scratch) failed: ") +
                                         hipGetErrorString(e));
+    void *d = nullptr;
+    e = hipGetSymbolAddress(&d, HIP_SYMBOL(scratch_done));
+    if (e != hipSuccess || !d)
+      return set_error(SNU_ERR_HIP, std::string("hipGetSymbolAddress(scratch_done) failed: ") + hipGetErrorString(e));
     g_scratch_base[device] = p;
+    g_scratch_done[device] = (int *)d;
   }
   *out = (unsigned char *)g_scratch_base[device];
   return SNU_OK;
@@ -562,7 +572,9 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
       VV.scratch_nrhs = -1;
       g = GemvPlan<T>();  // device pointers point into the scratch: nothing to free
       build_solve_plan<T>(h, bp, ys, k, g);
-      g.cap_part = layout_gemv_plan(g);
+      const SplitNeed need = layout_gemv_plan(g);
+      g.cap_part = need.part;
+      g.cap_done = need.done;
       VV.scratch_nrhs = k;
       VV.scratch_own_w = own_w;
     }
@@ -571,8 +583,9 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
     g.d_vp = (GemvProbT<T> *)carve(sizeof(GemvProbT<T>) * std::max<size_t>(1, g.vp.size()));
     g.d_vs = (GemvSegT<T> *)carve(sizeof(GemvSegT<T>) * std::max<size_t>(1, g.vs.size()));
     g.d_part = (T *)carve(sizeof(T) * std::max<size_t>(1, g.cap_part));
+    g.d_done = g_scratch_done[h->device];
     B.plan = &g;
-    return off <= kScratchBytes;
+    return off <= kScratchBytes && g.cap_done <= kScratchDone;
   };
   int step = nrhs;
   if (!layout(nrhs, true)) {

@@ -62,7 +62,8 @@ struct GemvPlan {
   GemvProbT<T> *d_vp = nullptr;
   GemvSegT<T> *d_vs = nullptr;
   T *d_part = nullptr;            // split-K partial sums (launches run in turn)
-  size_t cap_vp = 0, cap_vs = 0, cap_part = 0;  // device capacities (grow-only)
+  int *d_done = nullptr;          // their arrival counters (0 between launches)
+  size_t cap_vp = 0, cap_vs = 0, cap_part = 0, cap_done = 0;  // device capacities (grow-only)
 };
 
 // Multifrontal leaf factorization of a launch set (one matrix, or a batch
@@ -271,9 +272,12 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &out)
 template <typename T>
 int upload_gemv_plan(GemvPlan<T> &g, hipStream_t st = nullptr);
 // The split-K layout of the plan's launches (no device work); returns the
-// partial-sum values its largest launch needs.
+// partial-sum values and the arrival counters its largest launch needs.
+struct SplitNeed {
+  size_t part = 0, done = 0;
+};
 template <typename T>
-size_t layout_gemv_plan(GemvPlan<T> &g);
+SplitNeed layout_gemv_plan(GemvPlan<T> &g);
 template <typename T>
 void free_gemv_plan(GemvPlan<T> &g);
 template <typename T>

@@ -749,10 +749,11 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
 // Split-K layout: pieces per problem from its longest segment (the problem
 // alone decides), workgroup and partial-sum offsets per launch; a launch
 // whose problems are all single-piece runs unsplit.  Returns the partial-sum
-// values the largest launch needs (launches run in turn and share them).
+// values and counters the largest launch needs (launches run in turn and share
+// them).
 template <typename T>
-size_t layout_gemv_plan(GemvPlan<T> &g) {
-  size_t need_part = 0;
+SplitNeed layout_gemv_plan(GemvPlan<T> &g) {
+  SplitNeed need;
   for (std::vector<Launch> *ls : {&g.fwd, &g.bwd})
     for (Launch &L : *ls) {
       const bool one = L.kind == 7 || L.kind == 8;
@@ -780,9 +781,10 @@ size_t layout_gemv_plan(GemvPlan<T> &g) {
       }
       L.wgs = one && !split ? 0 : wgs;
       L.part = split ? off : 0;
-      need_part = std::max(need_part, (size_t)L.part);
+      need.part = std::max(need.part, (size_t)L.part);
+      if (split && one) need.done = std::max(need.done, (size_t)L.tiles);
     }
-  return need_part;
+  return need;
 }
 
 template <typename T>
@@ -796,11 +798,14 @@ int upload_gemv_plan(GemvPlan<T> &g, hipStream_t st) {
     cap = c;
     return SNU_OK;
   };
-  const size_t need_part = layout_gemv_plan(g);
+  const SplitNeed need = layout_gemv_plan(g);
+  const bool fresh = need.done && (!g.d_done || need.done > g.cap_done);
   int rc;
   if ((rc = grow(&g.d_vp, g.cap_vp, g.vp.size())) || (rc = grow(&g.d_vs, g.cap_vs, g.vs.size())) ||
-      (need_part && (rc = grow(&g.d_part, g.cap_part, need_part))))
+      (need.part && (rc = grow(&g.d_part, g.cap_part, need.part))) ||
+      (need.done && (rc = grow(&g.d_done, g.cap_done, need.done))))
     return rc;
+  if (fresh) launch_fill((float *)g.d_done, (long long)g.cap_done, st);
   if (!g.vp.empty())
     HIPCHK(hipMemcpyAsync(g.d_vp, g.vp.data(), g.vp.size() * sizeof(g.vp[0]), hipMemcpyHostToDevice, st));
   if (!g.vs.empty())
@@ -812,6 +817,7 @@ void free_gemv_plan(GemvPlan<T> &g) {
   if (g.d_vp) (void)hipFree(g.d_vp);
   if (g.d_vs) (void)hipFree(g.d_vs);
   if (g.d_part) (void)hipFree(g.d_part);
+  if (g.d_done) (void)hipFree(g.d_done);
   g = GemvPlan<T>();
 }
 template <typename T>
@@ -1640,7 +1646,7 @@ constexpr bool kSplit64 = true;
 template <typename T>
 void run_launch(const Launch &L, const GemmProbT<T> *gp, const GemmSegT<T> *gs,
                 const DiagProbT<T> *dp, const GemvProbT<T> *vp, const GemvSegT<T> *vs,
-                T *part, hipStream_t st, bool split = false) {
+                T *part, int *done, hipStream_t st, bool split = false) {
   if constexpr (std::is_same<T, float>::value) {
     if (split && (L.kind == 5 || L.kind == 10 || L.kind == 11)) {
       launch_gemm128_split(gp + L.p0, L.np, gs, L.tiles, L.kind == 5 ? 0 : L.kind == 10 ? 1 : 2, st);
@@ -1662,7 +1668,7 @@ void run_launch(const Launch &L, const GemmProbT<T> *gp, const GemmSegT<T> *gs,
     case 6: launch_gemm(gp + L.p0, L.np, gs, L.tiles, 2, st); break;
     case 7:
     case 8:
-      if (L.wgs > 0) launch_gemv_split(vp + L.p0, L.np, vs, L.tiles, L.wgs, L.kind == 7 ? 1 : 0, part, st);
+      if (L.wgs > 0) launch_gemv_split(vp + L.p0, L.np, vs, L.wgs, L.kind == 7 ? 1 : 0, part, done, st);
       else launch_gemv(vp + L.p0, L.np, vs, L.tiles, L.kind == 7 ? 1 : 0, st);
       break;
     case 17:
@@ -1743,7 +1749,7 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   auto run_timed = [&](const Launch &L, const DensePlan<T> &dp, hipStream_t on) -> int {
     const bool gm = prof && is_gemm(L.kind);
     if (gm) HIPCHK(hipEventRecord((*pev)[2 * g], st));
-    run_launch<T>(L, dp.d_gp, dp.d_gs, dp.d_dp, nullptr, nullptr, nullptr, on, fs.split);
+    run_launch<T>(L, dp.d_gp, dp.d_gs, dp.d_dp, nullptr, nullptr, nullptr, nullptr, on, fs.split);
     if (gm) HIPCHK(hipEventRecord((*pev)[2 * g++ + 1], st));
     return SNU_OK;
   };
@@ -1861,9 +1867,9 @@ void run_sweep(const SolveSet &ss, T *bp, T *wbuf, const GemvPlan<T> &plan, hipS
   launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, false, st);
   launch_assemble_rhs(wd.targets, wd.ntarget, wd.tsrc, ss.vec, wbuf, bp, ss.max_groups, ss.one, ss.many, st);
   for (const Launch &L : plan.fwd)
-    run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, st);
+    run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, plan.d_done, st);
   for (const Launch &L : plan.bwd)
-    run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, st);
+    run_launch<T>(L, nullptr, nullptr, nullptr, plan.d_vp, plan.d_vs, plan.d_part, plan.d_done, st);
   launch_leaf_sweep(wd.leaves, wd.nleaves, ss.vec, bp, wbuf, ss.max_groups, ss.one, ss.many, true, st);
 }
 template <typename T>
@@ -1929,7 +1935,7 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
 #define SNU_ENGINE_INST(T)                                                                    \
   template void build_solve_plan<T>(const snumat *, T *, T *, int, GemvPlan<T> &);            \
   template int upload_gemv_plan<T>(GemvPlan<T> &, hipStream_t);                               \
-  template size_t layout_gemv_plan<T>(GemvPlan<T> &);                                         \
+  template SplitNeed layout_gemv_plan<T>(GemvPlan<T> &);                                      \
   template void free_gemv_plan<T>(GemvPlan<T> &);                                             \
   template int upload_dense_plan<T>(DensePlan<T> &);                                          \
   template void free_dense_plan<T>(DensePlan<T> &);                                           \

@@ -228,11 +228,12 @@ template <typename T>
 void launch_gemm_variant(const GemmProbT<T> *probs, int nprob, const GemmSegT<T> *segs,
                          int total_tiles, int tile, int kb, int depth, hipStream_t st);
 // mode 0: y -= A x; 1: y = A x
-// Split-K GEMV: partial sums per (tile, piece) into part, then a fixed-order
-// sum per row applied to y (mode 1: y = sum, 0: y -= sum).
+// Split-K GEMV: partial sums per (tile, piece) into part, added in fixed order
+// by a tile's last workgroup.  done: an arrival counter per tile, 0 before the
+// launch and after it.
 template <typename T>
-void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
-                       int total_tiles, int total_wgs, int mode, T *part, hipStream_t st);
+void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_wgs, int mode,
+                       T *part, int *done, hipStream_t st);
 template <typename T>
 void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs,
                  int total_tiles, int mode, hipStream_t st);

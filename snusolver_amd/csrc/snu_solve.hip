@@ -772,16 +772,43 @@ __global__ __launch_bounds__(256) void k_gemv(const GemvProbT<T> *__restrict__ p
     else *y = *y - v;
   }
 }
-// Split-K GEMV, pass 1: workgroup (problem, tile lt, piece) sums
-// A[rows of lt][k] x[k] over k in [piece * kGemvPiece, (piece + 1) *
-// kGemvPiece) of every segment (within the triangle for tri problems), in
-// the order of the unsplit kernel, and stores the 64 partial sums.
-// Pass 2 adds the pieces in ascending order.  The decomposition depends on
-// the problem alone, so a problem gives the same bits in any launch.
+// Partial sums that another workgroup of the launch adds: written through to,
+// and read from, where the whole device sees them (the XCDs' L2 caches are not
+// coherent).  Release and acquire fences would do the same for plain accesses,
+// but write back and invalidate a whole L2 per workgroup (64^3, one column:
+// 1.83 ms per solve).
 template <typename T>
-__global__ __launch_bounds__(256) void k_gemv_part(const GemvProbT<T> *__restrict__ probs, int nprob,
-                                                   const GemvSegT<T> *__restrict__ segs,
-                                                   T *__restrict__ part) {
+__device__ __forceinline__ void put_part(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T get_part(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void parts_written() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Whether the calling wave's workgroup is the last of `parts` to arrive at
+// *done (left at 0 again for the next launch): what the others had written by
+// parts_written() before arriving can then be read.
+__device__ __forceinline__ bool last_to_arrive(int *done, int parts, int lane) {
+  int at = 0;
+  if (lane == 0) at = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool last = __builtin_amdgcn_readfirstlane(at) == parts - 1;
+  if (last && lane == 0) __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("" ::: "memory");
+  return last;
+}
+// Split-K GEMV: workgroup (problem, tile lt, piece) sums A[rows of lt][k] x[k]
+// over k in [piece * kGemvPiece, (piece + 1) * kGemvPiece) of every segment
+// (within the triangle for tri problems), in the order of the unsplit kernel,
+// and stores the 64 partial sums; the tile's last workgroup to arrive adds the
+// pieces in ascending order.  The decomposition depends on the problem alone,
+// so a problem gives the same bits in any launch.  64^3: 1.05 ms per solve, 1.12
+// with a second launch per product to add the pieces.  (The products of 16
+// columns keep theirs: there the last workgroup's sum takes as long, and with
+// several groups longer: six packed matrices 4.70 ms against 4.63.)
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void k_gemv_split(const GemvProbT<T> *__restrict__ probs, int nprob,
+                                                    const GemvSegT<T> *__restrict__ segs, T *part, int *done) {
   __shared__ T red[4][64];
   const int b = blockIdx.x;
   int lo = 0, hi = nprob - 1;
@@ -800,39 +827,36 @@ __global__ __launch_bounds__(256) void k_gemv_part(const GemvProbT<T> *__restric
     ke = min(P.tri == 1 ? min(K, m0 + 64) : K, (pc + 1) * kGemvPiece);
   });
   __syncthreads();
-  if (w == 0)
-    part[P.poff + (long long)(lt * P.parts + pc) * 64 + lane] =
-        red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
-}
-template <typename T, int MODE>
-__global__ __launch_bounds__(64) void k_gemv_sum(const GemvProbT<T> *__restrict__ probs, int nprob,
-                                                 const T *__restrict__ part) {
-  const int tile = blockIdx.x;
-  int lo = 0, hi = nprob - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (probs[mid].tile0 <= tile) lo = mid;
-    else hi = mid - 1;
+  if (w != 0) return;
+  T v = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+  if (P.parts > 1) {
+    T *in = part + P.poff + (long long)lt * P.parts * 64 + lane;
+    put_part(in + pc * 64, v);
+    parts_written();
+    if (!last_to_arrive(done + P.tile0 + lt, P.parts, lane)) return;
+    v = get_part(in);
+    int q = 1;
+    for (; q + 3 < P.parts; q += 4) {
+      const T a = get_part(in + q * 64), b1 = get_part(in + q * 64 + 64), c = get_part(in + q * 64 + 128),
+              d = get_part(in + q * 64 + 192);
+      v = v + a + b1 + c + d;
+    }
+    for (; q < P.parts; q++) v += get_part(in + q * 64);
   }
-  const GemvProbT<T> P = probs[lo];
-  const int lt = tile - P.tile0, m = lt * 64 + threadIdx.x;
-  if (m >= P.M) return;
-  const T *in = part + P.poff + (long long)lt * P.parts * 64 + threadIdx.x;
-  T v = in[0];
-  for (int pc = 1; pc < P.parts; pc++) v += in[(long long)pc * 64];
-  auto y = gptr(P.y) + m;
-  if (MODE == 1) *y = v;
-  else *y = *y - v;
+  if (m0 + lane < P.M) {
+    auto y = gptr(P.y) + m0 + lane;
+    if (MODE == 1) *y = v;
+    else *y = *y - v;
+  }
 }
 template <typename T>
-void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_tiles,
-                       int total_wgs, int mode, T *part, hipStream_t st) {
-  if (total_tiles <= 0 || nprob <= 0) return;
-  hipLaunchKernelGGL(k_gemv_part<T>, dim3(total_wgs), dim3(256), 0, st, probs, nprob, segs, part);
+void launch_gemv_split(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_wgs, int mode,
+                       T *part, int *done, hipStream_t st) {
+  if (total_wgs <= 0 || nprob <= 0) return;
   if (mode == 1)
-    hipLaunchKernelGGL((k_gemv_sum<T, 1>), dim3(total_tiles), dim3(64), 0, st, probs, nprob, part);
+    hipLaunchKernelGGL((k_gemv_split<T, 1>), dim3(total_wgs), dim3(256), 0, st, probs, nprob, segs, part, done);
   else
-    hipLaunchKernelGGL((k_gemv_sum<T, 0>), dim3(total_tiles), dim3(64), 0, st, probs, nprob, part);
+    hipLaunchKernelGGL((k_gemv_split<T, 0>), dim3(total_wgs), dim3(256), 0, st, probs, nprob, segs, part, done);
 }
 template <typename T>
 void launch_gemv(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs, int total_tiles, int mode,
@@ -986,7 +1010,7 @@ void launch_gemv16(const GemvProbT<T> *probs, int nprob, const GemvSegT<T> *segs
                                        bool, bool, hipStream_t);                                    \
   template void launch_leaf_sweep<T>(const LeafDev *, int, const VecDev *, T *, T *, int, bool, bool, bool, \
                                      hipStream_t);                                                  \
-  template void launch_gemv_split<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int, int, T *, \
+  template void launch_gemv_split<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int, T *, int *, \
                                      hipStream_t);                                                  \
   template void launch_gemv<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int, hipStream_t); \
   template void launch_gemv16<T>(const GemvProbT<T> *, int, const GemvSegT<T> *, int, int, int, int, int, T *, \

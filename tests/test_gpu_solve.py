@@ -12,6 +12,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -185,3 +186,26 @@ def test_one_wave_fronts_with_children(S, precision):
             with S.SnuMat(A, 1, order=o, sizes=[n], device=0, precision=precision, ir_tol=1e-12) as M:
                 M.factorize()
                 assert np.max(np.abs(M.solve(b) - x)) <= 1e-9 * np.max(np.abs(x))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_split_products_repeat_bitwise(S, prec):
+    """One-column products split over K (separators of more than 128 rows) give
+    the same bits solve after solve, in a batch, and from the fixed scratch, in
+    any order of these: the arrival counters are back at zero after each."""
+    A = S.gen_grid(30, 29, 28, 7, 0, 6.1, 2)
+    order, sizes = S.order_grid(30, 29, 28, 8)
+    b = np.ascontiguousarray(S.gen_rhs(A, 1, 1)[1][:, 0])
+    with S.SnuMat(A, 8, order=order, sizes=sizes, device=0, precision=prec) as M:
+        x = M.factorize().solve(b)
+        assert S.backward_error(A, x, b) <= 1e-12
+        db, dx = torch.from_numpy(b).cuda(), torch.zeros(A.n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        with S.Batch([M]) as B:
+            B.factorize()
+            for _ in range(3):
+                assert np.array_equal(M.solve(b), x)
+                M.solve(np.stack([b, b], 1))
+                assert np.array_equal(np.asarray(B.solve([b])[0]).reshape(-1), x)
+                M.solve_device_scratch_ptr(db.data_ptr(), dx.data_ptr(), 1)
+                assert np.array_equal(dx.cpu().numpy(), x)
