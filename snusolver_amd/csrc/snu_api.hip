@@ -213,7 +213,7 @@ extern "C" int snumat_construct(const snu_csr_t *A, const snu_opts_t *opts,
     }
     if (!rc && h->prec == SNU_FP32) {
       IrDev e = ir_entry(h, nullptr, 0, nullptr, 0, 0);
-      hipError_t he = hipMemcpy(h->d_ir, &e, sizeof(e), hipMemcpyHostToDevice);
+      hipError_t he = hipMemcpy(&h->d_tab->ir, &e, sizeof(e), hipMemcpyHostToDevice);
       if (he != hipSuccess) rc = set_error(SNU_ERR_HIP, hipGetErrorString(he));
     }
     if (!rc) rc = ensure_stream(h);
@@ -248,7 +248,7 @@ extern "C" int snumat_attach(snumat_t *h, int device, const double *values) {
   }
   if (!rc && h->prec == SNU_FP32) {
     IrDev e = ir_entry(h, nullptr, 0, nullptr, 0, 0);
-    hipError_t he = hipMemcpy(h->d_ir, &e, sizeof(e), hipMemcpyHostToDevice);
+    hipError_t he = hipMemcpy(&h->d_tab->ir, &e, sizeof(e), hipMemcpyHostToDevice);
     if (he != hipSuccess) rc = set_error(SNU_ERR_HIP, hipGetErrorString(he));
   }
   if (!rc) rc = ensure_stream(h);
@@ -309,7 +309,7 @@ int factorize_values(snumat *h, int stage) {
   fs.nmat = 1;
   fs.max_len = std::max(h->arena_len, h->inv_total);
   fs.max_nnz = h->nsep_ent;
-  fs.ir = h->prec == SNU_FP32 ? h->d_ir : nullptr;
+  fs.ir = h->prec == SNU_FP32 ? &h->d_tab->ir : nullptr;
   fs.anorm_out = h->d_norms;
   fs.max_n = h->P.n;
   fs.wd = &h->wd;
@@ -418,13 +418,12 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
   hipStream_t st = h->stream;
   h->t[15] = 0;
   const int n = h->P.n;
-  VecDev vd{0, 0, n, nrhs, h->wrows, 0};
-  const PermDev pd{h->d_order, d_b, d_x, ldb, ldx, n, 0};
-  HIPCHK(hipMemcpyAsync(h->d_vec, &vd, sizeof(vd), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(h->d_perm, &pd, sizeof(pd), hipMemcpyHostToDevice, st));
+  const SolveTab tab{VecDev{0, 0, n, nrhs, h->wrows, 0}, PermDev{h->d_order, d_b, d_x, ldb, ldx, n, 0},
+                     ir_entry(h, d_b, ldb, d_x, ldx, nrhs)};
+  HIPCHK(hipMemcpyAsync(h->d_tab, &tab, sizeof(tab), hipMemcpyHostToDevice, st));
   SolveSet ss;
-  ss.perm = h->d_perm;
-  ss.vec = h->d_vec;
+  ss.perm = &h->d_tab->perm;
+  ss.vec = &h->d_tab->vec;
   ss.nmat = 1;
   ss.max_groups = vec_groups(nrhs);
   ss.max_elems = (long long)n * ss.max_groups;
@@ -436,11 +435,9 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
   if (h->prec == SNU_FP32) {
     std::vector<int> slot_mat(nrhs, 0);
     std::vector<double> anorm{h->anorm};
-    IrDev e = ir_entry(h, d_b, ldb, d_x, ldx, nrhs);
-    HIPCHK(hipMemcpyAsync(h->d_ir, &e, sizeof(e), hipMemcpyHostToDevice, st));
     RefineSet rs;
     rs.sweep = ss;
-    rs.ir = h->d_ir;
+    rs.ir = &h->d_tab->ir;
     rs.nmat = 1;
     rs.max_n = n;
     rs.norms = B.colnorms;

@@ -129,6 +129,13 @@ struct Values {
   bool scratch_own_w = true;
 };
 
+// Tables of a standalone solve, one copy to the device.
+struct SolveTab {
+  VecDev vec;
+  PermDev perm;
+  IrDev ir;  // (SNU_FP32)
+};
+
 // Host copies of the per-leaf work lists (kept for batching).
 struct WorkLists {
   std::vector<TargetDev> targets;  // separator rows receiving leaf contributions
@@ -196,10 +203,8 @@ struct snumat {
   unsigned long long *d_norms = nullptr;     // |A|inf (bits of a double)
   double *d_colnorms = nullptr;              // refinement column norms (norm_values)
   int *d_active = nullptr;
-  snu::VecDev *d_vec = nullptr;
-  snu::PermDev *d_perm = nullptr;
+  snu::SolveTab *d_tab = nullptr;  // the tables of a standalone solve
   snu::PrepDev *d_prep = nullptr;
-  snu::IrDev *d_ir = nullptr;
   double anorm = 0;
   int nrhs_cap = 0;
   int ir_steps = 0;

@@ -1547,8 +1547,8 @@ int upload(snumat *h) {
     return rc;
   WorkDev &wd = h->wd;
   wd.nleaves = np;
-  if ((rc = dalloc(h, &h->d_vec, 1)) || (rc = dalloc(h, &h->d_perm, 1)) ||
-      (rc = dalloc(h, &h->d_prep, 1)) || (rc = dalloc(h, &h->d_ir, 1)) ||
+  if ((rc = dalloc(h, &h->d_tab, 1)) ||
+      (rc = dalloc(h, &h->d_prep, 1)) ||
       (rc = dalloc(h, &h->d_active, 1)) || (rc = dalloc(h, &h->d_norms, 1)))
     return rc;
   if (h->prec == SNU_FP32) {
