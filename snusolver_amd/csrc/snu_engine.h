@@ -112,7 +112,7 @@ struct Values {
   T *arena = nullptr;  // the separators' dense blocks
   T *inv = nullptr;    // per separator: full L^-1 then U^-1 (s x s each)
   T *lu = nullptr;     // per separator: LU of its 64 x 64 diagonal blocks
-  T *tmp = nullptr;    // products of the triangular inversion
+  T *tmp = nullptr;    // products of a level's panels, then of its triangular inversion
   T *farena = nullptr; // leaf fronts (each f x f, then the inverses of its pivot blocks)
   FrontPlan<T> fronts;
   DensePlan<T> fact;
@@ -195,7 +195,7 @@ struct snumat {
   int wrows = 0;       // update rows of the leaf fronts (solves)
   // dense tables
   std::vector<long long> inv_off, lu_off;
-  long long inv_total = 0, tmp_total = 0;
+  long long inv_total = 0, tmp_panels = 0, tmp_inversion = 0;
   snu::Values<double> v64;
   snu::Values<float> v32;
   // standalone solves

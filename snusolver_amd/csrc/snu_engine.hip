@@ -338,8 +338,8 @@ inline long long fkey(int height, long long step) { return height * kHeight + st
 //   recursive doubling (two grouped GEMMs per doubling step);
 //   then the panels in one pass each, Lp <- Lp U^-1 and Up <- L^-1 Up (GEMM
 //   into scratch over the structurally nonzero rows / columns, K limited by
-//   the triangle, then copied back): the panels are read and written once
-//   instead of once per 64-column step;
+//   the triangle; copied back for the solves): the panels are read and written
+//   once instead of once per 64-column step;
 //   then the Schur updates of the ancestors, K-concatenated over the level's
 //   separators below each of them: one grouped GEMM for the diagonal blocks of
 //   the next level (step kNextD), which that level starts from, and one for
@@ -365,6 +365,7 @@ void build_dense_plan(snumat *h) {
   h_gp.clear();
   h_gs.clear();
   out.clear();
+  std::vector<T *> outL(P.np), outU(P.np);  // the products of a level's panels
   for (int l = P.max_level - 1; l >= 0; l--) {
     const int height = P.max_level - l;
     int lo = 1 << l, hi = std::min((2 << l) - 1, P.np - 1);
@@ -445,9 +446,9 @@ void build_dense_plan(snumat *h) {
         int s = P.block_size[i];
         for (int r0 = 0; r0 + hh < s; r0 += 2 * hh) {
           int c0 = r0 + hh, hb = std::min(hh, s - c0);
-          T *TU = VV.tmp + toff;
+          T *TU = VV.tmp + h->tmp_panels + toff;
           toff += (long long)hh * hb;
-          T *TL = VV.tmp + toff;
+          T *TL = VV.tmp + h->tmp_panels + toff;
           toff += (long long)hb * hh;
           // TU = U12 X22, X22 upper triangular: columns [n0, n0 + W) need
           // its rows [0, n0 + W)
@@ -514,7 +515,7 @@ void build_dense_plan(snumat *h) {
       for (int i = lo; i <= hi; i++) {
         const int s = P.block_size[i], m = P.nL[i], nc = P.nU[i];
         if (m && s) {
-          T *dst = VV.tmp + toff;
+          T *dst = outL[i] = VV.tmp + toff;
           toff += (long long)m * s;
           T *src = Lp(i);
           for (int n0 = 0; n0 < s; n0 += W) {
@@ -525,7 +526,7 @@ void build_dense_plan(snumat *h) {
           cl.np += add_gemm(cp, h_gs, cl.tiles, src, m, m, s, {GemmSeg{dst, dst, m, m, 1}}, cfl);
         }
         if (nc && s) {
-          T *dst = VV.tmp + toff;
+          T *dst = outU[i] = VV.tmp + toff;
           toff += (long long)s * nc;
           T *src = R(i) + (long long)s * s;
           for (int m0 = 0; m0 < s; m0 += W) {
@@ -592,8 +593,8 @@ void build_dense_plan(snumat *h) {
           std::vector<GemmSeg> segs;
           for (int i : w) {
             const int si = P.block_size[i];
-            segs.push_back(GemmSeg{Lp(i) + P.lmap[i][ix(i, rows[a])],
-                                   R(i) + (long long)(si + P.umap[i][ix(i, cols[b])]) * si, P.nL[i], si, si});
+            segs.push_back(GemmSeg{outL[i] + P.lmap[i][ix(i, rows[a])],
+                                   outU[i] + (long long)P.umap[i][ix(i, cols[b])] * si, P.nL[i], si, si});
           }
           return segs;
         };
@@ -644,24 +645,28 @@ void build_dense_plan(snumat *h) {
   }
 }
 
-// Scratch needed by the products of the triangular inversion (max over the
-// doubling steps of every level) and by the panel products of a level.
-long long inversion_tmp_size(const Plan &P) {
-  long long best = 0;
+// Scratch of a level's panel products (they stay until the level's Schur
+// updates have read them) and of the products of the triangular inversion,
+// which run beside those: the most of any level, of any doubling step.
+struct TmpSize {
+  long long panels = 0, inversion = 0;
+};
+TmpSize tmp_size(const Plan &P) {
+  TmpSize best;
   for (int l = P.max_level - 1; l >= 0; l--) {
     int lo = 1 << l, hi = std::min((2 << l) - 1, P.np - 1);
     int smax = 0;
     for (int i = lo; i <= hi; i++) smax = std::max(smax, P.block_size[i]);
     long long panels = 0;
     for (int i = lo; i <= hi; i++) panels += (long long)(P.nL[i] + P.nU[i]) * P.block_size[i];
-    best = std::max(best, panels);
+    best.panels = std::max(best.panels, panels);
     for (int hh = 64; hh < smax; hh *= 2) {
       long long t = 0;
       for (int i = lo; i <= hi; i++) {
         int s = P.block_size[i];
         for (int r0 = 0; r0 + hh < s; r0 += 2 * hh) t += 2LL * hh * std::min(hh, s - r0 - hh);
       }
-      best = std::max(best, t);
+      best.inversion = std::max(best.inversion, t);
     }
   }
   return best;
@@ -950,7 +955,7 @@ int alloc_values(snumat *h) {
   Values<T> &VV = vals<T>(h);
   int rc;
   if ((rc = dalloc(h, &VV.arena, (size_t)h->arena_len)) || (rc = dalloc(h, &VV.inv, (size_t)h->inv_total)) ||
-      (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_total))) ||
+      (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_panels + h->tmp_inversion))) ||
       (rc = dalloc(h, &VV.lu, (size_t)std::max(1LL, h->lu_off[h->P.np]))))
     return rc;
   build_dense_plan<T>(h);
@@ -1534,7 +1539,9 @@ int upload(snumat *h) {
     inv_total += 2LL * P.block_size[p] * P.block_size[p];
   }
   h->inv_total = inv_total;
-  h->tmp_total = inversion_tmp_size(P);
+  const TmpSize tmp = tmp_size(P);
+  h->tmp_panels = tmp.panels;
+  h->tmp_inversion = tmp.inversion;
   h->arena_len = P.dense_total;
   // ---- structure uploads ----
   std::vector<long long> adest;
@@ -1598,8 +1605,8 @@ size_t estimate_device_bytes(const snumat *h) {
   }
   for (int p = 1; p < P.np; p++)
     inv += 2.0 * P.block_size[p] * P.block_size[p] + (P.block_size[p] + 63) / 64 * 4096.0;
-  double bytes = vs * ((double)P.dense_total + fronts + inv +
-                       (double)inversion_tmp_size(P));
+  const TmpSize tmp = tmp_size(P);
+  double bytes = vs * ((double)P.dense_total + fronts + inv + (double)(tmp.panels + tmp.inversion));
   bytes += 16.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block;
   if (h->prec == SNU_FP32) bytes += 4.0 * (P.n + 1 + P.nnz);
   bytes += 2 * vs * P.n + 16.0 * P.n;
@@ -1697,6 +1704,14 @@ bool beside(const DensePlan<T> &plan, size_t i) {
   for (; i < plan.launches.size() && plan.launches[i].key == key; i++) flops += plan.launches[i].flops;
   return beside(flops);
 }
+// The same for the height of launch i, one of its earlier launches.
+template <typename T>
+bool beside_later(const DensePlan<T> &plan, size_t i) {
+  const long long height = plan.launches[i].key / kHeight;
+  for (; i < plan.launches.size() && plan.launches[i].key / kHeight == height; i++)
+    if (plan.launches[i].key % kHeight == kNextD + 1) return beside(plan, i);
+  return false;
+}
 template <typename T>
 int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s) {
   std::map<long long, double> flops;
@@ -1777,10 +1792,16 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   if (ev) HIPCHK(hipEventRecord((*ev)[4], st));
   // the diagonal blocks of the height above and their inverses on the second
   // stream, from the updates of those blocks until its panels need them, beside
-  // the other Schur updates of the height (one stream when profiled: launches
-  // are timed one by one)
+  // the other Schur updates of the height; before them the copy of the height's
+  // panels to where the solves read them, beside the Schur updates of the
+  // diagonal blocks (one stream when profiled: launches are timed one by one)
   SideStream *side = prof ? nullptr : fs.side;
   bool forked = false;
+  auto fork = [&]() -> int {
+    HIPCHK(hipEventRecord(side->fork, st));
+    HIPCHK(hipStreamWaitEvent(side->st, side->fork, 0));
+    return SNU_OK;
+  };
   auto join = [&]() -> int {
     HIPCHK(hipEventRecord(side->join, side->st));
     HIPCHK(hipStreamWaitEvent(st, side->join, 0));
@@ -1791,9 +1812,13 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   for (size_t i = 0; i < plan.launches.size(); i++) {
     const Launch &L = plan.launches[i];
     const long long step = L.key % kHeight;
+    if (side && side->st && L.kind == 3 && beside_later(plan, i)) {
+      if ((rc = fork())) return rc;
+      if ((rc = run_timed(L, plan, side->st))) return rc;
+      continue;
+    }
     if (side && side->st && !forked && beside(plan, i)) {
-      HIPCHK(hipEventRecord(side->fork, st));
-      HIPCHK(hipStreamWaitEvent(side->st, side->fork, 0));
+      if ((rc = fork())) return rc;
       forked = true;
     }
     if (forked && step >= kPanels && step < kNextD && (rc = join())) return rc;
