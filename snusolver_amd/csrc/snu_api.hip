@@ -307,7 +307,7 @@ int factorize_values(snumat *h, int stage) {
   fs.side = &h->side;
   fs.prep = h->d_prep;
   fs.nmat = 1;
-  fs.max_len = std::max(h->arena_len, h->inv_total);
+  fs.max_len = h->arena_len;
   fs.max_nnz = h->nsep_ent;
   fs.ir = h->prec == SNU_FP32 ? &h->d_tab->ir : nullptr;
   fs.anorm_out = h->d_norms;

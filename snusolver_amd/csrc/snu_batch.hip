@@ -28,10 +28,8 @@ struct snubatch {
   std::vector<void *> allocs;
   // factor set
   WorkDev wd;
-  PrepDev *d_prep = nullptr;
   IrDev *d_ir_a = nullptr;  // |A| norm tables (FP32)
   unsigned long long *d_anorm = nullptr;
-  long long max_len = 0, max_nnz = 0;
   int max_n = 0;
   DensePlan<double> f64;
   DensePlan<float> f32;
@@ -182,10 +180,7 @@ template <typename T>
 int batch_factorize(snubatch *b) {
   FactorSet fs;
   fs.side = &b->side;
-  fs.prep = b->d_prep;
   fs.nmat = (int)b->mats.size();
-  fs.max_len = b->max_len;
-  fs.max_nnz = b->max_nnz;
   fs.ir = b->prec == SNU_FP32 ? b->d_ir_a : nullptr;
   fs.anorm_out = b->d_anorm;
   fs.max_n = b->max_n;
@@ -355,7 +350,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   // concatenated leaves and work lists
   std::vector<LeafDev> leaves;
   WorkLists W;
-  std::vector<PrepDev> prep;
   std::vector<IrDev> ira;
   for (int m = 0; m < count; m++) {
     snumat *h = b->mats[m];
@@ -367,16 +361,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
     const WorkLists &w = h->wl;
     for (TargetDev t : w.targets) W.targets.push_back(TargetDev{t.row, sbase + t.s0, sbase + t.s1, m});
     W.tsrc.insert(W.tsrc.end(), w.tsrc.begin(), w.tsrc.end());
-    PrepDev pd;
-    pd.arena = b->prec == SNU_FP32 ? (void *)h->v32.arena : (void *)h->v64.arena;
-    pd.inv = b->prec == SNU_FP32 ? (void *)h->v32.inv : (void *)h->v64.inv;
-    pd.arena_len = h->arena_len;
-    pd.inv_len = h->inv_total;
-    pd.aval = h->d_aval;
-    pd.adest = h->d_adest;
-    pd.asrc = h->d_asrc;
-    pd.nnz = h->nsep_ent;
-    prep.push_back(pd);
     IrDev e;
     std::memset(&e, 0, sizeof(e));
     e.rowptr = h->d_arow;
@@ -384,8 +368,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
     e.val = h->d_aval;
     e.n = h->P.n;
     ira.push_back(e);
-    b->max_len = std::max(b->max_len, std::max(h->arena_len, h->inv_total));
-    b->max_nnz = std::max(b->max_nnz, h->nsep_ent);
     b->max_n = std::max(b->max_n, h->P.n);
   }
   WorkDev &wd = b->wd;
@@ -393,7 +375,7 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   wd.ntarget = (int)W.targets.size();
   int rc;
   if ((rc = bupload(b, &wd.leaves, leaves)) || (rc = bupload(b, &wd.targets, W.targets)) ||
-      (rc = bupload(b, &wd.tsrc, W.tsrc)) || (rc = bupload(b, &b->d_prep, prep)) ||
+      (rc = bupload(b, &wd.tsrc, W.tsrc)) ||
       (rc = bupload(b, &b->d_ir_a, ira)))
     return fail(rc);
   // the members' leaf fronts, merged per height (descriptors point into the

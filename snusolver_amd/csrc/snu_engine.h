@@ -300,9 +300,9 @@ void merge_gemv(const std::vector<const GemvPlan<T> *> &in, GemvPlan<T> &out);
 // Executors over a launch set.
 struct FactorSet {
   SideStream *side = nullptr;  // (null: one stream)
-  const PrepDev *prep;
   int nmat;
-  long long max_len, max_nnz;
+  const PrepDev *prep = nullptr;  // scatter_only: its table, largest arena and entries
+  long long max_len = 0, max_nnz = 0;
   const IrDev *ir;           // FP32 only: |A| norms into anorm_out
   unsigned long long *anorm_out;
   int max_n;

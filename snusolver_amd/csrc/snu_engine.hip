@@ -3,12 +3,12 @@
 // and the executors of the factor and solve sweeps.
 //
 // Phase map (reference -> here):
-//   core_run (kernel_sparse.cu:1011-1037)        -> prepare (zero + scatter),
-//        the leaf fronts, k_front_schur, k_assemble_schur
+//   core_run (kernel_sparse.cu:1011-1037)        -> the leaf fronts, then
+//        k_extend_add into the separator blocks
 //   dense level loop (SnuMat_factorize.cu:258-284) -> per level: blocked
-//        getrf/trsm (k_diag_lu + k_gemm by the block inverses), then one
-//        grouped k_gemm for all Schur updates of the level (K-concatenated
-//        over siblings: replaces reduction_gpu, SnuMat_factorize.cu:78-124)
+//        getrf/trsm (k_diag_panel), then grouped k_gemm for the Schur updates
+//        of the level (K-concatenated over siblings: replaces reduction_gpu,
+//        SnuMat_factorize.cu:78-124)
 //   forward solve (core_trsm/core_update_b, trsm_Lxb/gemm on b; fused into
 //        the factorization in the reference) and backward solve
 //        (SnuMat_factorize.cu:286-345)     -> run_sweep
@@ -22,6 +22,7 @@
 #include <mutex>
 #include <tuple>
 #include <type_traits>
+#include <unordered_map>
 
 #include "snu_engine.h"
 
@@ -958,6 +959,10 @@ int alloc_values(snumat *h) {
       (rc = dalloc(h, &VV.tmp, (size_t)std::max(1LL, h->tmp_panels + h->tmp_inversion))) ||
       (rc = dalloc(h, &VV.lu, (size_t)std::max(1LL, h->lu_off[h->P.np]))))
     return rc;
+  // the inverses' other triangles stay zero: factorizations write within the
+  // 64 x 64 diagonal blocks and their own triangle alone
+  launch_fill(VV.inv, h->inv_total, nullptr);
+  HIPCHK(hipStreamSynchronize(nullptr));
   build_dense_plan<T>(h);
   return upload_dense_plan(VV.fact);
 }
@@ -1154,7 +1159,6 @@ int build_front_plan(snumat *h) {
           t.ldc = f;
           t.nr = std::min(64, f - 64 * rt);
           t.nc = std::min(64, f - 64 * ct);
-          t.keep = 0;
           t.s0 = (int)FP.src.size();
           for (int k = 0; k < nc; k++) {
             const int *bk = bound.data() + (size_t)k * (nt + 1);
@@ -1215,9 +1219,11 @@ int build_front_plan(snumat *h) {
     }
   }
   if ((rc = upload_dense_plan(DP))) return rc;
-  // extend-add tiles of the separator blocks: the root fronts' update blocks,
-  // per pair of 64-index tiles of the blocks their B entries belong to (pairs
-  // whose panel tile is not stored are structurally zero)
+  // extend-add tiles of the separator blocks, all that are stored: the root
+  // fronts' update blocks, per pair of 64-index tiles of the blocks their B
+  // entries belong to (pairs whose panel tile is not stored are structurally
+  // zero), and A's entries; every tile is written, so the blocks are not
+  // cleared before.  A piece without rows stands for a tile itself.
   FP.sep0 = (int)FP.tiles.size();
   struct Piece { long long key; T *C; long long ldc; int nr, nc; AddSrc s; };
   std::vector<Piece> pieces;
@@ -1225,6 +1231,27 @@ int build_front_plan(snumat *h) {
   std::vector<Group> gr;
   std::vector<long long> tbase(P.num_block + 2, 0);  // tiles of the blocks before each block
   for (int b = 1; b <= P.num_block; b++) tbase[b + 1] = tbase[b] + (P.block_size[b] + 63) / 64;
+  auto key_of = [&](int p, int t, int q, int u) { return (tbase[p] + t) * tbase[P.num_block + 1] + tbase[q] + u; };
+  for (int p = 1; p < np; p++) {
+    const int sp = P.block_size[p], tp = (sp + 63) / 64;
+    auto add = [&](long long key, long long off, long long ldc, int nr, int nc) {
+      pieces.push_back(Piece{key, VV.arena + off, ldc, nr, nc, AddSrc{}});
+    };
+    for (int t = 0; t < tp; t++)
+      for (int u = 0; u < tp; u++)
+        add(key_of(p, t, p, u), P.offR[p] + 64 * t + (long long)64 * u * sp, sp, std::min(64, sp - 64 * t), std::min(64, sp - 64 * u));
+    for (int q = p / 2; q; q /= 2) {
+      const int o = P.anc_off(p, q), sq = P.block_size[q];
+      for (int u = 0; 64 * u < sq; u++) {
+        const int cu = P.umap[p][o + 64 * u], rl = P.lmap[p][o + 64 * u], w = std::min(64, sq - 64 * u);
+        for (int t = 0; t < tp; t++) {
+          const int ht = std::min(64, sp - 64 * t);
+          if (cu >= 0) add(key_of(p, t, q, u), P.offR[p] + 64 * t + (long long)(sp + cu) * sp, sp, ht, w);
+          if (rl >= 0) add(key_of(q, u, p, t), P.offL[p] + rl + (long long)64 * t * P.nL[p], P.nL[p], w, ht);
+        }
+      }
+    }
+  }
   for (int r = 0; r < np; r++) {
     const LeafPlan &L = P.leaves[r];
     for (int f = 0; f < (int)L.ff.size(); f++) {
@@ -1258,7 +1285,7 @@ int build_front_plan(snumat *h) {
             C = VV.arena + P.offL[q] + l + (long long)64 * c.t * P.nL[q];
             ldc = P.nL[q];
           }
-          pieces.push_back(Piece{(tbase[p] + a.t) * tbase[P.num_block + 1] + tbase[q] + c.t, C, ldc,
+          pieces.push_back(Piece{key_of(p, a.t, q, c.t), C, ldc,
                                  std::min(64, sp - 64 * a.t), std::min(64, sq - 64 * c.t),
                                  AddSrc{U, d_rel + o_rel[r] + i0, fc, a.b0, a.b1 - a.b0, c.b0, c.b1 - c.b0,
                                         64 * a.t, 64 * c.t, 0}});
@@ -1282,11 +1309,49 @@ int build_front_plan(snumat *h) {
       t.nc = x.nc;
       t.s0 = t.s1 = (int)FP.src.size();
       t.nent = 0;
-      t.keep = 1;
       FP.tiles.push_back(t);
     }
+    if (x.s.rn == 0) continue;
     FP.src.push_back(x.s);
     FP.tiles.back().s1 = (int)FP.src.size();
+  }
+  // A's separator entries by tile
+  std::vector<std::pair<int, AEntry>> sent_of;  // tile from sep0 on, entry
+  {
+    std::unordered_map<long long, int> tile_at;  // by its first value's place in the arena
+    for (size_t q = FP.sep0; q < FP.tiles.size(); q++) tile_at[(T *)FP.tiles[q].C - VV.arena] = (int)q - FP.sep0;
+    // first stored column (row) of every tile of each separator's panels
+    std::vector<std::vector<int>> cu(np), rl(np);
+    for (int p = 1; p < np; p++)
+      for (int q = p / 2; q; q /= 2)
+        for (int u = 0, o = P.anc_off(p, q); u < P.block_size[q]; u += 64) {
+          if (P.umap[p][o + u] >= 0) cu[p].push_back(P.umap[p][o + u]);
+          if (P.lmap[p][o + u] >= 0) rl[p].push_back(P.lmap[p][o + u]);
+        }
+    auto start = [](const std::vector<int> &v, int x) { return *(std::upper_bound(v.begin(), v.end(), x) - 1); };
+    for (int q = 0; q < P.nnz; q++) {
+      if (P.a_dest[q] < P.leaf_total) continue;
+      const long long x = P.a_dest[q] - P.leaf_total;
+      const int p = (int)(std::upper_bound(P.offR.begin() + 1, P.offR.begin() + np, x) - P.offR.begin()) - 1;
+      const bool R = x < P.offL[p];
+      const long long ld = R ? P.block_size[p] : P.nL[p], y = x - (R ? P.offR[p] : P.offL[p]), sp = P.block_size[p];
+      const int row = (int)(y % ld), col = (int)(y / ld);
+      const int r0 = R ? row / 64 * 64 : start(rl[p], row);
+      const int c0 = !R || col < sp ? col / 64 * 64 : (int)sp + start(cu[p], col - (int)sp);
+      sent_of.push_back({tile_at.at((R ? P.offR[p] : P.offL[p]) + r0 + c0 * ld),
+                         AEntry{(int)(row - r0 + (col - c0) * ld), q}});
+    }
+    std::sort(sent_of.begin(), sent_of.end(), [](const std::pair<int, AEntry> &x, const std::pair<int, AEntry> &y) {
+      return x.first != y.first ? x.first < y.first : x.second.pos < y.second.pos;
+    });
+  }
+  std::vector<AEntry> sent;
+  for (const auto &e : sent_of) sent.push_back(e.second);
+  AEntry *d_sent = nullptr;
+  if ((rc = dupload(h, &d_sent, sent))) return rc;
+  for (size_t e = 0; e < sent_of.size(); e++) {
+    AddTile &t = FP.tiles[FP.sep0 + sent_of[e].first];
+    if (t.nent++ == 0) t.ent = d_sent + e, t.aval = h->d_aval;
   }
   list_inverse_blocks(FP);
   if ((rc = dupload(h, &FP.d_iblk, FP.iblk)) || (rc = dupload(h, &FP.d_small, FP.small)) ||
@@ -1573,9 +1638,7 @@ int upload(snumat *h) {
   if ((rc = dupload(h, &wd.leaves, h->h_leaves))) return rc;
   PrepDev pd;
   pd.arena = h->prec == SNU_FP32 ? (void *)h->v32.arena : (void *)h->v64.arena;
-  pd.inv = h->prec == SNU_FP32 ? (void *)h->v32.inv : (void *)h->v64.inv;
   pd.arena_len = h->arena_len;
-  pd.inv_len = h->inv_total;
   pd.aval = h->d_aval;
   pd.adest = h->d_adest;
   pd.asrc = h->d_asrc;
@@ -1607,7 +1670,7 @@ size_t estimate_device_bytes(const snumat *h) {
     inv += 2.0 * P.block_size[p] * P.block_size[p] + (P.block_size[p] + 63) / 64 * 4096.0;
   const TmpSize tmp = tmp_size(P);
   double bytes = vs * ((double)P.dense_total + fronts + inv + (double)(tmp.panels + tmp.inversion));
-  bytes += 16.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block;
+  bytes += 24.0 * P.nnz + 4.0 * (idx + P.n) + 48.0 * P.num_block + 56.0 / 2048 * (double)P.dense_total;
   if (h->prec == SNU_FP32) bytes += 4.0 * (P.n + 1 + P.nnz);
   bytes += 2 * vs * P.n + 16.0 * P.n;
   return (size_t)bytes;
@@ -1739,7 +1802,7 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
                    const std::vector<hipEvent_t> *ev, bool profile, std::vector<hipEvent_t> *pev) {
   const WorkDev &wd = *fs.wd;
   if (ev) HIPCHK(hipEventRecord((*ev)[0], st));
-  launch_prepare<T>(fs.prep, fs.nmat, fs.max_len, fs.max_nnz, st);
+  if (fs.scatter_only) launch_prepare<T>(fs.prep, fs.nmat, fs.max_len, fs.max_nnz, st);
   if (fs.ir) launch_rowabs_max(fs.ir, fs.nmat, fs.max_n, fs.anorm_out, st);
   if (ev) HIPCHK(hipEventRecord((*ev)[1], st));
   if (fs.scatter_only) {

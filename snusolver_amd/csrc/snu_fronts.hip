@@ -236,12 +236,14 @@ void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, h
 // 16 w + 15, lane = row, summed in registers and written once: every source
 // that lands in the tile (the host lists them, in order) is read through the
 // maps tile row -> its row, tile column -> its column, which each wave builds
-// in LDS from the source's ascending positions.  Bound by the update blocks
-// read and the target written; 64^3 7-point FP64, all heights and the
-// separator blocks together 1.6 ms.  (Fronts zeroed, filled from CSR factor
-// slots and added to child by child in memory took 3.5 ms, boundary Schur
-// blocks gathered and then added 2.1 ms, the factors' write-back into CSR
-// slots 1.5 ms.)
+// in LDS from the source's ascending positions; A's entries are added last.
+// Every stored tile is one, so nothing is cleared before (clearing the
+// separator blocks, 2.0 GB, and reading them back took 0.5 ms of a 64^3
+// factorization).  Bound by the update blocks read and the target written;
+// 64^3 7-point FP64, all heights and the separator blocks together 1.6 ms.
+// (Fronts zeroed, filled from CSR factor slots and added to child by child in
+// memory took 3.5 ms, boundary Schur blocks gathered and then added 2.1 ms, the
+// factors' write-back into CSR slots 1.5 ms.)
 template <typename T>
 __global__ __launch_bounds__(256) void k_extend_add(const AddTile *__restrict__ tiles,
                                                     const AddSrc *__restrict__ src) {
@@ -252,10 +254,6 @@ __global__ __launch_bounds__(256) void k_extend_add(const AddTile *__restrict__ 
   T v[16];
 #pragma unroll
   for (int j = 0; j < 16; j++) v[j] = T(0);
-  if (t.keep) {
-#pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = C[min(c0 + j, t.nc - 1) * t.ldc];
-  }
   for (int s = t.s0; s < t.s1; s++) {
     const AddSrc S = src[s];
     const auto pos = gptr(S.pos);

@@ -82,7 +82,7 @@ struct AddTile {
   int nr, nc;               // rows, columns of the tile
   int s0, s1;               // its sources
   int nent;                 // entries of A added after them
-  int keep;                 // 1: onto the values there, 0: onto zero
+  int pad;
 };
 
 // A matrix's right-hand sides in the packed solve vectors.  One column: n
@@ -112,11 +112,11 @@ struct PermDev {
   long long ldb, ldx;
   int n, vec;
 };
-// Factor set-up of one matrix: the separators' dense blocks and inverses are
+// Set-up of one matrix for the scatter alone: the separators' dense blocks are
 // zeroed, then A's separator entries put into place.
 struct PrepDev {
-  void *arena, *inv;
-  long long arena_len, inv_len;
+  void *arena;
+  long long arena_len;
   const double *aval;
   const long long *adest;   // per separator entry: place in the arena
   const int *asrc;          // and index in A's values
@@ -200,7 +200,7 @@ int device_lds_limit();
 
 template <typename T>
 void launch_fill(T *p, long long n, hipStream_t st);
-// zero arena / inverses, scatter A's values (one matrix per table entry)
+// zero arena, scatter A's values (one matrix per table entry)
 template <typename T>
 void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long max_nnz,
                     hipStream_t st);

@@ -1249,17 +1249,16 @@ void launch_rowabs_max(const IrDev *tab, int nmat, int max_n, unsigned long long
   if (max_n <= 0) return;
   hipLaunchKernelGGL(k_rowabs_max, dim3(ir_blocks(max_n), nmat), dim3(256), 0, st, tab, out);
 }
-// Factor set-up for a set of matrices (one per blockIdx.y): zero the
-// separators' blocks and inverses, then put A's separator entries into place.
+// The scatter alone, for a set of matrices (one per blockIdx.y): zero the
+// separators' blocks, then put A's separator entries into place.  (A
+// factorization writes every tile of them in k_extend_add.)
 template <typename T>
 __global__ void k_prep_fill(const PrepDev *__restrict__ tab) {
   const PrepDev M = tab[blockIdx.y];
-  const auto a = gptr((T *)M.arena), v = gptr((T *)M.inv);
+  const auto a = gptr((T *)M.arena);
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.arena_len; i += stride)
     a[i] = T(0);
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < M.inv_len; i += stride)
-    v[i] = T(0);
 }
 template <typename T>
 __global__ void k_prep_scatter(const PrepDev *__restrict__ tab) {
