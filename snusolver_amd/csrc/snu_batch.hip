@@ -103,13 +103,33 @@ void free_batch(snubatch *b) {
   b->stream = nullptr;
 }
 
+// What only factorizations need, on the first one: a batch that solves alone (a
+// server forms them per pack) does without.
 template <typename T>
 int build_factor_set(snubatch *b) {
   std::vector<const DensePlan<T> *> parts;
   for (snumat *h : b->mats) parts.push_back(&vals<T>(h).fact);
   DensePlan<T> &out = std::is_same<T, double>::value ? (DensePlan<T> &)b->f64 : (DensePlan<T> &)b->f32;
   merge_dense(parts, out);
-  return upload_dense_plan(out);
+  int rc = upload_dense_plan(out);
+  if (rc) return rc;
+  // the members' leaf fronts, merged per height (descriptors point into the
+  // members' own arrays)
+  FrontPlan<T> &fp = std::is_same<T, double>::value ? (FrontPlan<T> &)b->fr64 : (FrontPlan<T> &)b->fr32;
+  std::vector<const FrontPlan<T> *> fronts;
+  for (snumat *h : b->mats) fronts.push_back(&vals<T>(h).fronts);
+  merge_fronts(fronts, fp);
+  if ((rc = upload_dense_plan(fp.dense)) || (rc = bupload(b, &fp.d_iblk, fp.iblk)) || (rc = bupload(b, &fp.d_small, fp.small)) ||
+      (rc = bupload(b, &fp.d_tiles, fp.tiles)) || (rc = bupload(b, &fp.d_src, fp.src)))
+    return rc;
+  // both streams anew, one after the other (see SideStream)
+  if (b->stream) {
+    HIPCHK(hipStreamSynchronize(b->stream));
+    HIPCHK(hipStreamDestroy(b->stream));
+    b->stream = nullptr;
+  }
+  HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
+  return make_side<T>(parts, b->side);
 }
 
 // Solve plan and buffers for a right-hand-side pattern (columns per matrix;
@@ -337,13 +357,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
   hipError_t he = hipSetDevice(b->device);
   if (he == hipSuccess) he = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (he != hipSuccess) return fail(set_error(SNU_ERR_HIP, hipGetErrorString(he)));
-  {
-    std::vector<const DensePlan<double> *> d64;
-    std::vector<const DensePlan<float> *> d32;
-    for (const snumat *h : b->mats) d64.push_back(&h->v64.fact), d32.push_back(&h->v32.fact);
-    int rc = b->prec == SNU_FP32 ? make_side<float>(d32, b->side) : make_side<double>(d64, b->side);
-    if (rc) return fail(rc);
-  }
   b->ev.resize(8);
   for (auto &e : b->ev)
     if (hipEventCreate(&e) != hipSuccess) return fail(set_error(SNU_ERR_HIP, "event creation failed"));
@@ -378,23 +391,6 @@ extern "C" int snubatch_create(snumat_t *const *mats, int count, snubatch_t **ou
       (rc = bupload(b, &wd.tsrc, W.tsrc)) ||
       (rc = bupload(b, &b->d_ir_a, ira)))
     return fail(rc);
-  // the members' leaf fronts, merged per height (descriptors point into the
-  // members' own arrays)
-  {
-    auto fronts = [&](auto tag) -> int {
-      using T = decltype(tag);
-      FrontPlan<T> &fp = std::is_same<T, double>::value ? (FrontPlan<T> &)b->fr64 : (FrontPlan<T> &)b->fr32;
-      std::vector<const FrontPlan<T> *> parts;
-      for (snumat *h : b->mats) parts.push_back(&vals<T>(h).fronts);
-      merge_fronts(parts, fp);
-      int r;
-      if ((r = upload_dense_plan(fp.dense)) || (r = bupload(b, &fp.d_iblk, fp.iblk)) || (r = bupload(b, &fp.d_small, fp.small)) ||
-          (r = bupload(b, &fp.d_tiles, fp.tiles)) || (r = bupload(b, &fp.d_src, fp.src)))
-        return r;
-      return SNU_OK;
-    };
-    if ((rc = b->prec == SNU_FP32 ? fronts(float()) : fronts(double()))) return fail(rc);
-  }
   if ((rc = balloc(b, (void **)&b->d_anorm, sizeof(unsigned long long) * count)) ||
       (rc = balloc(b, (void **)&b->d_active, sizeof(int) * count)) ||
       (rc = balloc(b, (void **)&b->d_vec, sizeof(VecDev) * count)) ||
