@@ -407,6 +407,15 @@ int snu_bench_copy(size_t bytes, int reps, double *ms_out);
 /* in-place no-pivot LU of an nb x nb block (nb <= 64); Linv/Uinv: 64 x 64. */
 int snu_test_diag_lu(int nb, double *D, int ld, double *Linv, double *Uinv);
 int snu_test_diag_lu_f32(int nb, float *D, int ld, float *Linv, float *Uinv);
+/* the dense launches of a handle's factorization (also of a host-only
+ * handle), as run on two streams: key = height (from the leaves' parents, 1)
+ * x 1e8 + step (below 6e7: diagonal blocks and their inverses, 6e7: panels,
+ * 9e7: Schur updates of the next height's diagonal blocks, 9e7 + 1: the other
+ * Schur updates), kind (3: copy of the panels), side: 1: the first stream
+ * waits for the second, 2: the second for the first, 4: runs on the second.
+ * Fills at most cap entries, returns their number (negative: error). */
+int snu_test_dense_launches(snumat_t *h, int cap, int64_t *key, int *kind,
+                            int *side);
 
 #ifdef __cplusplus
 }

@@ -1098,6 +1098,27 @@ extern "C" int snu_test_diag_lu_f32(int nb, float *D, int ld, float *Linv,
   return test_diag_lu<float>(nb, D, ld, Linv, Uinv);
 }
 
+// The dense launches of a factorization with a second stream: per launch its
+// key, kind and kSide* flags.
+namespace {
+template <typename T>
+int dense_launches(snumat *h, int cap, int64_t *key, int *kind, int *side) {
+  const DensePlan<T> &plan = plan_of<T>(h);
+  const std::vector<int> how = side_schedule(plan);
+  for (int i = 0; i < cap && i < (int)how.size(); i++) {
+    key[i] = plan.launches[i].key;
+    kind[i] = plan.launches[i].kind;
+    side[i] = how[i];
+  }
+  return (int)how.size();
+}
+}  // namespace
+extern "C" int snu_test_dense_launches(snumat_t *h, int cap, int64_t *key, int *kind, int *side) {
+  if (!h || cap < 0 || (cap > 0 && (!key || !kind || !side))) return set_error(SNU_ERR_BAD_INPUT, "null");
+  return h->prec == SNU_FP32 ? dense_launches<float>(h, cap, key, kind, side)
+                             : dense_launches<double>(h, cap, key, kind, side);
+}
+
 // ---------------- device memory plumbing (bench, tests) ----------------
 extern "C" int snu_dev_alloc(size_t bytes, void **p) {
   if (!p) return set_error(SNU_ERR_BAD_INPUT, "null");

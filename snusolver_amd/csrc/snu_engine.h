@@ -160,6 +160,10 @@ struct SideStream {
   hipStream_t st = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
 };
+// What a launch of the dense plan does to it, before it runs (kSideJoin: the
+// first stream waits for the second; kSideFork: the second waits for the
+// first), and whether it runs on it.
+enum { kSideJoin = 1, kSideFork = 2, kSideRun = 4 };
 // A factorization's launch sequence captured once into a HIP graph and
 // replayed (no memset nodes: buffers are cleared by kernels).
 struct FactorGraph {
@@ -323,6 +327,14 @@ void free_graph(FactorGraph &g);
 template <typename T>
 int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s);
 void free_side(SideStream &s);
+// Per launch of the plan, the kSide* flags; at its end the first stream waits
+// for the second once more.
+template <typename T>
+std::vector<int> side_schedule(const DensePlan<T> &plan);
+// The dense plan of a handle (built for the structure alone if the handle is
+// on no device).
+template <typename T>
+const DensePlan<T> &plan_of(snumat *h);
 struct SolveSet {
   const PermDev *perm;
   const VecDev *vec;

@@ -1585,16 +1585,10 @@ template void merge_fronts<float>(const std::vector<const FrontPlan<float> *> &,
 template int build_front_plan<double>(snumat *);
 template int build_front_plan<float>(snumat *);
 
-int upload(snumat *h) {
-  Plan &P = h->P;
-  int rc;
-  HIPCHK(hipSetDevice(h->device));
-  if (h->prec == SNU_FP32) autotune_tiles<float>();
-  else autotune_tiles<double>();
+// Offsets of the separators' blocks, inverses and scratch (structure only).
+static void layout_dense(snumat *h) {
+  const Plan &P = h->P;
   const int np = P.np;
-  h->h_leaves.assign(np, LeafDev());
-  h->wl = WorkLists();
-  // ---- dense tables ----
   h->inv_off.assign(P.num_block + 1, 0);
   h->lu_off.assign(np + 1, 0);
   for (int p = 1; p < np; p++) h->lu_off[p + 1] = h->lu_off[p] + (P.block_size[p] + 63) / 64 * 4096LL;
@@ -1608,6 +1602,18 @@ int upload(snumat *h) {
   h->tmp_panels = tmp.panels;
   h->tmp_inversion = tmp.inversion;
   h->arena_len = P.dense_total;
+}
+
+int upload(snumat *h) {
+  Plan &P = h->P;
+  int rc;
+  HIPCHK(hipSetDevice(h->device));
+  if (h->prec == SNU_FP32) autotune_tiles<float>();
+  else autotune_tiles<double>();
+  const int np = P.np;
+  h->h_leaves.assign(np, LeafDev());
+  h->wl = WorkLists();
+  layout_dense(h);
   // ---- structure uploads ----
   std::vector<long long> adest;
   std::vector<int> asrc;
@@ -1775,6 +1781,47 @@ bool beside_later(const DensePlan<T> &plan, size_t i) {
     if (plan.launches[i].key % kHeight == kNextD + 1) return beside(plan, i);
   return false;
 }
+// The second stream's part in a factorization, launch by launch.  It takes the
+// copy of a height's panels to where the solves read them, beside the height's
+// Schur updates, and the diagonal blocks of the height above and their
+// inverses, from the updates of those blocks (step kNextD) on, beside the
+// height's other Schur updates.  Everything above those blocks waits for both
+// streams: that height's panels, and, where it has none (separators that are
+// empty or coupled to nothing above), the next launch of a greater height,
+// whose blocks the updates running beside may write.
+template <typename T>
+std::vector<int> side_schedule(const DensePlan<T> &plan) {
+  std::vector<int> out(plan.launches.size(), 0);
+  long long fork = -1;  // height of the last fork not joined yet
+  for (size_t i = 0; i < plan.launches.size(); i++) {
+    const Launch &L = plan.launches[i];
+    const long long height = L.key / kHeight, step = L.key % kHeight;
+    const bool next = fork >= 0 && height == fork + 1 && step < kPanels;
+    if (fork >= 0 && height > fork && !next) {
+      out[i] |= kSideJoin;
+      fork = -1;
+    }
+    if (next) out[i] |= kSideRun;
+    else if (L.kind == 3 && beside_later(plan, i)) out[i] |= kSideFork | kSideRun;
+    else if (fork < 0 && beside(plan, i)) {
+      out[i] |= kSideFork;
+      fork = height;
+    }
+  }
+  return out;
+}
+template std::vector<int> side_schedule<double>(const DensePlan<double> &);
+template std::vector<int> side_schedule<float>(const DensePlan<float> &);
+template <typename T>
+const DensePlan<T> &plan_of(snumat *h) {
+  if (!h->on_device) {  // (pointers from null: the launches alone are meant)
+    layout_dense(h);
+    build_dense_plan<T>(h);
+  }
+  return vals<T>(h).fact;
+}
+template const DensePlan<double> &plan_of<double>(snumat *);
+template const DensePlan<float> &plan_of<float>(snumat *);
 template <typename T>
 int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s) {
   std::map<long long, double> flops;
@@ -1853,13 +1900,9 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   launch_extend_add<T>(fp.d_tiles + fp.sep0, (int)fp.tiles.size() - fp.sep0, fp.d_src, st);
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[4], st));
-  // the diagonal blocks of the height above and their inverses on the second
-  // stream, from the updates of those blocks until its panels need them, beside
-  // the other Schur updates of the height; before them the copy of the height's
-  // panels to where the solves read them, beside the Schur updates of the
-  // diagonal blocks (one stream when profiled: launches are timed one by one)
-  SideStream *side = prof ? nullptr : fs.side;
-  bool forked = false;
+  // (one stream when profiled: launches are timed one by one)
+  SideStream *side = !prof && fs.side && fs.side->st ? fs.side : nullptr;
+  const std::vector<int> how = side ? side_schedule(plan) : std::vector<int>(plan.launches.size(), 0);
   auto fork = [&]() -> int {
     HIPCHK(hipEventRecord(side->fork, st));
     HIPCHK(hipStreamWaitEvent(side->st, side->fork, 0));
@@ -1868,26 +1911,17 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
   auto join = [&]() -> int {
     HIPCHK(hipEventRecord(side->join, side->st));
     HIPCHK(hipStreamWaitEvent(st, side->join, 0));
-    forked = false;
     return SNU_OK;
   };
   int rc;
+  bool pending = false;
   for (size_t i = 0; i < plan.launches.size(); i++) {
-    const Launch &L = plan.launches[i];
-    const long long step = L.key % kHeight;
-    if (side && side->st && L.kind == 3 && beside_later(plan, i)) {
-      if ((rc = fork())) return rc;
-      if ((rc = run_timed(L, plan, side->st))) return rc;
-      continue;
-    }
-    if (side && side->st && !forked && beside(plan, i)) {
-      if ((rc = fork())) return rc;
-      forked = true;
-    }
-    if (forked && step >= kPanels && step < kNextD && (rc = join())) return rc;
-    if ((rc = run_timed(L, plan, forked && step < kPanels ? side->st : st))) return rc;
+    if ((how[i] & kSideJoin) && (rc = join())) return rc;
+    if ((how[i] & kSideFork) && (rc = fork())) return rc;
+    pending = (pending && !(how[i] & kSideJoin)) || (how[i] & kSideFork);
+    if ((rc = run_timed(plan.launches[i], plan, how[i] & kSideRun ? side->st : st))) return rc;
   }
-  if (forked && (rc = join())) return rc;
+  if (pending && (rc = join())) return rc;
   HIPCHK(hipGetLastError());
   if (ev) HIPCHK(hipEventRecord((*ev)[5], st));
   return SNU_OK;
