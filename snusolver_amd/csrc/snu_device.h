@@ -49,6 +49,42 @@ __device__ __forceinline__ double bcast16(double v) {
                           __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + K, 0xf, 0xf, false));
 }
 
+// frexp, reciprocal, ldexp and division fixup in both precisions
+__device__ __forceinline__ double frexp_m(double x) { return __builtin_amdgcn_frexp_mant(x); }
+__device__ __forceinline__ float frexp_m(float x) { return __builtin_amdgcn_frexp_mantf(x); }
+__device__ __forceinline__ int frexp_e(double x) { return __builtin_amdgcn_frexp_exp(x); }
+__device__ __forceinline__ int frexp_e(float x) { return __builtin_amdgcn_frexp_expf(x); }
+__device__ __forceinline__ double recip(double x) { return __builtin_amdgcn_rcp(x); }
+__device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double scale2(double x, int e) { return __builtin_amdgcn_ldexp(x, e); }
+__device__ __forceinline__ float scale2(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
+__device__ __forceinline__ double div_special(double q, double d, double a) { return __builtin_amdgcn_div_fixup(q, d, a); }
+__device__ __forceinline__ float div_special(float q, float d, float a) { return __builtin_amdgcn_div_fixupf(q, d, a); }
+// Quotients by one divisor, rounded as by divisions, with one reciprocal: a few
+// Newton steps, and per quotient corrections by the exact remainder in FMA
+// (Markstein's division), on the mantissas of both so that nothing on the way
+// overflows or underflows (a dividend taken whole did beyond half the largest
+// value, and lost its remainder near the smallest); subnormal quotients are
+// rounded twice.
+template <typename T>
+struct Divisor {
+  T m, r;  // mantissa, its reciprocal
+  int e;   // exponent
+  __device__ __forceinline__ Divisor(T m_, T r_, int e_) : m(m_), r(r_), e(e_) {}
+  __device__ __forceinline__ explicit Divisor(T d) : m(frexp_m(d)), e(frexp_e(d)) {
+    r = recip(m);
+    r = fma(fma(-m, r, T(1)), r, r);
+    if constexpr (std::is_same<T, double>::value) r = fma(fma(-m, r, T(1)), r, r);
+  }
+  __device__ __forceinline__ T quotient(T a) const {
+    const T n = frexp_m(a);
+    T q = n * r;
+    q = fma(fma(-m, q, n), r, q);
+    if constexpr (std::is_same<T, float>::value) q = fma(fma(-m, q, n), r, q);
+    return div_special(scale2(q, frexp_e(a) - e), m, a);
+  }
+};
+
 // MFMA fragments, 16x16x4 products.  A 16 x 16 block of a vector group (16 rows, 16 columns)
 // is one fragment: register r of lane l holds row frag_row(r), column l % 16,
 // which is both the layout the product leaves its result in and, taking the

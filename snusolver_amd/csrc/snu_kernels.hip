@@ -726,26 +726,12 @@ __device__ __forceinline__ void rank1(T (&d)[16], T (&v)[16], T md, T mv) {
     rank1<T, J, C + N>(d, v, md, mv);
   }
 }
-// frexp, reciprocal, fixup and ldexp in both precisions
-__device__ __forceinline__ double frexp_m(double x) { return __builtin_amdgcn_frexp_mant(x); }
-__device__ __forceinline__ float frexp_m(float x) { return __builtin_amdgcn_frexp_mantf(x); }
-__device__ __forceinline__ int frexp_e(double x) { return __builtin_amdgcn_frexp_exp(x); }
-__device__ __forceinline__ int frexp_e(float x) { return __builtin_amdgcn_frexp_expf(x); }
-__device__ __forceinline__ double recip(double x) { return __builtin_amdgcn_rcp(x); }
-__device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double div_end(double z, int e, double p, double a) {
-  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_ldexp(z, e), p, a);
-}
-__device__ __forceinline__ float div_end(float z, int e, float p, float a) {
-  return __builtin_amdgcn_div_fixupf(__builtin_amdgcn_ldexpf(z, e), p, a);
-}
 // Column J of the diagonal block d (entry l16 of its columns per lane; becomes
 // its LU factors) and of what a wave carries along in v.  keep: v[J] stays as
 // it is instead of being divided by the pivot.  One code path for both waves:
 // fetching variants of the unrolled steps cost more than the arithmetic.
-// d[J] / pivot and v[J] / pivot are rounded as by two divisions, with one
-// reciprocal (Newton steps and a last correction by the exact remainder, in
-// FMA, on the pivot's mantissa: Markstein's division).
+// d[J] / pivot and v[J] / pivot are rounded as by two divisions (Divisor), with
+// one reciprocal.
 template <typename T, int J>
 __device__ __forceinline__ void diag_step(T (&d)[16], T (&v)[16], int l16, bool keep, T eps) {
   // pivots of magnitude below eps become +-eps (the leaf pivots' rule; eps = 0
@@ -753,15 +739,8 @@ __device__ __forceinline__ void diag_step(T (&d)[16], T (&v)[16], int l16, bool 
   T piv = bcast16<J>(d[J]);
   const T cl = piv < T(0) ? -eps : eps;
   piv = fabs(piv) < eps ? cl : piv;
-  const T m = frexp_m(piv);
-  const int e = -frexp_e(piv);
-  T r = recip(m);
-  r = fma(fma(-m, r, T(1)), r, r);
-  if constexpr (std::is_same<T, double>::value) r = fma(fma(-m, r, T(1)), r, r);
-  T a = d[J] * r, b = v[J] * r;
-  a = fma(fma(-m, a, d[J]), r, a), b = fma(fma(-m, b, v[J]), r, b);
-  if constexpr (std::is_same<T, float>::value) a = fma(fma(-m, a, d[J]), r, a), b = fma(fma(-m, b, v[J]), r, b);
-  a = div_end(a, e, piv, d[J]), b = div_end(b, e, piv, v[J]);
+  const Divisor<T> by(piv);
+  const T a = by.quotient(d[J]), b = by.quotient(v[J]);
   const T md = l16 > J ? a : T(0);
   d[J] = l16 > J ? a : l16 == J ? piv : d[J];
   v[J] = keep ? v[J] : b;
