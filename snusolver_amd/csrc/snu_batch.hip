@@ -119,7 +119,7 @@ int build_factor_set(snubatch *b) {
   std::vector<const FrontPlan<T> *> fronts;
   for (snumat *h : b->mats) fronts.push_back(&vals<T>(h).fronts);
   merge_fronts(fronts, fp);
-  if ((rc = upload_dense_plan(fp.dense)) || (rc = bupload(b, &fp.d_iblk, fp.iblk)) || (rc = bupload(b, &fp.d_small, fp.small)) ||
+  if ((rc = upload_dense_plan(fp.dense)) || (rc = bupload(b, &fp.d_small, fp.small)) ||
       (rc = bupload(b, &fp.d_tiles, fp.tiles)) || (rc = bupload(b, &fp.d_src, fp.src)))
     return rc;
   // both streams anew, one after the other (see SideStream)

@@ -70,7 +70,7 @@ template <typename T>
 struct Divisor {
   T m, r;  // mantissa, its reciprocal
   int e;   // exponent
-  __device__ __forceinline__ Divisor(T m_, T r_, int e_) : m(m_), r(r_), e(e_) {}
+  Divisor() = default;
   __device__ __forceinline__ explicit Divisor(T d) : m(frexp_m(d)), e(frexp_e(d)) {
     r = recip(m);
     r = fma(fma(-m, r, T(1)), r, r);
@@ -83,7 +83,47 @@ struct Divisor {
     if constexpr (std::is_same<T, float>::value) q = fma(fma(-m, q, n), r, q);
     return div_special(scale2(q, frexp_e(a) - e), m, a);
   }
+  // The same, a shorter chain for substitution: the dividend scaled whole, one
+  // correction.  (Rounded as by a division while remainders are normal numbers;
+  // where a division gives an infinity, any value that is not finite.)
+  __device__ __forceinline__ T quick(T a) const {
+    const T n = scale2(a, -e), q = n * r;
+    return fma(fma(-m, q, n), r, q);
+  }
+  // lane l's divisor
+  __device__ __forceinline__ Divisor of_lane(int l) const {
+    Divisor d;
+    d.m = rld(m, l), d.r = rld(r, l), d.e = rl(e, l);
+    return d;
+  }
 };
+
+// Between the four groups of 16 lanes (permlane swaps: VALU, no LDS).
+// every group's v, in all lanes
+__device__ __forceinline__ void gather_groups(double v, double (&s)[4]) {
+  unsigned w[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const unsigned x = h ? __double2hiint(v) : __double2loint(v);
+    const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(p[0], p[0], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(p[1], p[1], false, false);
+    w[h][0] = a[0], w[h][1] = a[1], w[h][2] = b[0], w[h][3] = b[1];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) s[i] = __hiloint2double((int)w[1][i], (int)w[0][i]);
+}
+// group G's s[i], in group i
+template <int G>
+__device__ __forceinline__ float spread_group(const float (&s)[4]) {
+  unsigned x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = __float_as_uint(s[i]);
+  const auto a = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+  const auto p = __builtin_amdgcn_permlane32_swap(a[G & 1], b[G & 1], false, false);
+  return __uint_as_float(p[G >> 1]);
+}
 
 // MFMA fragments, 16x16x4 products.  A 16 x 16 block of a vector group (16 rows, 16 columns)
 // is one fragment: register r of lane l holds row frag_row(r), column l % 16,

@@ -80,26 +80,18 @@ struct FrontLevel {
 template <typename T>
 struct FrontPlan {
   std::vector<FrontDev> small;
-  std::vector<int2> iblk;   // 16-pivot blocks of the small fronts: {front, first pivot}
   std::vector<AddTile> tiles;  // by height, then the separator tiles
   std::vector<AddSrc> src;
   int sep0 = 0;             // first separator tile
   std::vector<FrontLevel> levels;
   DensePlan<T> dense;
   FrontDev *d_small = nullptr;
-  int2 *d_iblk = nullptr;
   AddTile *d_tiles = nullptr;
   AddSrc *d_src = nullptr;
 };
-// Values of the inverses kept behind a front (FrontDev::inv).
+// Values kept behind a front for its pivot blocks (kFrontInv; larger fronts).
 inline long long front_inv_size(int f, int nk, int fmax) {
-  return f > fmax ? (nk + 63) / 64 * (long long)kFrontInv : (nk + 15) / 16 * 256LL;
-}
-template <typename T>
-void list_inverse_blocks(FrontPlan<T> &fp) {
-  fp.iblk.clear();
-  for (size_t f = 0; f < fp.small.size(); f++)
-    for (int k = 0; k < fp.small[f].nk; k += 16) fp.iblk.push_back(make_int2((int)f, k));
+  return f > fmax ? (nk + 63) / 64 * (long long)kFrontInv : 0;
 }
 inline long long front_key(int height, int step, int kind) {
   return (long long)height * 100000000LL + step * 8LL + kind;
@@ -113,7 +105,7 @@ struct Values {
   T *inv = nullptr;    // per separator: full L^-1 then U^-1 (s x s each)
   T *lu = nullptr;     // per separator: LU of its 64 x 64 diagonal blocks
   T *tmp = nullptr;    // products of a level's panels, then of its triangular inversion
-  T *farena = nullptr; // leaf fronts (each f x f, then the inverses of its pivot blocks)
+  T *farena = nullptr; // leaf fronts (each f x f, a larger one's pivot blocks behind it)
   FrontPlan<T> fronts;
   DensePlan<T> fact;
   // standalone solves: right-hand sides, dense-solve vectors, the fronts'

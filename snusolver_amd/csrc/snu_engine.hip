@@ -1104,7 +1104,6 @@ int build_front_plan(snumat *h) {
       }
       FrontDev D;
       D.F = F;
-      D.inv = inv;
       D.aval = h->d_aval;
       D.ent = d_ent + ent0[r][f];
       D.child = d_ch + ch0[r][f];
@@ -1353,8 +1352,7 @@ int build_front_plan(snumat *h) {
     AddTile &t = FP.tiles[FP.sep0 + sent_of[e].first];
     if (t.nent++ == 0) t.ent = d_sent + e, t.aval = h->d_aval;
   }
-  list_inverse_blocks(FP);
-  if ((rc = dupload(h, &FP.d_iblk, FP.iblk)) || (rc = dupload(h, &FP.d_small, FP.small)) ||
+  if ((rc = dupload(h, &FP.d_small, FP.small)) ||
       (rc = dupload(h, &FP.d_tiles, FP.tiles)) || (rc = dupload(h, &FP.d_src, FP.src)))
     return rc;
   return SNU_OK;
@@ -1401,7 +1399,6 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
   }
   out.sep0 = (int)out.tiles.size();
   for (size_t pi = 0; pi < in.size(); pi++) add_tiles(pi, in[pi]->sep0, (int)in[pi]->tiles.size() - in[pi]->sep0);
-  list_inverse_blocks(out);
   std::vector<const DensePlan<T> *> dp;
   for (const FrontPlan<T> *p : in) dp.push_back(&p->dense);
   merge_dense(dp, out.dense);
@@ -1661,7 +1658,7 @@ size_t estimate_device_bytes(const snumat *h) {
   double idx = 0, inv = 0, fronts = 0;
   const int fmax = h->prec == SNU_FP32 ? front_small_max<float>() : front_small_max<double>();
   for (const LeafPlan &L : P.leaves) {
-    // fronts: values with the inverses of their pivot blocks; solve units,
+    // fronts: values with larger ones' pivot blocks; solve units,
     // children's update rows, positions of the B entries; extend-add tiles
     // and their sources
     fronts += (double)L.fentries;
@@ -1891,7 +1888,6 @@ int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st
       if (rc) return rc;
     }
   }
-  launch_front_inverse<T>(fp.d_small, fp.d_iblk, (int)fp.iblk.size(), st);
   HIPCHK(hipGetLastError());
   if (ev) {
     HIPCHK(hipEventRecord((*ev)[2], st));

@@ -157,63 +157,6 @@ __global__ __launch_bounds__(64) void k_front_wave(const FrontDev *__restrict__ 
   }
 }
 
-// Inverses of the 16 x 16 diagonal blocks of L11 and U11 of the fronts factored
-// in LDS (the solves multiply by them): a group of 16 lanes per block, lane =
-// column, by substitution in registers; the multipliers come from the lane
-// that holds their column (DPP broadcast within 16 lanes).  A launch of its
-// own: inside k_front_small the unrolled substitution took its registers from
-// 30 to 256 and its workgroups per CU with them (batch of 96 2D matrices: 6.2
-// -> 9.2 ms per factorize + solve).
-template <typename T, int K>
-__device__ __forceinline__ void inv_step_l(T (&a)[16], T (&x)[16]) {
-#pragma unroll
-  for (int i = K + 1; i < 16; i++) x[i] -= bcast16<K>(a[i]) * x[K];
-  // opaque between steps: keeps broadcasts of later steps out of registers
-#pragma unroll
-  for (int i = K + 1; i < 16; i++) asm volatile("" : "+v"(x[i]), "+v"(a[i]));
-}
-template <typename T, int K>
-__device__ __forceinline__ void inv_step_u(T (&a)[16], T rc, T (&x)[16]) {
-  x[K] *= bcast16<K>(rc);
-#pragma unroll
-  for (int i = 0; i < K; i++) x[i] -= bcast16<K>(a[i]) * x[K];
-#pragma unroll
-  for (int i = 0; i < K; i++) asm volatile("" : "+v"(x[i]), "+v"(a[i]));
-}
-template <typename T, int... K>
-__device__ __forceinline__ void inv_steps(std::integer_sequence<int, K...>, T (&a)[16], T rc, T (&xl)[16],
-                                          T (&xu)[16]) {
-  (inv_step_l<T, K>(a, xl), ...);
-  (inv_step_u<T, 15 - K>(a, rc, xu), ...);
-}
-template <typename T>
-__global__ __launch_bounds__(256) void k_front_inverse(const FrontDev *__restrict__ fr, const int2 *__restrict__ blk,
-                                                       int nblk) {
-  const int t = blockIdx.x * 16 + (threadIdx.x >> 4), j = threadIdx.x & 15;
-  const int2 w = blk[min(t, nblk - 1)];
-  const FrontDev D = fr[w.x];
-  const int base = w.y, nbk = min(16, D.nk - base);
-  const T *F = (const T *)D.F + base + (long long)(base + min(j, nbk - 1)) * D.f;
-  T a[16], xl[16], xu[16], d = T(1);
-#pragma unroll
-  for (int i = 0; i < 16; i++) {
-    const T v = F[min(i, nbk - 1)];
-    a[i] = i < nbk && j < nbk ? v : T(0);
-    if (i == j && j < nbk) d = v;
-    xl[i] = xu[i] = i == j ? T(1) : T(0);
-  }
-  inv_steps<T>(std::make_integer_sequence<int, 16>{}, a, T(1) / d, xl, xu);
-  if (t >= nblk) return;
-  T *I = (T *)D.inv + (long long)base * 16 + j * 16;
-#pragma unroll
-  for (int i = 0; i < 16; i++) I[i] = i > j ? xl[i] : xu[i];
-}
-template <typename T>
-void launch_front_inverse(const FrontDev *fr, const int2 *blk, int nblk, hipStream_t st) {
-  if (nblk <= 0) return;
-  hipLaunchKernelGGL(k_front_inverse<T>, dim3((nblk + 15) / 16), dim3(256), 0, st, fr, blk, nblk);
-}
-
 // Largest front factored whole in LDS (order): above it a front goes
 // through HBM and the dense kernels.  Measured 64 / 80 / 96 / 128 (FP64) on
 // the 64^3, 96^3 and batch workloads: smaller LDS fronts keep more
@@ -305,7 +248,6 @@ void launch_extend_add(const AddTile *tiles, int ntile, const AddSrc *src, hipSt
   template int front_small_max<T>();                                                           \
   template void launch_front_small<T>(const FrontDev *, int, int, double, hipStream_t);        \
   template void launch_front_wave<T>(const FrontDev *, int, int, double, hipStream_t);         \
-  template void launch_front_inverse<T>(const FrontDev *, const int2 *, int, hipStream_t);     \
   template void launch_extend_add<T>(const AddTile *, int, const AddSrc *, hipStream_t);
 SNU_FRONT_INST(double)
 SNU_FRONT_INST(float)

@@ -16,7 +16,7 @@ namespace snu {
 // boundary columns (backward).
 enum SolveUnitKind { kFwdFront = 0, kFwdPivots, kFwdRows, kBwdFront, kBwdCols, kBwdPivots };
 struct SolveUnit {
-  const void *F, *inv;       // the front (column-major), its diagonal blocks' inverses
+  const void *F, *inv;       // the front (column-major), a larger one's pivot blocks (kFrontInv)
   int ld, nk, nb;            // front order, pivots, boundary entries B
   int kpos;                  // solve position of the first pivot (pivots are consecutive)
   int wrow;                  // first row of the front's update vector
@@ -56,9 +56,6 @@ struct AEntry {
 // A front factored whole in LDS.
 struct FrontDev {
   void *F;                  // the front's values (f x f, column-major)
-  void *inv;                // inverses of the pivot blocks' triangles: 16 x 16 blocks, L^-1 below
-                            // the diagonal, U^-1 on and above it (larger fronts: per 64-pivot
-                            // block L^-1, U^-1 and LU, 64 x 64 each)
   const double *aval;       // A's values
   const AEntry *ent;        // its entries of A
   const FrontChild *child;  // children in ascending order (their updates are added in it)
@@ -273,9 +270,6 @@ void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, h
 constexpr int kFrontWave = 48;
 template <typename T>
 void launch_front_wave(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st);
-// Inverses of their 16 x 16 diagonal blocks; blk: {front, first pivot}.
-template <typename T>
-void launch_front_inverse(const FrontDev *fr, const int2 *blk, int nblk, hipStream_t st);
 // Largest front order the LDS kernel takes for this value type.
 template <typename T>
 int front_small_max();

@@ -105,20 +105,29 @@ void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *
 // Forward, per front: w = (b of its pivots, 0) + the children's updates; y =
 // L11^-1 w_K replaces b, and w_B - L21 y is the front's update for its
 // parent (root fronts: for the separators, k_assemble_rhs).  Backward: x_K =
-// U11^-1 (y_K - U12 x_B).  A front's rows read their children's update rows
-// through lists in a fixed order, so no two units write one place and results
-// do not depend on scheduling.
+// U11^-1 (y_K - U12 x_B).  Both by substitution with divisions by the pivots.
+// (The inverses of triangles of 16 and 64 pivots in its place are shorter
+// chains, but their error grows with the triangle's condition number: one front
+// of a chain with diagonal 2, -3 below and -0.3 above, FP64, has backward error
+// 1.4e-12 at order 48 and 6e-3 at order 65 with them, 2e-16 by substitution.)
+// A row's products are summed and then taken from it, so that rounding goes
+// with their sum (errors of x against the exact solution 3.8e-16 to 4.6e-16 on
+// 2D and 3D grids; 4.7e-16 to 5.8e-16 taking them from the row one by one).
+// A front's rows read their children's update rows through lists in a fixed
+// order, so no two units write one place and results do not depend on
+// scheduling.
 // One workgroup per leaf and column group walks the leaf's front tree height
 // by height; between two barriers its waves take the units of a phase in turn.
 // That keeps the whole sweep in one launch (the tree is 3 to 12 heights of at
 // most a few hundred units) and a unit is sized so that a wave has 16 or more
-// loads in flight.  Bound by the latency of the units' loads down the chain of
-// heights; forward / backward, against row-by-row level sets over the leaf's
-// CSR factors (hundreds of levels, one row per wave): 64^3 7-point FP64, one
-// column 199 / 239 us (554 / 828); 48^3 27-point FP64, 16 columns 508 / 392 us
-// (2916 / 4719); 1000^2 5-point FP32, 64 columns 1.5 / 1.1 ms (3.8 / 4.8).
-// 1024 threads per leaf for one column (261 / 292 us with 512); the 16-column
-// fragments need 230 registers, so 512.
+// loads in flight.  Bound by the latency of the units' loads and substitutions
+// down the chain of heights; forward / backward: 64^3 7-point FP64, one column
+// 214 / 272 us (row by row over the leaf's CSR factors, hundreds of level sets:
+// 554 / 828; with the inverses 202 / 242); 48^3 27-point FP64, 16 columns 505 /
+// 436 us (2916 / 4719; 492 / 382); 1000^2 5-point FP32, 64 columns 1.45 / 1.27
+// ms (3.8 / 4.8; 1.53 / 1.15).
+// 1024 threads per leaf for one column (261 / 292 us with 512 and the
+// inverses); the 16-column fragments need over 200 registers, so 512.
 template <int NC>
 constexpr int leaf_threads() {
   return NC == 1 ? 1024 : 512;
@@ -136,6 +145,11 @@ __device__ __forceinline__ SolveUnit load_unit(const SolveUnit *p) {
 struct SweepCtx {
   int lane, l16, lk;
 };
+// LU of the unit's 64-pivot block of a larger front (64 x 64)
+template <typename T>
+__device__ __forceinline__ const T *pivot_block(const SolveUnit &U) {
+  return (const T *)U.inv + (long long)U.s * kFrontInv + 2 * 4096;
+}
 
 // ---- one column ----
 typedef int int2_v __attribute__((ext_vector_type(2)));
@@ -181,10 +195,72 @@ __device__ __forceinline__ T dot_cols(const T *a, long long ld, int K, int lane,
   }
   return (s0 + s1) + (s2 + s3);
 }
+// w -= L y for the `rows` rows of a lower trapezoid (unit diagonal, n columns;
+// y: w's first n rows on the way), RPL rows per lane.  A row's products are
+// summed and taken from it at once: rounding relative to their sum, not to the
+// row at every step.
+template <typename T, int RPL>
+__device__ __forceinline__ void solve_lower1(const T *A, int ld, int rows, int n, T (&w)[RPL], int lane) {
+  const auto F = gptr(A);
+  T s[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; i++) s[i] = T(0);
+  for (int k0 = 0; k0 < n; k0 += 16) {
+    T c[RPL][16];
+#pragma unroll
+    for (int i = 0; i < RPL; i++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) c[i][j] = F[min(lane + 64 * i, rows - 1) + min(k0 + j, n - 1) * ld];
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      const int k = k0 + j;
+      T yk = RPL == 1 || k < 64 ? rld(w[0] - s[0], k & 63) : rld(w[RPL - 1] - s[RPL - 1], k & 63);
+      if (k >= n) yk = T(0);
+#pragma unroll
+      for (int i = 0; i < RPL; i++) s[i] = lane + 64 * i > k ? s[i] + c[i][j] * yk : s[i];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RPL; i++) w[i] -= s[i];
+}
+// the divisors of an upper triangle's rows
+template <typename T, int RPL>
+__device__ __forceinline__ void pivots1(const T *A, int ld, int n, Divisor<T> (&by)[RPL], int lane) {
+#pragma unroll
+  for (int i = 0; i < RPL; i++) {
+    const int r = lane + 64 * i;
+    by[i] = Divisor<T>(r < n ? gptr(A)[(long long)r * (ld + 1)] : T(1));
+  }
+}
+// t = U^-1 (t - s), n rows
+template <typename T, int RPL>
+__device__ __forceinline__ void solve_upper1(const T *A, int ld, int n, const Divisor<T> (&by)[RPL], T (&t)[RPL],
+                                             T (&s)[RPL], int lane) {
+  const auto F = gptr(A);
+  for (int k0 = n - 1; k0 >= 0; k0 -= 16) {
+    T c[RPL][16];
+#pragma unroll
+    for (int i = 0; i < RPL; i++)
+#pragma unroll
+      for (int j = 0; j < 16; j++) c[i][j] = F[min(lane + 64 * i, n - 1) + max(k0 - j, 0) * ld];
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      const int k = k0 - j;
+      const int kk = max(k, 0);
+      T xk = RPL == 1 || kk < 64 ? rld(by[0].quick(t[0] - s[0]), kk & 63)
+                                 : rld(by[RPL - 1].quick(t[RPL - 1] - s[RPL - 1]), kk & 63);
+#pragma unroll
+      for (int i = 0; i < RPL; i++) {
+        const int r = lane + 64 * i;
+        if (r < k) s[i] += c[i][j] * xk;
+        else if (r == k) t[i] = xk, s[i] = T(0);
+      }
+    }
+  }
+}
 // RPL rows per lane (front order <= 64 RPL)
 template <typename T, int RPL>
 __device__ __forceinline__ void fwd_front1(const LeafDev &L, const SolveUnit &U, T *x, T *W, int lane) {
-  const auto F = gptr((const T *)U.F);
   const int f = U.ld, nk = U.nk;
   T w[RPL];
 #pragma unroll
@@ -193,21 +269,7 @@ __device__ __forceinline__ void fwd_front1(const LeafDev &L, const SolveUnit &U,
     w[i] = r < nk ? x[U.kpos + r] : T(0);
     w[i] += pull_sum<T, 1>(L, W, r < f ? pull_entry(L, U, r) : int2_v{-1, -1}, 0);
   }
-  for (int k0 = 0; k0 < nk; k0 += 16) {
-    T c[RPL][16];
-#pragma unroll
-    for (int i = 0; i < RPL; i++)
-#pragma unroll
-      for (int j = 0; j < 16; j++) c[i][j] = F[min(lane + 64 * i, f - 1) + min(k0 + j, nk - 1) * f];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      const int k = k0 + j;
-      T yk = RPL == 1 || k < 64 ? rld(w[0], k & 63) : rld(w[RPL - 1], k & 63);
-      if (k >= nk) yk = T(0);
-#pragma unroll
-      for (int i = 0; i < RPL; i++) w[i] = lane + 64 * i > k ? w[i] - c[i][j] * yk : w[i];
-    }
-  }
+  solve_lower1<T, RPL>((const T *)U.F, f, f, nk, w, lane);
 #pragma unroll
   for (int i = 0; i < RPL; i++) {
     const int r = lane + 64 * i;
@@ -219,13 +281,14 @@ template <typename T, int RPL>
 __device__ __forceinline__ void bwd_front1(const LeafDev &L, const SolveUnit &U, T *x, int lane) {
   const auto F = gptr((const T *)U.F);
   const int f = U.ld, nk = U.nk, nb = U.nb;
-  T xb[RPL], t[RPL], s[RPL], rc[RPL];
+  T xb[RPL], t[RPL], s[RPL];
+  Divisor<T> by[RPL];
+  pivots1<T, RPL>((const T *)U.F, f, nk, by, lane);
 #pragma unroll
   for (int i = 0; i < RPL; i++) {
     const int r = lane + 64 * i;
     xb[i] = r < nb ? x[gptr(L.bidx)[U.bidx + r]] : T(0);
     t[i] = r < nk ? x[U.kpos + r] : T(0);
-    rc[i] = r < nk ? T(1) / F[r + r * f] : T(0);
     s[i] = T(0);
   }
   // U12 x_B: 64 / gw columns per load when the pivots leave lanes free
@@ -255,40 +318,16 @@ __device__ __forceinline__ void bwd_front1(const LeafDev &L, const SolveUnit &U,
 #pragma unroll
   for (int i = 0; i < RPL; i++) {
     for (int o = gw; o < 64; o <<= 1) s[i] += __shfl_xor(s[i], o, 64);
-    t[i] -= s[i];
   }
-  for (int k0 = nk - 1; k0 >= 0; k0 -= 16) {
-    T c[RPL][16];
-#pragma unroll
-    for (int i = 0; i < RPL; i++)
-#pragma unroll
-      for (int j = 0; j < 16; j++) c[i][j] = F[min(lane + 64 * i, nk - 1) + max(k0 - j, 0) * f];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      const int k = k0 - j;
-      const int kk = max(k, 0);
-      T xk = RPL == 1 || kk < 64 ? rld(t[0] * rc[0], kk & 63) : rld(t[RPL - 1] * rc[RPL - 1], kk & 63);
-#pragma unroll
-      for (int i = 0; i < RPL; i++) {
-        const int r = lane + 64 * i;
-        if (r < k) t[i] -= c[i][j] * xk;
-        else if (r == k) t[i] = xk;
-      }
-    }
-  }
+  solve_upper1<T, RPL>((const T *)U.F, f, nk, by, t, s, lane);
 #pragma unroll
   for (int i = 0; i < RPL; i++)
     if (lane + 64 * i < nk) x[U.kpos + lane + 64 * i] = t[i];
 }
-// inverse of a 64-pivot block times v (lane = row; v zero beyond the block)
-template <typename T>
-__device__ __forceinline__ T block_inverse1(const T *inv, int nbk, T v, int lane) {
-  return dot_cols(inv + min(lane, nbk - 1), 64, nbk, lane, [&](int) { return v; });
-}
 template <typename T, bool BWD>
 __device__ __forceinline__ void unit1(const LeafDev &L, const SolveUnit &U, T *x, T *W, int lane) {
   constexpr int RPL = sizeof(T) == 8 ? 1 : 2;
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * kFrontInv;
+  const T *F = (const T *)U.F, *lu = pivot_block<T>(U);
   const int f = U.ld, nk = U.nk, r0 = 64 * U.s, nbk = min(64, nk - r0), r = r0 + min(lane, nbk - 1);
   if constexpr (!BWD) switch (U.kind) {
     case kFwdFront: fwd_front1<T, RPL>(L, U, x, W, lane); break;
@@ -299,8 +338,9 @@ __device__ __forceinline__ void unit1(const LeafDev &L, const SolveUnit &U, T *x
         const T p = dot_cols(F + r, f, r0, lane, [&](int k) { return x[U.kpos + k]; });
         if (lane < nbk) w -= p;
       }
-      const T y = block_inverse1(inv, nbk, w, lane);
-      if (lane < nbk) x[U.kpos + r] = y;
+      T y[1] = {w};
+      solve_lower1<T, 1>(lu, 64, nbk, nbk, y, lane);
+      if (lane < nbk) x[U.kpos + r] = y[0];
       break;
     }
     case kFwdRows: {
@@ -321,18 +361,15 @@ __device__ __forceinline__ void unit1(const LeafDev &L, const SolveUnit &U, T *x
       break;
     }
     case kBwdPivots: {
-      T t = lane < nbk ? x[U.kpos + r] : T(0);
-      for (int q = 0; q < U.nq; q++) {
-        const T p = W[U.wrow + (U.s * U.nq + q) * 64 + lane];
-        if (lane < nbk) t -= p;
-      }
-      if (r0 + 64 < nk) {
-        const T p = dot_cols(F + r + (long long)(r0 + 64) * f, f, nk - r0 - 64, lane,
-                             [&](int k) { return x[U.kpos + r0 + 64 + k]; });
-        if (lane < nbk) t -= p;
-      }
-      const T y = block_inverse1(inv + 4096, nbk, t, lane);
-      if (lane < nbk) x[U.kpos + r] = y;
+      Divisor<T> by[1];
+      pivots1<T, 1>(lu, 64, nbk, by, lane);
+      T y[1] = {lane < nbk ? x[U.kpos + r] : T(0)}, s[1] = {T(0)};
+      for (int q = 0; q < U.nq; q++) s[0] += W[U.wrow + (U.s * U.nq + q) * 64 + lane];
+      if (r0 + 64 < nk)
+        s[0] += dot_cols(F + r + (long long)(r0 + 64) * f, f, nk - r0 - 64, lane,
+                         [&](int k) { return x[U.kpos + r0 + 64 + k]; });
+      solve_upper1<T, 1>(lu, 64, nbk, by, y, s, lane);
+      if (lane < nbk) x[U.kpos + r] = y[0];
       break;
     }
   }
@@ -405,44 +442,92 @@ __device__ __forceinline__ void frag_mm(Frag<T> &acc, const T *a, int ld, int k0
 #pragma unroll
   for (int r = 0; r < 4; r++) acc = mfma4(v[r], b[r], acc);
 }
-// 16 x 16 inverse block times v: the strict lower triangle with a unit
-// diagonal, or the upper triangle
+// A 16 x 16 block of a triangle (unit lower, or upper), n of its rows and
+// columns used: entry (l16, 4 g + lk) of its strict part in a[g].
 template <typename T, bool UPPER>
-__device__ __forceinline__ Frag<T> inv16(const T *inv, const Frag<T> &v, const SweepCtx &c) {
-  const auto p = gptr(inv) + c.l16;
+struct Tri16 {
   T a[4];
+  Divisor<T> by;  // (UPPER) row l16's pivot
+  __device__ __forceinline__ void load(const T *F, int ld, int n, const SweepCtx &c) {
+    const auto p = gptr(F) + min(c.l16, n - 1);
 #pragma unroll
-  for (int r = 0; r < 4; r++) a[r] = p[frag_row<T>(r, c.lk) * 16];
-  Frag<T> acc = frag_zero<T>();
+    for (int g = 0; g < 4; g++) a[g] = p[(long long)min(4 * g + c.lk, n - 1) * ld];
+    if constexpr (UPPER) by = Divisor<T>(c.l16 < n ? p[(long long)min(c.l16, n - 1) * ld] : T(1));
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int k = frag_row<T>(r, c.lk);
-    const T m = UPPER ? (k >= c.l16 ? a[r] : T(0)) : (k < c.l16 ? a[r] : k == c.l16 ? T(1) : T(0));
-    acc = mfma4(m, v[r], acc);
+    for (int g = 0; g < 4; g++) {
+      const int k = 4 * g + c.lk;
+      if (!(UPPER ? k > c.l16 && k < n : k < c.l16 && c.l16 < n)) a[g] = T(0);
+    }
   }
-  return acc;
-}
+  // w - acc solved with it (both zero beyond n).  Four rows at a time: every
+  // lane (FP32: those that hold the four rows) solves them for its column, with
+  // the block's entries and pivots read lane by lane, then one product adds
+  // their share to the rows left.  (The four steps as a loop: half the code, but
+  // a block's loads are then waited for at its head: 1000^2, 64 columns 10.5 ->
+  // 12.5 ms per solve.)
+  template <int g>
+  __device__ __forceinline__ void rows(const Frag<T> &w, Frag<T> &acc, Frag<T> &y, const SweepCtx &c) const {
+    T v[4], p[4], s[4];
+    if constexpr (std::is_same<T, double>::value) {
+      gather_groups(w[g], v);
+      gather_groups(acc[g], p);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = w[i], p[i] = acc[i];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int j = UPPER ? 3 - q : q;
+      s[j] = v[j] - p[j];
+      if constexpr (UPPER) s[j] = by.of_lane(4 * g + j).quick(s[j]);
+#pragma unroll
+      for (int i = UPPER ? 0 : j + 1; i < (UPPER ? j : 4); i++) p[i] += rld(a[g], 4 * g + i + 16 * j) * s[j];
+    }
+    T b;  // row 4 g + lk
+    if constexpr (std::is_same<T, double>::value) {
+      b = c.lk == 0 ? s[0] : c.lk == 1 ? s[1] : c.lk == 2 ? s[2] : s[3];
+      y[g] = b;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) y[i] = c.lk == g ? s[i] : y[i];
+      b = spread_group<g>(s);
+    }
+    if (g != (UPPER ? 0 : 3)) acc = mfma4((UPPER ? c.l16 < 4 * g : c.l16 >= 4 * g + 4) ? a[g] : T(0), b, acc);
+  }
+  __device__ __forceinline__ Frag<T> solve(const Frag<T> &w, Frag<T> acc, const SweepCtx &c) const {
+    Frag<T> y = w;
+    if constexpr (UPPER) rows<3>(w, acc, y, c), rows<2>(w, acc, y, c), rows<1>(w, acc, y, c), rows<0>(w, acc, y, c);
+    else rows<0>(w, acc, y, c), rows<1>(w, acc, y, c), rows<2>(w, acc, y, c), rows<3>(w, acc, y, c);
+    return y;
+  }
+};
 // Whole front with at most 16 KB pivots and 16 BB boundary entries; EXACT: no
 // block is empty, so the code is straight-line and all its loads are in flight
 // before the first product (a branch per block would expose each block's
 // latency in turn).
 template <typename T, int KB, int BB, bool EXACT>
 __device__ __forceinline__ void fwd_front16(const LeafDev &L, const SolveUnit &U, T *x, T *W, const SweepCtx &c) {
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv;
+  const T *F = (const T *)U.F;
   const int f = U.ld, nk = U.nk, nb = U.nb;
   T *xk = x + (long long)U.kpos * kColGroup, *wb = W + (long long)U.wrow * kColGroup;
+  // (the stores to x last: the loads are not moved over them)
+  Tri16<T, false> t[KB];
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int b = 0; b < KB; b++) t[b].load(F + 16 * b * (f + 1), f, min(16, nk - 16 * b), c);
+  }
   Frag<T> y[KB];
 #pragma unroll
   for (int b = 0; b < KB; b++) {
     y[b] = frag_zero<T>();
     if (EXACT || 16 * b < nk) {
+      if constexpr (!EXACT) t[b].load(F + 16 * b * (f + 1), f, min(16, nk - 16 * b), c);
       Frag<T> acc = frag_zero<T>();
 #pragma unroll
       for (int a = 0; a < b; a++) frag_mm(acc, F + min(16 * b + c.l16, nk - 1), f, 16 * a, nk - 1, y[a], c);
-      Frag<T> w = load_frag(xk, 16 * b, nk, c) + pull_frag(L, U, W, 16 * b, nk, c) - acc;
-      mask_frag(w, 16 * b, nk, c);
-      y[b] = inv16<T, false>(inv + 256 * b, w, c);
-      store_frag(xk, 16 * b, nk, y[b], c);
+      Frag<T> w = load_frag(xk, 16 * b, nk, c) + pull_frag(L, U, W, 16 * b, nk, c);
+      mask_frag(acc, 16 * b, nk, c);
+      y[b] = t[b].solve(w, acc, c);
     }
   }
 #pragma unroll
@@ -454,6 +539,9 @@ __device__ __forceinline__ void fwd_front16(const LeafDev &L, const SolveUnit &U
         if (EXACT || 16 * a < nk) frag_mm(acc, F + min(nk + 16 * b + c.l16, f - 1), f, 16 * a, nk - 1, y[a], c);
       store_frag(wb, 16 * b, nb, pull_frag(L, U, W, nk + 16 * b, f, c) - acc, c);
     }
+#pragma unroll
+  for (int b = 0; b < KB; b++)
+    if (EXACT || 16 * b < nk) store_frag(xk, 16 * b, nk, y[b], c);
 }
 // rows of x at the positions idx[row0 ..], zero from n on
 template <typename T>
@@ -470,9 +558,14 @@ __device__ __forceinline__ Frag<T> gather_frag(const T *x, const int *idx, int r
 }
 template <typename T, int KB, int BB, bool EXACT>
 __device__ __forceinline__ void bwd_front16(const LeafDev &L, const SolveUnit &U, T *x, const SweepCtx &c) {
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv;
+  const T *F = (const T *)U.F;
   const int f = U.ld, nk = U.nk, nb = U.nb;
   T *xk = x + (long long)U.kpos * kColGroup;
+  Tri16<T, true> tri[KB];
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int b = 0; b < KB; b++) tri[b].load(F + 16 * b * (f + 1), f, min(16, nk - 16 * b), c);
+  }
   Frag<T> t[KB];
 #pragma unroll
   for (int b = 0; b < KB; b++) t[b] = frag_zero<T>();
@@ -488,15 +581,18 @@ __device__ __forceinline__ void bwd_front16(const LeafDev &L, const SolveUnit &U
 #pragma unroll
   for (int b = KB - 1; b >= 0; b--)
     if (EXACT || 16 * b < nk) {
+      if constexpr (!EXACT) tri[b].load(F + 16 * b * (f + 1), f, min(16, nk - 16 * b), c);
       Frag<T> acc = t[b];
 #pragma unroll
       for (int a = b + 1; a < KB; a++)
         if (EXACT || 16 * a < nk) frag_mm(acc, F + min(16 * b + c.l16, nk - 1), f, 16 * a, nk - 1, t[a], c);
-      Frag<T> w = load_frag(xk, 16 * b, nk, c) - acc;
-      mask_frag(w, 16 * b, nk, c);
-      t[b] = inv16<T, true>(inv + 256 * b, w, c);
-      store_frag(xk, 16 * b, nk, t[b], c);
+      const Frag<T> w = load_frag(xk, 16 * b, nk, c);
+      mask_frag(acc, 16 * b, nk, c);
+      t[b] = tri[b].solve(w, acc, c);
     }
+#pragma unroll
+  for (int b = 0; b < KB; b++)
+    if (EXACT || 16 * b < nk) store_frag(xk, 16 * b, nk, t[b], c);
 }
 // the straight-line form for the block counts of most fronts
 template <typename T, bool BWD>
@@ -557,22 +653,28 @@ __device__ __forceinline__ void tile_mm(Frag<T> (&acc)[4], const T *a, int ld, i
   }
   mul(x, v);
 }
-// the inverse of a 64-pivot block (lower or upper triangular) times w
+// the same with a 64-pivot block (64 x 64, nbk of its rows and columns used)
 template <typename T, bool UPPER>
-__device__ __forceinline__ void block_inverse16(Frag<T> (&y)[4], const T *inv, int nbk, const Frag<T> (&w)[4],
-                                                const SweepCtx &c) {
+__device__ __forceinline__ void tri64(Frag<T> (&y)[4], const T *lu, int nbk, const Frag<T> (&w)[4],
+                                      const Frag<T> (&sum)[4], const SweepCtx &c) {
 #pragma unroll
-  for (int b = 0; b < 4; b++) {
+  for (int q = 0; q < 4; q++) {
+    const int b = UPPER ? 3 - q : q;
     y[b] = frag_zero<T>();
+    if (16 * b >= nbk) continue;
+    Frag<T> acc = sum[b];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
-      if ((UPPER ? a >= b : a <= b) && 16 * a < nbk)
-        frag_mm(y[b], inv + min(16 * b + c.l16, nbk - 1), 64, 16 * a, nbk - 1, w[a], c);
+    for (int a = UPPER ? b + 1 : 0; a < (UPPER ? 4 : b); a++)
+      if (16 * a < nbk) frag_mm(acc, lu + min(16 * b + c.l16, nbk - 1), 64, 16 * a, nbk - 1, y[a], c);
+    Tri16<T, UPPER> t;
+    t.load(lu + 16 * b * 65, 64, min(16, nbk - 16 * b), c);
+    mask_frag(acc, 16 * b, nbk, c);
+    y[b] = t.solve(w[b], acc, c);
   }
 }
 template <typename T, bool BWD>
 __device__ __forceinline__ void unit16(const LeafDev &L, const SolveUnit &U, T *x, T *W, const SweepCtx &c) {
-  const T *F = (const T *)U.F, *inv = (const T *)U.inv + (long long)U.s * kFrontInv;
+  const T *F = (const T *)U.F, *lu = pivot_block<T>(U);
   const int f = U.ld, nk = U.nk, r0 = 64 * U.s, nbk = min(64, nk - r0);
   T *xk = x + (long long)U.kpos * kColGroup, *wf = W + (long long)U.wrow * kColGroup;
   Frag<T> acc[4];
@@ -584,10 +686,9 @@ __device__ __forceinline__ void unit16(const LeafDev &L, const SolveUnit &U, T *
       Frag<T> w[4], y[4];
 #pragma unroll
       for (int b = 0; b < 4; b++) {
-        w[b] = load_frag(xk, r0 + 16 * b, r0 + nbk, c) + pull_frag(L, U, W, r0 + 16 * b, r0 + nbk, c) - acc[b];
-        mask_frag(w[b], 16 * b, nbk, c);
+        w[b] = load_frag(xk, r0 + 16 * b, r0 + nbk, c) + pull_frag(L, U, W, r0 + 16 * b, r0 + nbk, c);
       }
-      block_inverse16<T, false>(y, inv, nbk, w, c);
+      tri64<T, false>(y, lu, nbk, w, acc, c);
 #pragma unroll
       for (int b = 0; b < 4; b++) store_frag(xk, r0 + 16 * b, r0 + nbk, y[b], c);
       break;
@@ -620,11 +721,8 @@ __device__ __forceinline__ void unit16(const LeafDev &L, const SolveUnit &U, T *
           acc[b] += load_frag(wf + (U.s * U.nq + q) * 64 * kColGroup, 16 * b, 64, c);
       Frag<T> w[4], y[4];
 #pragma unroll
-      for (int b = 0; b < 4; b++) {
-        w[b] = load_frag(xk, r0 + 16 * b, r0 + nbk, c) - acc[b];
-        mask_frag(w[b], 16 * b, nbk, c);
-      }
-      block_inverse16<T, true>(y, inv + 4096, nbk, w, c);
+      for (int b = 0; b < 4; b++) w[b] = load_frag(xk, r0 + 16 * b, r0 + nbk, c);
+      tri64<T, true>(y, lu, nbk, w, acc, c);
 #pragma unroll
       for (int b = 0; b < 4; b++) store_frag(xk, r0 + 16 * b, r0 + nbk, y[b], c);
       break;

@@ -33,3 +33,44 @@ def test_diagonal_block_quotients_at_the_ends_of_the_range(S, nb, prec, power):
     h = power // 2
     want = np.where(np.tri(nb, k=-1, dtype=bool), out[0], out[0] * t(2.0 ** h) * t(2.0 ** (power - h)))
     assert np.array_equal(out[1], want)
+
+
+def _chain(S, n):
+    """Diagonal 2, below it -3, above it -0.3, in a full pattern of explicit
+    zeros, so that the whole matrix is one front: elimination without pivoting
+    is stable (|L||U| is about |A|), but L's inverse grows as 2.3^n."""
+    D = 2.0 * np.eye(n) - 3.0 * np.eye(n, k=-1) - 0.3 * np.eye(n, k=1)
+    A = S.CSR(n, np.arange(0, n * n + 1, n), np.tile(np.arange(n), n), D.reshape(-1))
+    LU = D.copy()
+    for k in range(n - 1):
+        LU[k + 1, k] /= LU[k, k]
+        LU[k + 1, k + 1] -= LU[k + 1, k] * LU[k, k + 1]
+    growth = np.max((np.abs(np.tril(LU, -1) + np.eye(n)) @ np.abs(np.triu(LU))).sum(1)) / 5.3
+    return D, A, growth
+
+
+@pytest.mark.parametrize("precision,n", [("fp64", n) for n in (16, 33, 48, 64, 65, 96, 97, 130, 200)]
+                         + [("fp32", n) for n in (16, 33, 48, 64, 65, 96, 97)])
+def test_solves_through_badly_conditioned_triangles(S, precision, n):
+    """The backward error of substitution, 3 (order) u |L||U| / |A| at most,
+    whatever the condition of the triangles: one column, one group of columns
+    and more than one.  FP32: of the first iterate, A's and b's rounding added
+    (ir_max_steps < 0: no step, the scratch solve leaves it in x)."""
+    D, A, growth = _chain(S, n)
+    u = 2.0 ** -53 if precision == "fp64" else 2.0 ** -24
+    bar = (3 * n * growth + 2) * u
+    X = np.asfortranarray(np.random.default_rng(n).uniform(-1, 1, (n, 17)))
+    B = np.asfortranarray(D @ X)
+    with S.SnuMat(A, 1, order=np.arange(n), sizes=[n], device=0, precision=precision, ir_max_steps=-1) as M:
+        M.factorize()
+        for k in (1, 2, 17):
+            d_b, d_x = S.DeviceBuffer(8 * n * k), S.DeviceBuffer(8 * n * k)
+            d_b.upload(B[:, :k])
+            rc = S.lib().snumat_solve_device_scratch(M._h, d_b.ptr, d_x.ptr, k, n)
+            assert rc == 0 or precision == "fp32"  # (not converged)
+            x = np.zeros((n, k), order="F")
+            d_x.download(x)
+            d_b.free()
+            d_x.free()
+            for c in range(k):
+                assert S.backward_error(A, x[:, c], B[:, c]) <= bar, (k, c)
