@@ -2023,6 +2023,7 @@ int run_refined(const RefineSet &rs, float *bp, float *wbuf, const GemvPlan<floa
       const double den = (*rs.anorm)[m] * xn[i] + bn[i];
       double e = den > 0 ? rn[i] / den : (rn[i] > 0 ? INFINITY : 0.0);
       if (!(e == e)) e = INFINITY;
+      if (!std::isfinite(bn[i])) e = 0.0;  // no solution to refine: x as the sweep left it
       berr[m] = std::max(berr[m], e);
     }
     int nact = 0;

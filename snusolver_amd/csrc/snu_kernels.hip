@@ -1051,11 +1051,9 @@ __device__ __forceinline__ double block_max(double v, double *red) {
   for (int i = 1; i < (int)(blockDim.x >> 6); i++) v = fmax(v, red[i]);
   return v;
 }
-// Nonnegative doubles order like their bit patterns, so an integer atomic max
-// on the bits is exact.
-__device__ __forceinline__ void atomic_max_bits(unsigned long long *p, double v) {
-  atomicMax(p, (unsigned long long)__double_as_longlong(v));
-}
+// |v| for the norms, infinite for a NaN (fmax would leave it out, and a
+// solution of NaNs pass for an exact one)
+__device__ __forceinline__ double norm_abs(double v) { return v == v ? fabs(v) : HUGE_VAL; }
 // r = b - A x, rounded to T straight into the packed vectors (the next
 // sweep's right-hand sides, so no FP64 residual goes through memory), and the
 // column maxima of |b|, |r| and |x| in the same pass: each workgroup stores its
@@ -1091,9 +1089,9 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
       if (sub == 0) {
         const double b = rhs[row], r = b - s;
         out[order[row]] = (T)r;
-        mb = fmax(mb, fabs(b));
-        mr = fmax(mr, fabs(r));
-        mx = fmax(mx, fabs(x[row]));
+        mb = fmax(mb, norm_abs(b));
+        mr = fmax(mr, norm_abs(r));
+        mx = fmax(mx, norm_abs(x[row]));
       }
     }
     double *rd = &red[0][0][0];
@@ -1142,9 +1140,9 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
       for (int c = 0; c < NC; c++) {
         const double r = b[c] - s[c];
         o[c] = c0 + c < M.nrhs ? (T)r : T(0);
-        m[0][c] = fmax(m[0][c], fabs(b[c]));
-        m[1][c] = fmax(m[1][c], fabs(r));
-        m[2][c] = fmax(m[2][c], fabs(xr[c]));
+        m[0][c] = fmax(m[0][c], norm_abs(b[c]));
+        m[1][c] = fmax(m[1][c], norm_abs(r));
+        m[2][c] = fmax(m[2][c], norm_abs(xr[c]));
       }
     }
     __syncthreads();

@@ -31,7 +31,7 @@ def test_diagonal_block_quotients_at_the_ends_of_the_range(S, nb, prec, power):
         assert f(nb, ptr[0], nb, ptr[1], ptr[2]) == 0
         out.append(D)
     h = power // 2
-    want = np.where(np.tri(nb, k=-1, dtype=bool), out[0], out[0] * t(2.0 ** h) * t(2.0 ** (power - h)))
+    want = np.tril(out[0], -1) + np.triu(out[0]) * t(2.0 ** h) * t(2.0 ** (power - h))
     assert np.array_equal(out[1], want)
 
 
@@ -74,3 +74,51 @@ def test_solves_through_badly_conditioned_triangles(S, precision, n):
             d_x.free()
             for c in range(k):
                 assert S.backward_error(A, x[:, c], B[:, c]) <= bar, (k, c)
+
+
+def test_refinement_of_solutions_that_are_not_finite(S):
+    """FP32 factors that overflow give solutions of NaNs: on the device-pointer
+    paths too they are answered by FP64 factors, or reported.  A right-hand side
+    that is itself not finite is left as it is and does not ask for them."""
+    rng = np.random.default_rng(1)
+    A = S.gen_grid(20, 19, 1, 5, 0, 4.1, 1)
+    A.data = A.data * 1e39  # diagonal beyond FP32
+    n = A.n
+    for k in (1, 3):
+        B = np.asfortranarray(rng.uniform(-1, 1, (n, k)) * 1e39)
+        with S.SnuMat(A, 4, grid=(20, 19, 1), device=0, precision="fp32", ir_tol=1e-12) as M:
+            M.factorize()
+            d_b, d_x = S.DeviceBuffer(8 * n * k), S.DeviceBuffer(8 * n * k)
+            d_b.upload(B)
+            x = np.zeros((n, k), order="F")
+
+            def check():
+                d_x.download(x)
+                assert S.backward_error(A, x, B) <= 1e-12
+
+            assert S.lib().snumat_solve_device_scratch(M._h, d_b.ptr, d_x.ptr, k, n) == -10
+            M.solve_device_ptr(d_b.ptr.value, d_x.ptr.value, k)
+            assert M.timings()["fp64_fallback"] == 1
+            check()
+            with S.Batch([M]) as batch:
+                assert S.backward_error(A, np.asarray(batch.solve([B])[0]).reshape(n, k), B) <= 1e-12
+                assert batch.timings()["fp64_fallbacks"] == 1
+            d_b.free()
+            d_x.free()
+    A = S.gen_grid(20, 19, 1, 5, 0, 4.1, 1)
+    B = np.asfortranarray(rng.uniform(-1, 1, (n, 3)))
+    for bad in (np.nan, np.inf):
+        B[5, 1] = bad
+        with S.SnuMat(A, 4, grid=(20, 19, 1), device=0, precision="fp32", ir_tol=1e-12) as M:
+            M.factorize()
+            d_b, d_x = S.DeviceBuffer(8 * n * 3), S.DeviceBuffer(8 * n * 3)
+            d_b.upload(B)
+            M.solve_device_ptr(d_b.ptr.value, d_x.ptr.value, 3)
+            assert M.timings()["fp64_fallback"] == 0
+            x = np.zeros((n, 3), order="F")
+            d_x.download(x)
+            assert not np.all(np.isfinite(x[:, 1]))
+            for c in (0, 2):
+                assert S.backward_error(A, x[:, c], B[:, c]) <= 1e-12
+            d_b.free()
+            d_x.free()
