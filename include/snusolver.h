@@ -407,6 +407,9 @@ int snu_bench_copy(size_t bytes, int reps, double *ms_out);
 /* in-place no-pivot LU of an nb x nb block (nb <= 64); Linv/Uinv: 64 x 64. */
 int snu_test_diag_lu(int nb, double *D, int ld, double *Linv, double *Uinv);
 int snu_test_diag_lu_f32(int nb, float *D, int ld, float *Linv, float *Uinv);
+/* device allocations of more than `bytes` by this handle, and by batches whose
+ * first member it is, fail from now on (as out of memory). */
+int snu_test_alloc_limit(snumat_t *h, size_t bytes);
 /* the dense launches of a handle's factorization (also of a host-only
  * handle), as run on two streams: key = height (from the leaves' parents, 1)
  * x 1e8 + step (below 6e7: diagonal blocks and their inverses, 6e7: panels,

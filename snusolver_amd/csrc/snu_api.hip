@@ -61,6 +61,7 @@ void drop_alloc(snumat *h, void *p) {
 // them, so it is rebuilt after a reallocation).
 int ensure_rhs(snumat *h, int nrhs) {
   if (nrhs <= h->nrhs_cap) return SNU_OK;
+  h->nrhs_cap = 0;
   int rc;
   const size_t n = (size_t)h->P.n;
   const size_t cols = (size_t)vec_groups(nrhs) * vec_width(nrhs);  // columns of the packed vectors
@@ -91,6 +92,7 @@ template <typename T>
 int ensure_plan(snumat *h, int nrhs) {
   Values<T> &VV = vals<T>(h);
   if (VV.plan_nrhs == nrhs) return SNU_OK;
+  VV.plan_nrhs = -1;
   build_solve_plan<T>(h, VV.bp, VV.ys, nrhs, VV.sp);  // device arrays grow only
   int rc = upload_gemv_plan(VV.sp, h->stream);
   if (rc) return rc;
@@ -1117,6 +1119,12 @@ extern "C" int snu_test_dense_launches(snumat_t *h, int cap, int64_t *key, int *
   if (!h || cap < 0 || (cap > 0 && (!key || !kind || !side))) return set_error(SNU_ERR_BAD_INPUT, "null");
   return h->prec == SNU_FP32 ? dense_launches<float>(h, cap, key, kind, side)
                              : dense_launches<double>(h, cap, key, kind, side);
+}
+
+extern "C" int snu_test_alloc_limit(snumat_t *h, size_t bytes) {
+  if (!h) return set_error(SNU_ERR_BAD_INPUT, "null");
+  h->alloc_limit = bytes;
+  return SNU_OK;
 }
 
 // ---------------- device memory plumbing (bench, tests) ----------------

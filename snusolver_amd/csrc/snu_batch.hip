@@ -65,9 +65,10 @@ namespace {
 
 int balloc(snubatch *b, void **p, size_t bytes) {
   *p = nullptr;
-  hipError_t e = hipMalloc(p, std::max<size_t>(1, bytes));
+  const hipError_t e = bytes > b->mats[0]->alloc_limit ? hipErrorOutOfMemory : hipMalloc(p, std::max<size_t>(1, bytes));
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // (reported here; the next launch's check must not see it)
     return set_error(SNU_ERR_OOM, std::string("batch allocation failed: ") + hipGetErrorString(e));
   }
   b->allocs.push_back(*p);
@@ -168,6 +169,7 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   if (slots > b->slot_cap) {
     bfree(b, b->norms);
     b->norms = nullptr;
+    b->slot_cap = 0;
     if ((rc = balloc(b, (void **)&b->norms, sizeof(double) * norm_values(nm, b->max_n, slots)))) return rc;
     b->slot_cap = slots;
   }

@@ -196,6 +196,7 @@ struct snumat {
   snu::Values<float> v32;
   // standalone solves
   double *d_bx = nullptr;  // staging for host-pointer solves
+  size_t alloc_limit = ~size_t(0);  // larger device allocations fail (tests)
   unsigned long long *d_norms = nullptr;     // |A|inf (bits of a double)
   double *d_colnorms = nullptr;              // refinement column norms (norm_values)
   int *d_active = nullptr;

@@ -31,9 +31,10 @@ namespace snu {
 int device_alloc(snumat *h, void **p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 1;
-  hipError_t e = hipMalloc(p, bytes);
+  const hipError_t e = bytes > h->alloc_limit ? hipErrorOutOfMemory : hipMalloc(p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // (reported here; the next launch's check must not see it)
     return set_error(SNU_ERR_OOM, "hipMalloc of " + std::to_string(bytes) + " bytes failed (" +
                                       hipGetErrorString(e) + ")");
   }
@@ -799,8 +800,13 @@ int upload_gemv_plan(GemvPlan<T> &g, hipStream_t st) {
     if (need <= cap && *p) return SNU_OK;
     if (*p) HIPCHK(hipFree(*p));
     *p = nullptr;
+    cap = 0;
     const size_t c = std::max<size_t>(need + need / 2, 64);
-    HIPCHK(hipMalloc((void **)p, c * sizeof(**p)));
+    if (hipMalloc((void **)p, c * sizeof(**p)) != hipSuccess) {
+      *p = nullptr;
+      (void)hipGetLastError();
+      return set_error(SNU_ERR_OOM, "hipMalloc of " + std::to_string(c * sizeof(**p)) + " bytes for a solve failed");
+    }
     cap = c;
     return SNU_OK;
   };

@@ -1,0 +1,70 @@
+"""Solves whose working memory cannot be allocated (a limit set from the host:
+larger allocations fail as if the device were full)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+NO_LIMIT = 2 ** 64 - 1
+
+
+def _limit(S, M, nbytes):
+    S._check(S.lib().snu_test_alloc_limit(M._h, C.c_size_t(nbytes)))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_failed_allocation_leaves_no_buffer_behind(S, precision):
+    """A solve that cannot grow its buffers fails, and so does the next one,
+    with fewer columns than there were buffers for before; with memory again
+    the answers are the same.  Handle and batch."""
+    A = S.gen_grid(40, 31, 1, 9, 0, 8.1, 1)
+    B = np.asfortranarray(np.random.default_rng(2).standard_normal((A.n, 40)))
+    with S.SnuMat(A, 4, grid=(40, 31, 1), device=0, precision=precision, ir_tol=1e-12) as M:
+        M.factorize()
+        with S.Batch([M]) as batch:
+            solves = [lambda k: M.solve(B[:, :k]), lambda k: np.asarray(batch.solve([B[:, :k]])[0])]
+            for solve in solves:
+                first = {k: solve(k) for k in (1, 3)}
+                _limit(S, M, 0)
+                for k in (40, 3, 1):
+                    with pytest.raises(S.SnuError) as e:
+                        solve(k)
+                    assert e.value.code == -7
+                _limit(S, M, NO_LIMIT)
+                for k in (3, 1, 40):
+                    x = solve(k)
+                    assert k not in first or np.array_equal(x, first[k])
+                    assert S.backward_error(A, x, B[:, :k]) <= 1e-12
+
+
+def test_failed_norms_leave_no_buffer_behind(S):
+    """The same where the vectors fit and the norms of the refinement do not
+    (4 rows: 816 bytes of norms for 17 columns, 512 of vectors)."""
+    D = np.array([[4.0, 1, 0, 0], [1, 4, 1, 0], [0, 1, 4, 1], [0, 0, 1, 4]])
+    r, c = np.nonzero(D)
+    A = S.CSR(4, np.searchsorted(r, np.arange(5)), c, D[r, c])
+    B = np.asfortranarray(np.random.default_rng(3).standard_normal((4, 17)))
+    with S.SnuMat(A, 1, order=np.arange(4), sizes=[4], device=0, precision="fp32", ir_tol=1e-12) as M:
+        M.factorize()
+        d_b, d_x = S.DeviceBuffer(B.nbytes), S.DeviceBuffer(B.nbytes)
+        d_b.upload(B)
+        with S.Batch([M]) as batch:
+            one = lambda v: (C.c_void_p * 1)(v)
+            calls = [lambda k: S.lib().snumat_solve_device(M._h, d_b.ptr, d_x.ptr, k, 4),
+                     lambda k: S.lib().snubatch_solve_device(batch._h, one(d_b.ptr.value), one(d_x.ptr.value),
+                                                             (C.c_int * 1)(k), (C.c_int * 1)(4))]
+            for call in calls:
+                assert call(3) == 0
+                _limit(S, M, 600)
+                assert call(17) in (0, -7)
+                assert call(3) == 0
+                x = np.zeros((4, 17), order="F")
+                d_x.download(x)
+                assert np.max(np.abs(x[:, :3] - np.linalg.solve(D, B[:, :3]))) <= 1e-12
+                _limit(S, M, NO_LIMIT)
+                assert call(17) == 0
+                d_x.download(x)
+                assert np.max(np.abs(x - np.linalg.solve(D, B))) <= 1e-12
+        d_b.free()
+        d_x.free()
