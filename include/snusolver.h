@@ -138,7 +138,10 @@ int snumat_update_values(snumat_t *h, const double *values);
  * with the residual in FP64 until every column's backward error
  * |b - Ax|inf / (|A|inf |x|inf + |b|inf) <= ir_tol, or until a step stops
  * halving it; returns SNU_ERR_NOT_CONVERGED if it is then still above 1e-12
- * (x holds the last iterate). */
+ * (x holds the last iterate).
+ * Working memory, kept by the handle: one column takes its own, several take
+ * it in groups of 16 (2 columns as much as 16).  Where device memory for the
+ * groups is missing, the columns run one after the other in that of one. */
 int snumat_solve(snumat_t *h, const double *b, double *x, int nrhs, int ld);
 
 /* Same with device pointers (resident in HBM, no PCIe in the path). */
@@ -149,15 +152,17 @@ int snumat_solve_device(snumat_t *h, const double *d_b, double *d_x, int nrhs,
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Every working buffer of the solve (permuted right-hand sides,
- * dense-solve vectors and descriptors, split-K partial sums, and for
- * SNU_FP32 handles the FP64 residual, correction and column norms) comes
- * from one 256 MiB scratch array per device that the library holds until
- * the process ends; the call makes no hipMalloc / hipFree.  Needs a handle
- * constructed on a device and factorized.  A call whose buffers exceed the
- * scratch (about 16 n nrhs bytes for FP64 handles, 24 n nrhs for SNU_FP32)
- * returns SNU_ERR_BAD_INPUT with the size in the message.  All calls on one
- * device share the scratch: calls that overlap on one device (other host
- * threads, other handles) race and must be serialised by the caller.
+ * dense-solve vectors and descriptors, split-K partial sums, the leaf fronts'
+ * update rows, and for SNU_FP32 handles the column norms) comes from one 256
+ * MiB scratch array per device that the library holds until the process ends;
+ * the call makes no hipMalloc / hipFree.  Needs a handle constructed on a
+ * device and factorized.  A call of more than 256 MiB, counted as about 16 n
+ * nrhs bytes for FP64 handles and 24 n nrhs for SNU_FP32, returns
+ * SNU_ERR_BAD_INPUT with the size in the message.  Below that, columns whose
+ * groups of 16 (as in snumat_solve) do not fit run one after the other, in
+ * proportionally more time.  All calls on one device share the scratch:
+ * calls that overlap on one device (other host threads, other handles) race
+ * and must be serialised by the caller.
  * SNU_FP32 handles refine as snumat_solve_device does but have no FP64
  * fallback here (building it would allocate): a stalled refinement returns
  * SNU_ERR_NOT_CONVERGED with x holding the last iterate. */

@@ -62,7 +62,6 @@ void drop_alloc(snumat *h, void *p) {
 int ensure_rhs(snumat *h, int nrhs) {
   if (nrhs <= h->nrhs_cap) return SNU_OK;
   h->nrhs_cap = 0;
-  int rc;
   const size_t n = (size_t)h->P.n;
   const size_t cols = (size_t)vec_groups(nrhs) * vec_width(nrhs);  // columns of the packed vectors
   auto vec = [&](auto &VV) -> int {
@@ -77,15 +76,23 @@ int ensure_rhs(snumat *h, int nrhs) {
       return r;
     return SNU_OK;
   };
-  drop_alloc(h, h->d_bx);
+  int rc;
   drop_alloc(h, h->d_colnorms);
-  h->d_bx = nullptr;
   h->d_colnorms = nullptr;
   if ((rc = h->prec == SNU_FP32 ? vec(h->v32) : vec(h->v64))) return rc;
-  if ((rc = halloc(h, &h->d_bx, n * nrhs * 2))) return rc;
   if (h->prec == SNU_FP32 && (rc = halloc(h, &h->d_colnorms, norm_values(1, h->P.n, nrhs)))) return rc;
   h->nrhs_cap = nrhs;
   return SNU_OK;
+}
+// Device staging of a host-pointer solve: b, then x.
+int ensure_stage(snumat *h, int nrhs) {
+  if (nrhs <= h->stage_cap) return SNU_OK;
+  h->stage_cap = 0;
+  drop_alloc(h, h->d_bx);
+  h->d_bx = nullptr;
+  const int rc = halloc(h, &h->d_bx, (size_t)h->P.n * nrhs * 2);
+  if (!rc) h->stage_cap = nrhs;
+  return rc;
 }
 
 template <typename T>
@@ -478,24 +485,53 @@ int solve_core(snumat *h, const double *d_b, long long ldb, double *d_x, long lo
 }  // namespace snu
 
 namespace {
+// nrhs columns, `step` at a time on the buffers B (laid out for that many), the
+// timings and refinement figures over all of them.
+int solve_columns(snumat *h, const double *d_b, long long ldb, double *d_x, long long ldx, int nrhs, int step,
+                  const SolveBuffers &B, bool fallback) {
+  int worst = SNU_OK, steps = 0;
+  double berr = 0, ms = 0, twin = 0;
+  for (int c = 0; c < nrhs; c += step) {
+    const int rc = solve_core(h, d_b + (size_t)c * ldb, ldb, d_x + (size_t)c * ldx, ldx, step, B, fallback);
+    if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
+    if (rc) worst = rc;
+    steps = std::max(steps, h->ir_steps);
+    berr = std::max(berr, h->ir_berr);
+    twin = std::max(twin, h->t[15]);
+    ms += h->t[6];
+  }
+  h->ir_steps = steps;
+  h->ir_berr = berr;
+  h->t[6] = ms;
+  h->t[13] = steps;
+  h->t[14] = berr;
+  h->t[15] = twin;
+  return worst;
+}
+int ensure_solve(snumat *h, int nrhs) {
+  const int rc = ensure_rhs(h, nrhs);
+  if (rc) return rc;
+  return h->prec == SNU_FP32 ? ensure_plan<float>(h, nrhs) : ensure_plan<double>(h, nrhs);
+}
 int solve_dev(snumat *h, const double *d_b, long long ldb, double *d_x, long long ldx, int nrhs) {
   int rc = ensure_stream(h);
   if (rc) return rc;
-  if ((rc = ensure_rhs(h, nrhs))) return rc;
+  // several columns are padded to groups of 16 (vec_groups): where the memory
+  // for that is not there, one column after the other
+  int step = nrhs;
+  rc = ensure_solve(h, nrhs);
+  if (rc == SNU_ERR_OOM && nrhs > 1) rc = ensure_solve(h, step = 1);
+  if (rc) return rc;
   SolveBuffers B;
-  if (h->prec == SNU_FP32) {
-    if ((rc = ensure_plan<float>(h, nrhs))) return rc;
-    B.bp = h->v32.bp;
-    B.wbuf = h->v32.wbuf;
-    B.plan = &h->v32.sp;
-  } else {
-    if ((rc = ensure_plan<double>(h, nrhs))) return rc;
-    B.bp = h->v64.bp;
-    B.wbuf = h->v64.wbuf;
-    B.plan = &h->v64.sp;
-  }
+  auto use = [&](auto &VV) {
+    B.bp = VV.bp;
+    B.wbuf = VV.wbuf;
+    B.plan = &VV.sp;
+  };
+  if (h->prec == SNU_FP32) use(h->v32);
+  else use(h->v64);
   B.colnorms = h->d_colnorms;
-  return solve_core(h, d_b, ldb, d_x, ldx, nrhs, B, true);
+  return solve_columns(h, d_b, ldb, d_x, ldx, nrhs, step, B, true);
 }
 }  // namespace
 
@@ -527,12 +563,13 @@ namespace {
 // The solve of snumat_solve_device over buffers carved from the device's
 // scratch: permuted right-hand sides, dense-solve vectors, the leaf fronts'
 // update rows, (SNU_FP32) column norms, then the dense-solve descriptors and
-// split-K partial sums.  Every buffer is written
-// before it is read within the call (the column norms are zeroed by their
-// own kernel), so no clearing is needed; the descriptors are copied in on
+// split-K partial sums.  Every buffer is written before it is read within the
+// call, so no clearing is needed; the descriptors are copied in on
 // every call, as another handle's call may have overwritten them.  A call
 // whose padded column groups do not fit runs its columns one at a time, with
-// the handle's own one-column update rows when those do not fit either.
+// the handle's own one-column update rows when those do not fit either (1024^2
+// 5-point FP64: 1.8 ms for 2 columns in turn, 12.5 for 15; 1.4 for either as a
+// group).
 template <typename T>
 int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
   unsigned char *base = nullptr;
@@ -587,7 +624,8 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
     return off <= kScratchBytes && g.cap_done <= kScratchDone;
   };
   int step = nrhs;
-  if (!layout(nrhs, true)) {
+  if (nrhs >= VV.scratch_over || !layout(nrhs, true)) {
+    if (nrhs > 1) VV.scratch_over = std::min(VV.scratch_over, nrhs);
     step = 1;
     if (!layout(1, true) && !layout(1, false)) {
       VV.scratch_nrhs = -1;
@@ -597,21 +635,11 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
   }
   // no FP64 twin here: building one allocates (a stalled refinement
   // returns SNU_ERR_NOT_CONVERGED with x = the last iterate)
-  int worst = SNU_OK;
-  for (int c = 0; c < nrhs; c += step) {
-    if (c == 0) {
-      if (!g.vp.empty())
-        HIPCHK(hipMemcpyAsync(g.d_vp, g.vp.data(), g.vp.size() * sizeof(g.vp[0]), hipMemcpyHostToDevice,
-                              h->stream));
-      if (!g.vs.empty())
-        HIPCHK(hipMemcpyAsync(g.d_vs, g.vs.data(), g.vs.size() * sizeof(g.vs[0]), hipMemcpyHostToDevice,
-                              h->stream));
-    }
-    rc = solve_core(h, d_b + (size_t)c * ld, ld, d_x + (size_t)c * ld, ld, step, B, false);
-    if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
-    if (rc) worst = rc;
-  }
-  return worst;
+  if (!g.vp.empty())
+    HIPCHK(hipMemcpyAsync(g.d_vp, g.vp.data(), g.vp.size() * sizeof(g.vp[0]), hipMemcpyHostToDevice, h->stream));
+  if (!g.vs.empty())
+    HIPCHK(hipMemcpyAsync(g.d_vs, g.vs.data(), g.vs.size() * sizeof(g.vs[0]), hipMemcpyHostToDevice, h->stream));
+  return solve_columns(h, d_b, ld, d_x, ld, nrhs, step, B, false);
 }
 }  // namespace
 
@@ -638,7 +666,7 @@ extern "C" int snumat_solve(snumat_t *h, const double *b, double *x, int nrhs,
   HIPCHK(hipSetDevice(h->device));
   int rc = ensure_stream(h);
   if (rc) return rc;
-  if ((rc = ensure_rhs(h, nrhs))) return rc;
+  if ((rc = ensure_stage(h, nrhs))) return rc;
   double *db = h->d_bx, *dx = h->d_bx + (size_t)n * nrhs;
   HIPCHK(hipMemcpy2DAsync(db, sizeof(double) * n, b, sizeof(double) * ld, sizeof(double) * n, nrhs,
                           hipMemcpyHostToDevice, h->stream));

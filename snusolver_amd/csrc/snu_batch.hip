@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,7 @@ struct snubatch {
   std::vector<double> anorm;
   int ir_steps = 0;
   std::vector<double> berr;
+  std::vector<char> twin;  // members answered by FP64 factors
   double *stage = nullptr;  // host-pointer solves: packed b then x
   size_t stage_cap = 0;
   bool factor_plan = false;  // merged dense plan built (on first factorize)
@@ -234,13 +236,12 @@ int batch_factorize(snubatch *b) {
   return SNU_OK;
 }
 
+// One pass over all members, on the buffers of ensure_pattern.
 template <typename T>
-int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const int *nrhs,
-                const int *ld) {
+int solve_pattern(snubatch *b, const double *const *d_b, double *const *d_x, const int *nrhs,
+                  const int *ld) {
   const int nm = (int)b->mats.size();
-  std::vector<int> pat(nrhs, nrhs + nm);
-  int rc = ensure_pattern<T>(b, pat);
-  if (rc) return rc;
+  int rc = SNU_OK;
   hipStream_t st = b->stream;
   std::vector<PermDev> pd(nm);
   long long max_elems = 0;
@@ -305,7 +306,6 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
     rs.tol = o.ir_tol > 0 ? o.ir_tol : 1e-15;
     rc = run_refined(rs, (float *)b->bp, (float *)b->wbuf, b->s32, st, &b->ir_steps, &b->berr);
     if (rc && rc != SNU_ERR_NOT_CONVERGED) return rc;
-    b->t[15] = 0;
     if (rc == SNU_ERR_NOT_CONVERGED) {
       // members whose refinement stalled above 1e-12 are answered by FP64
       // factors of the same matrix (each member's FP64 twin); the batch's
@@ -313,7 +313,7 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
       for (int m = 0; m < nm; m++) {
         if (!nrhs[m] || b->berr[m] <= 1e-12) continue;
         if ((rc = fp64_fallback_solve(b->mats[m], d_b[m], ld[m], d_x[m], ld[m], nrhs[m]))) return rc;
-        b->t[15] += 1;
+        b->twin[m] = 1;
       }
       HIPCHK(hipSetDevice(b->device));
       rc = SNU_OK;
@@ -327,11 +327,47 @@ int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const
   HIPCHK(hipEventRecord(b->ev[7], st));
   HIPCHK(hipEventSynchronize(b->ev[7]));
   b->t[6] = ev_ms(b->ev[6], b->ev[7]);
-  b->t[13] = b->ir_steps;
-  double worst = 0;
-  for (double e : b->berr) worst = std::max(worst, e);
-  b->t[14] = worst;
   return rc;
+}
+// Several columns of a member are padded to groups of 16 (vec_groups): where the
+// memory for that is not there, one column of each member after the other.
+template <typename T>
+int batch_solve(snubatch *b, const double *const *d_b, double *const *d_x, const int *nrhs,
+                const int *ld) {
+  const int nm = (int)b->mats.size(), most = *std::max_element(nrhs, nrhs + nm);
+  b->twin.assign(nm, 0);
+  int rc = ensure_pattern<T>(b, std::vector<int>(nrhs, nrhs + nm)), steps = 0;
+  double ms = 0;
+  std::vector<double> berr(nm, 0.0);
+  auto pass = [&](const double *const *pb, double *const *px, const int *k) -> int {
+    const int r = solve_pattern<T>(b, pb, px, k, ld);
+    steps = std::max(steps, b->ir_steps);
+    for (int m = 0; m < nm && m < (int)b->berr.size(); m++) berr[m] = std::max(berr[m], b->berr[m]);
+    ms += b->t[6];
+    return r;
+  };
+  if (!rc) {
+    rc = pass(d_b, d_x, nrhs);
+  } else if (rc == SNU_ERR_OOM && most > 1) {
+    std::vector<const double *> pb(d_b, d_b + nm);
+    std::vector<double *> px(d_x, d_x + nm);
+    std::vector<int> k(nm);
+    for (int c = 0; c < most; c++) {
+      for (int m = 0; m < nm; m++) {
+        k[m] = nrhs[m] > c;
+        if (k[m] && c) pb[m] += ld[m], px[m] += ld[m];
+      }
+      if ((rc = ensure_pattern<T>(b, k)) || (rc = pass(pb.data(), px.data(), k.data()))) return rc;
+    }
+  }
+  if (rc) return rc;
+  b->ir_steps = steps;
+  b->berr = berr;
+  b->t[6] = ms;
+  b->t[13] = steps;
+  b->t[14] = *std::max_element(berr.begin(), berr.end());
+  b->t[15] = std::accumulate(b->twin.begin(), b->twin.end(), 0);
+  return SNU_OK;
 }
 
 }  // namespace

@@ -5,6 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -119,6 +120,7 @@ struct Values {
   GemvPlan<T> sp_scratch;
   int scratch_nrhs = -1;
   bool scratch_own_w = true;
+  int scratch_over = INT_MAX;  // columns known not to fit the scratch as groups
 };
 
 // Tables of a standalone solve, one copy to the device.
@@ -195,7 +197,8 @@ struct snumat {
   snu::Values<double> v64;
   snu::Values<float> v32;
   // standalone solves
-  double *d_bx = nullptr;  // staging for host-pointer solves
+  double *d_bx = nullptr;  // staging for host-pointer solves,
+  int stage_cap = 0;       // columns it holds
   size_t alloc_limit = ~size_t(0);  // larger device allocations fail (tests)
   unsigned long long *d_norms = nullptr;     // |A|inf (bits of a double)
   double *d_colnorms = nullptr;              // refinement column norms (norm_values)

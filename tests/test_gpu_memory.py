@@ -68,3 +68,57 @@ def test_failed_norms_leave_no_buffer_behind(S):
                 assert np.max(np.abs(x - np.linalg.solve(D, B))) <= 1e-12
         d_b.free()
         d_x.free()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_columns_in_turn_where_groups_do_not_fit(S, precision):
+    """Several columns take padded groups of 16; where the memory for those is
+    missing but one column's is there, the columns run in turn: the bits of
+    single solves, and refinement figures over all columns."""
+    A = S.gen_grid(40, 31, 1, 9, 0, 8.1, 1)
+    v = 8 if precision == "fp64" else 4
+    B = np.asfortranarray(np.random.default_rng(4).standard_normal((A.n, 18)))
+    B[:, 4:] = 0.0  # (no step of refinement after the fourth column)
+    d_b, d_x = S.DeviceBuffer(B.nbytes), S.DeviceBuffer(B.nbytes)
+    d_b.upload(B)
+    x = np.zeros((A.n, 18), order="F")
+    mats = [S.SnuMat(A, 4, grid=(40, 31, 1), device=0, precision=precision, ir_tol=1e-13) for _ in range(3)]
+    for M in mats:
+        M.factorize()
+    single = np.stack([mats[1].solve(B[:, c]) for c in range(18)], 1)
+    steps = []
+    for c in range(4):
+        mats[1].solve(B[:, c])
+        steps.append(mats[1].timings()["ir_steps"])
+    assert precision == "fp64" or max(steps) >= 1
+    for k in (2, 15, 18):
+        M = S.SnuMat(A, 4, grid=(40, 31, 1), device=0, precision=precision, ir_tol=1e-13)
+        M.factorize()
+        _limit(S, M, 12 * v * A.n)  # (the fronts' update rows of one column: up to 8 A.n)
+        M.solve_device_ptr(d_b.ptr.value, d_x.ptr.value, k)
+        d_x.download(x)
+        assert np.array_equal(x[:, :k], single[:, :k])
+        assert M.timings()["ir_steps"] == max(steps[:k])
+        _limit(S, M, NO_LIMIT)
+        M.solve_device_ptr(d_b.ptr.value, d_x.ptr.value, k)  # as groups again
+        d_x.download(x)
+        assert S.backward_error(A, x[:, :4], B[:, :4]) <= 1e-12 or k < 4
+        M.close()
+    ncol = (18, 1, 5)
+    with S.Batch(mats) as batch:
+        P = lambda q: (C.c_void_p * 3)(q, q, q)
+        outs = [S.DeviceBuffer(B.nbytes) for _ in range(3)]
+        _limit(S, mats[0], 3 * 12 * v * A.n)
+        rc = S.lib().snubatch_solve_device(batch._h, P(d_b.ptr.value), (C.c_void_p * 3)(*[o.ptr.value for o in outs]),
+                                           (C.c_int * 3)(*ncol), (C.c_int * 3)(A.n, A.n, A.n))
+        assert rc == 0
+        for o, k in zip(outs, ncol):
+            o.download(x)
+            assert np.array_equal(x[:, :k], single[:, :k])
+            o.free()
+        assert batch.timings()["ir_steps"] == max(steps)
+        _limit(S, mats[0], NO_LIMIT)
+    for M in mats:
+        M.close()
+    d_b.free()
+    d_x.free()
