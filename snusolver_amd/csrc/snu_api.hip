@@ -71,7 +71,7 @@ int ensure_rhs(snumat *h, int nrhs) {
     VV.bp = VV.wbuf = VV.ys = nullptr;
     VV.plan_nrhs = -1;
     int r;
-    if ((r = halloc(h, &VV.bp, n * cols)) || (r = halloc(h, &VV.ys, n * cols)) ||
+    if ((r = halloc(h, &VV.bp, n * cols)) || (r = halloc(h, &VV.ys, (size_t)h->sep_rows[h->P.np] * cols)) ||
         (r = halloc(h, &VV.wbuf, (size_t)h->wrows * cols)))
       return r;
     return SNU_OK;
@@ -599,7 +599,7 @@ int solve_scratch(snumat *h, const double *d_b, double *d_x, int nrhs, int ld) {
       return base + o;
     };
     const size_t cols = (size_t)vec_groups(k) * vec_width(k);
-    T *bp = (T *)carve(sizeof(T) * n * cols), *ys = (T *)carve(sizeof(T) * n * cols);
+    T *bp = (T *)carve(sizeof(T) * n * cols), *ys = (T *)carve(sizeof(T) * h->sep_rows[h->P.np] * cols);
     B.bp = bp;
     B.wbuf = own_w ? (void *)carve(sizeof(T) * (size_t)h->wrows * cols) : (void *)VV.w1;
     if (h->prec == SNU_FP32) B.colnorms = (double *)carve(sizeof(double) * norm_values(1, (int)n, k));

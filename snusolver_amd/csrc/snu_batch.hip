@@ -38,7 +38,7 @@ struct snubatch {
   FrontPlan<float> fr32;
   // solves (sized for the last right-hand-side pattern)
   std::vector<int> pattern;  // nrhs per matrix of the current solve plan
-  long long vec_cap = 0, w_cap = 0;
+  long long vec_cap = 0, y_cap = 0, w_cap = 0;
   int slot_cap = 0;
   void *bp = nullptr, *ys = nullptr, *wbuf = nullptr;
   double *norms = nullptr;
@@ -141,12 +141,13 @@ template <typename T>
 int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   if (b->pattern == nrhs) return SNU_OK;
   const int nm = (int)b->mats.size();
-  // packed vectors (padded column groups), update rows
-  long long tot = 0, wtot = 0;
+  // packed vectors (padded column groups; ys: separator rows), update rows
+  long long tot = 0, ytot = 0, wtot = 0;
   int slots = 0;
   for (int m = 0; m < nm; m++) {
     const long long cols = (long long)vec_groups(nrhs[m]) * vec_width(nrhs[m]);
     tot += (long long)b->mats[m]->P.n * cols;
+    ytot += (long long)b->mats[m]->sep_rows[b->mats[m]->P.np] * cols;
     wtot += (long long)b->mats[m]->wrows * cols;
     slots += nrhs[m];
   }
@@ -154,12 +155,17 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   b->pattern.clear();
   if (tot > b->vec_cap) {
     bfree(b, b->bp);
-    bfree(b, b->ys);
-    b->bp = b->ys = nullptr;
+    b->bp = nullptr;
     b->vec_cap = 0;
-    if ((rc = balloc(b, &b->bp, sizeof(T) * tot)) || (rc = balloc(b, &b->ys, sizeof(T) * tot)))
-      return rc;
+    if ((rc = balloc(b, &b->bp, sizeof(T) * tot))) return rc;
     b->vec_cap = tot;
+  }
+  if (ytot > b->y_cap) {
+    bfree(b, b->ys);
+    b->ys = nullptr;
+    b->y_cap = 0;
+    if ((rc = balloc(b, &b->ys, sizeof(T) * ytot))) return rc;
+    b->y_cap = ytot;
   }
   if (wtot > b->w_cap) {
     bfree(b, b->wbuf);
@@ -191,7 +197,8 @@ int ensure_pattern(snubatch *b, const std::vector<int> &nrhs) {
   T *bp = (T *)b->bp, *ys = (T *)b->ys;
   for (int m = 0; m < nm; m++) {
     if (!nrhs[m]) continue;
-    build_solve_plan<T>(b->mats[m], bp + b->h_vec[m].base, ys + b->h_vec[m].base, nrhs[m], parts[m]);
+    build_solve_plan<T>(b->mats[m], bp + b->h_vec[m].base, ys, nrhs[m], parts[m]);
+    ys += (long long)b->mats[m]->sep_rows[b->mats[m]->P.np] * vec_groups(nrhs[m]) * vec_width(nrhs[m]);
     ptrs.push_back(&parts[m]);
   }
   merge_gemv(ptrs, out);  // keeps out's device arrays, which grow only

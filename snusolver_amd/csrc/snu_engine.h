@@ -109,8 +109,8 @@ struct Values {
   T *farena = nullptr; // leaf fronts (each f x f, a larger one's pivot blocks behind it)
   FrontPlan<T> fronts;
   DensePlan<T> fact;
-  // standalone solves: right-hand sides, dense-solve vectors, the fronts'
-  // update rows; w1: update rows of one column (allocation-free solves)
+  // standalone solves: right-hand sides, dense-solve vectors (separator rows
+  // alone), the fronts' update rows; w1: update rows of one column (allocation-free solves)
   T *bp = nullptr, *ys = nullptr, *wbuf = nullptr, *w1 = nullptr;
   int plan_nrhs = -1;
   GemvPlan<T> sp;
@@ -193,6 +193,7 @@ struct snumat {
   int wrows = 0;       // update rows of the leaf fronts (solves)
   // dense tables
   std::vector<long long> inv_off, lu_off;
+  std::vector<int> sep_rows;  // separator rows before each separator (at np: all)
   long long inv_total = 0, tmp_panels = 0, tmp_inversion = 0;
   snu::Values<double> v64;
   snu::Values<float> v32;

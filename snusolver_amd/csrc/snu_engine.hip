@@ -690,13 +690,13 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
   // one column: groups 0, kinds 7 / 8; several: groups of 16, kinds 17 / 18
   const int w = vec_width(nrhs), groups = nrhs == 1 ? 0 : vec_groups(nrhs);
   const int kset = w == 1 ? 7 : 17, ksub = w == 1 ? 8 : 18;
-  const long long n = (long long)P.n * w;  // values per column (group)
+  const long long n = (long long)P.n * w, ny = (long long)h->sep_rows[P.np] * w;  // values per column (group)
   auto R = [&](int p) { return dense + P.offR[p]; };
   auto Lp = [&](int p) { return dense + P.offL[p]; };
   auto Li = [&](int p) { return VV.inv + h->inv_off[p]; };
   auto Ui = [&](int p) { return VV.inv + h->inv_off[p] + (long long)P.block_size[p] * P.block_size[p]; };
   auto bseg = [&](int p) { return bp + (long long)P.block_start[p] * w; };
-  auto yseg = [&](int p) { return ys + (long long)P.block_start[p] * w; };
+  auto yseg = [&](int p) { return ys + (long long)h->sep_rows[p] * w; };
   S.vp.clear();
   S.vs.clear();
   S.fwd.clear();
@@ -707,7 +707,7 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
     int lo = 1 << l, hi = std::min((2 << l) - 1, P.np - 1);
     for (int i = lo; i <= hi; i++) {
       int s = P.block_size[i];
-      g.add(S.vs, yseg(i), n, s, 1, groups, {GemvSeg{Li(i), bseg(i), s, n, s}});
+      g.add(S.vs, yseg(i), ny, s, 1, groups, {GemvSeg{Li(i), bseg(i), s, n, s}});
     }
     g.flush(kset, S.vp, S.fwd, height * 4LL + 0);
     for (int p = 1; p < lo; p++) {
@@ -720,7 +720,7 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
         for (int i = first; i <= last; i++) {
           const int r = P.lmap[i][P.anc_off(i, p) + m0];  // the tile's stored rows (or -1)
           if (r < 0) continue;
-          segs.push_back(GemvSeg{Lp(i) + r, yseg(i), P.nL[i], n, P.block_size[i]});
+          segs.push_back(GemvSeg{Lp(i) + r, yseg(i), P.nL[i], ny, P.block_size[i]});
         }
         g.add(S.vs, bseg(p) + m0 * w, n, mt, 0, groups, segs);
       }
@@ -742,12 +742,12 @@ void build_solve_plan(const snumat *h, T *bp, T *ys, int nrhs, GemvPlan<T> &S) {
           segs.push_back(GemvSeg{R(i) + (long long)(s + P.umap[i][off + cr.first]) * s, bseg(a) + cr.first * w, s, n,
                                  cr.second - cr.first});
       }
-      g.add(S.vs, yseg(i), n, s, 0, groups, segs);
+      g.add(S.vs, yseg(i), ny, s, 0, groups, segs);
     }
     g.flush(ksub, S.vp, S.bwd, bkey + 0);
     for (int i = lo; i <= hi; i++) {
       int s = P.block_size[i];
-      g.add(S.vs, bseg(i), n, s, 2, groups, {GemvSeg{Ui(i), yseg(i), s, n, s}});
+      g.add(S.vs, bseg(i), n, s, 2, groups, {GemvSeg{Ui(i), yseg(i), s, ny, s}});
     }
     g.flush(kset, S.vp, S.bwd, bkey + 1);
   }
@@ -1409,6 +1409,49 @@ void merge_fronts(const std::vector<const FrontPlan<T> *> &in, FrontPlan<T> &out
   for (const FrontPlan<T> *p : in) dp.push_back(&p->dense);
   merge_dense(dp, out.dense);
 }
+// Places of the fronts' update rows of one leaf (size: rows per front) and the
+// rows taken in all.  Rows live from their front's height to its parent's, where
+// they are read (root fronts: to the end); the backward sweep uses a front's
+// rows within its height.  Rows that are done with are given to fronts of later
+// heights, first fit: 35 to 45% fewer rows than side by side on 2D and 3D grids.
+static long long place_rows(const LeafPlan &L, const std::vector<long long> &size, std::vector<long long> &at) {
+  const int nf = (int)L.ff.size();
+  std::vector<std::vector<int>> begin(nf ? L.fheight_max + 1 : 0), done(begin.size());
+  for (int f = 0; f < nf; f++) {
+    begin[L.fheight[f]].push_back(f);
+    if (L.fpar[f] >= 0) done[L.fheight[L.fpar[f]]].push_back(f);
+  }
+  at.assign(nf, 0);
+  std::map<long long, long long> open;  // free rows below top: first, count (no two adjacent)
+  long long top = 0;
+  for (size_t h = 0; h < begin.size(); h++) {
+    for (int f : begin[h]) {
+      if (!size[f]) continue;
+      auto it = open.begin();
+      while (it != open.end() && it->second < size[f]) ++it;
+      if (it == open.end()) {
+        at[f] = top;
+        top += size[f];
+        continue;
+      }
+      at[f] = it->first;
+      const long long left = it->second - size[f];
+      open.erase(it);
+      if (left) open[at[f] + size[f]] = left;
+    }
+    for (int f : done[h]) {
+      if (!size[f]) continue;
+      auto it = open.emplace(at[f], size[f]).first;
+      auto next = std::next(it);
+      if (next != open.end() && it->first + it->second == next->first) it->second += next->second, open.erase(next);
+      if (it != open.begin()) {
+        auto prev = std::prev(it);
+        if (prev->first + prev->second == it->first) prev->second += it->second, open.erase(it);
+      }
+    }
+  }
+  return top;
+}
 // The leaf solves of one matrix: solve positions (leaf rows in front order, so
 // a front's pivots are consecutive), update rows, the children's
 // update rows each front row adds, the units of every phase (per height,
@@ -1443,6 +1486,16 @@ static int build_leaf_solve(snumat *h) {
     };
     std::vector<SolveUnit> base(nf);
     std::vector<std::vector<int>> byh(nf ? L.fheight_max + 1 : 0);
+    // update rows, which the backward sweep's partial products share
+    std::vector<long long> size(nf), at;
+    auto chunks = [&](int f) {
+      const int w = 64 * ((L.fnk[f] + 63) / 64);
+      return L.ff[f] > fmax ? (L.ff[f] - L.fnk[f] + w - 1) / w : 0;
+    };
+    for (int f = 0; f < nf; f++)
+      size[f] = std::max<long long>(L.ff[f] - L.fnk[f], 64LL * ((L.fnk[f] + 63) / 64) * chunks(f));
+    const long long row0 = wrows;
+    wrows += place_rows(L, size, at);
     for (int f = 0; f < nf; f++) {
       SolveUnit &U = base[f];
       std::memset(&U, 0, sizeof(U));
@@ -1453,10 +1506,8 @@ static int build_leaf_solve(snumat *h) {
       U.inv = VV.farena + ftotal + (long long)U.ld * U.ld;
       ftotal += (long long)U.ld * U.ld + front_inv_size(U.ld, U.nk, fmax);
       U.kpos = g0 + L.fkp[f];
-      U.wrow = (int)wrows;
-      U.nq = U.ld > fmax ? (U.nb + 64 * ((U.nk + 63) / 64) - 1) / (64 * ((U.nk + 63) / 64)) : 0;
-      // the backward sweep's partial products share the update rows
-      wrows += std::max<long long>(U.nb, 64LL * ((U.nk + 63) / 64) * U.nq);
+      U.wrow = (int)(row0 + at[f]);
+      U.nq = chunks(f);
       U.bidx = (int)bidx.size();
       for (int q = L.fidx_ptr[f]; q < L.fidx_ptr[f + 1]; q++) bidx.push_back(gpos(L.fidx[q]));
       U.pull = (int)(pull.size() / 2);
@@ -1594,6 +1645,8 @@ static void layout_dense(snumat *h) {
   const int np = P.np;
   h->inv_off.assign(P.num_block + 1, 0);
   h->lu_off.assign(np + 1, 0);
+  h->sep_rows.assign(np + 1, 0);
+  for (int p = 1; p < np; p++) h->sep_rows[p + 1] = h->sep_rows[p] + P.block_size[p];
   for (int p = 1; p < np; p++) h->lu_off[p + 1] = h->lu_off[p] + (P.block_size[p] + 63) / 64 * 4096LL;
   long long inv_total = 0;
   for (int p = 1; p < np; p++) {

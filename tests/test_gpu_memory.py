@@ -122,3 +122,24 @@ def test_columns_in_turn_where_groups_do_not_fit(S, precision):
         M.close()
     d_b.free()
     d_x.free()
+
+
+def test_working_memory_of_column_groups(S):
+    """A group of 16 columns takes its right-hand sides, the separators' vectors
+    and the update rows alive at once, not every front's side by side."""
+    for dims, st, np_ in (((33, 31, 29), 7, 16), ((250, 211, 1), 5, 32)):
+        A = S.gen_grid(*dims, st, 0, {7: 6.1, 5: 4.1}[st], 1)
+        order, sizes = S.order_grid(*dims, np_)
+        with S.SnuMat(A, np_, order=order, sizes=sizes, device=0) as M:
+            M.factorize()
+            rows = sum(int(np.sum(F["f"] - F["nk"])) for F in (M.leaf_fronts(r) for r in range(np_)))
+            seps = A.n - sum(M.leaf_sizes(r)[0] for r in range(np_))
+            before = M.info()["device_bytes"]
+            d_b, d_x = S.DeviceBuffer(8 * A.n * 2), S.DeviceBuffer(8 * A.n * 2)
+            d_b.upload(np.ones((A.n, 2), order="F"))
+            M.solve_device_ptr(d_b.ptr.value, d_x.ptr.value, 2)
+            d_b.free()
+            d_x.free()
+            taken = M.info()["device_bytes"] - before
+            print("case", dims, "bytes per row and column", taken / (16 * A.n), "rows", rows / A.n, flush=True)
+            assert taken <= 16 * 8 * (A.n + seps + 0.8 * rows)
