@@ -1051,9 +1051,18 @@ __device__ __forceinline__ double block_max(double v, double *red) {
   for (int i = 1; i < (int)(blockDim.x >> 6); i++) v = fmax(v, red[i]);
   return v;
 }
-// |v| for the norms, infinite for a NaN (fmax would leave it out, and a
-// solution of NaNs pass for an exact one)
-__device__ __forceinline__ double norm_abs(double v) { return v == v ? fabs(v) : HUGE_VAL; }
+// Maximum of |v| that takes a NaN for an infinity (fmax alone would leave it
+// out, and a solution of NaNs pass for an exact one): the largest high word
+// tells, which is cheaper per value than a comparison in FP64.
+struct NormMax {
+  double m = 0.0;
+  unsigned hi = 0;
+  __device__ __forceinline__ void add(double v) {
+    m = fmax(m, fabs(v));
+    hi = max(hi, (unsigned)__double2hiint(v) & 0x7fffffffu);
+  }
+  __device__ __forceinline__ double value() const { return hi < 0x7ff00000u ? m : HUGE_VAL; }
+};
 // r = b - A x, rounded to T straight into the packed vectors (the next
 // sweep's right-hand sides, so no FP64 residual goes through memory), and the
 // column maxima of |b|, |r| and |x| in the same pass: each workgroup stores its
@@ -1078,7 +1087,8 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
   const int sub = threadIdx.x & 7, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const long long first = ((long long)blockIdx.x * 256 + threadIdx.x) >> 3, step = ((long long)gridDim.x * 256) >> 3;
   if (M.nrhs == 1) {
-    double mb = 0.0, mr = 0.0, mx = 0.0;
+    NormMax nb, nr;
+    double mx = 0.0;
     for (long long row = first; row < M.n; row += step) {
       const int p0 = rowptr[row], p1 = rowptr[row + 1];
       double s = 0.0;
@@ -1089,14 +1099,13 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
       if (sub == 0) {
         const double b = rhs[row], r = b - s;
         out[order[row]] = (T)r;
-        mb = fmax(mb, norm_abs(b));
-        mr = fmax(mr, norm_abs(r));
-        mx = fmax(mx, norm_abs(x[row]));
+        nb.add(b);
+        nr.add(r);
+        mx = fmax(mx, fabs(x[row]));
       }
     }
     double *rd = &red[0][0][0];
-    mb = block_max(mb, rd);
-    mr = block_max(mr, rd);
+    const double mb = block_max(nb.value(), rd), mr = block_max(nr.value(), rd);
     mx = block_max(mx, rd);
     if (threadIdx.x == 0) {
       part[(long long)M.norm0 * nblk + blockIdx.x] = mb;
@@ -1114,11 +1123,10 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
   const int row_end = min((long long)M.n, (long long)(wg + 1) * chunk);
   for (int c0 = 0; c0 < M.nrhs; c0 += NC) {
     T *oc = out + (long long)(c0 / kColGroup) * V.n * kColGroup + c0 % kColGroup;
+    NormMax nb[NC], nr[NC];
     double m[3][NC];
 #pragma unroll
-    for (int q = 0; q < 3; q++)
-#pragma unroll
-      for (int c = 0; c < NC; c++) m[q][c] = 0.0;
+    for (int c = 0; c < NC; c++) m[2][c] = 0.0;
     for (int row = wg * chunk + threadIdx.x; row < row_end; row += 256) {
       const int p0 = rowptr[row], p1 = rowptr[row + 1];
       T *o = oc + (long long)order[row] * kColGroup;
@@ -1140,11 +1148,13 @@ __global__ __launch_bounds__(256) void k_residual(const IrDev *__restrict__ tab,
       for (int c = 0; c < NC; c++) {
         const double r = b[c] - s[c];
         o[c] = c0 + c < M.nrhs ? (T)r : T(0);
-        m[0][c] = fmax(m[0][c], norm_abs(b[c]));
-        m[1][c] = fmax(m[1][c], norm_abs(r));
-        m[2][c] = fmax(m[2][c], norm_abs(xr[c]));
+        nb[c].add(b[c]);
+        nr[c].add(r);
+        m[2][c] = fmax(m[2][c], fabs(xr[c]));
       }
     }
+#pragma unroll
+    for (int c = 0; c < NC; c++) m[0][c] = nb[c].value(), m[1][c] = nr[c].value();
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 3; q++)
