@@ -85,14 +85,23 @@ __global__ __launch_bounds__(256) void k_front_small(const FrontDev *__restrict_
 // us FP64, 32,898 of order 28 with 10 pivots 430 -> 252, 16 fronts 24 -> 13.
 // Orders above 48 would take more than 128 registers.
 constexpr int kFrontCol = 8;
+// (the pivot row's entries are read with every lane active: its own lane takes
+// no part in the update, and what the register holds there inside the branch is
+// the register allocator's affair)
 template <typename T, int P, int C>
-__device__ __forceinline__ void wave_update(T (&a)[kFrontWave], T q, int f) {
+__device__ __forceinline__ void wave_update(T (&a)[kFrontWave], T q, int f, int lane) {
   if constexpr (C < kFrontWave) {
     if (C < f) {
+      T u[kFrontCol];
 #pragma unroll
-      for (int c = C; c < C + kFrontCol; c++)
-        if (c > P) a[c] -= q * rld(a[c], P);
-      wave_update<T, P, C + kFrontCol>(a, q, f);
+      for (int c = 0; c < kFrontCol; c++)
+        if (C + c > P) u[c] = rld(a[C + c], P);
+      if (lane > P) {
+#pragma unroll
+        for (int c = 0; c < kFrontCol; c++)
+          if (C + c > P) a[C + c] -= q * u[c];
+      }
+      wave_update<T, P, C + kFrontCol>(a, q, f, lane);
     }
   }
 }
@@ -103,7 +112,7 @@ __device__ __forceinline__ void wave_step(T (&a)[kFrontWave], int f, int nk, int
   if (d < eps && d > -eps) d = d < T(0) ? -eps : eps;
   const T q = a[P] / d;
   a[P] = lane > P ? q : lane == P ? d : a[P];
-  if (lane > P) wave_update<T, P, (P + 1) / kFrontCol * kFrontCol>(a, q, f);
+  wave_update<T, P, (P + 1) / kFrontCol * kFrontCol>(a, q, f, lane);
 }
 template <typename T, int... P>
 __device__ __forceinline__ void wave_steps(std::integer_sequence<int, P...>, T (&a)[kFrontWave], int f, int nk,
@@ -213,11 +222,14 @@ __global__ __launch_bounds__(256) void k_extend_add(const AddTile *__restrict__ 
     if (!__any(lane >= c0 && lane < c0 + 16 && cc >= 0)) continue;
     const auto U = gptr((const T *)S.U) + max(rr, 0);
     T u[16];
+    int col[16];  // (read with every lane active)
 #pragma unroll
-    for (int j = 0; j < 16; j++) u[j] = U[(long long)max(rl(cc, c0 + j), S.cb) * S.ld];
+    for (int j = 0; j < 16; j++) col[j] = rl(cc, c0 + j);
+#pragma unroll
+    for (int j = 0; j < 16; j++) u[j] = U[(long long)max(col[j], S.cb) * S.ld];
 #pragma unroll
     for (int j = 0; j < 16; j++)
-      if (rr >= 0 && rl(cc, c0 + j) >= 0) v[j] += u[j];
+      if (rr >= 0 && col[j] >= 0) v[j] += u[j];
   }
   if (lane < t.nr) {
 #pragma unroll
