@@ -794,7 +794,7 @@ __device__ __forceinline__ void factor_block(DiagLds<T> &S, const DiagProbT<T> &
       for (int j = 0; j < 16; j++) v[j] = own ? (j == l16 ? T(1) : T(0)) : v[j];
       diag_block<T>(std::make_integer_sequence<int, 16>{}, d, v, l16, tr, P.eps);
       // (the diagonal block is read by both before wave 0 writes it)
-      __builtin_amdgcn_s_barrier();
+      __syncthreads();
       if (tr) {
         if (own) vs = &S.Xd[kb][l16][0];
 #pragma unroll
@@ -808,7 +808,7 @@ __device__ __forceinline__ void factor_block(DiagLds<T> &S, const DiagProbT<T> &
         }
       }
     } else {
-      __builtin_amdgcn_s_barrier();
+      __syncthreads();
     }
     __syncthreads();
     // tile (i, j) (16 x 16 blocks) -= (i, kb) (kb, j) for i > kb (column
