@@ -864,6 +864,7 @@ extern "C" int snumat_leaf_front_pivots(const snumat_t *h, int rank, int *k_ptr,
 extern "C" int snumat_leaf_values(const snumat_t *h, int rank, double *out) {
   if (!h || rank < 0 || rank >= h->P.np) return set_error(SNU_ERR_BAD_INPUT, "bad rank");
   if (!h->factored && !h->staged) return set_error(SNU_ERR_NOT_FACTORED, "not factored");
+  if (!out) return set_error(SNU_ERR_BAD_INPUT, "null output");
   const LeafPlan &L = h->P.leaves[rank];
   HIPCHK(hipSetDevice(h->device));
   std::fill(out, out + L.lu_nnz, 0.0);
@@ -894,6 +895,7 @@ static int overlay_diag(const snumat_t *h, int e, double *out) {
 extern "C" int snumat_sep_diag(const snumat_t *h, int e, double *out) {
   if (!h || e < 1 || e >= h->P.np) return set_error(SNU_ERR_BAD_INPUT, "bad separator");
   if (!h->factored) return set_error(SNU_ERR_NOT_FACTORED, "not factored");
+  if (!out) return set_error(SNU_ERR_BAD_INPUT, "null output");
   int s = h->P.block_size[e];
   int rc = read_values(h, h->P.offR[e], (size_t)s * s, out);
   return rc ? rc : h->prec == SNU_FP32 ? overlay_diag<float>(h, e, out) : overlay_diag<double>(h, e, out);

@@ -122,3 +122,14 @@ def test_refinement_of_solutions_that_are_not_finite(S):
                 assert S.backward_error(A, x[:, c], B[:, c]) <= 1e-12
             d_b.free()
             d_x.free()
+
+
+def test_introspection_without_an_output(S):
+    """A null output is refused, not written to."""
+    A = S.gen_grid(12, 11, 1, 5, 0, 4.1, 1)
+    for precision in ("fp64", "fp32"):
+        with S.SnuMat(A, 2, grid=(12, 11, 1), device=0, precision=precision) as M:
+            for stage in (0, 2):
+                S._check(S.lib().snumat_factorize_stage(M._h, stage))
+                assert S.lib().snumat_leaf_values(M._h, 0, None) == -1
+            assert S.lib().snumat_sep_diag(M._h, 1, None) == -1
