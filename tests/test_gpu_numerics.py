@@ -133,3 +133,56 @@ def test_introspection_without_an_output(S):
                 S._check(S.lib().snumat_factorize_stage(M._h, stage))
                 assert S.lib().snumat_leaf_values(M._h, 0, None) == -1
             assert S.lib().snumat_sep_diag(M._h, 1, None) == -1
+
+
+GRIDS = [((9, 9, 9), 27, 1), ((13, 7, 5), 7, 2), ((31, 23, 1), 9, 4), ((17, 16, 1), 5, 1), ((11, 10, 8), 27, 8),
+         ((24, 23, 22), 7, 8)]
+DIAG = {5: 4.1, 9: 8.1, 7: 6.1, 27: 0.0}
+
+
+def test_fp32_sweeps_without_refinement_or_fallback(S):
+    """FP32 sweeps on their own, where neither refinement nor the FP64 twin can
+    make up for a wrong one: the first iterate within 2 m u of the right-hand
+    side (m: the largest order of a dense block, growth at most 2: diagonally
+    dominant), then convergence in two steps at most and no fallback, for column
+    counts at the edges of the groups; as a batch too."""
+    u = 2.0 ** -24
+    mats, bs = [], []
+    for (dims, st, np_), kb in zip(GRIDS, (1, 17, 2, 16, 33, 3)):
+        A = S.gen_grid(*dims, st, 1 if st == 27 else 0, DIAG[st], 3)
+        order, sizes = S.order_grid(*dims, np_)
+        B = np.asfortranarray(np.random.default_rng(5).standard_normal((A.n, 65)))
+        args = dict(order=order, sizes=sizes, device=0, precision="fp32", ir_tol=1e-12)
+        m = 0
+        with S.SnuMat(A, np_, ir_max_steps=-1, **args) as M:
+            M.factorize()
+            m = max([int(np.max(F["f"])) for F in (M.leaf_fronts(r) for r in range(np_))] + [int(s) for s in sizes[np_:]])
+            d_b, d_x = S.DeviceBuffer(B.nbytes), S.DeviceBuffer(B.nbytes)
+            d_b.upload(B)
+            for k in (1, 2, 15, 16, 17, 33, 64, 65):
+                rc = S.lib().snumat_solve_device_scratch(M._h, d_b.ptr, d_x.ptr, k, A.n)
+                assert rc in (0, -10)
+                x = np.zeros((A.n, 65), order="F")
+                d_x.download(x)
+                err = S.backward_error(A, x[:, :k], B[:, :k])
+                print("case", dims, st, "columns", k, "order", m, "error / u", err / u, flush=True)
+                assert err <= 2 * m * u
+            d_b.free()
+            d_x.free()
+        M = S.SnuMat(A, np_, **args)
+        M.factorize()
+        for k in (1, 2, 16, 33):
+            x = M.solve(B[:, :k])
+            t = M.timings()
+            assert t["fp64_fallback"] == 0 and t["ir_steps"] <= 2
+            assert S.backward_error(A, x, B[:, :k]) <= 1e-12
+        mats.append(M)
+        bs.append(B[:, :kb])
+    with S.Batch(mats) as batch:
+        batch.factorize()
+        for M, b, x in zip(mats, bs, batch.solve(bs)):
+            assert S.backward_error(M.A, np.asarray(x).reshape(b.shape), b) <= 1e-12
+        t = batch.timings()
+        assert t["fp64_fallbacks"] == 0 and t["ir_steps"] <= 2
+    for M in mats:
+        M.close()
