@@ -180,7 +180,9 @@ int snumat_destroy(snumat_t *h);
  * dense step.  Each matrix's arithmetic is that of its standalone
  * factorization; after snubatch_factorize every member is factored and may
  * also be solved on its own.  The batch does not own the matrices, which
- * must outlive it. */
+ * must outlive it.  The first snubatch_factorize merges the members' launch
+ * lists (a batch that only solves does without), so it takes longer than the
+ * next. */
 typedef struct snubatch snubatch_t;
 int snubatch_create(snumat_t *const *mats, int count, snubatch_t **out);
 int snubatch_factorize(snubatch_t *b);

@@ -321,7 +321,6 @@ int factorize_values(snumat *h, int stage) {
   fs.ir = h->prec == SNU_FP32 ? &h->d_tab->ir : nullptr;
   fs.anorm_out = h->d_norms;
   fs.max_n = h->P.n;
-  fs.wd = &h->wd;
   fs.fronts = &vals<T>(h).fronts;
   fs.eps = h->opts.eps;
   fs.split = h->opts.fp32_gemm == SNU_GEMM_SPLIT;

@@ -215,7 +215,6 @@ int batch_factorize(snubatch *b) {
   fs.ir = b->prec == SNU_FP32 ? b->d_ir_a : nullptr;
   fs.anorm_out = b->d_anorm;
   fs.max_n = b->max_n;
-  fs.wd = &b->wd;
   fs.fronts = std::is_same<T, double>::value ? (const void *)&b->fr64 : (const void *)&b->fr32;
   fs.eps = b->mats[0]->opts.eps;
   fs.split = b->mats[0]->opts.fp32_gemm == SNU_GEMM_SPLIT;

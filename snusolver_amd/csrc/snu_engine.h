@@ -258,9 +258,6 @@ size_t estimate_device_bytes(const snumat *h);
 int device_alloc(snumat *h, void **p, size_t bytes);
 float ev_ms(hipEvent_t a, hipEvent_t b);
 
-template <typename T>
-int upload_list(T **p, const std::vector<T> &v);
-
 // Append problem C (M x N) -= / = sum_seg A_seg B_seg to a grouped GEMM
 // launch with tb x tb tiles; returns 1 if a problem was added.
 template <typename T>
@@ -307,7 +304,6 @@ struct FactorSet {
   const IrDev *ir;           // FP32 only: |A| norms into anorm_out
   unsigned long long *anorm_out;
   int max_n;
-  const WorkDev *wd;
   const void *fronts;  // FrontPlan of the set's value type
   double eps;
   bool split = false;  // FP32: GEMM tiles through bf16 splits (SNU_GEMM_SPLIT)

@@ -64,12 +64,6 @@ int upload_list(T **p, const std::vector<T> &v) {
   if (!v.empty()) HIPCHK(hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   return SNU_OK;
 }
-template int upload_list<int>(int **, const std::vector<int> &);
-template int upload_list<LeafDev>(LeafDev **, const std::vector<LeafDev> &);
-template int upload_list<VecDev>(VecDev **, const std::vector<VecDev> &);
-template int upload_list<PermDev>(PermDev **, const std::vector<PermDev> &);
-template int upload_list<PrepDev>(PrepDev **, const std::vector<PrepDev> &);
-template int upload_list<IrDev>(IrDev **, const std::vector<IrDev> &);
 
 float ev_ms(hipEvent_t a, hipEvent_t b) {
   float ms = 0;
@@ -1903,7 +1897,6 @@ int make_side(const std::vector<const DensePlan<T> *> &in, SideStream &s) {
 template <typename T>
 int enqueue_factor(const FactorSet &fs, const DensePlan<T> &plan, hipStream_t st,
                    const std::vector<hipEvent_t> *ev, bool profile, std::vector<hipEvent_t> *pev) {
-  const WorkDev &wd = *fs.wd;
   if (ev) HIPCHK(hipEventRecord((*ev)[0], st));
   if (fs.scatter_only) launch_prepare<T>(fs.prep, fs.nmat, fs.max_len, fs.max_nnz, st);
   if (fs.ir) launch_rowabs_max(fs.ir, fs.nmat, fs.max_n, fs.anorm_out, st);

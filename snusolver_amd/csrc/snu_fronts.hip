@@ -4,11 +4,11 @@
 // src/kernel_sparse.cu:740-781,953-971) runs as dense partial factorizations
 // of frontal matrices, level by level of the leaves' front trees, every leaf
 // of every matrix of a launch set sharing each launch:
-//   small fronts (the whole front fits the LDS): k_front_small does
-//     everything in one workgroup per front;
+//   small fronts (the whole front fits the LDS): k_front_wave does everything
+//     in one wave per front, k_front_small in one workgroup;
 //   larger fronts live in global memory: k_extend_add builds them, then the
-//     blocked partial LU on the dense kernels (k_diag_lu with the pivot clamp,
-//     the triangular solves and the update on the MFMA k_gemm);
+//     blocked partial LU on the dense kernels (k_diag_panel, or k_diag_lu and
+//     k_panel, with the pivot clamp; the update on the MFMA k_gemm);
 //   k_extend_add then adds the root fronts' updates into the separator blocks
 //     (the reference's boundary Schur assembly).
 // The factors stay in the fronts, where the solves read them.

@@ -193,7 +193,6 @@ using DiagProb = DiagProbT<double>;
 using GemvSeg = GemvSegT<double>;
 using GemvProb = GemvProbT<double>;
 
-int device_lds_limit();
 
 template <typename T>
 void launch_fill(T *p, long long n, hipStream_t st);
@@ -262,8 +261,9 @@ void launch_leaf_sweep(const LeafDev *leaves, int nleaves, const VecDev *vd, T *
                        int max_groups, bool one, bool many, bool bwd, hipStream_t st);
 
 // ---- multifrontal leaf factorization ----
-// Fronts held whole in LDS (f <= max_f): assembly, partial LU with the
-// pivot clamp, write-back of the owned slots, update block to global memory.
+// Fronts held whole in LDS (f <= max_f): assembly from A's entries and the
+// children's updates, partial LU with the pivot clamp, the whole front (factors
+// and update block) to global memory.
 template <typename T>
 void launch_front_small(const FrontDev *fr, int nfront, int max_f, double eps, hipStream_t st);
 // The same, one wave per front, for orders up to kFrontWave.

@@ -1269,13 +1269,6 @@ void launch_prepare(const PrepDev *tab, int nmat, long long max_len, long long m
   hipLaunchKernelGGL(k_prep_scatter<T>, dim3(blocks(max_nnz), nmat), dim3(256), 0, st, tab);
 }
 
-int device_lds_limit() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 65536;
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 65536;
-  return (int)prop.sharedMemPerBlock;
-}
 
 
 // ---- explicit instantiations: FP64 and FP32 value paths ----

@@ -994,7 +994,6 @@ __global__ __launch_bounds__(256) void k_gemv16(const GemvProbT<T> *__restrict__
   const int m0 = lt * 64, ng = min(GS, P.groups - g0);
   const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const SweepCtx c{lane, l16, lk};
   Frag<T> acc[GS][4];
 #pragma unroll
   for (int g = 0; g < GS; g++)
