@@ -60,12 +60,13 @@ __device__ __forceinline__ double scale2(double x, int e) { return __builtin_amd
 __device__ __forceinline__ float scale2(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
 __device__ __forceinline__ double div_special(double q, double d, double a) { return __builtin_amdgcn_div_fixup(q, d, a); }
 __device__ __forceinline__ float div_special(float q, float d, float a) { return __builtin_amdgcn_div_fixupf(q, d, a); }
-// Quotients by one divisor, rounded as by divisions, with one reciprocal: a few
-// Newton steps, and per quotient corrections by the exact remainder in FMA
-// (Markstein's division), on the mantissas of both so that nothing on the way
-// overflows or underflows (a dividend taken whole did beyond half the largest
-// value, and lost its remainder near the smallest); subnormal quotients are
-// rounded twice.
+// Quotients by one divisor with one reciprocal: a few Newton steps on its
+// mantissa, and per quotient corrections by the exact remainder in FMA
+// (Markstein's division).  The dividend is scaled by the divisor's exponent
+// first, so that nothing on the way overflows where the quotient does not (a
+// dividend beyond half the largest value did, taken whole).  Rounded as by a
+// division while remainders are normal numbers (quotients above 2^-969, FP32
+// 2^-101), within an ulp below.
 template <typename T>
 struct Divisor {
   T m, r;  // mantissa, its reciprocal
@@ -77,15 +78,14 @@ struct Divisor {
     if constexpr (std::is_same<T, double>::value) r = fma(fma(-m, r, T(1)), r, r);
   }
   __device__ __forceinline__ T quotient(T a) const {
-    const T n = frexp_m(a);
+    const T n = scale2(a, -e);
     T q = n * r;
     q = fma(fma(-m, q, n), r, q);
     if constexpr (std::is_same<T, float>::value) q = fma(fma(-m, q, n), r, q);
-    return div_special(scale2(q, frexp_e(a) - e), m, a);
+    return div_special(q, m, n);
   }
-  // The same, a shorter chain for substitution: the dividend scaled whole, one
-  // correction.  (Rounded as by a division while remainders are normal numbers;
-  // where a division gives an infinity, any value that is not finite.)
+  // The same, a shorter chain for substitution: one correction (FP32: within an
+  // ulp), and where a division gives an infinity any value that is not finite.
   __device__ __forceinline__ T quick(T a) const {
     const T n = scale2(a, -e), q = n * r;
     return fma(fma(-m, q, n), r, q);
