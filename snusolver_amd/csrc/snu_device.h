@@ -71,7 +71,6 @@ template <typename T>
 struct Divisor {
   T m, r;  // mantissa, its reciprocal
   int e;   // exponent
-  Divisor() = default;
   __device__ __forceinline__ explicit Divisor(T d) : m(frexp_m(d)), e(frexp_e(d)) {
     r = recip(m);
     r = fma(fma(-m, r, T(1)), r, r);
@@ -84,45 +83,63 @@ struct Divisor {
     if constexpr (std::is_same<T, float>::value) q = fma(fma(-m, q, n), r, q);
     return div_special(q, m, n);
   }
-  // The same, a shorter chain for substitution: one correction (FP32: within an
-  // ulp), and where a division gives an infinity any value that is not finite.
-  __device__ __forceinline__ T quick(T a) const {
-    const T n = scale2(a, -e), q = n * r;
-    return fma(fma(-m, q, n), r, q);
-  }
-  // lane l's divisor
-  __device__ __forceinline__ Divisor of_lane(int l) const {
-    Divisor d;
-    d.m = rld(m, l), d.r = rld(r, l), d.e = rl(e, l);
-    return d;
-  }
 };
 
-// Between the four groups of 16 lanes (permlane swaps: VALU, no LDS).
-// every group's v, in all lanes
-__device__ __forceinline__ void gather_groups(double v, double (&s)[4]) {
-  unsigned w[2][4];
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const unsigned x = h ? __double2hiint(v) : __double2loint(v);
-    const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    const auto a = __builtin_amdgcn_permlane16_swap(p[0], p[0], false, false);
-    const auto b = __builtin_amdgcn_permlane16_swap(p[1], p[1], false, false);
-    w[h][0] = a[0], w[h][1] = a[1], w[h][2] = b[0], w[h][3] = b[1];
+// A pivot of a substitution: its reciprocal in two parts, whose product with the
+// dividend has a division's rounding (to a few 2^-100) in two dependent
+// operations, and its scale.  The dividend v - s is scaled by the pivot's
+// exponent as it is formed, so that nothing on the way overflows where the
+// quotient does not.  (Where a division gives an infinity: any value that is
+// not finite.)
+template <typename T>
+struct Pivot {
+  T r, lo;  // 1 / (pivot 2^-e)
+  T neg;    // -2^-e
+  Pivot() = default;
+  __device__ __forceinline__ explicit Pivot(T d) {
+    const int e = max(frexp_e(d), std::is_same<T, double>::value ? -1021 : -125);  // (2^-e is finite)
+    const T m = scale2(d, -e);
+    r = recip(m);
+    r = fma(fma(-m, r, T(1)), r, r);
+    if constexpr (std::is_same<T, double>::value) r = fma(fma(-m, r, T(1)), r, r);
+    lo = fma(-m, r, T(1)) * r;
+    neg = -scale2(T(1), -e);
   }
-#pragma unroll
-  for (int i = 0; i < 4; i++) s[i] = __hiloint2double((int)w[1][i], (int)w[0][i]);
+  __device__ __forceinline__ T scaled(T v) const { return -(v * neg); }
+  // (v - s) / pivot, v scaled
+  __device__ __forceinline__ T solve(T v, T s) const {
+    const T n = fma(s, neg, v);
+    return fma(n, r, n * lo);
+  }
+  // lane l's
+  __device__ __forceinline__ Pivot of_lane(int l) const {
+    Pivot p;
+    p.r = rld(r, l), p.lo = rld(lo, l), p.neg = rld(neg, l);
+    return p;
+  }
+};
+// Of group G (of the four groups of 16 lanes) s[i], in group i, by permlane
+// swaps (VALU, no LDS).
+template <int G>
+__device__ __forceinline__ unsigned spread_words(const unsigned (&x)[4]) {
+  const auto a = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+  const auto p = __builtin_amdgcn_permlane32_swap(a[G & 1], b[G & 1], false, false);
+  return p[G >> 1];
 }
-// group G's s[i], in group i
 template <int G>
 __device__ __forceinline__ float spread_group(const float (&s)[4]) {
   unsigned x[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) x[i] = __float_as_uint(s[i]);
-  const auto a = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
-  const auto p = __builtin_amdgcn_permlane32_swap(a[G & 1], b[G & 1], false, false);
-  return __uint_as_float(p[G >> 1]);
+  return __uint_as_float(spread_words<G>(x));
+}
+template <int G>
+__device__ __forceinline__ double spread_group(const double (&s)[4]) {
+  unsigned lo[4], hi[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) lo[i] = __double2loint(s[i]), hi[i] = __double2hiint(s[i]);
+  return __hiloint2double((int)spread_words<G>(hi), (int)spread_words<G>(lo));
 }
 
 // MFMA fragments, 16x16x4 products.  A 16 x 16 block of a vector group (16 rows, 16 columns)

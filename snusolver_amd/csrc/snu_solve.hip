@@ -122,10 +122,10 @@ void launch_permute_out(const PermDev *pd, int nmat, const VecDev *vd, const T *
 // most a few hundred units) and a unit is sized so that a wave has 16 or more
 // loads in flight.  Bound by the latency of the units' loads and substitutions
 // down the chain of heights; forward / backward: 64^3 7-point FP64, one column
-// 214 / 272 us (row by row over the leaf's CSR factors, hundreds of level sets:
-// 554 / 828; with the inverses 202 / 242); 48^3 27-point FP64, 16 columns 505 /
-// 436 us (2916 / 4719; 492 / 382); 1000^2 5-point FP32, 64 columns 1.45 / 1.27
-// ms (3.8 / 4.8; 1.53 / 1.15).
+// 214 / 250 us (row by row over the leaf's CSR factors, hundreds of level sets:
+// 554 / 828; with the inverses 202 / 242); 48^3 27-point FP64, 16 columns 499 /
+// 428 us (2916 / 4719; 493 / 381); 1000^2 5-point FP32, 64 columns 1.42 / 1.23
+// ms (3.8 / 4.8; 1.54 / 1.15).
 // 1024 threads per leaf for one column (261 / 292 us with 512 and the
 // inverses); the 16-column fragments need over 200 registers, so 512.
 template <int NC>
@@ -142,9 +142,20 @@ __device__ __forceinline__ SolveUnit load_unit(const SolveUnit *p) {
   return __builtin_bit_cast(SolveUnit, *(__attribute__((address_space(4))) const int16_v *)p);
 }
 
+// l16: a fragment's column of the lane, lk: its row group (rows 4 lk .. 4 lk + 3,
+// one per register), ar: the row of A that the lane loads as the first operand.
+// For FP64 the product's register r of group lk is row 4 r + lk of the
+// instruction; loading A's rows in that order (ar) makes it row 4 lk + r of the
+// block as for FP32, so that four consecutive rows are in one lane, where
+// substitution needs them.
 struct SweepCtx {
-  int lane, l16, lk;
+  int lane, l16, lk, ar;
 };
+template <typename T>
+__device__ __forceinline__ constexpr int lane_of_row(int row) {
+  return std::is_same<T, double>::value ? 4 * (row & 3) + (row >> 2) : row;
+}
+__device__ __forceinline__ int sweep_row(int r, int lk) { return 4 * lk + r; }
 // LU of the unit's 64-pivot block of a larger front (64 x 64)
 template <typename T>
 __device__ __forceinline__ const T *pivot_block(const SolveUnit &U) {
@@ -198,13 +209,13 @@ __device__ __forceinline__ T dot_cols(const T *a, long long ld, int K, int lane,
 // w -= L y for the `rows` rows of a lower trapezoid (unit diagonal, n columns;
 // y: w's first n rows on the way), RPL rows per lane.  A row's products are
 // summed and taken from it at once: rounding relative to their sum, not to the
-// row at every step.
+// row at every step.  (Rows that are done go on summing, which nothing reads.)
 template <typename T, int RPL>
 __device__ __forceinline__ void solve_lower1(const T *A, int ld, int rows, int n, T (&w)[RPL], int lane) {
   const auto F = gptr(A);
-  T s[RPL];
+  T s[RPL], y[RPL];
 #pragma unroll
-  for (int i = 0; i < RPL; i++) s[i] = T(0);
+  for (int i = 0; i < RPL; i++) s[i] = y[i] = T(0);
   for (int k0 = 0; k0 < n; k0 += 16) {
     T c[RPL][16];
 #pragma unroll
@@ -214,29 +225,39 @@ __device__ __forceinline__ void solve_lower1(const T *A, int ld, int rows, int n
 #pragma unroll
     for (int j = 0; j < 16; j++) {
       const int k = k0 + j;
-      T yk = RPL == 1 || k < 64 ? rld(w[0] - s[0], k & 63) : rld(w[RPL - 1] - s[RPL - 1], k & 63);
-      if (k >= n) yk = T(0);
+      T yk;
+      auto take = [&](int i) __attribute__((always_inline)) {
+        const T d = w[i] - s[i];
+        y[i] = lane + 64 * i == k ? d : y[i];
+        yk = rld(d, k & 63);
+      };
+      if (RPL == 1 || k < 64) take(0);
+      else take(RPL - 1);
+      if (k >= n) yk = T(0);  // (no branch: the loads of later steps would move behind it)
 #pragma unroll
-      for (int i = 0; i < RPL; i++) s[i] = lane + 64 * i > k ? s[i] + c[i][j] * yk : s[i];
+      for (int i = 0; i < RPL; i++) s[i] += c[i][j] * yk;
     }
   }
 #pragma unroll
-  for (int i = 0; i < RPL; i++) w[i] -= s[i];
+  for (int i = 0; i < RPL; i++) w[i] = lane + 64 * i < n ? y[i] : w[i] - s[i];
 }
-// the divisors of an upper triangle's rows
+// an upper triangle's pivots
 template <typename T, int RPL>
-__device__ __forceinline__ void pivots1(const T *A, int ld, int n, Divisor<T> (&by)[RPL], int lane) {
+__device__ __forceinline__ void pivots1(const T *A, int ld, int n, Pivot<T> (&by)[RPL], int lane) {
 #pragma unroll
   for (int i = 0; i < RPL; i++) {
     const int r = lane + 64 * i;
-    by[i] = Divisor<T>(r < n ? gptr(A)[(long long)r * (ld + 1)] : T(1));
+    by[i] = Pivot<T>(r < n ? gptr(A)[(long long)r * (ld + 1)] : T(1));
   }
 }
 // t = U^-1 (t - s), n rows
 template <typename T, int RPL>
-__device__ __forceinline__ void solve_upper1(const T *A, int ld, int n, const Divisor<T> (&by)[RPL], T (&t)[RPL],
+__device__ __forceinline__ void solve_upper1(const T *A, int ld, int n, const Pivot<T> (&by)[RPL], T (&t)[RPL],
                                              T (&s)[RPL], int lane) {
   const auto F = gptr(A);
+  T v[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; i++) v[i] = by[i].scaled(t[i]);
   for (int k0 = n - 1; k0 >= 0; k0 -= 16) {
     T c[RPL][16];
 #pragma unroll
@@ -246,15 +267,17 @@ __device__ __forceinline__ void solve_upper1(const T *A, int ld, int n, const Di
 #pragma unroll
     for (int j = 0; j < 16; j++) {
       const int k = k0 - j;
-      const int kk = max(k, 0);
-      T xk = RPL == 1 || kk < 64 ? rld(by[0].quick(t[0] - s[0]), kk & 63)
-                                 : rld(by[RPL - 1].quick(t[RPL - 1] - s[RPL - 1]), kk & 63);
+      T xk;
+      auto take = [&](int i) __attribute__((always_inline)) {
+        const T q = by[i].solve(v[i], s[i]);
+        t[i] = lane + 64 * i == k ? q : t[i];
+        xk = rld(q, k & 63);
+      };
+      if (RPL == 1 || k < 64) take(0);
+      else take(RPL - 1);
+      if (k < 0) xk = T(0);
 #pragma unroll
-      for (int i = 0; i < RPL; i++) {
-        const int r = lane + 64 * i;
-        if (r < k) s[i] += c[i][j] * xk;
-        else if (r == k) t[i] = xk, s[i] = T(0);
-      }
+      for (int i = 0; i < RPL; i++) s[i] += c[i][j] * xk;
     }
   }
 }
@@ -282,7 +305,7 @@ __device__ __forceinline__ void bwd_front1(const LeafDev &L, const SolveUnit &U,
   const auto F = gptr((const T *)U.F);
   const int f = U.ld, nk = U.nk, nb = U.nb;
   T xb[RPL], t[RPL], s[RPL];
-  Divisor<T> by[RPL];
+  Pivot<T> by[RPL];
   pivots1<T, RPL>((const T *)U.F, f, nk, by, lane);
 #pragma unroll
   for (int i = 0; i < RPL; i++) {
@@ -367,7 +390,7 @@ __device__ __forceinline__ void unit1(const LeafDev &L, const SolveUnit &U, T *x
       break;
     }
     case kBwdPivots: {
-      Divisor<T> by[1];
+      Pivot<T> by[1];
       pivots1<T, 1>(lu, 64, nbk, by, lane);
       T y[1] = {lane < nbk ? x[U.kpos + r] : T(0)}, s[1] = {T(0)};
       for (int q = 0; q < U.nq; q++) s[0] += W[U.wrow + (U.s * U.nq + q) * 64 + lane];
@@ -388,7 +411,7 @@ __device__ __forceinline__ Frag<T> load_frag(const T *X, int row0, int nvalid, c
   Frag<T> v;
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const int row = row0 + frag_row<T>(r, c.lk);
+    const int row = row0 + sweep_row(r, c.lk);
     v[r] = row < nvalid ? X[(long long)row * kColGroup + c.l16] : T(0);
   }
   return v;
@@ -397,7 +420,7 @@ template <typename T>
 __device__ __forceinline__ void store_frag(T *X, int row0, int nvalid, const Frag<T> &v, const SweepCtx &c) {
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const int row = row0 + frag_row<T>(r, c.lk);
+    const int row = row0 + sweep_row(r, c.lk);
     if (row < nvalid) X[(long long)row * kColGroup + c.l16] = v[r];
   }
 }
@@ -408,7 +431,7 @@ __device__ __forceinline__ Frag<T> pull_frag(const LeafDev &L, const SolveUnit &
   int2_v e[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const int row = row0 + frag_row<T>(r, c.lk);
+    const int row = row0 + sweep_row(r, c.lk);
     e[r] = row < rend ? pull_entry(L, U, row) : int2_v{-1, -1};
   }
   Frag<T> v;
@@ -434,7 +457,7 @@ template <typename T>
 __device__ __forceinline__ void mask_frag(Frag<T> &v, int row0, int nvalid, const SweepCtx &c) {
 #pragma unroll
   for (int r = 0; r < 4; r++)
-    if (row0 + frag_row<T>(r, c.lk) >= nvalid) v[r] = T(0);
+    if (row0 + sweep_row(r, c.lk) >= nvalid) v[r] = T(0);
 }
 // acc += A[16 rows][columns k0 .. k0 + 15] b; a: this lane's row, columns
 // clamped to kmax (their b rows are zero)
@@ -444,61 +467,54 @@ __device__ __forceinline__ void frag_mm(Frag<T> &acc, const T *a, int ld, int k0
   const auto p = gptr(a);
   T v[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) v[r] = p[(long long)min(k0 + frag_row<T>(r, c.lk), kmax) * ld];
+  for (int r = 0; r < 4; r++) v[r] = p[(long long)min(k0 + sweep_row(r, c.lk), kmax) * ld];
 #pragma unroll
   for (int r = 0; r < 4; r++) acc = mfma4(v[r], b[r], acc);
 }
 // A 16 x 16 block of a triangle (unit lower, or upper), n of its rows and
-// columns used: entry (l16, 4 g + lk) of its strict part in a[g].
+// columns used: entry (ar, 4 g + lk) of its strict part in a[g].
 template <typename T, bool UPPER>
 struct Tri16 {
   T a[4];
-  Divisor<T> by;  // (UPPER) row l16's pivot
+  Pivot<T> by;  // (UPPER) row ar's pivot
   __device__ __forceinline__ void load(const T *F, int ld, int n, const SweepCtx &c) {
-    const auto p = gptr(F) + min(c.l16, n - 1);
+    const auto p = gptr(F) + min(c.ar, n - 1);
 #pragma unroll
     for (int g = 0; g < 4; g++) a[g] = p[(long long)min(4 * g + c.lk, n - 1) * ld];
-    if constexpr (UPPER) by = Divisor<T>(c.l16 < n ? p[(long long)min(c.l16, n - 1) * ld] : T(1));
+    if constexpr (UPPER) by = Pivot<T>(c.ar < n ? p[(long long)min(c.ar, n - 1) * ld] : T(1));
 #pragma unroll
     for (int g = 0; g < 4; g++) {
       const int k = 4 * g + c.lk;
-      if (!(UPPER ? k > c.l16 && k < n : k < c.l16 && c.l16 < n)) a[g] = T(0);
+      if (!(UPPER ? k > c.ar && k < n : k < c.ar && c.ar < n)) a[g] = T(0);
     }
   }
-  // w - acc solved with it (both zero beyond n).  Four rows at a time: every
-  // lane (FP32: those that hold the four rows) solves them for its column, with
-  // the block's entries and pivots read lane by lane, then one product adds
-  // their share to the rows left.  (The four steps as a loop: half the code, but
-  // a block's loads are then waited for at its head: 1000^2, 64 columns 10.5 ->
-  // 12.5 ms per solve.)
+  // w - acc solved with it (both zero beyond n).  Four rows at a time: the lanes
+  // that hold them (the others compute along) solve them with the block's
+  // entries and pivots read lane by lane, then one product adds their share to
+  // the rows left.  (The four steps as a loop: half the code, but a block's loads
+  // are then waited for at its head: 1000^2, 64 columns 10.5 -> 12.5 ms per solve.)
   template <int g>
   __device__ __forceinline__ void rows(const Frag<T> &w, Frag<T> &acc, Frag<T> &y, const SweepCtx &c) const {
-    T v[4], p[4], s[4];
-    if constexpr (std::is_same<T, double>::value) {
-      gather_groups(w[g], v);
-      gather_groups(acc[g], p);
-    } else {
+    T p[4], s[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = w[i], p[i] = acc[i];
-    }
+    for (int i = 0; i < 4; i++) p[i] = acc[i];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int j = UPPER ? 3 - q : q;
-      s[j] = v[j] - p[j];
-      if constexpr (UPPER) s[j] = by.of_lane(4 * g + j).quick(s[j]);
+      if constexpr (UPPER) {
+        const Pivot<T> d = by.of_lane(lane_of_row<T>(4 * g + j));
+        s[j] = d.solve(d.scaled(w[j]), p[j]);
+      } else {
+        s[j] = w[j] - p[j];
+      }
 #pragma unroll
-      for (int i = UPPER ? 0 : j + 1; i < (UPPER ? j : 4); i++) p[i] += rld(a[g], 4 * g + i + 16 * j) * s[j];
+      for (int i = UPPER ? 0 : j + 1; i < (UPPER ? j : 4); i++)
+        p[i] += rld(a[g], lane_of_row<T>(4 * g + i) + 16 * j) * s[j];
     }
-    T b;  // row 4 g + lk
-    if constexpr (std::is_same<T, double>::value) {
-      b = c.lk == 0 ? s[0] : c.lk == 1 ? s[1] : c.lk == 2 ? s[2] : s[3];
-      y[g] = b;
-    } else {
 #pragma unroll
-      for (int i = 0; i < 4; i++) y[i] = c.lk == g ? s[i] : y[i];
-      b = spread_group<g>(s);
-    }
-    if (g != (UPPER ? 0 : 3)) acc = mfma4((UPPER ? c.l16 < 4 * g : c.l16 >= 4 * g + 4) ? a[g] : T(0), b, acc);
+    for (int i = 0; i < 4; i++) y[i] = c.lk == g ? s[i] : y[i];
+    if (g != (UPPER ? 0 : 3))
+      acc = mfma4((UPPER ? c.ar < 4 * g : c.ar >= 4 * g + 4) ? a[g] : T(0), spread_group<g>(s), acc);
   }
   __device__ __forceinline__ Frag<T> solve(const Frag<T> &w, Frag<T> acc, const SweepCtx &c) const {
     Frag<T> y = w;
@@ -530,7 +546,7 @@ __device__ __forceinline__ void fwd_front16(const LeafDev &L, const SolveUnit &U
       if constexpr (!EXACT) t[b].load(F + 16 * b * (f + 1), f, min(16, nk - 16 * b), c);
       Frag<T> acc = frag_zero<T>();
 #pragma unroll
-      for (int a = 0; a < b; a++) frag_mm(acc, F + min(16 * b + c.l16, nk - 1), f, 16 * a, nk - 1, y[a], c);
+      for (int a = 0; a < b; a++) frag_mm(acc, F + min(16 * b + c.ar, nk - 1), f, 16 * a, nk - 1, y[a], c);
       Frag<T> w = load_frag(xk, 16 * b, nk, c) + pull_frag(L, U, W, 16 * b, nk, c);
       mask_frag(acc, 16 * b, nk, c);
       y[b] = t[b].solve(w, acc, c);
@@ -542,7 +558,7 @@ __device__ __forceinline__ void fwd_front16(const LeafDev &L, const SolveUnit &U
       Frag<T> acc = frag_zero<T>();
 #pragma unroll
       for (int a = 0; a < KB; a++)
-        if (EXACT || 16 * a < nk) frag_mm(acc, F + min(nk + 16 * b + c.l16, f - 1), f, 16 * a, nk - 1, y[a], c);
+        if (EXACT || 16 * a < nk) frag_mm(acc, F + min(nk + 16 * b + c.ar, f - 1), f, 16 * a, nk - 1, y[a], c);
       store_frag(wb, 16 * b, nb, pull_frag(L, U, W, nk + 16 * b, f, c) - acc, c);
     }
 #pragma unroll
@@ -555,11 +571,11 @@ __device__ __forceinline__ Frag<T> gather_frag(const T *x, const int *idx, int r
   const auto p = gptr(idx);
   int at[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) at[r] = p[min(row0 + frag_row<T>(r, c.lk), n - 1)];
+  for (int r = 0; r < 4; r++) at[r] = p[min(row0 + sweep_row(r, c.lk), n - 1)];
   Frag<T> v;
 #pragma unroll
   for (int r = 0; r < 4; r++)
-    v[r] = row0 + frag_row<T>(r, c.lk) < n ? x[(long long)at[r] * kColGroup + c.l16] : T(0);
+    v[r] = row0 + sweep_row(r, c.lk) < n ? x[(long long)at[r] * kColGroup + c.l16] : T(0);
   return v;
 }
 template <typename T, int KB, int BB, bool EXACT>
@@ -582,7 +598,7 @@ __device__ __forceinline__ void bwd_front16(const LeafDev &L, const SolveUnit &U
 #pragma unroll
       for (int b = 0; b < KB; b++)
         if (EXACT || 16 * b < nk)
-          frag_mm(t[b], F + min(16 * b + c.l16, nk - 1) + (long long)nk * f, f, 16 * a, nb - 1, xb, c);
+          frag_mm(t[b], F + min(16 * b + c.ar, nk - 1) + (long long)nk * f, f, 16 * a, nb - 1, xb, c);
     }
 #pragma unroll
   for (int b = KB - 1; b >= 0; b--)
@@ -591,7 +607,7 @@ __device__ __forceinline__ void bwd_front16(const LeafDev &L, const SolveUnit &U
       Frag<T> acc = t[b];
 #pragma unroll
       for (int a = b + 1; a < KB; a++)
-        if (EXACT || 16 * a < nk) frag_mm(acc, F + min(16 * b + c.l16, nk - 1), f, 16 * a, nk - 1, t[a], c);
+        if (EXACT || 16 * a < nk) frag_mm(acc, F + min(16 * b + c.ar, nk - 1), f, 16 * a, nk - 1, t[a], c);
       const Frag<T> w = load_frag(xk, 16 * b, nk, c);
       mask_frag(acc, 16 * b, nk, c);
       t[b] = tri[b].solve(w, acc, c);
@@ -626,13 +642,13 @@ __device__ __forceinline__ void tile_mm(Frag<T> (&acc)[4], const T *a, int ld, i
   const auto p = gptr(a);
   int row[4];
 #pragma unroll
-  for (int b = 0; b < 4; b++) row[b] = min(16 * b + c.l16, rmax);
+  for (int b = 0; b < 4; b++) row[b] = min(16 * b + c.ar, rmax);
   Frag<T> x;
   T v[4][4];
   auto load = [&](int k0, Frag<T> &xn, T (&vn)[4][4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const auto pc = p + (long long)min(k0 + frag_row<T>(r, c.lk), K - 1) * ld;
+      const auto pc = p + (long long)min(k0 + sweep_row(r, c.lk), K - 1) * ld;
 #pragma unroll
       for (int b = 0; b < 4; b++) vn[b][r] = pc[row[b]];
     }
@@ -671,7 +687,7 @@ __device__ __forceinline__ void tri64(Frag<T> (&y)[4], const T *lu, int nbk, con
     Frag<T> acc = sum[b];
 #pragma unroll
     for (int a = UPPER ? b + 1 : 0; a < (UPPER ? 4 : b); a++)
-      if (16 * a < nbk) frag_mm(acc, lu + min(16 * b + c.l16, nbk - 1), 64, 16 * a, nbk - 1, y[a], c);
+      if (16 * a < nbk) frag_mm(acc, lu + min(16 * b + c.ar, nbk - 1), 64, 16 * a, nbk - 1, y[a], c);
     Tri16<T, UPPER> t;
     t.load(lu + 16 * b * 65, 64, min(16, nbk - 16 * b), c);
     mask_frag(acc, 16 * b, nbk, c);
@@ -745,7 +761,7 @@ __global__ __launch_bounds__(leaf_threads<NC>()) void k_leaf_sweep(const LeafDev
   if (vec_width(V.nrhs) != NC || g >= vec_groups(V.nrhs)) return;
   T *x = bp + V.base + (long long)g * V.n * NC, *W = wbuf + V.wbase + (long long)g * V.wrows * NC;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const SweepCtx c{lane, lane & 15, lane >> 4};
+  const SweepCtx c{lane, lane & 15, lane >> 4, lane_of_row<T>(lane & 15)};
   const auto ph = cptr(BWD ? L.bphase : L.fphase);
   const int np = BWD ? L.nbphase : L.nfphase;
   int u0 = ph[0];
