@@ -186,3 +186,32 @@ def test_fp32_sweeps_without_refinement_or_fallback(S):
         assert t["fp64_fallbacks"] == 0 and t["ir_steps"] <= 2
     for M in mats:
         M.close()
+
+
+@pytest.mark.parametrize("precision,n", [("fp64", 20), ("fp64", 64), ("fp32", 20), ("fp32", 96)])
+def test_solves_divide_by_pivots_of_any_size(S, precision, n):
+    """x = b / d within an ulp for diagonal matrices (in a full pattern: one
+    front factored in LDS; larger ones' panels take the inverses of their pivot
+    blocks, which overflow for subnormal pivots) whose pivots go from subnormal
+    to the largest values, with no clamp; FP32: the first iterate."""
+    f64 = precision == "fp64"
+    t, lo, hi, u = (np.float64, -1070, 1022, 2.0 ** -52) if f64 else (np.float32, -145, 126, 2.0 ** -23)
+    rng = np.random.default_rng(n)
+    d = np.ldexp(rng.uniform(0.5, 1, n), np.linspace(lo, hi, n).astype(int)).astype(t) * rng.choice([-1, 1], n).astype(t)
+    q = rng.uniform(0.5, 1, (n, 17))
+    B = (q * d[:, None].astype(np.float64)).astype(t)  # (representable; subnormal where d is)
+    want = B.astype(np.float64) / d[:, None].astype(np.float64)
+    A = S.CSR(n, np.arange(0, n * n + 1, n), np.tile(np.arange(n), n), np.diag(d).astype(np.float64).reshape(-1))
+    B = np.asfortranarray(B.astype(np.float64))
+    with S.SnuMat(A, 1, order=np.arange(n), sizes=[n], device=0, precision=precision, eps=0.0, ir_max_steps=-1) as M:
+        M.factorize()
+        for k in (1, 2, 17):
+            d_b, d_x = S.DeviceBuffer(8 * n * k), S.DeviceBuffer(8 * n * k)
+            d_b.upload(B[:, :k])
+            rc = S.lib().snumat_solve_device_scratch(M._h, d_b.ptr, d_x.ptr, k, n)
+            assert rc == 0 or not f64
+            x = np.zeros((n, k), order="F")
+            d_x.download(x)
+            d_b.free()
+            d_x.free()
+            assert np.all(np.abs(x - want[:, :k]) <= u * np.abs(want[:, :k]))
