@@ -1071,7 +1071,7 @@ struct NormMax {
 // per row.  Several: a lane is a row, 8 columns at a time, so every load covers
 // 512 contiguous bytes of one column and A's entries are read once per 8
 // columns (16 rows x 4 columns per load: 1.18 ms against 0.84 for 1000^2
-// 5-point with 64 columns).  As separate passes, column by column, the same
+// 5-point with 64 columns; 0.69 now).  As separate passes, column by column, the same
 // work took 2.58 ms for the residual and 2 x 0.39 ms for the norms; the
 // vectors alone (1.3 GB) take 0.25 ms.
 template <typename T>
